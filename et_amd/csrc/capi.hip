@@ -402,6 +402,7 @@ int etg_test_gemm(char ta, char tb, int64_t m, int64_t n, int64_t k, double alph
     ETG_HIP(hipMemcpy(d.b.as<double>(), B, sizeof(double) * ldb * colsB, hipMemcpyHostToDevice));
     ETG_HIP(hipMemcpy(d.c.as<double>(), C, sizeof(double) * ldc * n, hipMemcpyHostToDevice));
     etg::GemmWorkspace ws;
+    ws.residue = std::make_shared<etg::ResidueWorkspace>(size_t(1500) << 20);
     etg::Gemm g = etg::make_gemm(ta, tb, m, n, k, alpha, d.a.as<double>(), lda, d.b.as<double>(), ldb, beta,
                                  d.c.as<double>(), ldc);
     g.split_any_shape = precision == ETG_BF16X3_ANY_SHAPE;
@@ -451,6 +452,7 @@ int etg_bench_gemm(char ta, char tb, int64_t m, int64_t n, int64_t k, int precis
     ETG_HIP(hipMemset(d.a.as<double>(), 0, sizeof(double) * m * k));
     ETG_HIP(hipMemset(d.b.as<double>(), 0, sizeof(double) * k * n));
     etg::GemmWorkspace ws;
+    ws.residue = std::make_shared<etg::ResidueWorkspace>(size_t(1500) << 20);
     etg::Gemm g = etg::make_gemm(ta, tb, m, n, k, 1.0, d.a.as<double>(), lda, d.b.as<double>(), ldb, 0.0,
                                  d.c.as<double>(), m);
     g.split_any_shape = precision == ETG_BF16X3_ANY_SHAPE;

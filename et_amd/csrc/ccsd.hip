@@ -46,6 +46,12 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   small_[1].resize(sizeof(double) * n * n);
   small_[2].resize(sizeof(double) * std::max(std::max(n * n, J), o * o * o * o));
   small_[3].resize(sizeof(double) * std::max(std::max(J * N, J * o * o), o * o * o * o));
+  // one workspace for the products that run as int8 ones, direct and in the
+  // transformation passes (one stream): a whole (ov)^3 product takes 45 n_t1^2 bytes
+  // (1.7 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
+  // 4 GB, 0.87 s with 2.5 GB)
+  const double residue_bytes = std::min(4.0e9, std::max(1.0e9, 64.0 * double(N) * double(N)));
+  gws_.residue = gws_pass_.residue = std::make_shared<ResidueWorkspace>(size_t(residue_bytes));
   // default ladder batch: G blocks of at most ~12 GB
   const double budget = 12e9 / 8.0;
   int64_t nb = int64_t(std::sqrt(budget) / double(v));

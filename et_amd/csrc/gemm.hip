@@ -353,6 +353,7 @@ const char* launch_tile(hipStream_t stream, const Gemm& g, const Params& p, int 
 
 struct Choice {
   int bm = 128, splits = 1;
+  double seconds = 0.0;              // the cost model's estimate
 };
 
 // only_bm != 0 restricts the search to that tile size
@@ -381,6 +382,7 @@ Choice choose_tiling(const Gemm& g, double peak, bool can_split, int only_bm = 0
         best_t = t;
         best.bm = c.bm;
         best.splits = s;
+        best.seconds = t;
       }
     }
   }
@@ -807,6 +809,9 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
   if (std::max(g.lda, g.ldb) >= (int64_t(1) << 24)) return gemm_tall(stream, g, ws);
   if (prec == Prec::BF16X3 && split_bf16_pays(g)) return gemm_bf16x3(stream, g, ws);
   if (prec == Prec::F32) return launch_typed<float>(stream, g, ws);
+  GemmLaunch info;
+  if (ws != nullptr && residue_pays(g, choose_tiling(g, 78.6e12, true).seconds) &&
+      gemm_residue(stream, g, ws, !capturing(stream), &info)) return info;
   return launch_typed<double>(stream, g, ws);
 }
 

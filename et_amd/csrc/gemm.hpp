@@ -6,6 +6,8 @@
 // op(X) = X ("N") or X^T ("T").  Batched products take element strides.
 #pragma once
 
+#include <memory>
+
 #include "common.hpp"
 
 namespace etg {
@@ -69,6 +71,17 @@ struct PackedOperand {
   DeviceBuffer buf;
 };
 
+// Packs, products and exponents of the FP64 products that run as int8 ones
+// (gemm_residue.hip).  Allocated once, at its first use, `capacity` bytes long:
+// larger products run in panels, and its address never changes (captured launch
+// sequences hold it).  Products queued on one stream only.
+struct ResidueWorkspace {
+  explicit ResidueWorkspace(size_t bytes) : capacity(bytes) {}
+  size_t capacity;
+  bool refused = false;              // could not be allocated: the FP64 kernels need none
+  DeviceBuffer buf;
+};
+
 // Scratch for split-K partial sums and the split-bf16 operand packs; grown on
 // demand.  `gen` counts the times one of its buffers moved (launch sequences
 // captured into a graph hold these addresses).
@@ -76,6 +89,7 @@ struct GemmWorkspace {
   DeviceBuffer buf, packA, packB;
   DeviceBuffer partials;             // per-entry products summed by the caller
   DeviceBuffer tune;                 // scratch output of the tile measurements
+  std::shared_ptr<ResidueWorkspace> residue;   // may be shared by workspaces of one stream; null: FP64 kernels only
   static constexpr int kCached = 4;
   PackedOperand cached[kCached];
   uint64_t clock = 0;
@@ -100,6 +114,13 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
 
 // The split-bf16 path (packs both operands into ws, then the bf16 matrix-core kernel).
 GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws);
+
+// FP64 products through exact int8 products (gemm_residue.hip): whether that is
+// the faster path for a product, and the product itself (false, with nothing
+// launched, when its workspace is not there and cannot be allocated or does not
+// hold the smallest panels).
+bool residue_pays(const Gemm& g, double fp64_seconds);
+bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may_allocate, GemmLaunch* info);
 
 // bf16 values of the split-bf16 pack of a rows x k operand (both splits, padded
 // to the product kernel's 256-row tile and 32-deep step).

@@ -1,0 +1,612 @@
+// FP64 products on the int8 matrix cores, exact modulo 15 coprime moduli
+// (residue.hpp has the arithmetic and its error).
+//
+// The FP64 matrix cores reach 78 TFLOP/s on this chip and the FP64 kernels 62
+// of them; the int8 matrix cores run v_mfma_i32_16x16x64_i8 at 4.2-4.9 POP/s,
+// so 15 int8 products per FP64 product are worth up to 280 TFLOP/s.  A product
+// runs as
+//   1. row norms of op(A) and op(B)^T            (reads each operand once)
+//   2. residue packs: 15 bytes per element, in the order the matrix cores read
+//   3. 15 int8 products, each sum reduced to one byte per output
+//   4. reconstruction of C from its 15 bytes     (writes C once)
+// on panels of A and B whose packs fit a bounded workspace.
+#include <algorithm>
+#include <string>
+
+#include "gemm.hpp"
+#include "residue.hpp"
+
+namespace etg {
+namespace {
+
+using residue::kC;
+using residue::kModuli;
+
+typedef int i4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+constexpr int kTileM = 256;                   // output rows of a tile of the int8 products
+constexpr int kDepth = 64;                    // k per step (one MFMA step)
+constexpr int kXcds = 8;
+constexpr int kGroupM = 8;
+
+// ---------------------------------------------------------------------------
+// 1. Scale exponents.  Element (r, k) of the rows x K operand is X[k + r ld]
+// (kcontig) or X[r + k ld].  Bound by HBM: each operand is read once.
+// ---------------------------------------------------------------------------
+
+// One workgroup per row.
+__global__ __launch_bounds__(256) void row_exponents_kcontig_kernel(const double* __restrict__ X, int64_t ld,
+                                                                    int64_t strideX, int64_t K,
+                                                                    int64_t exp_stride, int* __restrict__ e) {
+  __shared__ double ss[4];
+  __shared__ unsigned long long mm[4];
+  const int64_t r = blockIdx.x, bz = blockIdx.y;
+  const double* x = X + bz * strideX + r * ld;
+  double s = 0.0;
+  unsigned long long mx = 0;
+#pragma unroll 4
+  for (int64_t k = threadIdx.x; k < K; k += 256) {
+    const double v = x[k];
+    s += v * v;
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v) & 0x7fffffffffffffffull;
+    mx = b > mx ? b : mx;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    const unsigned long long o = __shfl_xor(mx, off, 64);
+    mx = o > mx ? o : mx;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    ss[threadIdx.x >> 6] = s;
+    mm[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < 4; ++q) {
+      s += ss[q];
+      mx = mm[q] > mx ? mm[q] : mx;
+    }
+    e[bz * exp_stride + r] = residue::scale_exponent(s, mx, K);
+  }
+}
+
+// 64 rows per workgroup (lanes along the contiguous rows), four k at a time, over
+// one of gridDim.y ranges of k; partial sums per range.
+__global__ __launch_bounds__(256) void row_norms_partial_kernel(const double* __restrict__ X, int64_t ld,
+                                                                int64_t strideX, int64_t rows, int64_t K,
+                                                                int64_t k_per, double* __restrict__ ps,
+                                                                unsigned long long* __restrict__ pm) {
+  __shared__ double ss[4][64];
+  __shared__ unsigned long long mm[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int64_t r = int64_t(blockIdx.x) * 64 + lane, bz = blockIdx.z;
+  const int64_t k0 = int64_t(blockIdx.y) * k_per, k1 = min(K, k0 + k_per);
+  const double* x = X + bz * strideX + r;
+  double s = 0.0;
+  unsigned long long mx = 0;
+  if (r < rows) {
+#pragma unroll 4
+    for (int64_t k = k0 + w; k < k1; k += 4) {
+      const double v = x[k * ld];
+      s += v * v;
+      const unsigned long long b = __builtin_bit_cast(unsigned long long, v) & 0x7fffffffffffffffull;
+      mx = b > mx ? b : mx;
+    }
+  }
+  ss[w][lane] = s;
+  mm[w][lane] = mx;
+  __syncthreads();
+  if (w == 0 && r < rows) {
+    for (int q = 1; q < 4; ++q) {
+      s += ss[q][lane];
+      mx = mm[q][lane] > mx ? mm[q][lane] : mx;
+    }
+    const int64_t at = (bz * gridDim.y + blockIdx.y) * rows + r;
+    ps[at] = s;
+    pm[at] = mx;
+  }
+}
+
+__global__ __launch_bounds__(256) void row_exponents_finish_kernel(const double* __restrict__ ps,
+                                                                   const unsigned long long* __restrict__ pm,
+                                                                   int64_t rows, int parts, int64_t K,
+                                                                   int64_t exp_stride, int* __restrict__ e) {
+  const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x, bz = blockIdx.y;
+  if (r >= rows) return;
+  double s = 0.0;
+  unsigned long long mx = 0;
+  for (int q = 0; q < parts; ++q) {
+    const int64_t at = (bz * parts + q) * rows + r;
+    s += ps[at];
+    mx = pm[at] > mx ? pm[at] : mx;
+  }
+  e[bz * exp_stride + r] = residue::scale_exponent(s, mx, K);
+}
+
+// ---------------------------------------------------------------------------
+// 2. Residue packs.  Per modulus one plane of 1 KB chunks (16 rows x 64 k: lane
+// l holds 16 consecutive k of row l % 16 from 16 (l / 16) on), row blocks
+// outermost, k steps contiguous.  One wave forms the 15 chunks of a (row block,
+// k step).  About 125 VALU operations per element (8 per modulus) against 8
+// bytes read and 15 written: close to balanced with HBM.
+// ---------------------------------------------------------------------------
+constexpr int kPackLd = kDepth + 2;           // LDS row of a staged chunk (doubles)
+
+__global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restrict__ X, int64_t ld, int64_t strideX,
+                                                           int kcontig, int64_t rows, int64_t K, int64_t KS,
+                                                           int64_t plane, const int* __restrict__ e,
+                                                           int64_t exp_stride, u4* __restrict__ P) {
+  __shared__ __attribute__((aligned(16))) double stage[4][16 * kPackLd];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t ks = int64_t(blockIdx.x) * 4 + wave;
+  const int64_t rb = blockIdx.y, bz = blockIdx.z;
+  const int64_t r = rb * 16 + (lane & 15), k0 = ks * kDepth + 16 * (lane >> 4);
+  const int ex = r < rows ? e[bz * exp_stride + r] : 0;
+  uint32_t lo[16], hi[16];
+  if (kcontig) {
+    // whole rows of the chunk (512 contiguous bytes per load) through LDS: read by
+    // each lane from global memory, 64 rows' lines per load, the pack took 2.7 times
+    // as long (6912 x 14400: 1150 us)
+    const double* x = X + bz * strideX + rb * 16 * ld;
+    const int64_t kl = ks * kDepth + lane;
+    double* t = stage[wave];
+#pragma unroll
+    for (int rr = 0; rr < 16; ++rr)
+      t[rr * kPackLd + lane] = (rb * 16 + rr < rows && kl < K) ? x[rr * ld + kl] : 0.0;
+    __syncthreads();
+    const double2* src = reinterpret_cast<const double2*>(&t[(lane & 15) * kPackLd + 16 * (lane >> 4)]);
+    const bool ok = ex != residue::kNotFinite;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const double2 v = src[j];
+      residue::to_integer(ok ? v.x : 0.0, ex, lo[2 * j], hi[2 * j]);
+      residue::to_integer(ok ? v.y : 0.0, ex, lo[2 * j + 1], hi[2 * j + 1]);
+    }
+  } else {
+    const double* x = X + bz * strideX + r + k0 * ld;
+    const int n = (r < rows && ex != residue::kNotFinite && k0 < K) ? int(min<int64_t>(16, K - k0)) : 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) residue::to_integer(j < n ? x[j * ld] : 0.0, ex, lo[j], hi[j]);
+  }
+  if (ks >= KS) return;
+  u4* dst = P + bz * kModuli * plane + (rb * KS + ks) * 64 + lane;
+#pragma unroll
+  for (int i = 0; i < kModuli; ++i) {
+    u4 w;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      uint32_t b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) b[j] = residue::residue_byte(lo[4 * q + j], hi[4 * q + j], i);
+      const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+      w[q] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+    }
+    dst[i * plane] = w;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 3. The int8 products.  Waves in 2 x WN, each 128 x 64 of the output (8 x 4
+// blocks, 128 int32 accumulators per lane): tiles of 256 x 128 (WN = 2, two
+// workgroups per CU, three LDS stages) or 256 x 256 (WN = 4, one, four stages).
+// Steps of 64 k (1 KB chunks) go from global memory straight into an LDS stage,
+// kStages - 1 steps ahead of their use; a wave waits for its own copies of the
+// step by count, then one barrier makes everyone's visible and frees the stage
+// read in the step before.  A step is 32 MFMAs (512 cycles) per wave against 12
+// KB of LDS reads.  Two workgroups per CU hide barriers, the first copies and the
+// byte epilogue under each other's products, but drift apart along k until their
+// tiles no longer meet in the L2: TOP/s with 15 moduli of random bytes for
+//   m = n = 6912, k =    1600    3200    14400   28800      m = n = k = 1536
+//   256 x 128            2360    2400     1780    1990                  1790
+//   256 x 256            2170    2440     2560    2480                  1470
+// so depths up to kShortDepth take the small tile.  Four waves of 128 x 128
+// reached 1890-2240 (one wave per SIMD), 128 x 128 tiles 2200 (LDS reads).
+// blockIdx.y is the modulus, blockIdx.z the batch entry.
+// ---------------------------------------------------------------------------
+constexpr int64_t kShortDepth = 3200;
+
+struct Params {
+  const u4 *A, *B;                 // packs (planes of the first modulus)
+  uint32_t* R;                     // one byte per output and modulus: tiles of 16 x 16 blocks in fragment order
+  int64_t KS;
+  int64_t planeA, planeB, planeR;  // from one modulus to the next (u4, u4, u32 units)
+  int64_t strideA, strideB, strideR;   // from one batch entry to the next
+  int tiles_m, tiles_n;
+};
+
+constexpr int kWaveM = 8, kWaveN = 4;         // 16 x 16 blocks of a wave
+constexpr int kBlocksM = kTileM / 16;
+
+__device__ inline void map_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int nb = tiles_m * tiles_n;
+  const int per = nb / kXcds, rem = nb % kXcds;
+  const int xcd = bid % kXcds, idx = bid / kXcds;
+  const int logical = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+  const int group = kGroupM * tiles_n;
+  const int first_m = (logical / group) * kGroupM;
+  const int gsize = min(tiles_m - first_m, kGroupM);
+  tm = first_m + (logical % group) % gsize;
+  tn = (logical % group) / gsize;
+}
+
+// Waits until at most N of this wave's vector-memory operations are outstanding.
+template <int N>
+__device__ inline void wait_copies() {
+  __builtin_amdgcn_s_waitcnt((N & 0xf) | 0x70 | 0xf00 | ((N >> 4) << 14));
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int WN, int kStages>
+__global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_kernel(Params p) {
+  constexpr int kBlocksN = WN * kWaveN;
+  constexpr int kCopiesA = kBlocksM / (2 * WN), kCopiesB = kBlocksN / (2 * WN);   // chunks a wave copies per step
+  __shared__ u4 lds[kStages][(kBlocksM + kBlocksN) * 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave & 1, wn = wave >> 1;
+  int tile_m, tile_n;
+  map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+  const int z = blockIdx.y;
+  const int64_t bz = blockIdx.z;
+  const u4* sa = p.A + bz * p.strideA + z * p.planeA + int64_t(tile_m) * kBlocksM * p.KS * 64;
+  const u4* sb = p.B + bz * p.strideB + z * p.planeB + int64_t(tile_n) * kBlocksN * p.KS * 64;
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<u4*>(sa), (short)0, 0x7fffffff, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<u4*>(sb), (short)0, 0x7fffffff, 0x00020000);
+  const uint32_t row_bytes = uint32_t(p.KS) * 1024u;     // one row block of a plane (at most 2 MB)
+  auto load = [&](int stage, int64_t s) {
+    const uint32_t voff = uint32_t(s) * 1024u + uint32_t(lane) * 16u;
+#pragma unroll
+    for (int q = 0; q < kCopiesA; ++q) {
+      const int c = wave * kCopiesA + q;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void*)(&lds[stage][c * 64]), 16, voff,
+                                               uint32_t(c) * row_bytes, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < kCopiesB; ++q) {
+      const int c = wave * kCopiesB + q;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void*)(&lds[stage][(kBlocksM + c) * 64]), 16, voff,
+                                               uint32_t(c) * row_bytes, 0, 0);
+    }
+  };
+  i4 acc[kWaveM][kWaveN];
+#pragma unroll
+  for (int i = 0; i < kWaveM; ++i)
+#pragma unroll
+    for (int j = 0; j < kWaveN; ++j) acc[i][j] = i4{0, 0, 0, 0};
+  // the four B fragments, then each row block's products with the next block's A
+  // fragment read ahead of them (order pinned by the scheduling groups)
+  auto compute = [&](int stage) {
+    const u4* As = &lds[stage][wm * kWaveM * 64];
+    const u4* Bs = &lds[stage][(kBlocksM + wn * kWaveN) * 64];
+    i4 a[2], b[kWaveN];
+    a[0] = __builtin_bit_cast(i4, As[lane]);
+#pragma unroll
+    for (int j = 0; j < kWaveN; ++j) b[j] = __builtin_bit_cast(i4, Bs[j * 64 + lane]);
+#pragma unroll
+    for (int i = 0; i < kWaveM; ++i) {
+      if (i + 1 < kWaveM) a[(i + 1) & 1] = __builtin_bit_cast(i4, As[(i + 1) * 64 + lane]);
+#pragma unroll
+      for (int j = 0; j < kWaveN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i & 1], b[j], acc[i][j], 0, 0, 0);
+      if (i == 0) __builtin_amdgcn_sched_group_barrier(0x100, kWaveN + 2, 0);
+      else if (i + 1 < kWaveM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, kWaveN, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  const int64_t ns = p.KS;
+#pragma unroll
+  for (int s = 0; s < kStages - 1; ++s)
+    if (s < ns) load(s, s);
+  int stage = 0;
+  int64_t s = 0;
+  for (; s + kStages - 1 < ns; ++s) {
+    wait_copies<(kStages - 2) * (kCopiesA + kCopiesB)>();
+    load(stage == 0 ? kStages - 1 : stage - 1, s + kStages - 1);
+    compute(stage);
+    stage = stage + 1 == kStages ? 0 : stage + 1;
+  }
+  for (; s < ns; ++s) {
+    wait_copies<0>();
+    compute(stage);
+    stage = stage + 1 == kStages ? 0 : stage + 1;
+  }
+  const double m = kC.md[z], inv = kC.invd[z];
+  uint32_t* R = p.R + bz * p.strideR + z * p.planeR +
+                (int64_t(tile_n) * p.tiles_m + tile_m) * (kBlocksM * kBlocksN * 64);
+#pragma unroll
+  for (int i = 0; i < kWaveM; ++i)
+#pragma unroll
+    for (int j = 0; j < kWaveN; ++j) {
+      uint32_t b[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[r] = residue::residue_byte_of_sum(acc[i][j][r], m, inv);
+      const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+      R[((wn * kWaveN + j) * kBlocksM + wm * kWaveM + i) * 64 + lane] =
+          __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// 4. Reconstruction: C = alpha op(A) op(B) + beta C from the 15 bytes of each
+// output.  A lane takes the four rows of one column that its word of each plane
+// holds.  Bound by HBM (15 bytes read, 8 written, 8 more read with beta).  A
+// row or column with an infinity or NaN is summed term by term from the
+// operands instead.
+// ---------------------------------------------------------------------------
+struct Output {
+  const uint32_t* R;
+  int64_t planeR, strideR;
+  int tiles_m, blocks_n;                  // tiles along m, 16-column blocks of a tile
+  int64_t m, n, K;                        // of this panel
+  const int *ea, *eb;
+  int64_t ea_stride, eb_stride;
+  double alpha, beta;
+  double* C;
+  int64_t ldc, strideC;
+  int vec_rows;                           // rows written four at a time (alignment checked on the host)
+  const double *A, *B;                    // panel operands, for the rows that are not finite
+  int64_t lda, strideA, ldb, strideB;
+  int a_kcontig, b_kcontig;
+};
+
+__device__ double plain_sum(const Output& p, int64_t bz, int64_t row, int64_t col) {
+  const double* a = p.A + bz * p.strideA + (p.a_kcontig ? row * p.lda : row);
+  const double* b = p.B + bz * p.strideB + (p.b_kcontig ? col * p.ldb : col);
+  const int64_t sa = p.a_kcontig ? 1 : p.lda, sb = p.b_kcontig ? 1 : p.ldb;
+  double s = 0.0;
+  for (int64_t k = 0; k < p.K; ++k) s += a[k * sa] * b[k * sb];
+  return s;
+}
+
+__global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
+  const int lane = threadIdx.x & 63;
+  const int per_tile = kBlocksM * p.blocks_n / 4;
+  const int64_t tile = blockIdx.x / unsigned(per_tile);
+  const int blk = int(blockIdx.x % unsigned(per_tile)) * 4 + int(threadIdx.x >> 6);
+  const int64_t bz = blockIdx.y;
+  const int64_t row = (tile % p.tiles_m) * kTileM + (blk % kBlocksM) * 16 + 4 * (lane >> 4);
+  const int64_t col = ((tile / p.tiles_m) * p.blocks_n + blk / kBlocksM) * 16 + (lane & 15);
+  if (row >= p.m || col >= p.n) return;
+  const uint32_t* R = p.R + bz * p.strideR + (tile * (kBlocksM * p.blocks_n) + blk) * 64 + lane;
+  uint32_t w[kModuli];
+#pragma unroll
+  for (int i = 0; i < kModuli; ++i) w[i] = R[i * p.planeR];
+  const int eb = p.eb[bz * p.eb_stride + col];
+  const int* ea = p.ea + bz * p.ea_stride + row;
+  const int rows = int(min<int64_t>(4, p.m - row));
+  double v[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    double hi = 0.0, lo = 0.0;
+#pragma unroll
+    for (int i = 0; i < kModuli; ++i) {
+      const double b = double(int(w[i] << (24 - 8 * r)) >> 24);
+      hi = fma(b, kC.fhi[i], hi);
+      lo = fma(b, kC.flo[i], lo);
+    }
+    v[r] = 0.0;
+    if (r < rows) {
+      const int e = ea[r];
+      v[r] = (e == residue::kNotFinite || eb == residue::kNotFinite) ? plain_sum(p, bz, row + r, col)
+                                                                    : residue::reconstruct(hi, lo, e, eb);
+    }
+  }
+  double* c = p.C + bz * p.strideC + row + col * p.ldc;
+  if (p.vec_rows) {
+    double2* c2 = reinterpret_cast<double2*>(c);
+    double2 x = {p.alpha * v[0], p.alpha * v[1]}, y = {p.alpha * v[2], p.alpha * v[3]};
+    if (p.beta != 0.0) {
+      const double2 o0 = c2[0], o1 = c2[1];
+      x.x += p.beta * o0.x; x.y += p.beta * o0.y;
+      y.x += p.beta * o1.x; y.y += p.beta * o1.y;
+    }
+    c2[0] = x;
+    c2[1] = y;
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    if (r < rows) c[r] = p.beta == 0.0 ? p.alpha * v[r] : p.alpha * v[r] + p.beta * c[r];
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+
+struct Panels {
+  int64_t KS, rows_m, rows_n, batch;          // panel rows of op(A) and op(B)^T, batch entries per group
+  int tile_n;                                 // columns of a tile
+  int64_t a_entries, b_entries;               // batch entries packed per group (1 for a shared operand)
+  int64_t rm_p, rn_p;                         // panel rows padded to whole tiles
+  int64_t parts;                              // k ranges of the row norms
+  size_t bytes_a, bytes_b, bytes_r, bytes_e, bytes_n;
+  size_t total() const { return bytes_a + bytes_b + bytes_r + bytes_e + bytes_n; }
+};
+
+size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+
+void size_panels(const Gemm& g, Panels& p) {
+  p.rm_p = ceil_div(p.rows_m, kTileM) * kTileM;
+  p.rn_p = ceil_div(p.rows_n, p.tile_n) * p.tile_n;
+  p.a_entries = g.strideA == 0 ? 1 : p.batch;
+  p.b_entries = g.strideB == 0 ? 1 : p.batch;
+  p.bytes_a = align256(size_t(p.a_entries * kModuli) * size_t(p.rm_p * p.KS * kDepth));
+  p.bytes_b = align256(size_t(p.b_entries * kModuli) * size_t(p.rn_p * p.KS * kDepth));
+  p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(p.rm_p * p.rn_p));
+  p.bytes_e = align256(sizeof(int) * size_t(p.a_entries * p.rm_p + p.b_entries * p.rn_p));
+  p.bytes_n = align256(16 * size_t(std::max(p.a_entries * p.rm_p, p.b_entries * p.rn_p) * p.parts));
+}
+
+// The whole product where it fits the capacity, else equal groups of the batch,
+// else (one entry at a time) equal panels of rows, the longer panel split first.
+// A panel more of one operand packs the other once more: 7.4 ps per element
+// against the 12.5 fs of products that each of its elements has with every row
+// of the panel, so panels of 2560 rows cost a quarter, of 6912 rows a twelfth.
+bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
+  p.KS = ceil_div(g.k, kDepth);
+  p.tile_n = g.k <= kShortDepth ? 128 : 256;
+  p.parts = std::max<int64_t>(1, std::min<int64_t>(64, g.k / 256));
+  p.rows_m = g.m;
+  p.rows_n = g.n;
+  p.batch = g.batch;
+  int64_t groups = 1, pm = 1, pn = 1;
+  for (;;) {
+    size_panels(g, p);
+    if (p.total() <= capacity) return true;
+    if (p.batch > 1) {
+      p.batch = ceil_div(g.batch, ++groups);
+    } else if (p.rows_m >= p.rows_n) {
+      if (p.rows_m <= kTileM) return false;
+      p.rows_m = std::min(g.m, ceil_div(ceil_div(g.m, ++pm), kTileM) * kTileM);
+    } else {
+      if (p.rows_n <= kTileM) return false;
+      p.rows_n = std::min(g.n, ceil_div(ceil_div(g.n, ++pn), kTileM) * kTileM);
+    }
+  }
+}
+
+// One operand panel: exponents, then the pack.
+void pack_operand(hipStream_t s, const double* X, int64_t ld, int64_t strideX, bool kcontig, int64_t rows, int64_t K,
+                  int64_t KS, int64_t rows_p, int64_t entries, int64_t parts, void* norms, int* e, u4* P) {
+  if (kcontig) {
+    row_exponents_kcontig_kernel<<<dim3(unsigned(rows), unsigned(entries)), 256, 0, s>>>(X, ld, strideX, K, rows_p, e);
+    ETG_LAUNCH("row_exponents");
+  } else {
+    const int64_t k_per = ceil_div(K, parts);
+    double* ps = static_cast<double*>(norms);
+    unsigned long long* pm = reinterpret_cast<unsigned long long*>(ps + entries * rows * parts);
+    row_norms_partial_kernel<<<dim3(unsigned(ceil_div(rows, 64)), unsigned(parts), unsigned(entries)), 256, 0, s>>>(
+        X, ld, strideX, rows, K, k_per, ps, pm);
+    ETG_LAUNCH("row_norms");
+    row_exponents_finish_kernel<<<dim3(unsigned(ceil_div(rows, 256)), unsigned(entries)), 256, 0, s>>>(
+        ps, pm, rows, int(parts), K, rows_p, e);
+    ETG_LAUNCH("row_exponents");
+  }
+  residue_pack_kernel<<<dim3(unsigned(ceil_div(KS, 4)), unsigned(ceil_div(rows, 16)), unsigned(entries)), 256, 0, s>>>(
+      X, ld, strideX, kcontig ? 1 : 0, rows, K, KS, rows_p * KS * (kDepth / 16), e, rows_p, P);
+  ETG_LAUNCH("residue_pack");
+}
+
+}  // namespace
+
+// Estimated seconds of the int8 path (2400 TOP/s over whole tiles, 7.4 ps per
+// operand element and 5.1 ps per output of packs and reconstruction, 45 us of
+// launches) against those of the FP64 kernels (`fp64_seconds`, at least the 35
+// TFLOP/s that products of a few hundred rows reach).  Measured per product, FP64
+// and int8: 1024^3 56 and 75 us, 1280^3 107 and 99, 1520^3 175 and 133, 2048^3
+// 311 and 193, 4096^3 2200 and 1069 us; m = n = 4096 with k = 279 / 600 / 1270:
+// 196 and 233, 364 and 295, 716 and 443 us; 210 x 2926 x 2926 100 and 132 us.
+// The estimate follows these to 20 % on either side of the crossing.
+bool residue_pays(const Gemm& g, double fp64_seconds) {
+  if (g.k > residue::kMaxDepth || std::min(g.m, g.n) < 128 || g.k < 128) return false;
+  const double b = double(g.batch), m = double(g.m), n = double(g.n), k = double(g.k);
+  const int64_t tile_n = g.k <= kShortDepth ? 128 : 256;
+  const double mp = double(ceil_div(g.m, kTileM) * kTileM), np = double(ceil_div(g.n, tile_n) * tile_n);
+  const double kp = double(ceil_div(g.k, kDepth) * kDepth);
+  const double products = 2.0 * kModuli * mp * np * kp * b / 2400e12;
+  const double packs = 7.4e-12 * ((g.strideA == 0 ? 1.0 : b) * m * k + (g.strideB == 0 ? 1.0 : b) * n * k);
+  const double output = 5.1e-12 * m * n * b;
+  return products + packs + output + 45e-6 < 0.95 * std::min(fp64_seconds, 2.0 * m * n * k * b / 35e12);
+}
+
+bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may_allocate, GemmLaunch* info) {
+  ResidueWorkspace* rw = ws->residue.get();
+  Panels p{};
+  if (rw == nullptr || rw->refused || !plan_panels(g, rw->capacity, p)) return false;
+  if (rw->buf.bytes() == 0) {
+    if (!may_allocate) return false;
+    try {
+      rw->buf.resize(rw->capacity);
+    } catch (const Error&) {
+      (void)hipGetLastError();
+      rw->refused = true;
+      return false;
+    }
+  }
+  char* base = rw->buf.as<char>();
+  u4* PA = reinterpret_cast<u4*>(base);
+  u4* PB = reinterpret_cast<u4*>(base + p.bytes_a);
+  uint32_t* R = reinterpret_cast<uint32_t*>(base + p.bytes_a + p.bytes_b);
+  int* ea = reinterpret_cast<int*>(base + p.bytes_a + p.bytes_b + p.bytes_r);
+  int* eb = ea + p.a_entries * p.rm_p;
+  void* norms = base + p.bytes_a + p.bytes_b + p.bytes_r + p.bytes_e;
+  const bool a_kcontig = g.ta, b_kcontig = !g.tb;
+  const int64_t pm = ceil_div(g.m, p.rows_m), pn = ceil_div(g.n, p.rows_n);
+  // one panel of op(A), group of batch entries and panel of op(B); an operand is
+  // packed again only where the last pack was another one
+  int64_t a_is = -1, b_is = -1;
+  auto panel = [&](int64_t mi, int64_t bi, int64_t ni) {
+    const int64_t m0 = mi * p.rows_m, b0 = bi * p.batch, n0 = ni * p.rows_n;
+    const int64_t m = std::min(p.rows_m, g.m - m0), n = std::min(p.rows_n, g.n - n0), nb = std::min(p.batch, g.batch - b0);
+    const double* A = g.A + b0 * g.strideA + (a_kcontig ? m0 * g.lda : m0);
+    const double* B = g.B + b0 * g.strideB + (b_kcontig ? n0 * g.ldb : n0);
+    const int64_t a_want = mi + (g.strideA == 0 ? 0 : pm * bi), b_want = ni + (g.strideB == 0 ? 0 : pn * bi);
+    if (a_want != a_is)
+      pack_operand(stream, A, g.lda, g.strideA, a_kcontig, m, g.k, p.KS, p.rm_p, g.strideA == 0 ? 1 : nb, p.parts, norms,
+                   ea, PA);
+    if (b_want != b_is)
+      pack_operand(stream, B, g.ldb, g.strideB, b_kcontig, n, g.k, p.KS, p.rn_p, g.strideB == 0 ? 1 : nb, p.parts, norms,
+                   eb, PB);
+    a_is = a_want;
+    b_is = b_want;
+    Params q{};
+    q.A = PA;
+    q.B = PB;
+    q.R = R;
+    q.KS = p.KS;
+    q.planeA = p.rm_p * p.KS * (kDepth / 16);
+    q.planeB = p.rn_p * p.KS * (kDepth / 16);
+    q.planeR = p.rm_p * p.rn_p / 4;
+    q.strideA = g.strideA == 0 ? 0 : kModuli * q.planeA;
+    q.strideB = g.strideB == 0 ? 0 : kModuli * q.planeB;
+    q.strideR = kModuli * q.planeR;
+    q.tiles_m = int(ceil_div(m, kTileM));
+    q.tiles_n = int(ceil_div(n, p.tile_n));
+    const unsigned tiles = unsigned(q.tiles_m) * unsigned(q.tiles_n);
+    const dim3 grid(tiles, kModuli, unsigned(nb));
+    if (p.tile_n == 128)
+      residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
+    else
+      residue_product_kernel<4, 4><<<grid, 512, 0, stream>>>(q);
+    ETG_LAUNCH("residue_product");
+    Output o{};
+    o.R = R;
+    o.planeR = q.planeR;
+    o.strideR = q.strideR;
+    o.tiles_m = q.tiles_m;
+    o.blocks_n = p.tile_n / 16;
+    o.m = m; o.n = n; o.K = g.k;
+    o.ea = ea; o.eb = eb;
+    o.ea_stride = g.strideA == 0 ? 0 : p.rm_p;
+    o.eb_stride = g.strideB == 0 ? 0 : p.rn_p;
+    o.alpha = g.alpha; o.beta = g.beta;
+    o.C = g.C + b0 * g.strideC + m0 + n0 * g.ldc;
+    o.ldc = g.ldc; o.strideC = g.strideC;
+    o.vec_rows = m % 4 == 0 && g.ldc % 2 == 0 && (g.batch == 1 || g.strideC % 2 == 0) &&
+                 reinterpret_cast<uintptr_t>(o.C) % 16 == 0;
+    o.A = A; o.lda = g.lda; o.strideA = g.strideA; o.a_kcontig = a_kcontig ? 1 : 0;
+    o.B = B; o.ldb = g.ldb; o.strideB = g.strideB; o.b_kcontig = b_kcontig ? 1 : 0;
+    residue_reconstruct_kernel<<<dim3(tiles * unsigned(kBlocksM * p.tile_n / 64), unsigned(nb)), 256, 0, stream>>>(o);
+    ETG_LAUNCH("residue_reconstruct");
+  };
+  // the outer operand's panels are packed once, the inner one's once per outer panel
+  // (and both once per group of the batch unless shared)
+  const int64_t ng = ceil_div(g.batch, p.batch);
+  const bool a_outer = g.batch > 1 ? g.strideA == 0 || g.strideB != 0
+                                   : (pn > 1 ? g.m + pm * g.n : g.m + g.n) <= (pm > 1 ? g.n + pn * g.m : g.n + g.m);
+  for (int64_t x = 0; x < (a_outer ? pm : pn); ++x)
+    for (int64_t bi = 0; bi < ng; ++bi)
+      for (int64_t y = 0; y < (a_outer ? pn : pm); ++y) panel(a_outer ? x : y, bi, a_outer ? y : x);
+  *info = GemmLaunch{p.tile_n == 128 ? "gemm_residue<256x128>" : "gemm_residue<256x256>", 1};
+  return true;
+}
+
+}  // namespace etg

@@ -1,0 +1,176 @@
+// FP64 products by exact integer arithmetic on the int8 matrix cores: the
+// number theory shared by the kernels (gemm_residue.hip) and the host checks.
+//
+// A row a of op(A) and a column b of op(B) are scaled by powers of two and
+// rounded to integers, a' = rint(2^ea a), b' = rint(2^eb b), with ||a'||_2 and
+// ||b'||_2 at most 2^kNormBits.  By Cauchy-Schwarz |a'.b'| < M / 2 for
+// M = m_0 m_1 ... m_14, the product of 15 pairwise coprime moduli of at most 8
+// bits, so the integer a'.b' is determined by its residues, and each residue
+// is an int8 product with int32 accumulation, without any rounding
+// (Chinese remainder theorem; the scheme is Ozaki, Uchino and Imamura's
+// "Ozaki scheme II", 2025).  The only errors are the rounding of the operands
+// to integers, at most 2^-(kNormBits - 1) ||a|| relative to a row's norm per
+// element, and one final rounding to double.
+//
+// An FP64 sum of k products rounds every partial sum: for terms of random sign
+// its error is about 2^-56 to 2^-55 of ||a|| ||b||, whatever k.  Rounding the
+// operands here costs about 2^-59 of ||a|| ||b|| (0.4 / 2^57.5), so 15 moduli
+// are about ten times closer to the exact product than the FP64 kernels;
+// 14 (2^-55) would not be.
+#pragma once
+
+#include <cmath>
+#include <cstdint>
+
+#ifndef ETG_HD
+#if defined(__HIPCC__)
+#define ETG_HD __host__ __device__
+#else
+#define ETG_HD
+#endif
+#endif
+
+namespace etg {
+namespace residue {
+
+constexpr int kModuli = 15;
+constexpr int kMod[kModuli] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197};
+constexpr int kNormBits = 58;                     // 2 kNormBits < log2(M / 2) = 116.78
+// |residue| <= 128 on both sides: the int32 sums hold this many terms
+constexpr int64_t kMaxDepth = (int64_t(1) << 17) - 1;
+constexpr int kNotFinite = INT32_MIN;             // exponent of a row with an infinity or NaN
+
+constexpr unsigned __int128 product_of_moduli() {
+  unsigned __int128 p = 1;
+  for (int i = 0; i < kModuli; ++i) p *= unsigned(kMod[i]);
+  return p;
+}
+constexpr unsigned __int128 kM = product_of_moduli();
+constexpr double kMDouble = double(kM);
+
+// 2^e mod m
+constexpr int pow2_mod(int e, int m) {
+  int r = 1 % m;
+  for (int i = 0; i < e; ++i) r = r * 2 % m;
+  return r;
+}
+
+// inverse of M / m_i modulo m_i
+constexpr int cofactor_inverse(int i) {
+  const int m = kMod[i], c = int((kM / unsigned(m)) % unsigned(m));
+  for (int x = 1; x < m; ++x)
+    if (c * x % m == 1) return x;
+  return 0;
+}
+
+// X = sum_i r_i inv_i (M / m_i)  (mod M), so X / M = sum_i r_i f_i (mod 1) with
+// f_i = inv_i / m_i.  f_i = (kHi + kLo 2^-40) 2^-40 to 2^-81: sums of 15 terms
+// |r_i| <= 128 of either part are exact in FP64, and the 2^-73 M that is left
+// out is below 2^-12 of the operands' rounding.
+constexpr uint64_t fraction80(int i, bool high) {
+  const unsigned __int128 num = (unsigned __int128)(unsigned(cofactor_inverse(i))) << 81;
+  const unsigned __int128 f = (num / unsigned(kMod[i]) + 1) >> 1;   // rounded to 2^-80
+  return high ? uint64_t(f >> 40) : uint64_t(f & ((uint64_t(1) << 40) - 1));
+}
+
+struct Constants {
+  // residues of an integer given as 8 unsigned bytes of (a' + 2^63): weights of
+  // the low and high four bytes, 256^j mod m, and -2^63 mod m
+  uint32_t low[kModuli], high[kModuli], offset[kModuli];
+  float mf[kModuli], invf[kModuli];
+  double md[kModuli], invd[kModuli];
+  double fhi[kModuli], flo[kModuli];
+};
+
+constexpr Constants make_constants() {
+  Constants c{};
+  for (int i = 0; i < kModuli; ++i) {
+    const int m = kMod[i];
+    uint32_t w[2] = {0, 0};
+    for (int j = 0; j < 8; ++j) w[j / 4] |= uint32_t(pow2_mod(8 * j, m) & 0xff) << (8 * (j % 4));
+    c.low[i] = w[0];
+    c.high[i] = w[1];
+    c.offset[i] = uint32_t((m - pow2_mod(63, m)) % m);
+    c.mf[i] = float(m);
+    c.invf[i] = 1.0f / float(m);
+    c.md[i] = double(m);
+    c.invd[i] = 1.0 / double(m);
+    c.fhi[i] = double(fraction80(i, true));
+    c.flo[i] = double(fraction80(i, false));
+  }
+  return c;
+}
+constexpr Constants kC = make_constants();
+
+// Scale exponent of a row from its sum of squares, the bits of its largest
+// magnitude and its length: ||2^e a|| <= 2^kNormBits.  Where the squares leave
+// the range in which their sum is accurate, the norm is bounded by
+// sqrt(k) max |a|.
+ETG_HD inline int scale_exponent(double sumsq, uint64_t max_bits, int64_t k) {
+  if (max_bits == 0) return 0;
+  if (max_bits >= 0x7ff0000000000000ull) return kNotFinite;
+  int x;
+  if (sumsq > 1e-270 && sumsq < 1e290) {
+    (void)frexp(sumsq, &x);                       // sumsq < 2^x
+    return kNormBits - ((x + 1) >> 1);
+  }
+  double big;
+  static_assert(sizeof(big) == sizeof(max_bits), "double bits");
+  __builtin_memcpy(&big, &max_bits, sizeof(big));
+  (void)frexp(big, &x);                           // big < 2^x
+  int lk = 0;
+  while ((int64_t(1) << lk) < k) ++lk;
+  return kNormBits - x - ((lk + 1) >> 1);
+}
+
+// a' = rint(2^e x) + 2^63 as two 32-bit halves (|a'| < 2^60)
+ETG_HD inline void to_integer(double x, int e, uint32_t& lo, uint32_t& hi) {
+  const double v = rint(ldexp(x, e));
+  const double h = floor(v * 0x1p-32);
+  lo = uint32_t(fma(h, -0x1p32, v));
+  hi = uint32_t(int32_t(h)) ^ 0x80000000u;
+}
+
+ETG_HD inline uint32_t byte_dot(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_udot4(a, b, c, false);
+#else
+  for (int j = 0; j < 4; ++j) c += ((a >> (8 * j)) & 0xffu) * ((b >> (8 * j)) & 0xffu);
+  return c;
+#endif
+}
+
+// Symmetric residue of the integer modulo m_i: its two's complement in the low
+// byte of the returned word.  The byte dot products are below 2^20, so the FP32
+// arithmetic is exact; rounding to the nearest multiple cannot err, as a tie
+// occurs for m = 256 only, where 128 and -128 are the same byte.
+ETG_HD inline uint32_t residue_byte(uint32_t lo, uint32_t hi, int i) {
+  constexpr float kMagic = 12582912.0f;           // 1.5 2^23: adding it rounds to an integer
+  const float f = float(byte_dot(hi, kC.high[i], byte_dot(lo, kC.low[i], kC.offset[i])));
+  const float q = fmaf(f, kC.invf[i], kMagic) - kMagic;
+  const float r = fmaf(-q, kC.mf[i], f) + kMagic;
+  uint32_t bits;
+  __builtin_memcpy(&bits, &r, sizeof(bits));
+  return bits;
+}
+
+// The same of an int32 sum (FP64 arithmetic, exact).
+ETG_HD inline uint32_t residue_byte_of_sum(int32_t s, double m, double inv) {
+  constexpr double kMagic = 6755399441055744.0;   // 1.5 2^52
+  const double t = double(s);
+  const double q = fma(t, inv, kMagic) - kMagic;
+  const double r = fma(-q, m, t) + kMagic;
+  uint64_t bits;
+  __builtin_memcpy(&bits, &r, sizeof(bits));
+  return uint32_t(bits);
+}
+
+// a'.b' 2^-(ea + eb) from the sums hi = sum_i r_i kHi_i and lo = sum_i r_i kLo_i.
+ETG_HD inline double reconstruct(double hi, double lo, int ea, int eb) {
+  const double t = hi * 0x1p-40;
+  const double frac = (t - rint(t)) + lo * 0x1p-80;   // X / M in [-1/2, 1/2], the first term exact
+  return ldexp(frac * kMDouble, -ea - eb);
+}
+
+}  // namespace residue
+}  // namespace etg
