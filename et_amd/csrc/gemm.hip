@@ -75,6 +75,8 @@ struct Mfma<double> {
   }
   static __device__ inline double cvt(double x) { return x; }
   static __device__ inline int row(int lrow, int r) { return lrow + 4 * r; }
+  static __device__ inline int lane_row(int row) { return row & 3; }      // lane / 16 and element of a row
+  static __device__ inline int element(int row) { return row >> 2; }
 };
 
 template <>
@@ -85,6 +87,8 @@ struct Mfma<float> {
   }
   static __device__ inline float cvt(double x) { return static_cast<float>(x); }
   static __device__ inline int row(int lrow, int r) { return 4 * lrow + r; }
+  static __device__ inline int lane_row(int row) { return row >> 2; }
+  static __device__ inline int element(int row) { return row & 3; }
 };
 
 // Raw buffer access (gfx9 descriptor word 3).  Offsets at or past kOutOfRange
@@ -288,6 +292,112 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p) {
       }
 }
 
+// ---- products of few output tiles ---------------------------------------------
+// A product with fewer tiles than the chip has CUs is bound by latency: the tiled
+// kernel above walks k in steps of 16, each of them a trip to memory and a barrier
+// (95 x 95 x 279: 18 us).  Here the WK waves of a workgroup share one tile of
+// 16 TM x 16 TN outputs and take every WK-th chunk of 16 k each, operands straight
+// from global memory into the fragments, a chunk ahead of its use, no barrier until
+// the waves' sums meet in LDS (summed in wave order).  Within a chunk lane group
+// l / 16 holds k = 4 (l / 16) .. + 3 and MFMA step s takes element s of each: every
+// lane reads 32 contiguous bytes of a k-contiguous operand, 16 lanes 128 of the other.
+template <typename T, bool TA, bool TB, int TM, int TN, int WK>
+__global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
+  using M = Mfma<T>;
+  using acc_t = typename M::acc_t;
+  __shared__ double red[WK][TM * TN * 256];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lcol = lane & 15, lk = 4 * (lane >> 4);
+  const int64_t m0 = int64_t(blockIdx.x % p.tiles_m) * (16 * TM), n0 = int64_t(blockIdx.x / p.tiles_m) * (16 * TN);
+  const int64_t bz = blockIdx.z, split = blockIdx.y;
+  const int64_t kbeg = split * p.k_per_split, kend = min(p.k, kbeg + p.k_per_split);
+  const int64_t sa = TA ? 1 : p.lda, sb = TB ? p.ldb : 1;   // from one k to the next
+  const double* pa[TM];
+  const double* pb[TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {                           // rows past the edge repeat the last one
+    const int64_t r = min(m0 + 16 * i + lcol, p.m - 1);
+    pa[i] = p.A + bz * p.strideA + (TA ? r * p.lda : r);
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int64_t c = min(n0 + 16 * j + lcol, p.n - 1);
+    pb[j] = p.B + bz * p.strideB + (TB ? c : c * p.ldb);
+  }
+  acc_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  T a[2][TM][4], b[2][TN][4];
+  auto load = [&](int at, int64_t k0) {
+    if (k0 + 16 <= kend) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[at][i][s] = M::cvt(pa[i][(k0 + lk + s) * sa]);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) b[at][j][s] = M::cvt(pb[j][(k0 + lk + s) * sb]);
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool ok = k0 + lk + s < kend;
+        const int64_t k = ok ? k0 + lk + s : kbeg;
+#pragma unroll
+        for (int i = 0; i < TM; ++i) a[at][i][s] = ok ? M::cvt(pa[i][k * sa]) : T(0);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) b[at][j][s] = ok ? M::cvt(pb[j][k * sb]) : T(0);
+      }
+    }
+  };
+  auto multiply = [&](int at) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = M::run(a[at][i][s], b[at][j][s], acc[i][j]);
+  };
+  int64_t k0 = kbeg + 16 * wave;
+  if (k0 < kend) load(0, k0);
+  while (k0 < kend) {
+    if (k0 + 16 * WK < kend) load(1, k0 + 16 * WK);
+    multiply(0);
+    k0 += 16 * WK;
+    if (k0 >= kend) break;
+    if (k0 + 16 * WK < kend) load(0, k0 + 16 * WK);
+    multiply(1);
+    k0 += 16 * WK;
+  }
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) red[wave][(i * TN + j) * 256 + r * 64 + lane] = double(acc[i][j][r]);
+  __syncthreads();
+  for (int e = tid; e < TM * TN * 256; e += 64 * WK) {
+    // output e: rows fastest, 16 TM per column of the tile
+    const int rr = e % (16 * TM), cc = e / (16 * TM);
+    const int row16 = rr & 15;
+    const int lrow = M::lane_row(row16), r = M::element(row16);
+    const int at = ((rr >> 4) * TN + (cc >> 4)) * 256 + r * 64 + 16 * lrow + (cc & 15);
+    double v = red[0][at];
+#pragma unroll
+    for (int w = 1; w < WK; ++w) v += red[w][at];
+    const int64_t row = m0 + rr, col = n0 + cc;
+    if (row >= p.m || col >= p.n) continue;
+    if (p.W) {
+      p.W[(split + bz * gridDim.y) * p.m * p.n + row + col * p.m] = v;
+    } else {
+      double* c = p.C + bz * p.strideC + row + col * p.ldc;
+      *c = (p.beta == 0.0) ? p.alpha * v : p.alpha * v + p.beta * *c;
+    }
+  }
+}
+
 // C = beta * C (a product with k = 0).
 __global__ void scale_matrix(double* C, int64_t m, int64_t n, int64_t ldc, int64_t strideC,
                              double beta) {
@@ -310,6 +420,42 @@ __global__ void splitk_reduce(const double* __restrict__ W, int splits, int64_t 
   double* c = C + bz * strideC + row + col * ldc;
   const double v = alpha * s;
   *c = (beta == 0.0) ? v : v + beta * *c;
+}
+
+// The same for many splits of few outputs: 32 outputs per workgroup, eight threads
+// an output over every eighth split, their sums added in order (one thread per
+// output would wait for a load per split: 95 us for 380 splits of 400 outputs).
+__global__ __launch_bounds__(256) void splitk_reduce_deep(const double* __restrict__ W, int splits, int64_t m, int64_t n,
+                                                          double alpha, double beta, double* C, int64_t ldc,
+                                                          int64_t strideC) {
+  __shared__ double part[8][32];
+  const int64_t bz = blockIdx.z;
+  const int o = threadIdx.x & 31, g = threadIdx.x >> 5;
+  const int64_t idx = int64_t(blockIdx.x) * 32 + o;
+  double s = 0.0;
+  if (idx < m * n) {
+    const double* w = W + bz * splits * m * n + idx;
+#pragma unroll 4
+    for (int q = g; q < splits; q += 8) s += w[int64_t(q) * m * n];
+  }
+  part[g][o] = s;
+  __syncthreads();
+  if (g != 0 || idx >= m * n) return;
+  for (int q = 1; q < 8; ++q) s += part[q][o];
+  double* c = C + bz * strideC + (idx % m) + (idx / m) * ldc;
+  const double v = alpha * s;
+  *c = (beta == 0.0) ? v : v + beta * *c;
+}
+
+void reduce_splits(hipStream_t stream, const Gemm& g, const double* W, int splits) {
+  const int64_t mn = g.m * g.n;
+  if (splits >= 16)
+    splitk_reduce_deep<<<dim3(unsigned(ceil_div(mn, 32)), 1, unsigned(g.batch)), 256, 0, stream>>>(
+        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC);
+  else
+    splitk_reduce<<<dim3(unsigned(ceil_div(mn, 256)), 1, unsigned(g.batch)), 256, 0, stream>>>(
+        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC);
+  ETG_LAUNCH("splitk_reduce");
 }
 
 template <typename T, bool TA, bool TB, int BM, int BN, bool WIDE>
@@ -389,9 +535,9 @@ Choice choose_tiling(const Gemm& g, double peak, bool can_split, int only_bm = 0
   return best;
 }
 
-// Runs the product with a given tile size and split-K count.
-template <typename T>
-GemmLaunch run_choice(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, Choice ch) {
+// Kernel parameters of a product in (up to) `want` splits of k, each a multiple of 16
+// long; their partial sums go to the workspace.
+Params split_params(const Gemm& g, GemmWorkspace* ws, int want, int* splits) {
   Params p{};
   p.m = g.m; p.n = g.n; p.k = g.k;
   p.alpha = g.alpha; p.beta = g.beta;
@@ -400,27 +546,43 @@ GemmLaunch run_choice(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, Choi
   p.C = g.C; p.ldc = g.ldc; p.strideC = g.strideC;
   p.W = nullptr;
   p.k_per_split = g.k;
-  int splits = ch.splits;
-  if (splits > 1) {
-    const int64_t kps = ceil_div(ceil_div(g.k, splits), 16) * 16;
-    splits = int(ceil_div(g.k, kps));
+  *splits = want;
+  if (want > 1) {
+    const int64_t kps = ceil_div(ceil_div(g.k, want), 16) * 16;
+    *splits = int(ceil_div(g.k, kps));
+    if (*splits == 1) return p;
     p.k_per_split = kps;
-    const size_t need = size_t(splits) * size_t(g.m) * size_t(g.n) * size_t(g.batch) * sizeof(double);
+    const size_t need = size_t(*splits) * size_t(g.m) * size_t(g.n) * size_t(g.batch) * sizeof(double);
     if (ws->buf.resize(need)) ++ws->gen;
     p.W = ws->buf.as<double>();
   }
+  return p;
+}
+
+// Runs the product with a given tile size and split-K count.
+template <typename T>
+GemmLaunch run_choice(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, Choice ch) {
+  int splits = 1;
+  const Params p = split_params(g, ws, ch.splits, &splits);
   GemmLaunch info;
   info.splits = splits;
   if (ch.bm == 128) info.kernel = launch_tile<T, 128, 128, 16>(stream, g, p, splits);
   else info.kernel = launch_tile<T, 64, 64, 16>(stream, g, p, splits);
-  if (splits > 1) {
-    const int64_t mn = g.m * g.n;
-    dim3 grid(unsigned(ceil_div(mn, 256)), 1, unsigned(g.batch));
-    splitk_reduce<<<grid, 256, 0, stream>>>(p.W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc,
-                                            g.strideC);
-    ETG_LAUNCH("splitk_reduce");
-  }
+  if (splits > 1) reduce_splits(stream, g, p.W, splits);
   return info;
+}
+
+template <typename T, int TM, int TN, int WK>
+const char* launch_few(hipStream_t stream, const Gemm& g, Params p, int splits) {
+  p.tiles_m = int(ceil_div(g.m, 16 * TM));
+  p.tiles_n = int(ceil_div(g.n, 16 * TN));
+  const dim3 grid(unsigned(p.tiles_m) * unsigned(p.tiles_n), unsigned(splits), unsigned(g.batch));
+  if (!g.ta && !g.tb) gemm_few_tiles<T, false, false, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
+  else if (!g.ta && g.tb) gemm_few_tiles<T, false, true, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
+  else if (g.ta && !g.tb) gemm_few_tiles<T, true, false, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
+  else gemm_few_tiles<T, true, true, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
+  ETG_LAUNCH("gemm_few_tiles");
+  return sizeof(T) == 8 ? "gemm_few_tiles<f64>" : "gemm_few_tiles<f32>";
 }
 
 // ---- measured tile choice ---------------------------------------------------
@@ -509,8 +671,54 @@ Choice tuned_choice(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, Choice
   return best;
 }
 
+// Tile (16 or 32 square), k splits and estimated microseconds of gemm_few_tiles.
+// A wave's chunk of 16 k takes 0.26 us (16 x 16, four matrix products) or 0.56 us
+// (32 x 32, sixteen), the chip as a whole 26 or 50 TFLOP/s over whole tiles, and a
+// split costs the second launch and its partial sums' traffic: within 20 % of the
+// measured times over m, n = 1 .. 5776 and k = 5 .. 115520.
+struct FewChoice {
+  int tile = 16, splits = 1;
+  double us = 1e300;
+};
+
+FewChoice choose_few(const Gemm& g, bool can_split) {
+  FewChoice best;
+  const double b = double(g.batch), mn = double(g.m) * double(g.n) * b;
+  for (int tile : {16, 32}) {
+    const double start = tile == 16 ? 2.4 : 3.4, chunk = tile == 16 ? 0.26 : 0.56, rate = tile == 16 ? 26e6 : 50e6;
+    const double work = 2.0 * double(ceil_div(g.m, tile) * tile) * double(ceil_div(g.n, tile) * tile) * double(g.k) * b;
+    for (int s = 1; s <= 256; s *= 2) {
+      if (s > 1 && (!can_split || g.k < int64_t(s) * 128 || 8.0 * s * mn > 1e9)) break;
+      const int64_t kps = ceil_div(ceil_div(g.k, s), 16) * 16;
+      const double us = start + chunk * double(ceil_div(kps, 64)) + work / rate + (s > 1 ? 2.6 + 16.0 * s * mn / 3e6 : 0.0);
+      if (us < best.us) best = FewChoice{tile, s, us};
+    }
+  }
+  return best;
+}
+
+// Products that run on gemm_few_tiles: at most 1.5 GFLOP (us, tiled and this:
+// 95 x 95 x 279 18 and 4, 19 x 5 x 5301 19 and 6, 380^3 25 and 8, 741^3 41 and 32, 76 x 20
+// x 96520 40 and 26; beyond, 400 x 400 x 5776 63 and 64, 210 x 2926 x 2926 99 and 112),
+// except short k over many outputs, which the larger tiles read fewer times
+// (76 x 30400 x 76: 20 and 26).
+bool few_tiles_pay(const Gemm& g) {
+  if (gemm_flops(g) > 1.5e9 || ceil_div(g.m, 16) * ceil_div(g.n, 16) > (int64_t(1) << 30)) return false;
+  return g.k > 128 || double(g.m) * double(g.n) * double(g.batch) < 4e5;
+}
+
 template <typename T>
 GemmLaunch launch_rows(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
+  if (few_tiles_pay(g)) {
+    const FewChoice c = choose_few(g, ws != nullptr);
+    int splits = 1;
+    const Params p = split_params(g, ws, c.splits, &splits);
+    GemmLaunch info;
+    info.splits = splits;
+    info.kernel = c.tile == 16 ? launch_few<T, 1, 1, 4>(stream, g, p, splits) : launch_few<T, 2, 2, 4>(stream, g, p, splits);
+    if (splits > 1) reduce_splits(stream, g, p.W, splits);
+    return info;
+  }
   // Tile size and split-K count from a cost model: a launch runs in rounds of
   // `slots` concurrent tiles (two 128 x 128 or four 64 x 64 workgroups per CU
   // on 256 CUs), each round at the tile's sustained matrix-core efficiency;
