@@ -990,6 +990,11 @@ int64_t gemm_tuned_shapes() {
   return int64_t(g_tuned.size());
 }
 
+bool runs_as_residues(const Gemm& g, Prec prec, const GemmWorkspace* ws) {
+  return prec == Prec::F64 && ws != nullptr && residue_pays(g, choose_tiling(g, 78.6e12, true).seconds) &&
+         residue_fits(g, ws);
+}
+
 GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws) {
   if (g.m < 0 || g.n < 0 || g.k < 0 || g.batch < 1) fail("gemm: negative dimension");
   if (g.m == 0 || g.n == 0) return GemmLaunch{};
@@ -1018,8 +1023,7 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
   if (prec == Prec::BF16X3 && split_bf16_pays(g)) return gemm_bf16x3(stream, g, ws);
   if (prec == Prec::F32) return launch_typed<float>(stream, g, ws);
   GemmLaunch info;
-  if (ws != nullptr && residue_pays(g, choose_tiling(g, 78.6e12, true).seconds) &&
-      gemm_residue(stream, g, ws, !capturing(stream), &info)) return info;
+  if (runs_as_residues(g, Prec::F64, ws) && gemm_residue(stream, g, ws, !capturing(stream), &info)) return info;
   return launch_typed<double>(stream, g, ws);
 }
 

@@ -41,6 +41,9 @@ struct Gemm {
   // Split-bf16 products only: C written in FP32 (the products' accumulation
   // type) to Cf instead of C; beta must be 0.
   float* Cf = nullptr;
+  // Nonzero: the caller reads C(i, j) only for i >= lower (j / lower), a lower
+  // triangle of lower x lower blocks; the other outputs may be left as they are.
+  int64_t lower = 0;
   // Split-bf16 products only: run the split-bf16 kernel whatever the shape
   // (diagnostics; see split_bf16_pays).
   bool split_any_shape = false;
@@ -120,7 +123,10 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws);
 // launched, when its workspace is not there and cannot be allocated or does not
 // hold the smallest panels).
 bool residue_pays(const Gemm& g, double fp64_seconds);
+bool residue_fits(const Gemm& g, const GemmWorkspace* ws);
 bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may_allocate, GemmLaunch* info);
+// Whether gemm() would run g so (the caller then need not cut g.lower's triangle itself).
+bool runs_as_residues(const Gemm& g, Prec prec, const GemmWorkspace* ws);
 
 // bf16 values of the split-bf16 pack of a rows x k operand (both splits, padded
 // to the product kernel's 256-row tile and 32-deep step).
@@ -158,8 +164,10 @@ inline Gemm make_gemm(char ta, char tb, int64_t m, int64_t n, int64_t k, double 
   return g;
 }
 
-// Floating-point operations the product performs (2 m n k per batch entry).
+// Floating-point operations the product performs (2 m n k per batch entry; of a
+// lower block triangle those of its blocks).
 inline double gemm_flops(const Gemm& g) {
+  if (g.lower > 0) return double(g.m + g.lower) * double(g.n) * double(g.k);
   return 2.0 * double(g.m) * double(g.n) * double(g.k) * double(g.batch);
 }
 

@@ -423,7 +423,9 @@ __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
 
 struct Panels {
   int64_t KS, rows_m, rows_n, batch;          // panel rows of op(A) and op(B)^T, batch entries per group
+  int64_t out_m, out_n;                       // outputs of a panel taken at once (their residues)
   int tile_n;                                 // columns of a tile
+  bool same;                                  // op(A)^T and op(B) are one array, packed once
   int64_t a_entries, b_entries;               // batch entries packed per group (1 for a shared operand)
   int64_t rm_p, rn_p;                         // panel rows padded to whole tiles
   int64_t parts;                              // k ranges of the row norms
@@ -432,22 +434,40 @@ struct Panels {
 };
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
+int64_t round_up(int64_t x, int64_t to) { return ceil_div(x, to) * to; }
 
-void size_panels(const Gemm& g, Panels& p) {
-  p.rm_p = ceil_div(p.rows_m, kTileM) * kTileM;
-  p.rn_p = ceil_div(p.rows_n, p.tile_n) * p.tile_n;
+// Buffer sizes of the panels; what the packs leave is the room for the residues,
+// which go by columns (at least 512, or all), then rows.  False when that does not fit.
+bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
+  p.rm_p = round_up(p.rows_m, kTileM);
+  p.rn_p = round_up(p.rows_n, p.tile_n);
   p.a_entries = g.strideA == 0 ? 1 : p.batch;
   p.b_entries = g.strideB == 0 ? 1 : p.batch;
+  if (p.same) p.rm_p = p.rn_p = std::max(p.rm_p, p.rn_p);
   p.bytes_a = align256(size_t(p.a_entries * kModuli) * size_t(p.rm_p * p.KS * kDepth));
-  p.bytes_b = align256(size_t(p.b_entries * kModuli) * size_t(p.rn_p * p.KS * kDepth));
-  p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(p.rm_p * p.rn_p));
+  p.bytes_b = p.same ? 0 : align256(size_t(p.b_entries * kModuli) * size_t(p.rn_p * p.KS * kDepth));
   p.bytes_e = align256(sizeof(int) * size_t(p.a_entries * p.rm_p + p.b_entries * p.rn_p));
   p.bytes_n = align256(16 * size_t(std::max(p.a_entries * p.rm_p, p.b_entries * p.rn_p) * p.parts));
+  p.bytes_r = 0;
+  if (p.total() >= capacity) return false;
+  const int64_t room = int64_t(capacity - p.total()) / (p.batch * kModuli) - 256;   // outputs
+  p.out_m = p.rm_p;
+  p.out_n = p.rn_p;
+  // a quarter of the capacity (or all) for the residues: thinner pieces leave CUs idle
+  if (room < std::min(p.rm_p * p.rn_p, int64_t(capacity / 4) / (p.batch * kModuli))) return false;
+  // a lower block triangle goes by columns: a sixteenth of them at once wastes 3 %
+  if (g.lower > 0) p.out_n = std::min(p.out_n, round_up(std::max<int64_t>(1, p.rn_p / 16), p.tile_n));
+  const int64_t least = std::min<int64_t>(p.out_n, 512);
+  if (p.out_m * p.out_n > room) p.out_n = std::max(least, room / p.out_m / p.tile_n * p.tile_n);
+  if (p.out_m * p.out_n > room) p.out_m = room / p.out_n / kTileM * kTileM;
+  if (p.out_m < std::min<int64_t>(p.rm_p, 1024)) return false;
+  p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(p.out_m * p.out_n));
+  return p.total() <= capacity;
 }
 
-// The whole product where it fits the capacity, else equal groups of the batch,
-// else (one entry at a time) equal panels of rows, the longer panel split first.
-// A panel more of one operand packs the other once more: 7.4 ps per element
+// The whole product where its packs fit the capacity, else equal groups of the
+// batch, else (one entry at a time) equal panels of rows, the longer panel split
+// first.  A panel more of one operand packs the other once more: 7.4 ps per element
 // against the 12.5 fs of products that each of its elements has with every row
 // of the panel, so panels of 2560 rows cost a quarter, of 6912 rows a twelfth.
 bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
@@ -457,20 +477,22 @@ bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
   p.rows_m = g.m;
   p.rows_n = g.n;
   p.batch = g.batch;
+  p.same = g.A == g.B && g.ta != g.tb && g.lda == g.ldb && g.m == g.n && g.batch == 1;
   int64_t groups = 1, pm = 1, pn = 1;
-  for (;;) {
-    size_panels(g, p);
-    if (p.total() <= capacity) return true;
-    if (p.batch > 1) {
+  while (!size_panels(g, capacity, p)) {
+    if (p.same) {
+      p.same = false;
+    } else if (p.batch > 1) {
       p.batch = ceil_div(g.batch, ++groups);
     } else if (p.rows_m >= p.rows_n) {
       if (p.rows_m <= kTileM) return false;
-      p.rows_m = std::min(g.m, ceil_div(ceil_div(g.m, ++pm), kTileM) * kTileM);
+      p.rows_m = std::min(g.m, round_up(ceil_div(g.m, ++pm), kTileM));
     } else {
       if (p.rows_n <= kTileM) return false;
-      p.rows_n = std::min(g.n, ceil_div(ceil_div(g.n, ++pn), kTileM) * kTileM);
+      p.rows_n = std::min(g.n, round_up(ceil_div(g.n, ++pn), kTileM));
     }
   }
+  return true;
 }
 
 // One operand panel: exponents, then the pack.
@@ -517,6 +539,11 @@ bool residue_pays(const Gemm& g, double fp64_seconds) {
   return products + packs + output + 45e-6 < 0.95 * std::min(fp64_seconds, 2.0 * m * n * k * b / 35e12);
 }
 
+bool residue_fits(const Gemm& g, const GemmWorkspace* ws) {
+  Panels p{};
+  return ws->residue && !ws->residue->refused && plan_panels(g, ws->residue->capacity, p);
+}
+
 bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may_allocate, GemmLaunch* info) {
   ResidueWorkspace* rw = ws->residue.get();
   Panels p{};
@@ -533,10 +560,10 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
   }
   char* base = rw->buf.as<char>();
   u4* PA = reinterpret_cast<u4*>(base);
-  u4* PB = reinterpret_cast<u4*>(base + p.bytes_a);
+  u4* PB = p.same ? PA : reinterpret_cast<u4*>(base + p.bytes_a);
   uint32_t* R = reinterpret_cast<uint32_t*>(base + p.bytes_a + p.bytes_b);
   int* ea = reinterpret_cast<int*>(base + p.bytes_a + p.bytes_b + p.bytes_r);
-  int* eb = ea + p.a_entries * p.rm_p;
+  int* eb = p.same ? ea : ea + p.a_entries * p.rm_p;
   void* norms = base + p.bytes_a + p.bytes_b + p.bytes_r + p.bytes_e;
   const bool a_kcontig = g.ta, b_kcontig = !g.tb;
   const int64_t pm = ceil_div(g.m, p.rows_m), pn = ceil_div(g.n, p.rows_n);
@@ -552,50 +579,57 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
     if (a_want != a_is)
       pack_operand(stream, A, g.lda, g.strideA, a_kcontig, m, g.k, p.KS, p.rm_p, g.strideA == 0 ? 1 : nb, p.parts, norms,
                    ea, PA);
-    if (b_want != b_is)
+    if (b_want != b_is && !p.same)
       pack_operand(stream, B, g.ldb, g.strideB, b_kcontig, n, g.k, p.KS, p.rn_p, g.strideB == 0 ? 1 : nb, p.parts, norms,
                    eb, PB);
     a_is = a_want;
     b_is = b_want;
-    Params q{};
-    q.A = PA;
-    q.B = PB;
-    q.R = R;
-    q.KS = p.KS;
-    q.planeA = p.rm_p * p.KS * (kDepth / 16);
-    q.planeB = p.rn_p * p.KS * (kDepth / 16);
-    q.planeR = p.rm_p * p.rn_p / 4;
-    q.strideA = g.strideA == 0 ? 0 : kModuli * q.planeA;
-    q.strideB = g.strideB == 0 ? 0 : kModuli * q.planeB;
-    q.strideR = kModuli * q.planeR;
-    q.tiles_m = int(ceil_div(m, kTileM));
-    q.tiles_n = int(ceil_div(n, p.tile_n));
-    const unsigned tiles = unsigned(q.tiles_m) * unsigned(q.tiles_n);
-    const dim3 grid(tiles, kModuli, unsigned(nb));
-    if (p.tile_n == 128)
-      residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
-    else
-      residue_product_kernel<4, 4><<<grid, 512, 0, stream>>>(q);
-    ETG_LAUNCH("residue_product");
-    Output o{};
-    o.R = R;
-    o.planeR = q.planeR;
-    o.strideR = q.strideR;
-    o.tiles_m = q.tiles_m;
-    o.blocks_n = p.tile_n / 16;
-    o.m = m; o.n = n; o.K = g.k;
-    o.ea = ea; o.eb = eb;
-    o.ea_stride = g.strideA == 0 ? 0 : p.rm_p;
-    o.eb_stride = g.strideB == 0 ? 0 : p.rn_p;
-    o.alpha = g.alpha; o.beta = g.beta;
-    o.C = g.C + b0 * g.strideC + m0 + n0 * g.ldc;
-    o.ldc = g.ldc; o.strideC = g.strideC;
-    o.vec_rows = m % 4 == 0 && g.ldc % 2 == 0 && (g.batch == 1 || g.strideC % 2 == 0) &&
-                 reinterpret_cast<uintptr_t>(o.C) % 16 == 0;
-    o.A = A; o.lda = g.lda; o.strideA = g.strideA; o.a_kcontig = a_kcontig ? 1 : 0;
-    o.B = B; o.ldb = g.ldb; o.strideB = g.strideB; o.b_kcontig = b_kcontig ? 1 : 0;
-    residue_reconstruct_kernel<<<dim3(tiles * unsigned(kBlocksM * p.tile_n / 64), unsigned(nb)), 256, 0, stream>>>(o);
-    ETG_LAUNCH("residue_reconstruct");
+    for (int64_t c0 = 0; c0 < n; c0 += p.out_n) {
+      // first row of the panel that these columns need, down to a whole tile
+      const int64_t first = g.lower > 0 ? (n0 + c0) / g.lower * g.lower - m0 : 0;
+      for (int64_t r0 = first > 0 ? first / kTileM * kTileM : 0; r0 < m; r0 += p.out_m) {
+        const int64_t mo = std::min(p.out_m, m - r0), no = std::min(p.out_n, n - c0);
+        Params q{};
+        q.A = PA + r0 * p.KS * (kDepth / 16);
+        q.B = PB + c0 * p.KS * (kDepth / 16);
+        q.R = R;
+        q.KS = p.KS;
+        q.tiles_m = int(ceil_div(mo, kTileM));
+        q.tiles_n = int(ceil_div(no, p.tile_n));
+        q.planeA = p.rm_p * p.KS * (kDepth / 16);
+        q.planeB = p.rn_p * p.KS * (kDepth / 16);
+        q.planeR = int64_t(q.tiles_m) * kTileM * q.tiles_n * p.tile_n / 4;
+        q.strideA = g.strideA == 0 ? 0 : kModuli * q.planeA;
+        q.strideB = g.strideB == 0 ? 0 : kModuli * q.planeB;
+        q.strideR = kModuli * q.planeR;
+        const unsigned tiles = unsigned(q.tiles_m) * unsigned(q.tiles_n);
+        const dim3 grid(tiles, kModuli, unsigned(nb));
+        if (p.tile_n == 128)
+          residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
+        else
+          residue_product_kernel<4, 4><<<grid, 512, 0, stream>>>(q);
+        ETG_LAUNCH("residue_product");
+        Output o{};
+        o.R = R;
+        o.planeR = q.planeR;
+        o.strideR = q.strideR;
+        o.tiles_m = q.tiles_m;
+        o.blocks_n = p.tile_n / 16;
+        o.m = mo; o.n = no; o.K = g.k;
+        o.ea = ea + r0; o.eb = eb + c0;
+        o.ea_stride = g.strideA == 0 ? 0 : p.rm_p;
+        o.eb_stride = g.strideB == 0 ? 0 : p.rn_p;
+        o.alpha = g.alpha; o.beta = g.beta;
+        o.C = g.C + b0 * g.strideC + m0 + r0 + (n0 + c0) * g.ldc;
+        o.ldc = g.ldc; o.strideC = g.strideC;
+        o.vec_rows = mo % 4 == 0 && g.ldc % 2 == 0 && (g.batch == 1 || g.strideC % 2 == 0) &&
+                     reinterpret_cast<uintptr_t>(o.C) % 16 == 0;
+        o.A = A + (a_kcontig ? r0 * g.lda : r0); o.lda = g.lda; o.strideA = g.strideA; o.a_kcontig = a_kcontig ? 1 : 0;
+        o.B = B + (b_kcontig ? c0 * g.ldb : c0); o.ldb = g.ldb; o.strideB = g.strideB; o.b_kcontig = b_kcontig ? 1 : 0;
+        residue_reconstruct_kernel<<<dim3(tiles * unsigned(kBlocksM * p.tile_n / 64), unsigned(nb)), 256, 0, stream>>>(o);
+        ETG_LAUNCH("residue_reconstruct");
+      }
+    }
   };
   // the outer operand's panels are packed once, the inner one's once per outer panel
   // (and both once per group of the batch unless shared)

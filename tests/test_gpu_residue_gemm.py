@@ -106,3 +106,23 @@ def test_transformations_of_a_group():
             assert np.abs(one[:, 0] - R[:, 1]).max() < 1e-13 * np.abs(R[:, 1]).max()
         left, right = Y.T @ AX, AtY.T @ X
         assert np.abs(left - right).max() < 1e-12 * np.linalg.norm(Y[:, 0]) * np.linalg.norm(AX[:, 0])
+
+
+@pytest.mark.parametrize('o,v,J', [(12, 61, 700), (10, 76, 1270)])
+def test_ladder_blocks(o, v, J):
+    """The residual with the G of the ladder as one triangle, as triangles and off-diagonal blocks,
+    and as blocks too small for the int8 path; oddly aligned columns of a block row too."""
+    s = syn.system(5, o, v, J, t2_sigma=1e-3, t1_sigma=1e-2, L_scale=0.02)
+    with ccsd.CCSD(o, v, J) as wf:
+        wf.set_cholesky(s['L'])
+        wf.set_oei(s['h'])
+        wf.set_amplitudes(np.concatenate([s['t1'].ravel(order='F'), s['t2']]))
+        wf.construct_t1_cholesky()
+        ref = wf.construct_omega()
+        wf.set_kernel_ledger(True)
+        wf.construct_omega(copy_out=False)
+        assert any('gemm_residue' in r[0] for r in wf.kernel_ledger())
+        wf.set_kernel_ledger(False)
+        for nb in (v // 2 + 1, 33, 5):
+            wf.set_ladder_batch(nb)
+            assert np.abs(wf.construct_omega() - ref).max() < 1e-13 * np.abs(ref).max()
