@@ -50,7 +50,7 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   // transformation passes (one stream): a whole (ov)^3 product takes 45 n_t1^2 bytes
   // (1.7 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
   // 4 GB, 0.87 s with 2.5 GB)
-  const double residue_bytes = std::min(4.0e9, std::max(1.0e9, 64.0 * double(N) * double(N)));
+  const double residue_bytes = std::min(4.0e9, std::max(0.4e9, 64.0 * double(N) * double(N)));
   gws_.residue = gws_pass_.residue = std::make_shared<ResidueWorkspace>(size_t(residue_bytes));
   // default ladder batch: G blocks of at most ~12 GB
   const double budget = 12e9 / 8.0;
@@ -241,15 +241,13 @@ void CCSD::set_amplitudes(const double* t) {
 
 void CCSD::get_amplitudes(double* t) {
   require(t != nullptr, "etg_get_amplitudes: null pointer");
-  ETG_HIP(hipMemcpyAsync(t, t_.as<double>(), sizeof(double) * (n_t1 + n_t2),
-                         hipMemcpyDeviceToHost, stream_));
+  host_copy_.to_host(stream_, t, t_.as<double>(), sizeof(double) * (n_t1 + n_t2));
   synchronize();
 }
 
 void CCSD::get_omega(double* out) {
   require(out != nullptr, "etg_get_omega: null pointer");
-  ETG_HIP(hipMemcpyAsync(out, omega_.as<double>(), sizeof(double) * (n_t1 + n_t2),
-                         hipMemcpyDeviceToHost, stream_));
+  host_copy_.to_host(stream_, out, omega_.as<double>(), sizeof(double) * (n_t1 + n_t2));
   synchronize();
 }
 
@@ -1157,8 +1155,7 @@ void CCSD::transform_batch(int side, int64_t n_vec, const double* X, double* R, 
         tgraphs_.push_back(e);
       }
     }
-    ETG_HIP(hipMemcpyAsync(R + k0 * n, jout_.as<double>(), sizeof(double) * n * nb, hipMemcpyDefault,
-                           stream_));
+    host_copy_.to_host(stream_, R + k0 * n, jout_.as<double>(), sizeof(double) * n * nb);
   }
   pack_cache_ = true;
   synchronize();

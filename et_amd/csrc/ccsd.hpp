@@ -8,6 +8,7 @@
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "host_copy.hpp"
 #include "ops.hpp"
 
 namespace etg {
@@ -210,6 +211,7 @@ class CCSD {
   void omega_c2_d2(Ops& X, Prec prec, const double* T, const double* U);
 
   hipStream_t stream_ = nullptr;
+  HostCopy host_copy_;
   GemmWorkspace gws_;
 
   DeviceBuffer Lmo_oo_, Lmo_ov_, Lmo_vo_, Lmo_vv_;

@@ -645,7 +645,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     if (converged || stalled) {
       if (vectors) {
         for (int64_t j = 0; j < s; ++j) scale(stream_, Y + j * n, n, 1.0 / std::sqrt(ynorm[j]));
-        ETG_HIP(hipMemcpyAsync(vectors, Y, sizeof(double) * n * s, hipMemcpyDefault, stream_));
+        host_copy_.to_host(stream_, vectors, Y, sizeof(double) * n * s);
         synchronize();
       }
       return converged ? it : -it;

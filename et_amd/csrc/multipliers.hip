@@ -99,8 +99,7 @@ void CCSD::set_multipliers(const double* host) {
 void CCSD::get_multipliers(double* host) {
   require(have_tbar_, "get_multipliers: no multipliers set");
   require(host != nullptr, "get_multipliers: null pointer");
-  ETG_HIP(hipMemcpyAsync(host, tbar_.as<double>(), sizeof(double) * (n_t1 + n_t2),
-                         hipMemcpyDeviceToHost, stream_));
+  host_copy_.to_host(stream_, host, tbar_.as<double>(), sizeof(double) * (n_t1 + n_t2));
   synchronize();
 }
 
@@ -111,8 +110,7 @@ void CCSD::construct_eta(double* host) {
   eta_kernel<<<grid_for_m(n), kBlock, 0, stream_>>>(F_.as<double>(), g_ovov_.as<double>(),
                                                     eta_.as<double>(), n_o, n_v);
   ETG_LAUNCH("eta");
-  if (host)
-    ETG_HIP(hipMemcpyAsync(host, eta_.as<double>(), sizeof(double) * n, hipMemcpyDeviceToHost, stream_));
+  if (host) host_copy_.to_host(stream_, host, eta_.as<double>(), sizeof(double) * n);
   synchronize();
 }
 
@@ -125,8 +123,7 @@ void CCSD::construct_multiplier_equation(double* host, Prec prec) {
   mres_.resize(sizeof(double) * n);
   transform_batch(1, 1, tbar_.as<double>(), mres_.as<double>(), prec);
   axpy(stream_, n, 1.0, eta_.as<double>(), mres_.as<double>());
-  if (host)
-    ETG_HIP(hipMemcpyAsync(host, mres_.as<double>(), sizeof(double) * n, hipMemcpyDeviceToHost, stream_));
+  if (host) host_copy_.to_host(stream_, host, mres_.as<double>(), sizeof(double) * n);
   synchronize();
   have_mres_ = true;
 }
