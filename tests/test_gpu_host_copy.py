@@ -22,15 +22,15 @@ def _round_trip(o, v, seed, out=None):
                 out.append(ok)
 
 
-# 4 MB and below (runtime's copy), just above, several pieces, more than the ring holds
-@pytest.mark.parametrize('o,v', [(7, 70), (16, 63), (16, 64), (13, 79), (20, 101), (30, 152), (31, 200)])
+# 16 MB and below (runtime's copy), just above, several pieces, more than the ring holds
+@pytest.mark.parametrize('o,v', [(7, 70), (32, 63), (32, 64), (23, 101), (30, 152), (31, 200)])
 def test_lengths(o, v):
     _round_trip(o, v, o * v)
 
 
 def test_two_threads():
     out = []
-    ts = [threading.Thread(target=_round_trip, args=(12 + k, 90, k, out)) for k in range(2)]
+    ts = [threading.Thread(target=_round_trip, args=(30 + k, 90, k, out)) for k in range(2)]
     for t in ts:
         t.start()
     for t in ts:
