@@ -774,12 +774,10 @@ void CCSD::ladder_tangent(const double* t2, const double* dt2, int64_t s_dt2, co
     g.strideC = sC;
     run_gemm(g, prec);
   };
-  for (int64_t k = 0; k < nb; ++k) {
-    if (split)
-      ladder_t_pm_blocked(s, dt2 + k * s_dt2, dtp + k * lsz_tp_, dtm + k * lsz_tm_, o, v);
-    else
-      ladder_t_pm(s, dt2 + k * s_dt2, dtp + k * lsz_tp_, dtm + k * lsz_tm_, o, v);
-  }
+  if (split)
+    ladder_t_pm_blocked(s, dt2, dtp, dtm, o, v, LadderBatch{nb, s_dt2, lsz_tp_, lsz_tm_});
+  else
+    ladder_t_pm(s, dt2, dtp, dtm, o, v, LadderBatch{nb, s_dt2, lsz_tp_, lsz_tm_});
   for (const Block& b : blocks_) {
     ladder_G(b, LT, prec, split, 0);
     Gemm gpl = make_gemm('N', 'N', op, b.npairs, kp, 0.5, dtp, op, gp_.as<double>(), kp, 0.0,
@@ -799,19 +797,15 @@ void CCSD::ladder_tangent(const double* t2, const double* dt2, int64_t s_dt2, co
     batched(gpl, lsz_tp_, 0, lsz_wp_);
     if (minus) batched(gmi, lsz_tm_, 0, lsz_wm_);
   }
-  for (int64_t k = 0; k < nb; ++k)
-    ladder_gather(s, dwp + k * lsz_wp_, dwm + k * lsz_wm_, pair_col_.as<int32_t>(), dom2 + k * s_dom2,
-                  o, v);
+  ladder_gather(s, dwp, dwm, pair_col_.as<int32_t>(), dom2, o, v, LadderBatch{nb, s_dom2, lsz_wp_, lsz_wm_});
   // T1 part: Z(a, b, i, j) = -dt1(a, k) W(k, bij), then (a, i, b, j), then symmetrised into packed
   double* Z = lz1_.as<double>();
   double* Zf = lz2_.as<double>();
   batched(make_gemm('N', 'N', v, v * o * o, o, -1.0, dt2 - n_t1, v, lw_.as<double>(), o, 0.0, Z, v),
           s_dt2, 0, N * N);
   const int64_t dZ[4] = {v, v, o, o};
-  for (int64_t k = 0; k < nb; ++k) {
-    sort4(s, Z + k * N * N, dZ, "1324", Zf + k * N * N, 1.0, 0.0);
-    symmetrize_and_pack(s, Zf + k * N * N, dom2 + k * s_dom2, v, o, 1.0, 1.0, 0.0);
-  }
+  sort4(s, Z, dZ, "1324", Zf, 1.0, 0.0, Batch{nb, N * N, N * N});
+  symmetrize_and_pack(s, Zf, dom2, v, o, 1.0, 1.0, 0.0, Batch{nb, N * N, s_dom2});
 }
 
 // Adjoint of the ladder term for nb vectors: from om2b + k s_om2b, accumulates
@@ -841,34 +835,27 @@ void CCSD::ladder_adjoint(const double* t2, double* t2b, int64_t s_t2b, const do
     g.strideC = sC;
     run_gemm(g, prec);
   };
-  ladder_t_pm(s, t2, tp_.as<double>(), tm_.as<double>(), o, v);
-  for (int64_t k = 0; k < nb; ++k)
-    ladder_gather_adjoint(s, om2b + k * s_om2b, pcol_a_.as<int32_t>(), pcol_b_.as<int32_t>(),
-                          wpb + k * lsz_wp_, wmb + k * lsz_wm_, o, v);
-  fill(s, tpb, nb * lsz_tp_, 0.0);
-  if (om > 0 && vm > 0) fill(s, tmb, nb * lsz_tm_, 0.0);
+  ladder_gather_adjoint(s, om2b, pcol_a_.as<int32_t>(), pcol_b_.as<int32_t>(), wpb, wmb, o, v,
+                        LadderBatch{nb, s_om2b, lsz_wp_, lsz_wm_});
   for (const Block& b : blocks_) {
+    const double acc = &b == &blocks_.front() ? 0.0 : 1.0;
     ladder_G(b, LT, prec, false, 0);
     ladder_g_pm(s, gblk_.as<double>(), v, b.la, b.lb, pair_a_.as<int32_t>() + b.col0,
                 pair_b_.as<int32_t>() + b.col0, b.npairs, gp_.as<double>(), gm_.as<double>());
     // w+ = 1/2 t+ g+  ->  t+_bar += 1/2 w+_bar g+^T
     batched(make_gemm('N', 'T', op, vp, b.npairs, 0.5, wpb + op * b.col0, op, gp_.as<double>(), vp,
-                      1.0, tpb, op), lsz_wp_, 0, lsz_tp_);
+                      acc, tpb, op), lsz_wp_, 0, lsz_tp_);
     if (om > 0 && vm > 0)
       batched(make_gemm('N', 'T', om, vm, b.npairs, 0.5, wmb + om * b.col0, om, gm_.as<double>(), vm,
-                        1.0, tmb, om), lsz_wm_, 0, lsz_tm_);
+                        acc, tmb, om), lsz_wm_, 0, lsz_tm_);
   }
-  for (int64_t k = 0; k < nb; ++k)
-    ladder_t_pm_adjoint(s, tpb + k * lsz_tp_, tmb + k * lsz_tm_, t2b + k * s_t2b, o, v);
+  ladder_t_pm_adjoint(s, tpb, tmb, t2b, o, v, LadderBatch{nb, s_t2b, lsz_tp_, lsz_tm_});
   // T1 part: Zf_bar from the packed adjoint, to (a, b, i, j), then t1_bar -= Z_bar W^T
   double* Zb = lz1_.as<double>();
   double* Zfb = lz2_.as<double>();
-  fill(s, Zfb, nb * N * N, 0.0);
   const int64_t dZf[4] = {v, o, v, o};
-  for (int64_t k = 0; k < nb; ++k) {
-    symmetrize_and_pack_adjoint(s, om2b + k * s_om2b, Zfb + k * N * N, v, o, 1.0, 1.0, 0.0);
-    sort4(s, Zfb + k * N * N, dZf, "1324", Zb + k * N * N, 1.0, 0.0);
-  }
+  symmetrize_and_pack_adjoint(s, om2b, Zfb, v, o, 1.0, 1.0, 0.0, false, Batch{nb, s_om2b, N * N});
+  sort4(s, Zfb, dZf, "1324", Zb, 1.0, 0.0, Batch{nb, N * N, N * N});
   batched(make_gemm('N', 'T', v, o, v * o * o, -1.0, Zb, v, lw_.as<double>(), o, 1.0, t2b - n_t1, v),
           N * N, 0, s_t2b);
 }

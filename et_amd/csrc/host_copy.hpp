@@ -96,7 +96,7 @@ class HostCopy {
   static constexpr int kRing = 8, kThreads = 8;
 
   static size_t piece_bytes(size_t bytes) {
-    const size_t even = (bytes / (2 * kRing) + 4095) / 4096 * 4096;
+    const size_t even = (bytes / (4 * kRing) + 4095) / 4096 * 4096;
     return std::max(size_t(256) << 10, std::min(kPiece, even));
   }
   static bool known_to_runtime(const void* p) {

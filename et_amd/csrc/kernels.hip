@@ -17,6 +17,9 @@ inline unsigned grid_for(int64_t n, int64_t per_block = kBlock, int64_t cap = 1 
   return unsigned(g);
 }
 
+// The same over the vectors of a batch (blockIdx.z).
+inline dim3 grid_z(int64_t n, int64_t batch) { return dim3(grid_for(n), 1, unsigned(batch)); }
+
 // Largest X with X (X + 1) / 2 <= k.
 __device__ inline int64_t tri_root(int64_t k) {
   int64_t x = int64_t((sqrt(8.0 * double(k) + 1.0) - 1.0) * 0.5);
@@ -34,7 +37,9 @@ __device__ inline int64_t pidx(int64_t x, int64_t y) {
 // element-wise divisions then cost a fraction of the 64-bit ones)
 template <typename I>
 __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict__ y, I e0, I e1, I e2,
-                                I e3, I s0, I s1, I s2, I s3, double alpha, double beta) {
+                                I e3, I s0, I s1, I s2, I s3, double alpha, double beta, int64_t sx, int64_t sy) {
+  x += int64_t(blockIdx.z) * sx;
+  y += int64_t(blockIdx.z) * sy;
   const I n = e0 * e1 * e2 * e3;
   for (I idx = I(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += I(gridDim.x) * blockDim.x) {
     I r = idx;
@@ -54,7 +59,9 @@ __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict
 __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __restrict__ y,
                                       int64_t e0, int64_t ep, int64_t eq, int64_t er, int64_t s0,
                                       int64_t sq, int64_t sr, int64_t yp, int64_t yq, int64_t yr,
-                                      double alpha, double beta) {
+                                      double alpha, double beta, int64_t bx, int64_t by) {
+  x += int64_t(blockIdx.z) * bx;
+  y += int64_t(blockIdx.z) * by;
   __shared__ double tile[32][33];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t nt0 = (e0 + 31) / 32;
@@ -81,7 +88,9 @@ __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __re
 }
 
 __global__ void squareup_kernel(const double* __restrict__ packed, double* __restrict__ full,
-                                int64_t N) {
+                                int64_t N, int64_t sx, int64_t sy) {
+  packed += int64_t(blockIdx.z) * sx;
+  full += int64_t(blockIdx.z) * sy;
   const int64_t n = N * N;
   for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n;
        idx += int64_t(gridDim.x) * blockDim.x) {
@@ -93,7 +102,9 @@ __global__ void squareup_kernel(const double* __restrict__ packed, double* __res
 // X block) reads packed elements (X, Y), Y <= X, along Y and writes full(Y, X)
 // along Y and its mirror full(X, Y) along X.
 __global__ __launch_bounds__(256) void squareup_tiled_kernel(const double* __restrict__ packed,
-                                                             double* __restrict__ full, int64_t N) {
+                                                             double* __restrict__ full, int64_t N, int64_t sx, int64_t sy) {
+  packed += int64_t(blockIdx.z) * sx;
+  full += int64_t(blockIdx.z) * sy;
   __shared__ double P[32][33];                          // P[xl][yl] = packed(X0 + xl, Y0 + yl)
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t xb = tri_root(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
@@ -113,7 +124,9 @@ __global__ __launch_bounds__(256) void squareup_tiled_kernel(const double* __res
 
 // packed element k = (X, Y), X >= Y, reads full(Y, X) (column X is contiguous in Y)
 __global__ void packin_kernel(const double* __restrict__ full, double* __restrict__ packed,
-                              int64_t N, double alpha, double beta, double diag_scale) {
+                              int64_t N, double alpha, double beta, double diag_scale, int64_t sx, int64_t sy) {
+  full += int64_t(blockIdx.z) * sx;
+  packed += int64_t(blockIdx.z) * sy;
   const int64_t n = N * (N + 1) / 2;
   for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n;
        k += int64_t(gridDim.x) * blockDim.x) {
@@ -126,7 +139,9 @@ __global__ void packin_kernel(const double* __restrict__ full, double* __restric
 
 // y = x + x^T through 32 x 32 LDS tiles
 __global__ void symmetric_sum_kernel(const double* __restrict__ x, double* __restrict__ y,
-                                     int64_t N) {
+                                     int64_t N, int64_t sx, int64_t sy) {
+  x += int64_t(blockIdx.z) * sx;
+  y += int64_t(blockIdx.z) * sy;
   __shared__ double tile[32][33];
   const int64_t bx = blockIdx.x, by = blockIdx.y;
   const int tx = threadIdx.x, ty = threadIdx.y;  // 32 x 8
@@ -150,7 +165,9 @@ __global__ void symmetric_sum_kernel(const double* __restrict__ x, double* __res
 __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const double* __restrict__ x,
                                                                         double* __restrict__ y, int64_t n_v,
                                                                         int64_t N, double alpha, double f1,
-                                                                        double f2) {
+                                                                        double f2, int64_t sx, int64_t sy) {
+  x += int64_t(blockIdx.z) * sx;
+  y += int64_t(blockIdx.z) * sy;
   __shared__ double A[32][33], B[32][33];              // A[xl][yl] = x(Y, X), B[yl][xl] = x(X, Y)
   __shared__ double C[32][33], D[32][33];              // C[xl][yl] = x(p + v s, r + v q), D[yl][xl] = mirror
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
@@ -191,7 +208,9 @@ __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const do
 
 __global__ void symmetrize_and_pack_kernel(const double* __restrict__ x, double* __restrict__ y,
                                            int64_t n_v, int64_t n_o, double alpha, double f1,
-                                           double f2) {
+                                           double f2, int64_t sx, int64_t sy) {
+  x += int64_t(blockIdx.z) * sx;
+  y += int64_t(blockIdx.z) * sy;
   const int64_t N = n_v * n_o;
   const int64_t n = N * (N + 1) / 2;
   for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n;
@@ -209,7 +228,10 @@ __global__ void symmetrize_and_pack_kernel(const double* __restrict__ x, double*
 }
 
 __global__ void ladder_t_pm_kernel(const double* __restrict__ t2, double* __restrict__ tp,
-                                   double* __restrict__ tm, int64_t n_o, int64_t n_v) {
+                                   double* __restrict__ tm, int64_t n_o, int64_t n_v, int64_t st, int64_t sp, int64_t sm) {
+  t2 += int64_t(blockIdx.z) * st;
+  tp += int64_t(blockIdx.z) * sp;
+  tm += int64_t(blockIdx.z) * sm;
   const int64_t op = n_o * (n_o + 1) / 2, vp = n_v * (n_v + 1) / 2;
   const int64_t om = n_o * (n_o - 1) / 2, vm = n_v * (n_v - 1) / 2;
   const int64_t n = op * vp;
@@ -233,7 +255,10 @@ __global__ void ladder_t_pm_kernel(const double* __restrict__ t2, double* __rest
 // order of ladder_order.hpp (zero at padding positions).
 __global__ void ladder_t_pm_blocked_kernel(const double* __restrict__ t2, double* __restrict__ tp,
                                            double* __restrict__ tm, int64_t n_o, int64_t n_v, int64_t KP,
-                                           int64_t KM) {
+                                           int64_t KM, int64_t st, int64_t sp, int64_t sm) {
+  t2 += int64_t(blockIdx.z) * st;
+  tp += int64_t(blockIdx.z) * sp;
+  tm += int64_t(blockIdx.z) * sm;
   const int64_t op = n_o * (n_o + 1) / 2, om = n_o * (n_o - 1) / 2;
   const int64_t np = op * KP, n = np + om * KM;
   for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n;
@@ -293,7 +318,10 @@ __global__ void ladder_g_pm_tiled_kernel(const double* __restrict__ G, int64_t n
 
 __global__ void ladder_gather_kernel(const double* __restrict__ wp, const double* __restrict__ wm,
                                      const int32_t* __restrict__ col, double* __restrict__ om,
-                                     int64_t n_o, int64_t n_v) {
+                                     int64_t n_o, int64_t n_v, int64_t so, int64_t sp, int64_t sm) {
+  wp += int64_t(blockIdx.z) * sp;
+  wm += int64_t(blockIdx.z) * sm;
+  om += int64_t(blockIdx.z) * so;
   const int64_t N = n_o * n_v;
   const int64_t n = N * (N + 1) / 2;
   const int64_t op = n_o * (n_o + 1) / 2, omn = n_o * (n_o - 1) / 2;
@@ -430,7 +458,7 @@ __global__ void fill_kernel(double* __restrict__ x, int64_t n, double value) {
 }  // namespace
 
 void permute4(hipStream_t s, const double* x, double* y, const int64_t e[4], const int64_t st[4],
-              double alpha, double beta) {
+              double alpha, double beta, const Batch& b) {
   const int64_t n = e[0] * e[1] * e[2] * e[3];
   if (n == 0) return;
   int p = -1;                                   // output position of the input-fastest index
@@ -443,26 +471,26 @@ void permute4(hipStream_t s, const double* x, double* y, const int64_t e[4], con
     const int64_t ostride[4] = {1, e[0], e[0] * e[1], e[0] * e[1] * e[2]};
     const int64_t tiles = ceil_div(e[0], 32) * ceil_div(e[p], 32);
     const int64_t others = e[oth[0]] * e[oth[1]];
-    dim3 grid(unsigned(tiles), unsigned(std::min<int64_t>(others, 65535)));
+    dim3 grid(unsigned(tiles), unsigned(std::min<int64_t>(others, 65535)), unsigned(b.n));
     permute4_tiled_kernel<<<grid, kBlock, 0, s>>>(x, y, e[0], e[p], e[oth[0]], e[oth[1]], st[0],
                                                   st[oth[0]], st[oth[1]], ostride[p], ostride[oth[0]],
-                                                  ostride[oth[1]], alpha, beta);
+                                                  ostride[oth[1]], alpha, beta, b.x, b.y);
     ETG_LAUNCH("permute4_tiled");
     return;
   }
   // (32-bit indices: the grid-stride step stays below 2^32 - n as well)
   if (n + int64_t(kBlock) * grid_for(n) <= int64_t(UINT32_MAX))
-    permute4_kernel<uint32_t><<<grid_for(n), kBlock, 0, s>>>(
+    permute4_kernel<uint32_t><<<grid_z(n, b.n), kBlock, 0, s>>>(
         x, y, uint32_t(e[0]), uint32_t(e[1]), uint32_t(e[2]), uint32_t(e[3]), uint32_t(st[0]), uint32_t(st[1]),
-        uint32_t(st[2]), uint32_t(st[3]), alpha, beta);
+        uint32_t(st[2]), uint32_t(st[3]), alpha, beta, b.x, b.y);
   else
-    permute4_kernel<int64_t><<<grid_for(n), kBlock, 0, s>>>(x, y, e[0], e[1], e[2], e[3], st[0], st[1], st[2],
-                                                            st[3], alpha, beta);
+    permute4_kernel<int64_t><<<grid_z(n, b.n), kBlock, 0, s>>>(x, y, e[0], e[1], e[2], e[3], st[0], st[1], st[2],
+                                                               st[3], alpha, beta, b.x, b.y);
   ETG_LAUNCH("permute4");
 }
 
 void sort4(hipStream_t s, const double* x, const int64_t d[4], const char* perm, double* y,
-           double alpha, double beta) {
+           double alpha, double beta, const Batch& b) {
   if (std::strlen(perm) != 4) fail("sort4: permutation must have 4 digits");
   const int64_t in_stride[4] = {1, d[0], d[0] * d[1], d[0] * d[1] * d[2]};
   int64_t e[4], st[4];
@@ -474,59 +502,60 @@ void sort4(hipStream_t s, const double* x, const int64_t d[4], const char* perm,
     e[k] = d[q];
     st[k] = in_stride[q];
   }
-  permute4(s, x, y, e, st, alpha, beta);
+  permute4(s, x, y, e, st, alpha, beta, b);
 }
 
-void squareup(hipStream_t s, const double* packed, double* full, int64_t N) {
+void squareup(hipStream_t s, const double* packed, double* full, int64_t N, const Batch& b) {
   if (N >= 32) {
     const int64_t nb = ceil_div(N, 32);
-    squareup_tiled_kernel<<<unsigned(nb * (nb + 1) / 2), kBlock, 0, s>>>(packed, full, N);
+    squareup_tiled_kernel<<<dim3(unsigned(nb * (nb + 1) / 2), 1, unsigned(b.n)), kBlock, 0, s>>>(packed, full, N, b.x, b.y);
     ETG_LAUNCH("squareup_tiled");
     return;
   }
-  squareup_kernel<<<grid_for(N * N), kBlock, 0, s>>>(packed, full, N);
+  squareup_kernel<<<grid_z(N * N, b.n), kBlock, 0, s>>>(packed, full, N, b.x, b.y);
   ETG_LAUNCH("squareup");
 }
 
 void packin(hipStream_t s, const double* full, double* packed, int64_t N, double alpha, double beta,
-            double diag_scale) {
-  packin_kernel<<<grid_for(N * (N + 1) / 2), kBlock, 0, s>>>(full, packed, N, alpha, beta, diag_scale);
+            double diag_scale, const Batch& b) {
+  packin_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(full, packed, N, alpha, beta, diag_scale, b.x, b.y);
   ETG_LAUNCH("packin");
 }
 
-void symmetric_sum(hipStream_t s, const double* x, double* y, int64_t N) {
+void symmetric_sum(hipStream_t s, const double* x, double* y, int64_t N, const Batch& b) {
   if (x == y) fail("symmetric_sum: out of place only");
-  dim3 grid(unsigned(ceil_div(N, 32)), unsigned(ceil_div(N, 32)));
-  symmetric_sum_kernel<<<grid, dim3(32, 8), 0, s>>>(x, y, N);
+  dim3 grid(unsigned(ceil_div(N, 32)), unsigned(ceil_div(N, 32)), unsigned(b.n));
+  symmetric_sum_kernel<<<grid, dim3(32, 8), 0, s>>>(x, y, N, b.x, b.y);
   ETG_LAUNCH("symmetric_sum");
 }
 
 void symmetrize_and_pack(hipStream_t s, const double* x, double* packed, int64_t n_v, int64_t n_o,
-                         double alpha, double f1, double f2) {
+                         double alpha, double f1, double f2, const Batch& b) {
   const int64_t N = n_v * n_o;
   if (N >= 32) {
     const int64_t nb = ceil_div(N, 32);
-    symmetrize_and_pack_tiled_kernel<<<unsigned(nb * (nb + 1) / 2), kBlock, 0, s>>>(x, packed, n_v, N, alpha,
-                                                                                   f1, f2);
+    symmetrize_and_pack_tiled_kernel<<<dim3(unsigned(nb * (nb + 1) / 2), 1, unsigned(b.n)), kBlock, 0, s>>>(
+        x, packed, n_v, N, alpha, f1, f2, b.x, b.y);
     ETG_LAUNCH("symmetrize_and_pack_tiled");
     return;
   }
-  symmetrize_and_pack_kernel<<<grid_for(N * (N + 1) / 2), kBlock, 0, s>>>(x, packed, n_v, n_o,
-                                                                          alpha, f1, f2);
+  symmetrize_and_pack_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(x, packed, n_v, n_o, alpha, f1, f2, b.x,
+                                                                             b.y);
   ETG_LAUNCH("symmetrize_and_pack");
 }
 
-void ladder_t_pm(hipStream_t s, const double* t2, double* tp, double* tm, int64_t n_o, int64_t n_v) {
+void ladder_t_pm(hipStream_t s, const double* t2, double* tp, double* tm, int64_t n_o, int64_t n_v,
+                 const LadderBatch& b) {
   const int64_t n = (n_o * (n_o + 1) / 2) * (n_v * (n_v + 1) / 2);
-  ladder_t_pm_kernel<<<grid_for(n), kBlock, 0, s>>>(t2, tp, tm, n_o, n_v);
+  ladder_t_pm_kernel<<<grid_z(n, b.n), kBlock, 0, s>>>(t2, tp, tm, n_o, n_v, b.vec, b.plus, b.minus);
   ETG_LAUNCH("ladder_t_pm");
 }
 
 void ladder_t_pm_blocked(hipStream_t s, const double* t2, double* tp, double* tm, int64_t n_o,
-                         int64_t n_v) {
+                         int64_t n_v, const LadderBatch& b) {
   const int64_t KP = ladder_blocked_len(n_v, true), KM = ladder_blocked_len(n_v, false);
   const int64_t n = (n_o * (n_o + 1) / 2) * KP + (n_o * (n_o - 1) / 2) * KM;
-  ladder_t_pm_blocked_kernel<<<grid_for(n), kBlock, 0, s>>>(t2, tp, tm, n_o, n_v, KP, KM);
+  ladder_t_pm_blocked_kernel<<<grid_z(n, b.n), kBlock, 0, s>>>(t2, tp, tm, n_o, n_v, KP, KM, b.vec, b.plus, b.minus);
   ETG_LAUNCH("ladder_t_pm_blocked");
 }
 
@@ -542,9 +571,10 @@ void ladder_g_pm(hipStream_t s, const double* G, int64_t n_v, int64_t lenA, int6
 }
 
 void ladder_gather(hipStream_t s, const double* wp, const double* wm, const int32_t* col,
-                   double* omega2, int64_t n_o, int64_t n_v) {
+                   double* omega2, int64_t n_o, int64_t n_v, const LadderBatch& b) {
   const int64_t N = n_o * n_v;
-  ladder_gather_kernel<<<grid_for(N * (N + 1) / 2), kBlock, 0, s>>>(wp, wm, col, omega2, n_o, n_v);
+  ladder_gather_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(wp, wm, col, omega2, n_o, n_v, b.vec, b.plus,
+                                                                       b.minus);
   ETG_LAUNCH("ladder_gather");
 }
 
@@ -633,7 +663,9 @@ __global__ void scale_kernel(double* x, int64_t n, double beta) {
 }
 
 __global__ void symmetric_sum_acc_kernel(const double* __restrict__ x, double* __restrict__ y,
-                                         int64_t N, double beta) {
+                                         int64_t N, double beta, int64_t sx, int64_t sy) {
+  x += int64_t(blockIdx.z) * sx;
+  y += int64_t(blockIdx.z) * sy;
   __shared__ double tile[32][33];
   const int64_t bx = blockIdx.x, by = blockIdx.y;
   const int tx = threadIdx.x, ty = threadIdx.y;
@@ -652,7 +684,9 @@ __global__ void symmetric_sum_acc_kernel(const double* __restrict__ x, double* _
 }
 
 __global__ void packsum_kernel(const double* __restrict__ full, double* __restrict__ packed,
-                               int64_t N) {
+                               int64_t N, int64_t sx, int64_t sy) {
+  full += int64_t(blockIdx.z) * sx;
+  packed += int64_t(blockIdx.z) * sy;
   GRID_LOOP(k, N * (N + 1) / 2) {
     const int64_t X = tri_root2(k), Y = k - X * (X + 1) / 2;
     double v = full[X + N * Y];
@@ -662,7 +696,9 @@ __global__ void packsum_kernel(const double* __restrict__ full, double* __restri
 }
 
 __global__ void unpack_upper_add_kernel(const double* __restrict__ packed, double* __restrict__ full,
-                                        int64_t N, double alpha, double diag_scale) {
+                                        int64_t N, double alpha, double diag_scale, int64_t sx, int64_t sy) {
+  packed += int64_t(blockIdx.z) * sx;
+  full += int64_t(blockIdx.z) * sy;
   GRID_LOOP(k, N * (N + 1) / 2) {
     const int64_t X = tri_root2(k), Y = k - X * (X + 1) / 2;
     double v = alpha * packed[k];
@@ -674,7 +710,9 @@ __global__ void unpack_upper_add_kernel(const double* __restrict__ packed, doubl
 // x(R, C) += alpha * [R == C ? p{R,R} : f1 p{R,C} + f2 p{U,W}],
 // U = (R_a, C_i), W = (C_a, R_i)  (the element the psrq terms of the forward pass read)
 __global__ void sympack_adjoint_kernel(const double* __restrict__ p, double* __restrict__ x,
-                                       int64_t n_v, int64_t n_o, double alpha, double f1, double f2) {
+                                       int64_t n_v, int64_t n_o, double alpha, double f1, double f2, bool acc, int64_t sx, int64_t sy) {
+  p += int64_t(blockIdx.z) * sx;
+  x += int64_t(blockIdx.z) * sy;
   const int64_t N = n_v * n_o;
   GRID_LOOP(idx, N * N) {
     const int64_t R = idx % N, C = idx / N;
@@ -689,7 +727,7 @@ __global__ void sympack_adjoint_kernel(const double* __restrict__ p, double* __r
         if (U != W) v += f2 * p[pidx2(U, W)];
       }
     }
-    x[idx] += alpha * v;
+    x[idx] = acc ? x[idx] + alpha * v : alpha * v;
   }
 }
 
@@ -698,7 +736,10 @@ __global__ void sympack_adjoint_kernel(const double* __restrict__ p, double* __r
 // and x(X, Y) along X).
 __global__ __launch_bounds__(256) void sympack_adjoint_tiled_kernel(const double* __restrict__ p,
                                                                     double* __restrict__ x, int64_t N,
-                                                                    double alpha, double f1) {
+                                                                    double alpha, double f1, bool acc, int64_t sx,
+                                                                    int64_t sy) {
+  p += int64_t(blockIdx.z) * sx;
+  x += int64_t(blockIdx.z) * sy;
   __shared__ double P[32][33];                          // P[xl][yl] = p(X0 + xl, Y0 + yl)
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t xb = tri_root2(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
@@ -710,15 +751,18 @@ __global__ __launch_bounds__(256) void sympack_adjoint_tiled_kernel(const double
   __syncthreads();
   for (int k = ty; k < 32; k += 8) {
     const int64_t X = X0 + k, Y = Y0 + tx;              // x(Y, X), along Y
-    if (X < N && Y <= X) x[Y + N * X] += P[k][tx];
+    if (X < N && Y <= X) x[Y + N * X] = acc ? x[Y + N * X] + P[k][tx] : P[k][tx];
     const int64_t Xr = X0 + tx, Yc = Y0 + k;            // x(Xr, Yc), along Xr (the diagonal once)
-    if (Xr < N && Yc < Xr) x[Xr + N * Yc] += P[tx][k];
+    if (Xr < N && Yc < Xr) x[Xr + N * Yc] = acc ? x[Xr + N * Yc] + P[tx][k] : P[tx][k];
   }
 }
 
 // t2[{(c,i),(d,j)}] += coef * tp[ij, cd] + sgn * tm[ij, cd]
 __global__ void ladder_t_pm_adjoint_kernel(const double* __restrict__ tp, const double* __restrict__ tm,
-                                           double* __restrict__ t2, int64_t n_o, int64_t n_v) {
+                                           double* __restrict__ t2, int64_t n_o, int64_t n_v, int64_t st, int64_t sp, int64_t sm) {
+  tp += int64_t(blockIdx.z) * sp;
+  tm += int64_t(blockIdx.z) * sm;
+  t2 += int64_t(blockIdx.z) * st;
   const int64_t Nov = n_o * n_v;
   const int64_t op = n_o * (n_o + 1) / 2, om = n_o * (n_o - 1) / 2;
   GRID_LOOP(k, Nov * (Nov + 1) / 2) {
@@ -769,7 +813,10 @@ __global__ void ladder_g_pm_adjoint_kernel(const double* __restrict__ gp, const 
 __global__ void ladder_gather_adjoint_kernel(const double* __restrict__ om,
                                              const int32_t* __restrict__ pa,
                                              const int32_t* __restrict__ pb, double* __restrict__ wp,
-                                             double* __restrict__ wm, int64_t n_o, int64_t n_v) {
+                                             double* __restrict__ wm, int64_t n_o, int64_t n_v, int64_t so, int64_t sp, int64_t sm) {
+  om += int64_t(blockIdx.z) * so;
+  wp += int64_t(blockIdx.z) * sp;
+  wm += int64_t(blockIdx.z) * sm;
   const int64_t op = n_o * (n_o + 1) / 2, omn = n_o * (n_o - 1) / 2;
   const int64_t vp = n_v * (n_v + 1) / 2;
   GRID_LOOP(idx, op * vp) {
@@ -787,7 +834,10 @@ __global__ void ladder_gather_adjoint_kernel(const double* __restrict__ om,
 }
 
 __global__ void t1_xy_kernel2(const double* t1, double* X, double* Y, int64_t n_o, int64_t n_v,
-                              double diag) {
+                              double diag, int64_t st, int64_t sm) {
+  t1 += int64_t(blockIdx.z) * st;
+  X += int64_t(blockIdx.z) * sm;
+  Y += int64_t(blockIdx.z) * sm;
   const int64_t n = n_o + n_v;
   GRID_LOOP(k, n * n) {
     const int64_t p = k % n, q = k / n;
@@ -800,7 +850,10 @@ __global__ void t1_xy_kernel2(const double* t1, double* X, double* Y, int64_t n_
 }
 
 __global__ void t1_xy_adjoint_kernel(const double* Xb, const double* Yb, double* t1b, int64_t n_o,
-                                     int64_t n_v) {
+                                     int64_t n_v, int64_t st, int64_t sm) {
+  Xb += int64_t(blockIdx.z) * sm;
+  Yb += int64_t(blockIdx.z) * sm;
+  t1b += int64_t(blockIdx.z) * st;
   const int64_t n = n_o + n_v;
   GRID_LOOP(k, n_o * n_v) {
     const int64_t a = k % n_v, i = k / n_v;
@@ -808,7 +861,9 @@ __global__ void t1_xy_adjoint_kernel(const double* Xb, const double* Yb, double*
   }
 }
 
-__global__ void trace_oo_kernel2(const double* Loo, double* XJ, int64_t nJ, int64_t n_o) {
+__global__ void trace_oo_kernel2(const double* Loo, double* XJ, int64_t nJ, int64_t n_o, int64_t sx, int64_t sy) {
+  Loo += int64_t(blockIdx.z) * sx;
+  XJ += int64_t(blockIdx.z) * sy;
   GRID_LOOP(J, nJ) {
     double s = 0.0;
     for (int64_t k = 0; k < n_o; ++k) s += Loo[J + nJ * (k + n_o * k)];
@@ -816,14 +871,18 @@ __global__ void trace_oo_kernel2(const double* Loo, double* XJ, int64_t nJ, int6
   }
 }
 
-__global__ void trace_oo_adjoint_kernel(const double* XJb, double* Loob, int64_t nJ, int64_t n_o) {
+__global__ void trace_oo_adjoint_kernel(const double* XJb, double* Loob, int64_t nJ, int64_t n_o, int64_t sx, int64_t sy) {
+  XJb += int64_t(blockIdx.z) * sx;
+  Loob += int64_t(blockIdx.z) * sy;
   GRID_LOOP(idx, nJ * n_o) {
     const int64_t J = idx % nJ, k = idx / nJ;
     Loob[J + nJ * (k + n_o * k)] += XJb[J];
   }
 }
 
-__global__ void fock_ov_vector_kernel2(const double* F, double* f, int64_t n_o, int64_t n_v) {
+__global__ void fock_ov_vector_kernel2(const double* F, double* f, int64_t n_o, int64_t n_v, int64_t sx, int64_t sy) {
+  F += int64_t(blockIdx.z) * sx;
+  f += int64_t(blockIdx.z) * sy;
   const int64_t n = n_o + n_v;
   GRID_LOOP(k, n_o * n_v) {
     const int64_t b = k % n_v, j = k / n_v;
@@ -831,7 +890,9 @@ __global__ void fock_ov_vector_kernel2(const double* F, double* f, int64_t n_o, 
   }
 }
 
-__global__ void fock_ov_vector_adjoint_kernel(const double* fb, double* Fb, int64_t n_o, int64_t n_v) {
+__global__ void fock_ov_vector_adjoint_kernel(const double* fb, double* Fb, int64_t n_o, int64_t n_v, int64_t sx, int64_t sy) {
+  fb += int64_t(blockIdx.z) * sx;
+  Fb += int64_t(blockIdx.z) * sy;
   const int64_t n = n_o + n_v;
   GRID_LOOP(k, n_o * n_v) {
     const int64_t b = k % n_v, j = k / n_v;
@@ -840,7 +901,9 @@ __global__ void fock_ov_vector_adjoint_kernel(const double* fb, double* Fb, int6
 }
 
 __global__ void copy_sub_kernel2(const double* src, int64_t lds, double* dst, int64_t ldd, int64_t m,
-                                 int64_t n, double alpha, double beta) {
+                                 int64_t n, double alpha, double beta, int64_t sx, int64_t sy) {
+  src += int64_t(blockIdx.z) * sx;
+  dst += int64_t(blockIdx.z) * sy;
   GRID_LOOP(k, m * n) {
     const int64_t r = k % m, c = k / m;
     const double v = alpha * src[r + lds * c];
@@ -876,41 +939,42 @@ void scale(hipStream_t s, double* x, int64_t n, double beta) {
   ETG_LAUNCH("scale");
 }
 
-void symmetric_sum_acc(hipStream_t s, const double* x, double* y, int64_t N, double beta) {
+void symmetric_sum_acc(hipStream_t s, const double* x, double* y, int64_t N, double beta, const Batch& b) {
   if (x == y) fail("symmetric_sum_acc: out of place only");
-  dim3 grid(unsigned(ceil_div(N, 32)), unsigned(ceil_div(N, 32)));
-  symmetric_sum_acc_kernel<<<grid, dim3(32, 8), 0, s>>>(x, y, N, beta);
+  dim3 grid(unsigned(ceil_div(N, 32)), unsigned(ceil_div(N, 32)), unsigned(b.n));
+  symmetric_sum_acc_kernel<<<grid, dim3(32, 8), 0, s>>>(x, y, N, beta, b.x, b.y);
   ETG_LAUNCH("symmetric_sum_acc");
 }
 
-void packsum(hipStream_t s, const double* full, double* packed, int64_t N) {
-  packsum_kernel<<<g2(N * (N + 1) / 2), kBlock, 0, s>>>(full, packed, N);
+void packsum(hipStream_t s, const double* full, double* packed, int64_t N, const Batch& b) {
+  packsum_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(full, packed, N, b.x, b.y);
   ETG_LAUNCH("packsum");
 }
 
 void unpack_upper_add(hipStream_t s, const double* packed, double* full, int64_t N, double alpha,
-                      double diag_scale) {
-  unpack_upper_add_kernel<<<g2(N * (N + 1) / 2), kBlock, 0, s>>>(packed, full, N, alpha, diag_scale);
+                      double diag_scale, const Batch& b) {
+  unpack_upper_add_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(packed, full, N, alpha, diag_scale, b.x, b.y);
   ETG_LAUNCH("unpack_upper_add");
 }
 
 void symmetrize_and_pack_adjoint(hipStream_t s, const double* packed, double* x, int64_t n_v,
-                                 int64_t n_o, double alpha, double f1, double f2) {
+                                 int64_t n_o, double alpha, double f1, double f2, bool acc, const Batch& b) {
   const int64_t N = n_v * n_o;
   if (f2 == 0.0 && N >= 32) {
     const int64_t nb = ceil_div(N, 32);
-    sympack_adjoint_tiled_kernel<<<unsigned(nb * (nb + 1) / 2), kBlock, 0, s>>>(packed, x, N, alpha, f1);
+    sympack_adjoint_tiled_kernel<<<dim3(unsigned(nb * (nb + 1) / 2), 1, unsigned(b.n)), kBlock, 0, s>>>(
+        packed, x, N, alpha, f1, acc, b.x, b.y);
     ETG_LAUNCH("sympack_adjoint_tiled");
     return;
   }
-  sympack_adjoint_kernel<<<g2(N * N), kBlock, 0, s>>>(packed, x, n_v, n_o, alpha, f1, f2);
+  sympack_adjoint_kernel<<<grid_z(N * N, b.n), kBlock, 0, s>>>(packed, x, n_v, n_o, alpha, f1, f2, acc, b.x, b.y);
   ETG_LAUNCH("sympack_adjoint");
 }
 
 void ladder_t_pm_adjoint(hipStream_t s, const double* tp, const double* tm, double* t2, int64_t n_o,
-                         int64_t n_v) {
+                         int64_t n_v, const LadderBatch& b) {
   const int64_t N = n_o * n_v;
-  ladder_t_pm_adjoint_kernel<<<g2(N * (N + 1) / 2), kBlock, 0, s>>>(tp, tm, t2, n_o, n_v);
+  ladder_t_pm_adjoint_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(tp, tm, t2, n_o, n_v, b.vec, b.plus, b.minus);
   ETG_LAUNCH("ladder_t_pm_adjoint");
 }
 
@@ -924,49 +988,51 @@ void ladder_g_pm_adjoint(hipStream_t s, const double* gp, const double* gm, doub
 }
 
 void ladder_gather_adjoint(hipStream_t s, const double* omega2, const int32_t* pcol_a,
-                           const int32_t* pcol_b, double* wp, double* wm, int64_t n_o, int64_t n_v) {
+                           const int32_t* pcol_b, double* wp, double* wm, int64_t n_o, int64_t n_v,
+                           const LadderBatch& b) {
   const int64_t n = (n_o * (n_o + 1) / 2) * (n_v * (n_v + 1) / 2);
-  ladder_gather_adjoint_kernel<<<g2(n), kBlock, 0, s>>>(omega2, pcol_a, pcol_b, wp, wm, n_o, n_v);
+  ladder_gather_adjoint_kernel<<<grid_z(n, b.n), kBlock, 0, s>>>(omega2, pcol_a, pcol_b, wp, wm, n_o, n_v, b.vec, b.plus,
+                                                                 b.minus);
   ETG_LAUNCH("ladder_gather_adjoint");
 }
 
 void t1_xy(hipStream_t s, const double* t1, double* X, double* Y, int64_t n_o, int64_t n_v,
-           double diag) {
+           double diag, const Batch& b) {
   const int64_t n = n_o + n_v;
-  t1_xy_kernel2<<<g2(n * n), kBlock, 0, s>>>(t1, X, Y, n_o, n_v, diag);
+  t1_xy_kernel2<<<grid_z(n * n, b.n), kBlock, 0, s>>>(t1, X, Y, n_o, n_v, diag, b.x, b.y);
   ETG_LAUNCH("t1_xy");
 }
 
 void t1_xy_adjoint(hipStream_t s, const double* Xb, const double* Yb, double* t1b, int64_t n_o,
-                   int64_t n_v) {
-  t1_xy_adjoint_kernel<<<g2(n_o * n_v), kBlock, 0, s>>>(Xb, Yb, t1b, n_o, n_v);
+                   int64_t n_v, const Batch& b) {
+  t1_xy_adjoint_kernel<<<grid_z(n_o * n_v, b.n), kBlock, 0, s>>>(Xb, Yb, t1b, n_o, n_v, b.x, b.y);
   ETG_LAUNCH("t1_xy_adjoint");
 }
 
-void trace_oo(hipStream_t s, const double* Loo, double* XJ, int64_t nJ, int64_t n_o) {
-  trace_oo_kernel2<<<g2(nJ), kBlock, 0, s>>>(Loo, XJ, nJ, n_o);
+void trace_oo(hipStream_t s, const double* Loo, double* XJ, int64_t nJ, int64_t n_o, const Batch& b) {
+  trace_oo_kernel2<<<grid_z(nJ, b.n), kBlock, 0, s>>>(Loo, XJ, nJ, n_o, b.x, b.y);
   ETG_LAUNCH("trace_oo");
 }
 
-void trace_oo_adjoint(hipStream_t s, const double* XJb, double* Loob, int64_t nJ, int64_t n_o) {
-  trace_oo_adjoint_kernel<<<g2(nJ * n_o), kBlock, 0, s>>>(XJb, Loob, nJ, n_o);
+void trace_oo_adjoint(hipStream_t s, const double* XJb, double* Loob, int64_t nJ, int64_t n_o, const Batch& b) {
+  trace_oo_adjoint_kernel<<<grid_z(nJ * n_o, b.n), kBlock, 0, s>>>(XJb, Loob, nJ, n_o, b.x, b.y);
   ETG_LAUNCH("trace_oo_adjoint");
 }
 
-void fock_ov_vector(hipStream_t s, const double* F, double* f, int64_t n_o, int64_t n_v) {
-  fock_ov_vector_kernel2<<<g2(n_o * n_v), kBlock, 0, s>>>(F, f, n_o, n_v);
+void fock_ov_vector(hipStream_t s, const double* F, double* f, int64_t n_o, int64_t n_v, const Batch& b) {
+  fock_ov_vector_kernel2<<<grid_z(n_o * n_v, b.n), kBlock, 0, s>>>(F, f, n_o, n_v, b.x, b.y);
   ETG_LAUNCH("fock_ov_vector");
 }
 
-void fock_ov_vector_adjoint(hipStream_t s, const double* fb, double* Fb, int64_t n_o, int64_t n_v) {
-  fock_ov_vector_adjoint_kernel<<<g2(n_o * n_v), kBlock, 0, s>>>(fb, Fb, n_o, n_v);
+void fock_ov_vector_adjoint(hipStream_t s, const double* fb, double* Fb, int64_t n_o, int64_t n_v, const Batch& b) {
+  fock_ov_vector_adjoint_kernel<<<grid_z(n_o * n_v, b.n), kBlock, 0, s>>>(fb, Fb, n_o, n_v, b.x, b.y);
   ETG_LAUNCH("fock_ov_vector_adjoint");
 }
 
 void copy_sub(hipStream_t s, const double* src, int64_t lds, double* dst, int64_t ldd, int64_t m,
-              int64_t n, double alpha, double beta) {
+              int64_t n, double alpha, double beta, const Batch& b) {
   if (m * n == 0) return;
-  copy_sub_kernel2<<<g2(m * n), kBlock, 0, s>>>(src, lds, dst, ldd, m, n, alpha, beta);
+  copy_sub_kernel2<<<grid_z(m * n, b.n), kBlock, 0, s>>>(src, lds, dst, ldd, m, n, alpha, beta, b.x, b.y);
   ETG_LAUNCH("copy_sub");
 }
 

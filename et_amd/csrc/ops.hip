@@ -241,12 +241,60 @@ void Tape::zero_derivatives(int64_t nb) {
   }
 }
 
-// nb derivative vectors of each listed intermediate (contiguous from its slot's start).
-void Tape::zero_starting(const std::vector<int>& bufs, int64_t nb) {
-  for (int k : bufs) {
-    const Buf& b = *bufs_[size_t(k)];
-    fill(wf_.stream(), slots_[size_t(b.slot)].as<double>(), nb * std::max<int64_t>(b.elems, 1), 0.0);
+// nb derivative vectors of intermediate k (contiguous from its slot's start).
+void Tape::zero_intermediate(int k, int64_t nb) {
+  const Buf& b = *bufs_[size_t(k)];
+  fill(wf_.stream(), slots_[size_t(b.slot)].as<double>(), nb * std::max<int64_t>(b.elems, 1), 0.0);
+}
+
+// Whether the forward rule of an operation writes the whole derivative of buffer k
+// without reading it: its lifetime then needs no zeroes to start from.
+bool Tape::writes_whole(const Op& op, int k) const {
+  const Buf& b = *bufs_[size_t(k)];
+  auto is = [&](const double* p, int64_t elems) { return p == b.base && elems == b.elems; };
+  switch (op.kind) {
+    case GEMM: {
+      const Gemm& g = op.g;
+      return g.beta == 0.0 && g.ldc == g.m && (g.batch == 1 || g.strideC == g.m * g.n) && is(g.C, g.m * g.n * g.batch);
+    }
+    case SORT4: return op.beta == 0.0 && is(op.y, op.d[0] * op.d[1] * op.d[2] * op.d[3]);
+    case SQUAREUP:
+    case SYMSUM: return is(op.y, op.N * op.N);
+    case PACKIN: return op.beta == 0.0 && is(op.y, op.N * (op.N + 1) / 2);
+    case COPY_SUB: return op.beta == 0.0 && op.ldd == op.m && is(op.y, op.m * op.n);
+    case FILL0: return is(op.y, op.n);
+    case T1_XY: return is(op.y, wf_.n_mo * wf_.n_mo) || is(op.y2, wf_.n_mo * wf_.n_mo);
+    case TRACE_OO: return is(op.y, wf_.n_J);
+    case FOCK_OV_VEC: return is(op.y, wf_.n_o * wf_.n_v);
+    case SYMPACK:
+    case LADDER: break;
   }
+  return false;
+}
+
+// Whether the backward rule of an operation can write the whole adjoint of its
+// input buffer k (the first contribution to it) instead of adding to zeroes.
+bool Tape::adjoint_writes_whole(const Op& op, int k) const {
+  const Buf& b = *bufs_[size_t(k)];
+  auto is = [&](const double* p, int64_t elems) { return p == b.base && elems == b.elems; };
+  switch (op.kind) {
+    case GEMM: {
+      const Gemm& g = op.g;
+      if (find(g.C) == k) return false;
+      const int64_t ra = g.ta ? g.k : g.m, ca = g.ta ? g.m : g.k, rb = g.tb ? g.n : g.k, cb = g.tb ? g.k : g.n;
+      // an operand shared by a recorded batch collects the entries' sum; the adjoint
+      // of A is formed first, so that of B may only come first where A has none there
+      if (find(g.A) == k)
+        return g.lda == ra && (g.batch == 1 || g.strideA == ra * ca) && is(g.A, ra * ca * g.batch);
+      return g.ldb == rb && (g.batch == 1 || g.strideB == rb * cb) && is(g.B, rb * cb * g.batch);
+    }
+    case SORT4: return find(op.y) != k && is(op.x, op.d[0] * op.d[1] * op.d[2] * op.d[3]);
+    case SYMSUM: return is(op.x, op.N * op.N);
+    case SYMPACK: return is(op.x, op.nv * op.no * op.nv * op.no);
+    case COPY_SUB: return find(op.y) != k && op.lds == op.m && is(op.x, op.m * op.n);
+    default: break;
+  }
+  return false;
 }
 
 void Tape::gemm(const Gemm& g, Prec prec) {
@@ -659,32 +707,36 @@ void Tape::tangent_gemm(const Gemm& g, Prec prec, int64_t nb) {
       base.strideA = 0;
       base.strideB = 0;
     }
-    if (g.beta != 1.0) {
+    if (!dA && !dB && g.beta != 1.0) {
       Gemm z = base;
       z.k = 0;
       z.beta = g.beta;
       wf_.run_gemm(z, prec);
     }
+    double beta = g.beta;                 // of the first product; the second adds to it
     if (dA) {
       Gemm h = base;
       h.A = dA + k * sA;
       if (vec_batch) h.strideA = sA;
-      h.beta = 1.0;
+      h.beta = beta;
       wf_.run_gemm(h, prec);
+      beta = 1.0;
     }
     if (dB) {
       Gemm h = base;
       h.B = dB + k * sB;
       if (vec_batch) h.strideB = sB;
-      h.beta = 1.0;
+      h.beta = beta;
       wf_.run_gemm(h, prec);
     }
   }
 }
 
 // A_bar_k += alpha C_bar_k op(B)^T (or its transpose), B_bar_k likewise, then
-// C_bar_k *= beta; batched over the vectors as in tangent_gemm.
-void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb) {
+// C_bar_k *= beta; batched over the vectors as in tangent_gemm.  `fresh`: buffers
+// whose adjoints start here (their first product has beta = 0); `c_ends`: nothing
+// reads the adjoint of C after this.
+void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb, const std::vector<int>& fresh, bool c_ends) {
   double* Cb0 = deriv(g0.C);
   double* Ab0 = deriv(g0.A);
   double* Bb0 = deriv(g0.B);
@@ -696,6 +748,8 @@ void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb) {
   const int64_t sC = dstride(g0.C), sA = Ab0 ? dstride(g0.A) : 0, sB = Bb0 ? dstride(g0.B) : 0;
   const bool vec_batch = g.batch == 1 && nb > 1;
   const int64_t reps = vec_batch ? 1 : nb;
+  auto starts = [&](const double* p) { return std::find(fresh.begin(), fresh.end(), find(p)) != fresh.end(); };
+  const bool a_fresh = Ab0 && starts(g0.A), b_fresh = Bb0 && find(g0.A) != find(g0.B) && starts(g0.B);
   for (int64_t v = 0; v < reps; ++v) {
     const double* Cb = Cb0 + v * sC;
     double* Ab = Ab0 ? Ab0 + v * sA : nullptr;
@@ -737,7 +791,7 @@ void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb) {
         h.C = Bo; h.ldc = g.ldb; h.strideC = g.strideB;
       }
       h.alpha = g.alpha;
-      h.beta = 1.0;
+      h.beta = (for_A ? a_fresh : b_fresh) ? 0.0 : 1.0;
       if (vec_batch) {             // one product per vector: adjoints at their strides, primal shared
         h.batch = nb;
         h.strideA = (h.A == C) ? sC : 0;
@@ -774,7 +828,7 @@ void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb) {
       if (g.batch > 1 && g.strideB == 0) shared(false);
       else wf_.run_gemm(pair(false, 0, g.batch), prec);
     }
-    if (g.beta != 1.0) {
+    if (g.beta != 1.0 && !(g.beta == 0.0 && c_ends)) {
       Gemm z = g;
       z.a_tag = 0;
       z.k = 0;
@@ -791,16 +845,14 @@ void Tape::adjoint_gemm(const Gemm& g0, Prec prec, int64_t nb) {
 
 void Tape::tangent(Prec prec, int64_t nb) {
   hipStream_t s = wf_.stream();
-  auto D = [&](const double* p, int64_t k) -> double* {
-    double* d = deriv(p);
-    return d ? d + k * dstride(p) : nullptr;
-  };
   plan_derivatives();
   reset_rebuilt();
   for (size_t i = 0; i < ops_.size(); ++i) {
     const Op& op = ops_[i];
-    zero_starting(starts_fwd_[i], nb);
-    if (!op_active_.empty() && !op_active_[i]) continue;   // no output carries a derivative
+    const bool runs = op_active_.empty() || op_active_[i];
+    for (int k : starts_fwd_[i])
+      if (!runs || !writes_whole(op, k)) zero_intermediate(k, nb);
+    if (!runs) continue;                  // no output carries a derivative
     unpin_all();
     if (op.kind == GEMM) {
       tangent_gemm(op.g, prec, nb);
@@ -811,86 +863,83 @@ void Tape::tangent(Prec prec, int64_t nb) {
                          deriv(op.y), dstride(op.y), nb, prec);
       continue;
     }
-    for (int64_t k = 0; k < nb; ++k) {
-      switch (op.kind) {
-        case SORT4: {
-          double* dy = D(op.y, k);
-          const double* dx = D(op.x, k);
-          if (dx) etg::sort4(s, dx, op.d, op.perm, dy, op.alpha, op.beta);
-          else scale(s, dy, dense_size(op.d), op.beta);
-          break;
-        }
-        case SQUAREUP: {
-          const double* dp = D(op.x, k);
-          double* df = D(op.y, k);
-          if (dp) etg::squareup(s, dp, df, op.N);
-          else fill(s, df, op.N * op.N, 0.0);
-          break;
-        }
-        case PACKIN: {
-          const double* df = D(op.x, k);
-          double* dp = D(op.y, k);
-          if (df) etg::packin(s, df, dp, op.N, op.alpha, op.beta, op.diag);
-          else scale(s, dp, op.N * (op.N + 1) / 2, op.beta);
-          break;
-        }
-        case SYMSUM: {
-          const double* dx = D(op.x, k);
-          double* dy = D(op.y, k);
-          if (dx) etg::symmetric_sum(s, dx, dy, op.N);
-          else fill(s, dy, op.N * op.N, 0.0);
-          break;
-        }
-        case SYMPACK: {
-          const double* dx = D(op.x, k);
-          if (dx) etg::symmetrize_and_pack(s, dx, D(op.y, k), op.nv, op.no, op.alpha, op.f1, op.f2);
-          break;
-        }
-        case COPY_SUB: {
-          const double* dsrc = D(op.x, k);
-          double* ddst = D(op.y, k);
-          if (dsrc) etg::copy_sub(s, dsrc, op.lds, ddst, op.ldd, op.m, op.n, op.alpha, op.beta);
-          else etg::copy_sub(s, ddst, op.ldd, ddst, op.ldd, op.m, op.n, 0.0, op.beta);
-          break;
-        }
-        case FILL0:
-          fill(s, D(op.y, k), op.n, 0.0);
-          break;
-        case T1_XY:
-          etg::t1_xy(s, D(op.x, k), D(op.y, k), D(op.y2, k), wf_.n_o, wf_.n_v, 0.0);
-          break;
-        case TRACE_OO: {
-          const double* dL = D(op.x, k);
-          if (dL) etg::trace_oo(s, dL, D(op.y, k), wf_.n_J, wf_.n_o);
-          else fill(s, D(op.y, k), wf_.n_J, 0.0);
-          break;
-        }
-        case FOCK_OV_VEC:
-          etg::fock_ov_vector(s, D(op.x, k), D(op.y, k), wf_.n_o, wf_.n_v);
-          break;
-        case GEMM:
-        case LADDER:
-          break;
-      }
+    const double* dx = op.x ? deriv(op.x) : nullptr;
+    double* dy = deriv(op.y);
+    const Batch b{nb, op.x ? dstride(op.x) : 0, dstride(op.y)};
+    switch (op.kind) {
+      case SORT4:
+        if (dx) etg::sort4(s, dx, op.d, op.perm, dy, op.alpha, op.beta, b);
+        else scale_vectors(dy, dense_size(op.d), b.y, nb, op.beta);
+        break;
+      case SQUAREUP:
+        if (dx) etg::squareup(s, dx, dy, op.N, b);
+        else scale_vectors(dy, op.N * op.N, b.y, nb, 0.0);
+        break;
+      case PACKIN:
+        if (dx) etg::packin(s, dx, dy, op.N, op.alpha, op.beta, op.diag, b);
+        else scale_vectors(dy, op.N * (op.N + 1) / 2, b.y, nb, op.beta);
+        break;
+      case SYMSUM:
+        if (dx) etg::symmetric_sum(s, dx, dy, op.N, b);
+        else scale_vectors(dy, op.N * op.N, b.y, nb, 0.0);
+        break;
+      case SYMPACK:
+        if (dx) etg::symmetrize_and_pack(s, dx, dy, op.nv, op.no, op.alpha, op.f1, op.f2, b);
+        break;
+      case COPY_SUB:
+        if (dx) etg::copy_sub(s, dx, op.lds, dy, op.ldd, op.m, op.n, op.alpha, op.beta, b);
+        else etg::copy_sub(s, dy, op.ldd, dy, op.ldd, op.m, op.n, 0.0, op.beta, Batch{nb, b.y, b.y});
+        break;
+      case FILL0:
+        scale_vectors(dy, op.n, b.y, nb, 0.0);
+        break;
+      case T1_XY:
+        etg::t1_xy(s, dx, dy, deriv(op.y2), wf_.n_o, wf_.n_v, 0.0, b);
+        break;
+      case TRACE_OO:
+        if (dx) etg::trace_oo(s, dx, dy, wf_.n_J, wf_.n_o, b);
+        else scale_vectors(dy, wf_.n_J, b.y, nb, 0.0);
+        break;
+      case FOCK_OV_VEC:
+        etg::fock_ov_vector(s, dx, dy, wf_.n_o, wf_.n_v, b);
+        break;
+      case GEMM:
+      case LADDER:
+        break;
     }
   }
 }
 
+// The first n elements of nb vectors at stride, times beta (0 stores zeroes).
+void Tape::scale_vectors(double* x, int64_t n, int64_t stride, int64_t nb, double beta) {
+  if (n == stride || nb == 1) {
+    scale(wf_.stream(), x, nb * n, beta);
+    return;
+  }
+  for (int64_t k = 0; k < nb; ++k) scale(wf_.stream(), x + k * stride, n, beta);
+}
+
 void Tape::adjoint(Prec prec, int64_t nb) {
   hipStream_t s = wf_.stream();
-  auto D = [&](const double* p, int64_t k) -> double* {
-    double* d = deriv(p);
-    return d ? d + k * dstride(p) : nullptr;
-  };
   plan_derivatives();
   reset_rebuilt();
   for (size_t i = ops_.size(); i-- > 0;) {
     const Op& op = ops_[i];
-    zero_starting(starts_bwd_[i], nb);
-    if (!op_active_.empty() && !op_active_[i]) continue;   // no output carries a derivative
+    const bool runs = op_active_.empty() || op_active_[i];
+    std::vector<int> fresh;               // start with this operation's own contribution
+    for (int k : starts_bwd_[i]) {
+      if (runs && adjoint_writes_whole(op, k)) fresh.push_back(k);
+      else zero_intermediate(k, nb);
+    }
+    if (!runs) continue;                  // no output carries a derivative
+    // an output whose lifetime begins with this operation is not read again
+    auto ends = [&](const double* p) {
+      const Buf& b = *bufs_[size_t(find(p))];
+      return b.intermediate && b.first == int(i);
+    };
     unpin_all();
     if (op.kind == GEMM) {
-      adjoint_gemm(op.g, prec, nb);
+      adjoint_gemm(op.g, prec, nb, fresh, ends(op.g.C));
       continue;
     }
     if (op.kind == LADDER) {
@@ -898,87 +947,67 @@ void Tape::adjoint(Prec prec, int64_t nb) {
                          deriv(op.y), dstride(op.y), nb, prec);
       continue;
     }
-    for (int64_t k = 0; k < nb; ++k) {
-      switch (op.kind) {
-        case SORT4: {
-          double* yb = D(op.y, k);
-          double* xb = D(op.x, k);
-          if (xb) {
-            int64_t e[4];
-            char inv[5] = {0, 0, 0, 0, 0};
-            for (int q = 0; q < 4; ++q) {
-              const int r = op.perm[q] - '1';
-              e[q] = op.d[r];
-              inv[r] = char('1' + q);
-            }
-            etg::sort4(s, yb, e, inv, xb, op.alpha, 1.0);
+    double* xb = op.x ? deriv(op.x) : nullptr;
+    double* yb = deriv(op.y);
+    const int64_t sx = op.x ? dstride(op.x) : 0, sy = dstride(op.y);
+    const Batch b{nb, sy, sx};
+    const bool y_ends = ends(op.y);
+    const double acc = fresh.empty() ? 1.0 : 0.0;
+    switch (op.kind) {
+      case SORT4:
+        if (xb) {
+          int64_t e[4];
+          char inv[5] = {0, 0, 0, 0, 0};
+          for (int q = 0; q < 4; ++q) {
+            const int r = op.perm[q] - '1';
+            e[q] = op.d[r];
+            inv[r] = char('1' + q);
           }
-          scale(s, yb, dense_size(op.d), op.beta);
-          break;
+          etg::sort4(s, yb, e, inv, xb, op.alpha, acc, b);
         }
-        case SQUAREUP: {
-          double* pb = D(op.x, k);
-          double* fb = D(op.y, k);
-          if (pb) packsum(s, fb, pb, op.N);
-          fill(s, fb, op.N * op.N, 0.0);
-          break;
-        }
-        case PACKIN: {
-          double* fb = D(op.x, k);
-          double* pb = D(op.y, k);
-          if (fb) unpack_upper_add(s, pb, fb, op.N, op.alpha, op.diag);
-          scale(s, pb, op.N * (op.N + 1) / 2, op.beta);
-          break;
-        }
-        case SYMSUM: {
-          double* xb = D(op.x, k);
-          double* yb = D(op.y, k);
-          if (xb) symmetric_sum_acc(s, yb, xb, op.N, 1.0);
-          fill(s, yb, op.N * op.N, 0.0);
-          break;
-        }
-        case SYMPACK: {
-          double* xb = D(op.x, k);
-          if (xb) symmetrize_and_pack_adjoint(s, D(op.y, k), xb, op.nv, op.no, op.alpha, op.f1, op.f2);
-          break;
-        }
-        case COPY_SUB: {
-          double* sb = D(op.x, k);
-          double* db = D(op.y, k);
-          if (sb) etg::copy_sub(s, db, op.ldd, sb, op.lds, op.m, op.n, op.alpha, 1.0);
-          etg::copy_sub(s, db, op.ldd, db, op.ldd, op.m, op.n, 0.0, op.beta);
-          break;
-        }
-        case FILL0:
-          fill(s, D(op.y, k), op.n, 0.0);
-          break;
-        case T1_XY: {
-          double* tb = D(op.x, k);
-          double* Xb = D(op.y, k);
-          double* Yb = D(op.y2, k);
-          if (tb) t1_xy_adjoint(s, Xb, Yb, tb, wf_.n_o, wf_.n_v);
-          fill(s, Xb, wf_.n_mo * wf_.n_mo, 0.0);
-          fill(s, Yb, wf_.n_mo * wf_.n_mo, 0.0);
-          break;
-        }
-        case TRACE_OO: {
-          double* Lb = D(op.x, k);
-          double* Xb = D(op.y, k);
-          if (Lb) trace_oo_adjoint(s, Xb, Lb, wf_.n_J, wf_.n_o);
-          fill(s, Xb, wf_.n_J, 0.0);
-          break;
-        }
-        case FOCK_OV_VEC: {
-          double* Fb = D(op.x, k);
-          double* fb = D(op.y, k);
-          if (Fb) fock_ov_vector_adjoint(s, fb, Fb, wf_.n_o, wf_.n_v);
-          fill(s, fb, wf_.n_o * wf_.n_v, 0.0);
-          break;
-        }
-        case GEMM:
-        case LADDER:
-          break;
+        if (!y_ends) scale_vectors(yb, dense_size(op.d), sy, nb, op.beta);
+        break;
+      case SQUAREUP:
+        if (xb) packsum(s, yb, xb, op.N, b);
+        if (!y_ends) scale_vectors(yb, op.N * op.N, sy, nb, 0.0);
+        break;
+      case PACKIN:
+        if (xb) unpack_upper_add(s, yb, xb, op.N, op.alpha, op.diag, b);
+        if (!y_ends) scale_vectors(yb, op.N * (op.N + 1) / 2, sy, nb, op.beta);
+        break;
+      case SYMSUM:
+        if (xb) symmetric_sum_acc(s, yb, xb, op.N, acc, b);
+        if (!y_ends) scale_vectors(yb, op.N * op.N, sy, nb, 0.0);
+        break;
+      case SYMPACK:
+        if (xb) symmetrize_and_pack_adjoint(s, yb, xb, op.nv, op.no, op.alpha, op.f1, op.f2, fresh.empty(), b);
+        break;
+      case COPY_SUB:
+        if (xb) etg::copy_sub(s, yb, op.ldd, xb, op.lds, op.m, op.n, op.alpha, acc, b);
+        if (!y_ends && op.beta != 1.0)
+          etg::copy_sub(s, yb, op.ldd, yb, op.ldd, op.m, op.n, 0.0, op.beta, Batch{nb, sy, sy});
+        break;
+      case FILL0:
+        if (!y_ends) scale_vectors(yb, op.n, sy, nb, 0.0);
+        break;
+      case T1_XY: {
+        double* Yb = deriv(op.y2);
+        if (xb) t1_xy_adjoint(s, yb, Yb, xb, wf_.n_o, wf_.n_v, Batch{nb, sx, sy});
+        if (!y_ends) scale_vectors(yb, wf_.n_mo * wf_.n_mo, sy, nb, 0.0);
+        if (!ends(op.y2)) scale_vectors(Yb, wf_.n_mo * wf_.n_mo, dstride(op.y2), nb, 0.0);
+        break;
       }
+      case TRACE_OO:
+        if (xb) trace_oo_adjoint(s, yb, xb, wf_.n_J, wf_.n_o, b);
+        if (!y_ends) scale_vectors(yb, wf_.n_J, sy, nb, 0.0);
+        break;
+      case FOCK_OV_VEC:
+        if (xb) fock_ov_vector_adjoint(s, yb, xb, wf_.n_o, wf_.n_v, b);
+        if (!y_ends) scale_vectors(yb, wf_.n_o * wf_.n_v, sy, nb, 0.0);
+        break;
+      case GEMM:
+      case LADDER:
+        break;
     }
   }
 }

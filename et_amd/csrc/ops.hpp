@@ -159,7 +159,7 @@ class Tape : public DirectOps {
   const double* primal(const double* p);
   // Zeroes the first nb derivative vectors of the buffers that exist outside
   // the tape (allocating on first use); the passes zero each intermediate's
-  // derivative where its lifetime starts.
+  // derivative where its lifetime starts, unless the operation there writes all of it.
   void zero_derivatives(int64_t nb = 1);
   // Derivative buffer matching a primal pointer (nullptr for constants), vector 0.
   double* deriv(const double* p);
@@ -229,9 +229,12 @@ class Tape : public DirectOps {
   uint64_t rclock_ = 0;
   bool finalized_ = false;
   void tangent_gemm(const Gemm& g, Prec prec, int64_t nb);
-  void adjoint_gemm(const Gemm& g, Prec prec, int64_t nb);
+  void adjoint_gemm(const Gemm& g, Prec prec, int64_t nb, const std::vector<int>& fresh, bool c_ends);
   void plan_derivatives();
-  void zero_starting(const std::vector<int>& bufs, int64_t nb);
+  void zero_intermediate(int k, int64_t nb);
+  void scale_vectors(double* x, int64_t n, int64_t stride, int64_t nb, double beta);
+  bool writes_whole(const Op& op, int k) const;
+  bool adjoint_writes_whole(const Op& op, int k) const;
   std::vector<Op> ops_;
   std::vector<std::unique_ptr<Buf>> bufs_;
   std::map<std::string, DeviceBuffer> named_;
