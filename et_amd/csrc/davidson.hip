@@ -13,17 +13,19 @@
 // cc_es_amplitudes_solver_factory_class.F90:307), linear-dependence threshold
 // min(1e-11, 0.1 threshold) (:315).
 //
-// The reduced eigenproblem (non-symmetric, dimension <= 128) is solved by one
-// wavefront: Householder reduction to upper Hessenberg form, the implicitly
-// double-shifted QR iteration for the eigenvalues (francis.hpp), then inverse
-// iteration on G - w I with a partially pivoted LU for the wanted eigenvectors
-// (for a complex pair a +- ib, the real 2k system of u + i v).  Complex pairs are carried as (u, v) column pairs with
-// real and imaginary residuals, as eT's Davidson tool does.
+// The reduced eigenproblem (non-symmetric, dimension <= 128): one wavefront does
+// the Householder reduction to upper Hessenberg form and the implicitly double-
+// shifted QR iteration for the eigenvalues (francis.hpp), then one wavefront per
+// wanted real root the inverse iteration on G - w I with a partially pivoted LU
+// (for a complex pair a +- ib, the real 2k system of u + i v).  Complex pairs are
+// carried as (u, v) column pairs with real and imaginary residuals, as eT's
+// Davidson tool does.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -40,11 +42,72 @@ constexpr int kLanes = 64;
 
 __device__ inline double sgn(double a, double b) { return b >= 0.0 ? fabs(a) : -fabs(a); }
 
+// Adds (or takes the larger of) each lane's value and that of the lane that the
+// DPP control names; lanes outside the row mask and past the row's edge add 0.
+template <int kCtrl, int kRows>
+__device__ inline double dpp_add(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(u)), kCtrl, kRows, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(u >> 32), kCtrl, kRows, 0xf, true);
+  return v + __builtin_bit_cast(double, (uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
+}
+template <int kCtrl, int kRows>
+__device__ inline uint32_t dpp_max(uint32_t v) {
+  return max(v, uint32_t(__builtin_amdgcn_update_dpp(0, int(v), kCtrl, kRows, 0xf, true)));
+}
+
+// Lane `from`'s value (from is the same in every lane).
+__device__ inline double lane_value(double v, int from) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), from));
+  const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(u >> 32), from));
+  return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+
+// Sum / largest over the wavefront, in every lane.  Six DPP steps: a shuffle
+// through LDS costs a round trip per step, and these reductions sit in the
+// middle of serial chains.
+__device__ inline double wave_sum(double v) {
+  v = dpp_add<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8: lane 15 of each row of 16 has the row's sum
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
+  return lane_value(v, kLanes - 1);
+}
+__device__ inline uint32_t wave_max(uint32_t v) {
+  v = dpp_max<0x111, 0xf>(v);
+  v = dpp_max<0x112, 0xf>(v);
+  v = dpp_max<0x114, 0xf>(v);
+  v = dpp_max<0x118, 0xf>(v);
+  v = dpp_max<0x142, 0xa>(v);
+  v = dpp_max<0x143, 0xc>(v);
+  return uint32_t(__builtin_amdgcn_readlane(int(v), kLanes - 1));
+}
+
+// Orders the memory accesses of one wavefront: they execute in program order, so
+// only the compiler has to keep it.
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The reduced eigensolver's team: one wavefront.
 struct WaveTeam {
   __device__ int rank() const { return int(threadIdx.x); }
   __device__ int size() const { return kLanes; }
-  __device__ void sync() const { __syncthreads(); }
+  __device__ void sync() const { wave_sync(); }
+  __device__ double sum(double v) const { return wave_sum(v); }
+  template <class F>
+  __device__ int highest(int top, F f) const {
+    for (; top > 0; top -= kLanes) {
+      const int l = top - rank();
+      const uint64_t hit = __ballot(l > 0 && f(l));
+      if (hit != 0) return top - __builtin_ctzll(hit);
+    }
+    return 0;
+  }
 };
 
 // H(i, j) of the k x k working matrix in LDS, column-major with the odd leading
@@ -52,246 +115,338 @@ struct WaveTeam {
 constexpr int kLdH = kMaxRed + 1;
 #define HH(i, j) H[(i) + (j) * kLdH]
 
-// Inverse iteration on the nm x nm matrix M (ld ldm; LDS or global): LU with
-// partial pivoting in place, then three solves M y = y starting from a fixed
-// pattern, each normalised to unit 2-norm (largest component positive).  For
-// real roots M = G - (w + d) I; for a complex pair a +- ib the real 2k system
-// [[G - a I, b I], [-b I, G - a I]] acting on [u; v] (eigenvector u + i v).
-__device__ void inverse_iteration(double* M, int ldm, int nm, double anorm, int* piv, double* y,
+// G - shift I into LDS, eight columns per round: their global loads are in flight together.
+__device__ void load_shifted(double* H, const double* __restrict__ G, int k, int64_t ldg, double shift) {
+  for (int i = threadIdx.x; i < k; i += kLanes)
+    for (int j0 = 0; j0 < k; j0 += 8) {
+      double g[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) g[u] = j0 + u < k ? G[i + (j0 + u) * ldg] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (j0 + u < k) HH(i, j0 + u) = g[u] - (i == j0 + u ? shift : 0.0);
+    }
+  wave_sync();
+}
+
+// Inverse iteration on the nm x nm matrix M (ld ldm; LDS or global; nm at most
+// 64 kRows): LU with partial pivoting in place, then three solves M y = y
+// starting from a fixed pattern, each normalised to unit 2-norm (largest
+// component positive).  Row i of y is yv[i / 64] of lane i % 64; perm holds the
+// row order of the pivoting.  For real roots M = G - (w + d) I; for a complex
+// pair a +- ib the real 2k system [[G - a I, b I], [-b I, G - a I]] acting on
+// [u; v] (eigenvector u + i v).
+//
+// One dependent chain: what costs is the latency of each of its steps.  The
+// solves keep y in registers and broadcast one element per column by readlane
+// (the columns of M do not depend on it and are read ahead), the pivot is the
+// largest high word (20 bits of the mantissa: as stable as the largest value).
+template <int kRows>
+__device__ void inverse_iteration(double* M, int ldm, int nm, double anorm, int* perm, double (&yv)[kRows],
                                   int seed, int lane) {
 #define MM(i, j) M[(i) + (j) * ldm]
+  for (int i = lane; i < nm; i += kLanes) perm[i] = i;
+  wave_sync();
   for (int c = 0; c < nm; ++c) {
-    // pivot: the first row of largest magnitude, found across the lanes (each
-    // lane scans every kLanes-th row, then the wave keeps the larger value and,
-    // on a tie, the smaller row)
-    int p = c;
-    double best = fabs(MM(c, c));
-    for (int r = c + 1 + lane; r < nm; r += kLanes) {
-      const double v = fabs(MM(r, c));
-      if (v > best) {
-        best = v;
-        p = r;
+    uint32_t key = 0;
+    int row = c;
+    for (int r = c + lane; r < nm; r += kLanes) {
+      const uint32_t v = uint32_t(__builtin_bit_cast(uint64_t, MM(r, c)) >> 32) & 0x7fffffffu;
+      if (v > key) {
+        key = v;
+        row = r;
       }
     }
-    for (int off = kLanes / 2; off > 0; off >>= 1) {
-      const double ob = __shfl_xor(best, off, kLanes);
-      const int op = __shfl_xor(p, off, kLanes);
-      if (ob > best || (ob == best && op < p)) {
-        best = ob;
-        p = op;
-      }
-    }
-    __syncthreads();
-    if (lane == 0) {
-      piv[c] = p;
-      if (MM(p, c) == 0.0) MM(p, c) = 1e-300 + 1e-16 * anorm;
-    }
-    __syncthreads();
-    if (p != c)
+    const uint32_t top = wave_max(key);
+    const int p = top == 0 ? c : __builtin_amdgcn_readlane(row, __builtin_ctzll(__ballot(key == top)));
+    if (p != c) {
       for (int j = lane; j < nm; j += kLanes) {
         const double tmp = MM(c, j);
         MM(c, j) = MM(p, j);
         MM(p, j) = tmp;
       }
-    __syncthreads();
-    const double d = MM(c, c);
-    for (int r = c + 1 + lane; r < nm; r += kLanes) {
+      if (lane == 0) {
+        const int tmp = perm[c];
+        perm[c] = perm[p];
+        perm[p] = tmp;
+      }
+      wave_sync();
+    }
+    double d = MM(c, c);
+    if (d == 0.0) {
+      d = 1e-300 + 1e-16 * anorm;
+      wave_sync();
+      if (lane == 0) MM(c, c) = d;
+    }
+    // rows across the lanes; at most half a wavefront of them: two lanes per row,
+    // each with every other column
+    const int rows = nm - c - 1;
+    const int step = rows <= kLanes / 2 ? 2 : 1;
+    const int first = step == 2 ? lane % (kLanes / 2) : lane, half = step == 2 ? lane / (kLanes / 2) : 0;
+    for (int r = c + 1 + first; r < nm; r += kLanes) {
       const double f = MM(r, c) / d;
-      MM(r, c) = f;
       // four columns per round: their loads go out before the stores
-      int j = c + 1;
-      for (; j + 4 <= nm; j += 4) {
-        const double p0 = MM(c, j), p1 = MM(c, j + 1), p2 = MM(c, j + 2), p3 = MM(c, j + 3);
-        const double a0 = MM(r, j), a1 = MM(r, j + 1), a2 = MM(r, j + 2), a3 = MM(r, j + 3);
+      int j = c + 1 + half;
+      for (; j + 3 * step < nm; j += 4 * step) {
+        const double p0 = MM(c, j), p1 = MM(c, j + step), p2 = MM(c, j + 2 * step), p3 = MM(c, j + 3 * step);
+        const double a0 = MM(r, j), a1 = MM(r, j + step), a2 = MM(r, j + 2 * step), a3 = MM(r, j + 3 * step);
         MM(r, j) = a0 - f * p0;
-        MM(r, j + 1) = a1 - f * p1;
-        MM(r, j + 2) = a2 - f * p2;
-        MM(r, j + 3) = a3 - f * p3;
+        MM(r, j + step) = a1 - f * p1;
+        MM(r, j + 2 * step) = a2 - f * p2;
+        MM(r, j + 3 * step) = a3 - f * p3;
       }
-      for (; j < nm; ++j) MM(r, j) -= f * MM(c, j);
+      for (; j < nm; j += step) MM(r, j) -= f * MM(c, j);
+      wave_sync();                                       // both lanes of the row have read MM(r, c)
+      if (half == 0) MM(r, c) = f;
     }
-    __syncthreads();
+    wave_sync();
   }
-  for (int i = lane; i < nm; i += kLanes) y[i] = 1.0 + 0.01 * ((i * 7 + seed * 3) % 11);
-  __syncthreads();
+  double rd[kRows];                                      // 1 / diagonal
+  int src[kRows];
+#pragma unroll
+  for (int s = 0; s < kRows; ++s) {
+    const int i = lane + s * kLanes;
+    rd[s] = i < nm ? 1.0 / MM(i, i) : 0.0;
+    src[s] = i < nm ? perm[i] : i;
+    yv[s] = i < nm ? 1.0 + 0.01 * ((i * 7 + seed * 3) % 11) : 0.0;
+  }
+  auto element = [&](const double (&v)[kRows], int c) {  // element c of a vector, to all lanes
+    double e = v[0];
+#pragma unroll
+    for (int s = 1; s < kRows; ++s)
+      if (c / kLanes == s) e = v[s];
+    return lane_value(e, c % kLanes);
+  };
   for (int iter = 0; iter < 3; ++iter) {
-    if (lane == 0)
-      for (int c = 0; c < nm; ++c) {
-        const int p = piv[c];
-        const double tmp = y[c];
-        y[c] = y[p];
-        y[p] = tmp;
+    double t[kRows];
+#pragma unroll
+    for (int s = 0; s < kRows; ++s) {                    // y in the pivots' order
+      t[s] = 0.0;
+#pragma unroll
+      for (int u = 0; u < kRows; ++u) {
+        const double v = __shfl(yv[u], src[s] % kLanes, kLanes);
+        if (src[s] / kLanes == u) t[s] = v;
       }
-    __syncthreads();
-    // triangular solves column by column, the updates of each column across the lanes
-    for (int c = 0; c < nm; ++c) {                     // unit lower L
-      const double yc = y[c];
-      for (int r = c + 1 + lane; r < nm; r += kLanes) y[r] -= MM(r, c) * yc;
-      __syncthreads();
     }
-    for (int c = nm - 1; c >= 0; --c) {                // upper U
-      const double yc = y[c] / MM(c, c);
-      for (int r = lane; r < c; r += kLanes) y[r] -= MM(r, c) * yc;
-      __syncthreads();
-      if (lane == 0) y[c] = yc;
-      __syncthreads();
+    // triangular solves column by column, four columns' entries read ahead
+    for (int c0 = 0; c0 < nm; c0 += 4) {                 // unit lower L
+      double m[4][kRows];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < kRows; ++s) {
+          const int i = lane + s * kLanes;
+          m[q][s] = c0 + q < nm && i > c0 + q && i < nm ? MM(i, c0 + q) : 0.0;
+        }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (c0 + q < nm) {
+          const double yc = element(t, c0 + q);
+#pragma unroll
+          for (int s = 0; s < kRows; ++s) t[s] -= m[q][s] * yc;
+        }
     }
-    if (lane == 0) {
-      double nrm = 0.0, big = 0.0;
-      int ib = 0;
-      for (int i = 0; i < nm; ++i) {
-        nrm += y[i] * y[i];
-        if (fabs(y[i]) > big) { big = fabs(y[i]); ib = i; }
+    for (int c0 = nm - 1; c0 >= 0; c0 -= 4) {            // upper U
+      double m[4][kRows];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < kRows; ++s) {
+          const int i = lane + s * kLanes;
+          m[q][s] = i < c0 - q ? MM(i, c0 - q) : 0.0;
+        }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (c0 - q >= 0) {
+          const int c = c0 - q;
+          const double yc = element(t, c) * element(rd, c);
+#pragma unroll
+          for (int s = 0; s < kRows; ++s) t[s] = lane + s * kLanes == c ? yc : t[s] - m[q][s] * yc;
+        }
+    }
+    double sq = 0.0, big = 0.0;
+    int ib = 0;
+#pragma unroll
+    for (int s = 0; s < kRows; ++s) {
+      sq += t[s] * t[s];
+      if (fabs(t[s]) > big) {
+        big = fabs(t[s]);
+        ib = lane + s * kLanes;
       }
-      nrm = sqrt(nrm);
-      const double sg = y[ib] < 0.0 ? -1.0 : 1.0;
-      for (int i = 0; i < nm; ++i) y[i] = sg * y[i] / nrm;
     }
-    __syncthreads();
+    const double nrm = sqrt(wave_sum(sq));
+    for (int off = kLanes / 2; off > 0; off >>= 1) {     // the first of the largest components
+      const double ob = __shfl_xor(big, off, kLanes);
+      const int oi = __shfl_xor(ib, off, kLanes);
+      if (ob > big || (ob == big && oi < ib)) {
+        big = ob;
+        ib = oi;
+      }
+    }
+    const double sg = element(t, __builtin_amdgcn_readfirstlane(ib)) < 0.0 ? -1.0 : 1.0;
+#pragma unroll
+    for (int s = 0; s < kRows; ++s) yv[s] = sg * t[s] / nrm;
   }
 #undef MM
 }
 
-__global__ __launch_bounds__(kLanes) void reduced_eigen_kernel(const double* __restrict__ G, int k,
-                                                               int ldg, int n_want,
-                                                               double* __restrict__ wr_out,
-                                                               double* __restrict__ wi_out,
-                                                               double* __restrict__ X, int ldx,
-                                                               double* __restrict__ work,
-                                                               int* __restrict__ info) {
+// Eigenvalues, ordered by real part then imaginary part, the matrix's norm and
+// the status (1: no convergence).  One wavefront, bound by its chain of dependent
+// steps (about 0.6 us per step of the bulge chase).  With the vectors' kernel, for
+// 4 roots: 95 us at k = 10, 0.27 ms at 20, 0.97 at 40, 6.7 at 100; as one kernel
+// with two barriers and two round trips through LDS per step, and the roots one
+// after another: 0.20, 0.54, 1.70 and 9.8 ms.
+__global__ __launch_bounds__(kLanes) void reduced_eigenvalues_kernel(const double* __restrict__ G, int k,
+                                                                     int ldg, double* __restrict__ wr_out,
+                                                                     double* __restrict__ wi_out,
+                                                                     double* __restrict__ norm_out,
+                                                                     int* __restrict__ info) {
   __shared__ double H[kLdH * kMaxRed];
-  __shared__ double wr[kMaxRed], wi[kMaxRed], ort[kMaxRed], y[2 * kMaxRed];
-  __shared__ int order[kMaxRed], piv[2 * kMaxRed];
-  __shared__ int status;
+  __shared__ double wr[kMaxRed], wi[kMaxRed], ort[kMaxRed];
   const int lane = threadIdx.x;
-  if (lane == 0) status = 0;
-  for (int q = lane; q < k * k; q += kLanes) HH(q % k, q / k) = G[q % k + (q / k) * int64_t(ldg)];
-  __syncthreads();
+  load_shifted(H, G, k, ldg, 0.0);
 
   // ---- Householder reduction to upper Hessenberg form (orthes) ----
   for (int m = 1; m < k - 1; ++m) {
-    double scale = 0.0;
-    for (int i = m; i < k; ++i) scale += fabs(HH(i, m - 1));
+    const int i0 = m + lane, i1 = i0 + kLanes;
+    const double u0 = i0 < k ? HH(i0, m - 1) : 0.0, u1 = i1 < k ? HH(i1, m - 1) : 0.0;
+    const double scale = wave_sum(fabs(u0) + fabs(u1));
     if (scale == 0.0) continue;
-    double h = 0.0;
-    for (int i = m; i < k; ++i) {
-      const double u = HH(i, m - 1) / scale;
-      h += u * u;
+    const double s0 = u0 / scale, s1 = u1 / scale;
+    double h = wave_sum(s0 * s0 + s1 * s1);
+    const double x = lane_value(s0, 0);                  // the entry that stays
+    const double g = -sgn(sqrt(h), x);
+    h -= x * g;
+    if (i0 < k) {
+      ort[i0] = s0 - (lane == 0 ? g : 0.0);
+      HH(i0, m - 1) = lane == 0 ? scale * g : 0.0;
     }
-    const double g = -sgn(sqrt(h), HH(m, m - 1));
-    h -= HH(m, m - 1) / scale * g;
-    __syncthreads();
-    for (int i = m + lane; i < k; i += kLanes) ort[i] = HH(i, m - 1) / scale - (i == m ? g : 0.0);
-    __syncthreads();
-    for (int j = m + lane; j < k; j += kLanes) {           // (I - u u^T / h) H
-      double f = 0.0;
-      for (int i = m; i < k; ++i) f += ort[i] * HH(i, j);
-      f /= h;
-      for (int i = m; i < k; ++i) HH(i, j) -= f * ort[i];
+    if (i1 < k) {
+      ort[i1] = s1;
+      HH(i1, m - 1) = 0.0;
     }
-    __syncthreads();
-    for (int i = lane; i < k; i += kLanes) {               // H (I - u u^T / h)
-      double f = 0.0;
-      for (int j = m; j < k; ++j) f += ort[j] * HH(i, j);
-      f /= h;
-      for (int j = m; j < k; ++j) HH(i, j) -= f * ort[j];
+    wave_sync();
+    const double rh = 1.0 / h;
+    // (I - u u^T / h) H: a column per lane, then H (I - u u^T / h): a row per lane
+    for (int side = 0; side < 2; ++side) {
+      const int st = side == 0 ? 1 : kLdH;
+      for (int q = (side == 0 ? m : 0) + lane; q < k; q += kLanes) {
+        double* p = side == 0 ? &HH(0, q) : &HH(q, 0);
+        double f[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int i = m; i < k; i += 4)
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (i + u < k) f[u] += ort[i + u] * p[(i + u) * st];
+        const double w = ((f[0] + f[1]) + (f[2] + f[3])) * rh;
+        for (int i = m; i < k; i += 4) {
+          double v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = i + u < k ? p[(i + u) * st] - w * ort[i + u] : 0.0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (i + u < k) p[(i + u) * st] = v[u];
+        }
+      }
+      wave_sync();
     }
-    __syncthreads();
-    for (int i = m + lane; i < k; i += kLanes) HH(i, m - 1) = (i == m) ? scale * g : 0.0;
-    __syncthreads();
   }
 
   // ---- eigenvalues of the Hessenberg matrix (implicit double-shift QR) ----
   double anorm = 0.0;
-  {
-    const int st = francis::hessenberg_eigenvalues(WaveTeam(), H, kLdH, k, wr, wi, &anorm);
-    if (lane == 0 && st != 0) status = st;
-  }
-  __syncthreads();
-
-  // ---- order by real part ----
+  const int st = francis::hessenberg_eigenvalues(WaveTeam(), H, kLdH, k, wr, wi, &anorm);
   if (lane == 0) {
-    for (int i = 0; i < k; ++i) order[i] = i;
-    for (int i = 1; i < k; ++i) {
-      const int o = order[i];
-      int j = i - 1;
-      while (j >= 0 && (wr[order[j]] > wr[o] || (wr[order[j]] == wr[o] && wi[order[j]] > wi[o]))) {
-        order[j + 1] = order[j];
-        --j;
-      }
-      order[j + 1] = o;
-    }
-    for (int i = 0; i < k; ++i) {
-      wr_out[i] = wr[order[i]];
-      wi_out[i] = wi[order[i]];
-    }
+    *norm_out = anorm;
+    *info = st;
   }
-  __syncthreads();
+  if (st != 0) return;
+  for (int i = lane; i < k; i += kLanes) {
+    int rank = 0;
+    for (int j = 0; j < k; ++j) {
+      const bool eq = wr[j] == wr[i];
+      rank += wr[j] < wr[i] || (eq && (wi[j] < wi[i] || (wi[j] == wi[i] && j < i)));
+    }
+    wr_out[rank] = wr[i];
+    wi_out[rank] = wi[i];
+  }
+}
 
-  // ---- eigenvectors by inverse iteration ----
-  // Real root: column w.  Complex pair a -+ ib (ordered a - ib first): columns
-  // w and w + 1 hold u and v of the eigenvector u + i v of a + ib.
-  for (int w = 0; w < n_want && status == 0; ++w) {
-    const double lam = wr[order[w]], mu = wi[order[w]];
-    if (mu == 0.0) {
-      const double shift = lam + 1e-13 * fmax(anorm / k, fabs(lam));
-      // eight elements per lane and round: their global loads are in flight together
-      for (int q0 = 0; q0 < k * k; q0 += 8 * kLanes) {
-        double g[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int q = q0 + u * kLanes + lane;
-          g[u] = q < k * k ? G[q % k + (q / k) * int64_t(ldg)] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const int q = q0 + u * kLanes + lane;
-          if (q < k * k) {
-            const int i = q % k, j = q / k;
-            HH(i, j) = g[u] - (i == j ? shift : 0.0);
-          }
-        }
+// Eigenvectors of the n_want lowest roots by inverse iteration.  Real root w:
+// column w of X.  Complex pair a -+ ib (ordered a - ib first): columns w and
+// w + 1 hold u and v of the eigenvector u + i v of a + ib.  Block w < n_want: the
+// real root w with those after it that are numerically the same (each made
+// orthogonal to the earlier ones), unless it belongs to an earlier root; block
+// n_want: the complex pairs, one after another in the one 2k x 2k workspace.
+// Bound by each block's chain of dependent steps: 63 us at k = 40 for 4 roots.
+__global__ __launch_bounds__(kLanes) void reduced_eigenvectors_kernel(
+    const double* __restrict__ G, int k, int ldg, int n_want, const double* __restrict__ wr,
+    const double* __restrict__ wi, const double* __restrict__ norm, const int* __restrict__ info,
+    double* __restrict__ X, int ldx, double* __restrict__ work) {
+  __shared__ double H[kLdH * kMaxRed];
+  __shared__ int perm[2 * kMaxRed];
+  const int lane = threadIdx.x;
+  if (*info != 0) return;
+  const double anorm = *norm;
+  if (int(blockIdx.x) < n_want) {
+    // the same root: within 1e-8; a chain of them is taken with twice that, so that
+    // no two roots that are the same end up in different blocks
+    auto near = [&](int u, int w, double tol) { return fabs(wr[u] - wr[w]) <= tol * fmax(1.0, fabs(wr[w])); };
+    auto after = [&](int w) {                            // next real root, or n_want
+      for (++w; w < n_want && wi[w] != 0.0; ++w) {
       }
-      __syncthreads();
-      inverse_iteration(H, kLdH, k, anorm, piv, y, w, lane);
-      if (lane == 0) {
-        // orthogonal to earlier vectors of (numerically) the same eigenvalue
-        for (int u = 0; u < w; ++u) {
-          if (wi[order[u]] != 0.0 || fabs(wr[order[u]] - lam) > 1e-8 * fmax(1.0, fabs(lam))) continue;
-          double dp = 0.0;
-          for (int i = 0; i < k; ++i) dp += X[i + u * int64_t(ldx)] * y[i];
-          for (int i = 0; i < k; ++i) y[i] -= dp * X[i + u * int64_t(ldx)];
-        }
-        double nrm = 0.0;
-        for (int i = 0; i < k; ++i) nrm += y[i] * y[i];
-        nrm = sqrt(nrm);
-        for (int i = 0; i < k; ++i) y[i] /= nrm;
+      return w;
+    };
+    int w = blockIdx.x;
+    if (wi[w] != 0.0) return;
+    int before = w - 1;
+    while (before >= 0 && wi[before] != 0.0) --before;
+    if (before >= 0 && near(before, w, 2e-8)) return;
+    for (const int head = w;;) {
+      const double lam = wr[w];
+      load_shifted(H, G, k, ldg, lam + 1e-13 * fmax(anorm / k, fabs(lam)));
+      double y[2];
+      inverse_iteration<2>(H, kLdH, k, anorm, perm, y, w, lane);
+      const int i0 = lane, i1 = lane + kLanes;
+      for (int u = head; u < w; ++u) {
+        if (wi[u] != 0.0 || !near(u, w, 1e-8)) continue;
+        const double x0 = i0 < k ? X[i0 + u * int64_t(ldx)] : 0.0, x1 = i1 < k ? X[i1 + u * int64_t(ldx)] : 0.0;
+        const double dp = wave_sum(x0 * y[0] + x1 * y[1]);
+        y[0] -= dp * x0;
+        y[1] -= dp * x1;
       }
-      __syncthreads();
-      for (int i = lane; i < k; i += kLanes) X[i + w * int64_t(ldx)] = y[i];
-      __syncthreads();
-    } else if (mu < 0.0) {
-      const double a = lam + 1e-13 * fmax(anorm / k, fabs(lam)), b = -mu;
-      const int n2 = 2 * k;
-      for (int q = lane; q < n2 * n2; q += kLanes) {
-        const int i = q % n2, j = q / n2;
-        const int bi = i / k, bj = j / k, ii = i % k, jj = j % k;
-        double v;
-        if (bi == bj) v = G[ii + jj * int64_t(ldg)] - (ii == jj ? a : 0.0);
-        else v = (ii == jj) ? (bi == 0 ? b : -b) : 0.0;
-        work[i + int64_t(j) * n2] = v;
-      }
-      __syncthreads();
-      inverse_iteration(work, n2, n2, anorm, piv, y, w, lane);
-      for (int i = lane; i < k; i += kLanes) {
-        X[i + w * int64_t(ldx)] = y[i];
-        if (w + 1 < n_want) X[i + (w + 1) * int64_t(ldx)] = y[k + i];
-      }
-      __syncthreads();
-      ++w;                                  // the partner a + ib is done
+      const double nrm = sqrt(wave_sum(y[0] * y[0] + y[1] * y[1]));
+      if (i0 < k) X[i0 + w * int64_t(ldx)] = y[0] / nrm;
+      if (i1 < k) X[i1 + w * int64_t(ldx)] = y[1] / nrm;
+      const int next = after(w);
+      if (next >= n_want || !near(w, next, 2e-8)) return;
+      w = next;
+      wave_sync();
     }
   }
-  if (lane == 0) *info = status;
+  for (int w = 0; w < n_want; ++w) {
+    const double lam = wr[w], mu = wi[w];
+    if (!(mu < 0.0)) continue;
+    const double a = lam + 1e-13 * fmax(anorm / k, fabs(lam)), b = -mu;
+    const int n2 = 2 * k;
+    for (int q = lane; q < n2 * n2; q += kLanes) {
+      const int i = q % n2, j = q / n2;
+      const int bi = i / k, bj = j / k, ii = i % k, jj = j % k;
+      double v;
+      if (bi == bj) v = G[ii + jj * int64_t(ldg)] - (ii == jj ? a : 0.0);
+      else v = (ii == jj) ? (bi == 0 ? b : -b) : 0.0;
+      work[i + int64_t(j) * n2] = v;
+    }
+    __syncthreads();
+    double y[4];
+    inverse_iteration<4>(work, n2, n2, anorm, perm, y, w, lane);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int i = lane + s * kLanes;
+      if (i < k) X[i + w * int64_t(ldx)] = y[s];
+      else if (i < n2 && w + 1 < n_want) X[i - k + (w + 1) * int64_t(ldx)] = y[s];
+    }
+    __syncthreads();
+    ++w;                                  // the partner a + ib is done
+  }
 }
 #undef HH
 
@@ -331,8 +486,9 @@ __global__ void precondition_kernel(const double* r, const double* __restrict__ 
 namespace {
 
 // Doubles of the reduced eigensolver's device workspace: eigenvalues (2 x 128),
-// the real 2k x 2k systems of complex pairs (4 x 128^2), the status flag.
-constexpr size_t kEigenWork = 2 * kMaxRed + 4 * kMaxRed * kMaxRed + 1;
+// the real 2k x 2k system of a complex pair (4 x 128^2), the matrix's norm, the
+// status flag.
+constexpr size_t kEigenWork = 2 * kMaxRed + 4 * kMaxRed * kMaxRed + 2;
 
 // The same workspace as a file-scope array, for the entry point that allocates
 // nothing (one copy per GPU, 526 KB, held until the process ends).  Host code
@@ -346,18 +502,25 @@ void reduced_eigen_launch(hipStream_t stream, double* base, const double* G_dev,
   if (k < 1 || k > kMaxRed) fail("reduced eigenproblem: dimension must be in [1, 128]");
   if (n_want < 0 || n_want > k) fail("reduced eigenproblem: invalid number of wanted roots");
   if (ldg < k || ldx < k) fail("reduced eigenproblem: leading dimension below the dimension");
-  double* dwr = base;
+  double* dwr = base;                       // wr, wi, norm, status: one copy to the host
   double* dwi = dwr + kMaxRed;
-  double* work = dwi + kMaxRed;             // (2k)^2: complex-pair systems
-  int* dinfo = reinterpret_cast<int*>(work + 4 * kMaxRed * kMaxRed);
-  reduced_eigen_kernel<<<1, kLanes, 0, stream>>>(G_dev, int(k), int(ldg), int(n_want), dwr, dwi, X_dev,
-                                                 int(ldx), work, dinfo);
-  ETG_LAUNCH("reduced_eigen");
-  int info = 0;
-  ETG_HIP(hipMemcpyAsync(wr, dwr, sizeof(double) * k, hipMemcpyDeviceToHost, stream));
-  ETG_HIP(hipMemcpyAsync(wi, dwi, sizeof(double) * k, hipMemcpyDeviceToHost, stream));
-  ETG_HIP(hipMemcpyAsync(&info, dinfo, sizeof(int), hipMemcpyDeviceToHost, stream));
+  double* dnorm = dwi + kMaxRed;
+  int* dinfo = reinterpret_cast<int*>(dnorm + 1);
+  double* work = dnorm + 2;                 // (2k)^2: a complex pair's system
+  reduced_eigenvalues_kernel<<<1, kLanes, 0, stream>>>(G_dev, int(k), int(ldg), dwr, dwi, dnorm, dinfo);
+  ETG_LAUNCH("reduced_eigenvalues");
+  if (n_want > 0) {
+    reduced_eigenvectors_kernel<<<unsigned(n_want + 1), kLanes, 0, stream>>>(
+        G_dev, int(k), int(ldg), int(n_want), dwr, dwi, dnorm, dinfo, X_dev, int(ldx), work);
+    ETG_LAUNCH("reduced_eigenvectors");
+  }
+  double host[2 * kMaxRed + 2];
+  ETG_HIP(hipMemcpyAsync(host, base, sizeof host, hipMemcpyDeviceToHost, stream));
   ETG_HIP(hipStreamSynchronize(stream));
+  std::copy(host, host + k, wr);
+  std::copy(host + kMaxRed, host + kMaxRed + k, wi);
+  int info = 0;
+  std::memcpy(&info, host + 2 * kMaxRed + 1, sizeof info);
   if (info == 1) fail("reduced eigenproblem: QR iteration did not converge");
 }
 

@@ -7,9 +7,15 @@
 //
 // The routine is written once for a team of lanes: on the device the team is
 // one wavefront (64 lanes, scalar control computed redundantly by every lane
-// from the same LDS values, row and column sweeps split across lanes, a
-// barrier between dependent phases); on the host it is one lane with no-op
-// barriers, so the same code is checked against LAPACK from the CPU.
+// from the same LDS values, row and column sweeps split across lanes); on the
+// host it is one lane, so the same code is checked against LAPACK from the CPU.
+//
+// On the device the bulge chase is one chain of dependent steps.  A step's left
+// and right updates meet only in the 3 x 3 block on the diagonal and in the one
+// entry below it; every lane computes these in registers, and the other columns
+// (left only) and rows (right only) are independent of each other.  So a step
+// is one round of reads and one of writes, and the next reflector is made from
+// registers while the writes and reads are under way.
 #pragma once
 
 #include <cmath>
@@ -31,14 +37,14 @@ struct Reflector {
 
 ETG_HD inline Reflector make_reflector(double a0, double a1, double a2, int nr) {
   Reflector r;
-  const double tail = nr == 3 ? std::sqrt(a1 * a1 + a2 * a2) : std::fabs(a1);
-  if (tail == 0.0) {
+  const double tail2 = nr == 3 ? a1 * a1 + a2 * a2 : a1 * a1;
+  if (nr == 3 ? tail2 == 0.0 : a1 == 0.0) {
     r.tau = 0.0;
     r.v1 = r.v2 = 0.0;
     r.alpha = a0;
     return r;
   }
-  const double len = std::sqrt(a0 * a0 + tail * tail);
+  const double len = std::sqrt(a0 * a0 + tail2);
   const double beta = a0 >= 0.0 ? -len : len;            // opposite sign of a0: no cancellation
   r.tau = (beta - a0) / beta;
   const double inv = 1.0 / (a0 - beta);
@@ -70,12 +76,92 @@ ETG_HD inline void block2_eigenvalues(double a, double b, double c, double d, do
   }
 }
 
-// Team of lanes: rank, size, barrier.
+// Team of lanes: rank, size, barrier, the sum of one value per lane, and the
+// highest l in [1, top] with f(l) (0 if there is none).
 struct HostTeam {
   int rank() const { return 0; }
   int size() const { return 1; }
   void sync() const {}
+  double sum(double v) const { return v; }
+  template <class F>
+  int highest(int top, F f) const {
+    while (top > 0 && !f(top)) --top;
+    return top;
+  }
 };
+
+// One step of the bulge chase at column c of the active block lo .. hi: the
+// reflector of (x, y, z) on rows and columns c .. c + kRows - 1.  kBelow: row
+// c + 3 is in the block.  On return (x, y, z) is the next step's column.
+template <int kRows, bool kBelow, class Team>
+ETG_HD inline void chase_step(const Team& team, double* H, int ldh, int lo, int hi, int c, double& x, double& y,
+                              double& z) {
+  const int me = team.rank(), lanes = team.size();
+  double* D = H + c + c * ldh;                            // the diagonal block b, and t below its last column
+  double b[kRows][kRows], t = 0.0;
+  for (int j = 0; j < kRows; ++j)
+    for (int i = 0; i < kRows; ++i) b[i][j] = D[i + j * ldh];
+  if (kBelow) t = D[3 + 2 * ldh];
+  // the columns right of the block (updated from the left), then the rows above
+  // it (updated from the right): three entries p[0], p[st], p[2 st] each
+  const int cols = kBelow ? hi - c - 2 : 0, items = cols + c - lo;
+  int q = me, st = 1;
+  double *p = H, p0 = 0.0, p1 = 0.0, p2 = 0.0;
+  auto fetch = [&]() {
+    if (q >= items) return;
+    st = q < cols ? 1 : ldh;
+    p = H + (q < cols ? c + (c + 3 + q) * ldh : lo + q - cols + c * ldh);
+    p0 = p[0];
+    p1 = p[st];
+    if (kRows == 3) p2 = p[2 * st];
+  };
+  fetch();
+  const Reflector r = make_reflector(x, y, z, kRows);
+  const double tv1 = r.tau * r.v1, tv2 = r.tau * r.v2;
+  for (int j = 0; j < kRows; ++j) {                       // from the left
+    double w = r.tau * b[0][j] + tv1 * b[1][j];
+    if (kRows == 3) w += tv2 * b[kRows - 1][j];
+    b[0][j] -= w;
+    b[1][j] -= w * r.v1;
+    if (kRows == 3) b[kRows - 1][j] -= w * r.v2;
+  }
+  for (int i = 0; i < kRows; ++i) {                       // from the right
+    double w = r.tau * b[i][0] + tv1 * b[i][1];
+    if (kRows == 3) w += tv2 * b[i][kRows - 1];
+    b[i][0] -= w;
+    b[i][1] -= w * r.v1;
+    if (kRows == 3) b[i][kRows - 1] -= w * r.v2;
+  }
+  const double wt = tv2 * t;                              // row c + 3: (0, 0, t), from the right
+  while (q < items) {
+    double w = r.tau * p0 + tv1 * p1;
+    if (kRows == 3) w += tv2 * p2;
+    p[0] = p0 - w;
+    p[st] = p1 - w * r.v1;
+    if (kRows == 3) p[2 * st] = p2 - w * r.v2;
+    q += lanes;
+    fetch();
+  }
+  // column c below the diagonal stays in registers: the next reflector takes it,
+  // and leaves alpha and zeros
+  if (me == 0) {
+    if (c > lo) {
+      D[-ldh] = r.alpha;
+      D[1 - ldh] = 0.0;
+    }
+    D[0] = b[0][0];
+    for (int j = 1; j < kRows; ++j)
+      for (int i = 0; i < kRows; ++i) D[i + j * ldh] = b[i][j];
+    if (kBelow) {
+      D[3 + ldh] = -wt * r.v1;
+      D[3 + 2 * ldh] = t - wt * r.v2;
+    }
+  }
+  x = b[1][0];
+  y = kRows == 3 ? b[kRows - 1][0] : 0.0;
+  z = -wt;
+  team.sync();
+}
 
 // Eigenvalues of the k x k upper Hessenberg matrix H (column-major, leading
 // dimension ldh; overwritten) into wr, wi (complex pairs as re +- i im with the
@@ -91,21 +177,20 @@ ETG_HD int hessenberg_eigenvalues(const Team& team, double* H, int ldh, int k, d
 #define ETG_H(i, j) H[(i) + (j) * ldh]
   const int me = team.rank(), lanes = team.size();
   double scale = 0.0;
-  for (int j = 0; j < k; ++j)
+  for (int j = me; j < k; j += lanes)
     for (int i = 0; i <= (j + 1 < k ? j + 1 : k - 1); ++i) scale += std::fabs(ETG_H(i, j));
+  scale = team.sum(scale);
   *hnorm = scale;
   if (scale == 0.0) scale = 1.0;
   int hi = k - 1;             // the active block ends at row/column hi
   int sweeps = 0;             // double-shift steps since the last deflation
   while (hi >= 0) {
     // smallest lo such that H(lo:hi, lo:hi) has no negligible subdiagonal entry
-    int lo = hi;
-    while (lo > 0) {
-      double ref = std::fabs(ETG_H(lo, lo)) + std::fabs(ETG_H(lo - 1, lo - 1));
+    const int lo = team.highest(hi, [&](int l) {
+      double ref = std::fabs(ETG_H(l, l)) + std::fabs(ETG_H(l - 1, l - 1));
       if (ref == 0.0) ref = scale;
-      if (std::fabs(ETG_H(lo, lo - 1)) <= kEps * ref) break;
-      --lo;
-    }
+      return std::fabs(ETG_H(l, l - 1)) <= kEps * ref;
+    });
     team.sync();
     if (lo > 0 && me == 0) ETG_H(lo, lo - 1) = 0.0;
     team.sync();
@@ -171,45 +256,14 @@ ETG_HD int hessenberg_eigenvalues(const Team& team, double* H, int ldh, int k, d
       y /= sz;
       z /= sz;
     }
-    // chase the bulge down the block
-    for (int c = lo; c < hi; ++c) {
-      const int nr = hi - c + 1 < 3 ? hi - c + 1 : 3;
-      double a0 = x, a1 = y, a2 = z;
-      if (c > lo) {
-        a0 = ETG_H(c, c - 1);
-        a1 = ETG_H(c + 1, c - 1);
-        a2 = nr == 3 ? ETG_H(c + 2, c - 1) : 0.0;
-      }
-      const Reflector r = make_reflector(a0, a1, a2, nr);
-      team.sync();                                        // every lane has read the column
-      if (r.tau == 0.0) continue;
-      if (c > lo && me == 0) {
-        ETG_H(c, c - 1) = r.alpha;
-        ETG_H(c + 1, c - 1) = 0.0;
-        if (nr == 3) ETG_H(c + 2, c - 1) = 0.0;
-      }
-      // rows c .. c + nr - 1, columns c .. hi, from the left
-      for (int j = c + me; j <= hi; j += lanes) {
-        double w = ETG_H(c, j) + r.v1 * ETG_H(c + 1, j);
-        if (nr == 3) w += r.v2 * ETG_H(c + 2, j);
-        w *= r.tau;
-        ETG_H(c, j) -= w;
-        ETG_H(c + 1, j) -= w * r.v1;
-        if (nr == 3) ETG_H(c + 2, j) -= w * r.v2;
-      }
-      team.sync();
-      // columns c .. c + nr - 1, rows lo .. min(c + 3, hi), from the right
-      const int last = c + 3 < hi ? c + 3 : hi;
-      for (int i = lo + me; i <= last; i += lanes) {
-        double w = ETG_H(i, c) + r.v1 * ETG_H(i, c + 1);
-        if (nr == 3) w += r.v2 * ETG_H(i, c + 2);
-        w *= r.tau;
-        ETG_H(i, c) -= w;
-        ETG_H(i, c + 1) -= w * r.v1;
-        if (nr == 3) ETG_H(i, c + 2) -= w * r.v2;
-      }
-      team.sync();
-    }
+    // chase the bulge down the block; (x, y, z) is the column that the next
+    // reflector maps onto a multiple of e1
+    int c = lo;
+    for (; c + 3 <= hi; ++c) chase_step<3, true>(team, H, ldh, lo, hi, c, x, y, z);
+    chase_step<3, false>(team, H, ldh, lo, hi, c, x, y, z);
+    chase_step<2, false>(team, H, ldh, lo, hi, c + 1, x, y, z);
+    if (me == 0) ETG_H(hi, hi - 1) = x;
+    team.sync();
   }
   return 0;
 #undef ETG_H
