@@ -38,7 +38,7 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   t_.resize(sizeof(double) * (n_t1 + n_t2));
   omega_.resize(sizeof(double) * (n_t1 + n_t2));
   g_ovov_.resize(sizeof(double) * N * N);
-  red_partial_.resize(sizeof(double) * kReduceBlocks);
+  red_partial_.resize(sizeof(double) * kReduceBlocks * kDotBatch);
   red_result_.resize(sizeof(double) * 8);
   work_.resize(kBigSlots);
   // small scratch, sized once for every use in the programs below

@@ -469,16 +469,82 @@ __global__ void ritz_residual_kernel(const double* __restrict__ AY, const double
   }
 }
 
-// x_i = r_i / (w - d_i), guarded where the denominator vanishes (diagonal preconditioner)
-// x = r / (w - d) elementwise (x may be r itself)
-__global__ void precondition_kernel(const double* r, const double* __restrict__ d, double w, int64_t n,
-                                    double* x) {
+// The residuals that become new trial vectors: column c from column src[c] >= c
+// (increasing) of the block, preconditioned with root w[c].
+constexpr int kMaxRoots = kMaxRed / 2 - 1;
+struct NewColumns {
+  int n;
+  int src[kMaxRoots];
+  double w[kMaxRoots];
+};
+
+// R[:, c] = R[:, src] / (w - d), guarded where the denominator vanishes (diagonal
+// preconditioner).  A thread takes its element of all columns in turn: each is
+// read before the column that it is in is written.
+__global__ void precondition_kernel(double* R, const double* __restrict__ d, NewColumns cols, int64_t n) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += int64_t(gridDim.x) * blockDim.x) {
-    double den = w - d[i];
-    if (fabs(den) < 1e-8) den = den < 0.0 ? -1e-8 : 1e-8;
-    x[i] = r[i] / den;
+    const double di = d[i];
+    for (int c = 0; c < cols.n; ++c) {
+      double den = cols.w[c] - di;
+      if (fabs(den) < 1e-8) den = den < 0.0 ? -1e-8 : 1e-8;
+      R[i + c * n] = R[i + cols.src[c] * n] / den;
+    }
   }
+}
+
+// Columns to unit norm, from their squared norms on the device (zero columns stay
+// zero: they are dropped as linearly dependent).
+__global__ void normalize_kernel(double* X, const double* __restrict__ sq, int64_t n) {
+  double* x = X + blockIdx.y * n;
+  const double s = sq[blockIdx.y];
+  const double f = s > 0.0 ? 1.0 / sqrt(s) : 0.0;
+  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * blockDim.x)
+    x[i] = f * x[i];
+}
+
+// T = R^-1 of the Cholesky factor R (upper) of the q x q Gram matrix, q <= 64, by
+// one wavefront: lane j holds column j's row of work.  *ok = 0 (and T the identity)
+// when a pivot falls below 1e-8 of its diagonal entry.  The host would need the
+// matrix, its factor and two waits, 40-60 us for a few columns.
+__global__ __launch_bounds__(kLanes) void cholesky_inverse_kernel(const double* __restrict__ gram, int q,
+                                                                  double* __restrict__ T, double* __restrict__ ok) {
+  __shared__ double A[kLanes][kLanes + 1], V[kLanes][kLanes + 1];
+  const int j = threadIdx.x;
+  if (j < q)
+    for (int i = 0; i < q; ++i) A[i][j] = gram[i + j * q];
+  const double diag = j < q ? gram[j + j * q] : 0.0;
+  wave_sync();
+  bool good = true;
+  for (int c = 0; c < q; ++c) {
+    const double pivot = A[c][c];
+    if (!(pivot > 1e-8 * lane_value(diag, c))) {
+      good = false;
+      break;
+    }
+    const double r = sqrt(pivot);
+    wave_sync();
+    if (j >= c && j < q) A[c][j] = j == c ? r : A[c][j] / r;
+    wave_sync();
+    if (j > c && j < q)
+      for (int i = c + 1; i <= j; ++i) A[i][j] -= A[c][i] * A[c][j];
+    wave_sync();
+  }
+  if (j < q) {
+    for (int i = q - 1; i >= 0; --i) {
+      double v = i == j ? 1.0 : 0.0;
+      if (good && i == j) v = 1.0 / A[j][j];
+      if (good && i < j) {
+        double s = 0.0;
+        for (int l = i + 1; l <= j; ++l) s += A[i][l] * V[l][j];
+        v = -s / A[i][i];
+      }
+      V[i][j] = v;
+      T[i + j * q] = v;
+    }
+  }
+  if (j == 0) *ok = good ? 1.0 : 0.0;
 }
 
 }  // namespace
@@ -593,7 +659,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   // otherwise AV, and then V as well, in pinned host memory that the kernels
   // read and write over PCIe (etg_set_davidson_space overrides the choice).
   dav_Y_.resize(sizeof(double) * size_t(n) * size_t(3 * s1));
-  dav_small_.resize(sizeof(double) * size_t(max_dim * max_dim + 2 * max_dim * s1 + 3 * s1 + max_dim + 2 * s1 * s1));
+  dav_small_.resize(sizeof(double) * size_t(max_dim * max_dim + 2 * max_dim * s1 + 3 * s1 + max_dim + 2 * s1 * s1 + 2 * s1 + 2));
   {
     const size_t space = sizeof(double) * size_t(n) * size_t(max_dim);
     size_t free_b = 0, total_b = 0;
@@ -639,6 +705,8 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   double* cvec = coef + 3 * s1;              // Gram-Schmidt coefficients (max_dim)
   double* gram = cvec + max_dim;             // Gram matrix of a block (s1 x s1)
   double* tmat = gram + s1 * s1;             // inverse Cholesky factor of a block (s1 x s1)
+  double* sums = tmat + s1 * s1;             // squared norms (2 s1)
+  double* flags = sums + 2 * s1;             // success of the two Cholesky factorisations
   diff_.resize(sizeof(double) * n);
   double* d = diff_.as<double>();
   orbital_differences(stream_, eps_.as<double>(), d, n_o, n_v, n);
@@ -651,39 +719,29 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     synchronize();
     return v;
   };
-  // Cholesky QR of q columns at X: W = X T with T = R^-1, R^T R = X^T X (and
-  // WA = XA T alongside when XA is given).  It gives the Q of Gram-Schmidt when
-  // every column keeps more than 1e-4 of its norm against the ones before it
-  // (Cholesky pivots above 1e-8 of the diagonal); false otherwise, with nothing
-  // written.
-  auto cholqr = [&](const double* X, const double* XA, int64_t q, double* W, double* WA) {
-    run_gemm(make_gemm('T', 'N', q, q, n, 1.0, X, n, X, n, 0.0, gram, q), Prec::F64);
-    std::vector<double> hg(size_t(q * q)), R(size_t(q * q), 0.0), T(size_t(q * q), 0.0);
-    ETG_HIP(hipMemcpyAsync(hg.data(), gram, sizeof(double) * q * q, hipMemcpyDeviceToHost, stream_));
+  // Cholesky QR twice of q columns at X, through W: X T with T = R^-1, R^T R =
+  // X^T X, both times (and XA T alongside, through WA, when XA is given).  It gives
+  // the Q of Gram-Schmidt when every column keeps more than 1e-4 of its norm
+  // against the ones before it (Cholesky pivots above 1e-8 of the diagonal); false
+  // otherwise, with X and XA as they were.
+  auto cholqr = [&](double* X, double* XA, int64_t q, double* W, double* WA) {
+    auto factor = [&](const double* x, double* flag) {
+      run_gemm(make_gemm('T', 'N', q, q, n, 1.0, x, n, x, n, 0.0, gram, q), Prec::F64);
+      cholesky_inverse_kernel<<<1, kLanes, 0, stream_>>>(gram, int(q), tmat, flag);
+      ETG_LAUNCH("cholesky_inverse");
+    };
+    auto multiply = [&](const double* x, const double* xa, double* w, double* wa) {
+      run_gemm(make_gemm('N', 'N', n, q, q, 1.0, x, n, tmat, q, 0.0, w, n), Prec::F64);
+      if (xa) run_gemm(make_gemm('N', 'N', n, q, q, 1.0, xa, n, tmat, q, 0.0, wa, n), Prec::F64);
+    };
+    factor(X, flags);
+    multiply(X, XA, W, WA);
+    factor(W, flags + 1);
+    double ok[2];
+    ETG_HIP(hipMemcpyAsync(ok, flags, sizeof ok, hipMemcpyDeviceToHost, stream_));
     synchronize();
-    for (int64_t c = 0; c < q; ++c) {
-      for (int64_t i = 0; i < c; ++i) {
-        double v = hg[i + c * q];
-        for (int64_t l = 0; l < i; ++l) v -= R[l + i * q] * R[l + c * q];
-        R[i + c * q] = v / R[i + i * q];
-      }
-      double dcc = hg[c + c * q];
-      for (int64_t l = 0; l < c; ++l) dcc -= R[l + c * q] * R[l + c * q];
-      if (!(dcc > 1e-8 * hg[c + c * q])) return false;
-      R[c + c * q] = std::sqrt(dcc);
-    }
-    for (int64_t c = 0; c < q; ++c) {
-      T[c + c * q] = 1.0 / R[c + c * q];
-      for (int64_t i = c - 1; i >= 0; --i) {
-        double v = 0.0;
-        for (int64_t l = i + 1; l <= c; ++l) v += R[i + l * q] * T[l + c * q];
-        T[i + c * q] = -v / R[i + i * q];
-      }
-    }
-    ETG_HIP(hipMemcpyAsync(tmat, T.data(), sizeof(double) * q * q, hipMemcpyHostToDevice, stream_));
-    run_gemm(make_gemm('N', 'N', n, q, q, 1.0, X, n, tmat, q, 0.0, W, n), Prec::F64);
-    if (XA) run_gemm(make_gemm('N', 'N', n, q, q, 1.0, XA, n, tmat, q, 0.0, WA, n), Prec::F64);
-    synchronize();                        // T (host) is read by the copy above
+    if (ok[0] == 0.0 || ok[1] == 0.0) return false;
+    multiply(W, WA, X, XA);
     return true;
   };
   if (start) {
@@ -770,14 +828,18 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     ETG_HIP(hipMemcpyAsync(coef, packed.data(), sizeof(double) * 3 * se, hipMemcpyHostToDevice, stream_));
     ritz_residual_kernel<<<grid_for_d(n * se), kBlock, 0, stream_>>>(AY, Y, coef, n, int(se), Rb);
     ETG_LAUNCH("ritz_residual");
-    synchronize();                        // packed (host) is read by the copy above
+    // squared norms of the Ritz vectors and of the residuals
+    dots(stream_, Y, n, Y, n, n, se, red_partial_.as<double>(), sums, 1);
+    dots(stream_, Rb, n, Rb, n, n, se, red_partial_.as<double>(), sums + se, 1);
+    std::vector<double> ynorm(2 * se);
+    ETG_HIP(hipMemcpyAsync(ynorm.data(), sums, sizeof(double) * 2 * se, hipMemcpyDeviceToHost, stream_));
+    synchronize();                        // also: packed (host) is read by the copy above
+    const double* rnorm = ynorm.data() + se;
     bool converged = true;
-    std::vector<double> ynorm(se);
-    for (int64_t j = 0; j < se; ++j) ynorm[j] = dot_host(Y + j * n, Y + j * n);
     for (int64_t j = 0; j < se; ++j) {
       const int64_t p = int64_t(hcoef[2 * s1 + j]);
       const double yy = std::sqrt(ynorm[j] + (p != j ? ynorm[p] : 0.0));
-      norms[j] = std::sqrt(dot_host(Rb + j * n, Rb + j * n)) / yy;
+      norms[j] = std::sqrt(rnorm[j]) / yy;
       if (norms[j] >= threshold) converged = false;
     }
     for (int64_t j = 0; j < s; ++j) {
@@ -820,7 +882,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
       // orthonormalise the Ritz vectors (and their transforms alike), then they
       // become the space: Cholesky QR twice (through V and AV, which are
       // replaced anyway), or one vector at a time in HBM
-      if (se > 1 && cholqr(Y, AY, se, V, AV) && cholqr(V, AV, se, Y, AY)) {
+      if (se > 1 && cholqr(Y, AY, se, V, AV)) {
         run_gemm(make_gemm('T', 'N', se, se, n, 1.0, Y, n, AY, n, 0.0, G, max_dim), Prec::F64);
         ETG_HIP(hipMemcpyAsync(V, Y, sizeof(double) * n * se, hipMemcpyDefault, stream_));
         ETG_HIP(hipMemcpyAsync(AV, AY, sizeof(double) * n * se, hipMemcpyDefault, stream_));
@@ -845,17 +907,20 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
       k = se;
     }
     // preconditioned residuals of the unconverged roots, normalised, in the
-    // first columns of the residual block (column j moves to nc <= j, already read)
-    int64_t nc = 0;
-    for (int64_t j = 0; j < se; ++j) {
-      if (norms[j] < threshold) continue;
-      double* x = Rb + nc * n;
-      precondition_kernel<<<grid_for_d(n), kBlock, 0, stream_>>>(Rb + j * n, d, hcoef[j], n, x);
+    // first columns of the residual block
+    NewColumns cols{};
+    for (int64_t j = 0; j < se; ++j)
+      if (norms[j] >= threshold) {
+        cols.src[cols.n] = int(j);
+        cols.w[cols.n++] = hcoef[j];
+      }
+    const int64_t nc = cols.n;
+    if (nc > 0) {
+      precondition_kernel<<<grid_for_d(n), kBlock, 0, stream_>>>(Rb, d, cols, n);
       ETG_LAUNCH("precondition");
-      const double nx = std::sqrt(dot_host(x, x));
-      if (nx == 0.0) continue;
-      scale(stream_, x, n, 1.0 / nx);
-      ++nc;
+      dots(stream_, Rb, n, Rb, n, n, nc, red_partial_.as<double>(), sums, 1);
+      normalize_kernel<<<dim3(grid_for_d(n), unsigned(nc)), kBlock, 0, stream_>>>(Rb, sums, n);
+      ETG_LAUNCH("normalize");
     }
     // orthogonalised against the space as one block (two passes: one read of V
     // per product however many vectors are new) ...
@@ -869,7 +934,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     // vectors), otherwise one vector at a time (two passes), dropping linearly
     // dependent ones
     m = 0;
-    if (nc > 1 && cholqr(Rb, nullptr, nc, Y, nullptr) && cholqr(Y, nullptr, nc, Rb, nullptr)) m = nc;
+    if (nc > 1 && cholqr(Rb, nullptr, nc, Y, nullptr)) m = nc;
     for (int64_t c = m; c < nc; ++c) {
       double* x = Rb + c * n;
       if (m > 0)
@@ -878,7 +943,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
           run_gemm(make_gemm('N', 'N', n, 1, m, -1.0, Rb, n, cvec, max_dim, 1.0, x, n), Prec::F64);
         }
       const double nx = std::sqrt(dot_host(x, x));
-      if (nx < lindep) continue;
+      if (nx == 0.0 || nx < lindep) continue;
       scale(stream_, x, n, 1.0 / nx);
       if (c != m)
         ETG_HIP(hipMemcpyAsync(Rb + m * n, x, sizeof(double) * n, hipMemcpyDeviceToDevice, stream_));

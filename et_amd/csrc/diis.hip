@@ -208,9 +208,7 @@ void CCSD::diis_step(DiisSpace& d, const double* e, double* x) {
                          stream_));
   // new row of G (construct_new_G_elements, diis_tool_class.F90:503-546)
   auto new_row = [&] {
-    for (int i = 0; i < dim; ++i)
-      dot(stream_, E + int64_t(slot) * n, E + int64_t(i) * n, n, red_partial_.as<double>(),
-          G + slot + int64_t(i) * kMaxDiis);
+    dots(stream_, E + int64_t(slot) * n, 0, E, n, n, dim, red_partial_.as<double>(), G + slot, kMaxDiis);
     mirror_row_kernel<<<1, kMaxDiis, 0, stream_>>>(G, kMaxDiis, slot, dim);
     ETG_LAUNCH("diis_mirror_row");
   };

@@ -76,7 +76,11 @@ void ccsd_energy(hipStream_t s, const double* t1, const double* t2, const double
 void sum_squares(hipStream_t s, const double* x, int64_t n, double* partial, double* result);
 // result = x . y
 void dot(hipStream_t s, const double* x, const double* y, int64_t n, double* partial, double* result);
+// result[q sr] = (x + q sx) . (y + q sy) for q < count; partial holds kReduceBlocks * kDotBatch.
+void dots(hipStream_t s, const double* x, int64_t sx, const double* y, int64_t sy, int64_t n, int64_t count,
+          double* partial, double* result, int64_t sr);
 constexpr int kReduceBlocks = 1024;
+constexpr int kDotBatch = 64;
 
 // Amplitude-space helpers ----------------------------------------------------
 // MP2 guess: t2[aibj] = g_vovo(a,i,b,j) / (e_i - e_a + e_j - e_b)
