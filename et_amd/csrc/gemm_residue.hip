@@ -208,29 +208,84 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
 // ---------------------------------------------------------------------------
 constexpr int64_t kShortDepth = 3200;
 
+constexpr int kWaveM = 8, kWaveN = 4;         // 16 x 16 blocks of a wave
+constexpr int kBlocksM = kTileM / 16;
+
+// The tiles of one launch.  A slot is a tile's place in the order of work (groups of
+// row tiles, in each column tile by column tile) and in the array of residues.  Of a
+// lower block triangle (Gemm::lower) a group holds the column tiles that its last row
+// needs; the few above the diagonal among them do nothing.  Cut into sixteen column
+// pieces instead, each from its first row on, a triangle of 5776 rows (k = 1270) took
+// 16 launches of 1035 workgroups and fewer, two or three rounds of the chip each: 0.60
+// ms against 0.35.  At 23104 rows both run at the kernel's rate (9.5 ms).
+constexpr int kMaxGroups = 64;
+struct TileMap {
+  int tiles_m, tiles_n, tile_n;
+  int64_t lower, row0, col0;       // of the product's output, for the triangle
+  int group, groups, count;        // row tiles of a group; slots
+  uint32_t first[kMaxGroups];      // first slot of each group
+};
+
+// Tile of a slot; false: nothing to do.  Called by whole wavefronts.
+__device__ inline bool tile_of(const TileMap& t, int slot, int& tm, int& tn) {
+  if (t.lower == 0) {
+    const int group = kGroupM * t.tiles_n;
+    const int first_m = (slot / group) * kGroupM;
+    const int gsize = min(t.tiles_m - first_m, kGroupM);
+    tm = first_m + (slot % group) % gsize;
+    tn = (slot % group) / gsize;
+    return true;
+  }
+  const int lane = threadIdx.x & 63;
+  const uint32_t f = lane < t.groups ? t.first[lane] : ~0u;
+  const int g = __popcll(__ballot(uint32_t(slot) >= f)) - 1;
+  const int first_m = g * t.group;
+  const int gsize = min(t.tiles_m - first_m, t.group);
+  const int l = slot - __builtin_amdgcn_readlane(int(f), g);
+  tm = first_m + l % gsize;
+  tn = l / gsize;
+  return t.row0 + (tm + 1) * int64_t(kTileM) > (t.col0 + tn * int64_t(t.tile_n)) / t.lower * t.lower;
+}
+
+// Slot of a workgroup: contiguous ranges of slots per XCD (their tiles share an L2).
+__device__ inline int slot_of(int bid, int nb) {
+  const int per = nb / kXcds, rem = nb % kXcds;
+  const int xcd = bid % kXcds, idx = bid / kXcds;
+  return (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
+}
+
+TileMap map_tiles(int64_t m, int64_t n, int tile_n, int64_t lower, int64_t row0, int64_t col0) {
+  TileMap t{};
+  t.tiles_m = int(ceil_div(m, kTileM));
+  t.tiles_n = int(ceil_div(n, tile_n));
+  t.tile_n = tile_n;
+  t.lower = lower;
+  t.row0 = row0;
+  t.col0 = col0;
+  if (lower == 0) {
+    t.count = t.tiles_m * t.tiles_n;
+    return t;
+  }
+  t.group = std::max(kGroupM, int(ceil_div(t.tiles_m, kMaxGroups)));
+  t.groups = int(ceil_div(t.tiles_m, t.group));
+  for (int g = 0; g < t.groups; ++g) {
+    const int64_t end = std::min(t.tiles_m, (g + 1) * t.group);          // first row tile after the group
+    // its last row needs the columns before the end of that row's block
+    const int64_t columns = ceil_div(row0 + end * kTileM, lower) * lower - col0;
+    t.first[g] = uint32_t(t.count);
+    t.count += int(end - g * t.group) * int(std::clamp<int64_t>(ceil_div(columns, tile_n), 0, t.tiles_n));
+  }
+  return t;
+}
+
 struct Params {
   const u4 *A, *B;                 // packs (planes of the first modulus)
   uint32_t* R;                     // one byte per output and modulus: tiles of 16 x 16 blocks in fragment order
   int64_t KS;
   int64_t planeA, planeB, planeR;  // from one modulus to the next (u4, u4, u32 units)
   int64_t strideA, strideB, strideR;   // from one batch entry to the next
-  int tiles_m, tiles_n;
+  TileMap tiles;
 };
-
-constexpr int kWaveM = 8, kWaveN = 4;         // 16 x 16 blocks of a wave
-constexpr int kBlocksM = kTileM / 16;
-
-__device__ inline void map_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int nb = tiles_m * tiles_n;
-  const int per = nb / kXcds, rem = nb % kXcds;
-  const int xcd = bid % kXcds, idx = bid / kXcds;
-  const int logical = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-  const int group = kGroupM * tiles_n;
-  const int first_m = (logical / group) * kGroupM;
-  const int gsize = min(tiles_m - first_m, kGroupM);
-  tm = first_m + (logical % group) % gsize;
-  tn = (logical % group) / gsize;
-}
 
 // Waits until at most N of this wave's vector-memory operations are outstanding.
 template <int N>
@@ -248,8 +303,9 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
   __shared__ u4 lds[kStages][(kBlocksM + kBlocksN) * 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;
+  const int slot = slot_of(blockIdx.x, gridDim.x);
   int tile_m, tile_n;
-  map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+  if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
   const int z = blockIdx.y;
   const int64_t bz = blockIdx.z;
   const u4* sa = p.A + bz * p.strideA + z * p.planeA + int64_t(tile_m) * kBlocksM * p.KS * 64;
@@ -319,7 +375,7 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
   }
   const double m = kC.md[z], inv = kC.invd[z];
   uint32_t* R = p.R + bz * p.strideR + z * p.planeR +
-                (int64_t(tile_n) * p.tiles_m + tile_m) * (kBlocksM * kBlocksN * 64);
+                int64_t(slot) * (kBlocksM * kBlocksN * 64);
 #pragma unroll
   for (int i = 0; i < kWaveM; ++i)
 #pragma unroll
@@ -344,7 +400,7 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
 struct Output {
   const uint32_t* R;
   int64_t planeR, strideR;
-  int tiles_m, blocks_n;                  // tiles along m, 16-column blocks of a tile
+  TileMap tiles;
   int64_t m, n, K;                        // of this panel
   const int *ea, *eb;
   int64_t ea_stride, eb_stride;
@@ -368,14 +424,17 @@ __device__ double plain_sum(const Output& p, int64_t bz, int64_t row, int64_t co
 
 __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
   const int lane = threadIdx.x & 63;
-  const int per_tile = kBlocksM * p.blocks_n / 4;
-  const int64_t tile = blockIdx.x / unsigned(per_tile);
+  const int blocks_n = p.tiles.tile_n / 16;
+  const int per_tile = kBlocksM * blocks_n / 4;
+  const int slot = int(blockIdx.x / unsigned(per_tile));
   const int blk = int(blockIdx.x % unsigned(per_tile)) * 4 + int(threadIdx.x >> 6);
+  int tile_m, tile_n;
+  if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
   const int64_t bz = blockIdx.y;
-  const int64_t row = (tile % p.tiles_m) * kTileM + (blk % kBlocksM) * 16 + 4 * (lane >> 4);
-  const int64_t col = ((tile / p.tiles_m) * p.blocks_n + blk / kBlocksM) * 16 + (lane & 15);
+  const int64_t row = int64_t(tile_m) * kTileM + (blk % kBlocksM) * 16 + 4 * (lane >> 4);
+  const int64_t col = (int64_t(tile_n) * blocks_n + blk / kBlocksM) * 16 + (lane & 15);
   if (row >= p.m || col >= p.n) return;
-  const uint32_t* R = p.R + bz * p.strideR + (tile * (kBlocksM * p.blocks_n) + blk) * 64 + lane;
+  const uint32_t* R = p.R + bz * p.strideR + (int64_t(slot) * (kBlocksM * blocks_n) + blk) * 64 + lane;
   uint32_t w[kModuli];
 #pragma unroll
   for (int i = 0; i < kModuli; ++i) w[i] = R[i * p.planeR];
@@ -455,8 +514,22 @@ bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
   p.out_n = p.rn_p;
   // a quarter of the capacity (or all) for the residues: thinner pieces leave CUs idle
   if (room < std::min(p.rm_p * p.rn_p, int64_t(capacity / 4) / (p.batch * kModuli))) return false;
-  // a lower block triangle goes by columns: a sixteenth of them at once wastes 3 %
-  if (g.lower > 0) p.out_n = std::min(p.out_n, round_up(std::max<int64_t>(1, p.rn_p / 16), p.tile_n));
+  // of a lower block triangle as many columns as have room: the first ones are the
+  // longest, and only tiles of the triangle are kept
+  const int64_t tile = int64_t(kTileM) * p.tile_n;
+  if (g.lower > 0 && p.rows_m == g.m && p.rows_n == g.n) {
+    auto outputs = [&](int64_t cols) { return map_tiles(p.rm_p, cols, p.tile_n, g.lower, 0, 0).count * tile; };
+    int64_t fit = 0, over = p.rn_p / p.tile_n + 1;                       // column tiles
+    while (over - fit > 1) {
+      const int64_t mid = (fit + over) / 2;
+      (outputs(mid * p.tile_n) <= room ? fit : over) = mid;
+    }
+    if (fit * p.tile_n >= std::min<int64_t>(p.rn_p, 512)) {
+      p.out_n = fit * p.tile_n;
+      p.bytes_r = align256(size_t(kModuli) * size_t(outputs(p.out_n)));
+      return p.total() <= capacity;
+    }
+  }
   const int64_t least = std::min<int64_t>(p.out_n, 512);
   if (p.out_m * p.out_n > room) p.out_n = std::max(least, room / p.out_m / p.tile_n * p.tile_n);
   if (p.out_m * p.out_n > room) p.out_m = room / p.out_n / kTileM * kTileM;
@@ -594,15 +667,14 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
         q.B = PB + c0 * p.KS * (kDepth / 16);
         q.R = R;
         q.KS = p.KS;
-        q.tiles_m = int(ceil_div(mo, kTileM));
-        q.tiles_n = int(ceil_div(no, p.tile_n));
+        q.tiles = map_tiles(mo, no, p.tile_n, g.lower, m0 + r0, n0 + c0);
         q.planeA = p.rm_p * p.KS * (kDepth / 16);
         q.planeB = p.rn_p * p.KS * (kDepth / 16);
-        q.planeR = int64_t(q.tiles_m) * kTileM * q.tiles_n * p.tile_n / 4;
+        q.planeR = int64_t(q.tiles.count) * kTileM * p.tile_n / 4;
         q.strideA = g.strideA == 0 ? 0 : kModuli * q.planeA;
         q.strideB = g.strideB == 0 ? 0 : kModuli * q.planeB;
         q.strideR = kModuli * q.planeR;
-        const unsigned tiles = unsigned(q.tiles_m) * unsigned(q.tiles_n);
+        const unsigned tiles = unsigned(q.tiles.count);
         const dim3 grid(tiles, kModuli, unsigned(nb));
         if (p.tile_n == 128)
           residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
@@ -613,8 +685,7 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
         o.R = R;
         o.planeR = q.planeR;
         o.strideR = q.strideR;
-        o.tiles_m = q.tiles_m;
-        o.blocks_n = p.tile_n / 16;
+        o.tiles = q.tiles;
         o.m = mo; o.n = no; o.K = g.k;
         o.ea = ea + r0; o.eb = eb + c0;
         o.ea_stride = g.strideA == 0 ? 0 : p.rm_p;
