@@ -613,10 +613,11 @@ bool CCSD::reserve_ladder_packs() {
 // G of ladder block b: G(c + v aa, d + v bb) = sum_J L_t1(J, c, a0 + aa)
 // L_t1(J, d, b0 + bb), in FP32 when `fp32` (the split-bf16 path).  The pairs
 // of a diagonal block (a0 == b0) have aa >= bb, so it is formed as a lower block
-// triangle, or on the FP64 and bf16 kernels in column strips of 8 b's, each from
-// the row block of its first b on (a little over half of the full block's work).
+// triangle, or on the FP64 kernels in column strips of 8 b's, each from the row
+// block of its first b on (a little over half of the full block's work).
 // One triangle packs L once for both operands: 19 strips at (H2O)8 packed it 38
-// times, 9 ms of a 72 ms residual.  `tag` names the full block's A operand for the pack cache
+// times, 9 ms of a 72 ms residual in FP64, and split their k, 9 of 41 ms with the
+// packs in split-bf16.  `tag` names the full block's A operand for the pack cache
 // (0: no tag).
 void CCSD::ladder_G(const Block& b, const double* LT, Prec prec, bool fp32, uint64_t tag) {
   const int64_t v = n_v, J = n_J, ldg = v * b.la;
@@ -638,7 +639,11 @@ void CCSD::ladder_G(const Block& b, const double* LT, Prec prec, bool fp32, uint
   }
   Gemm whole = block_product(0, 0, b.lb);
   whole.lower = v;
-  if (!fp32 && runs_as_residues(whole, prec, gws_cur_)) {
+  if (fp32) {
+    whole.C = nullptr;
+    whole.Cf = gblk_.as<float>();
+  }
+  if ((prec == Prec::BF16X3 && split_bf16_pays(whole)) || runs_as_residues(whole, prec, gws_cur_)) {
     run_gemm(whole, prec);
     return;
   }

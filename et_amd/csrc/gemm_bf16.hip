@@ -18,6 +18,7 @@
 
 #include "gemm.hpp"
 #include "ladder_order.hpp"
+#include "tile_map.hpp"
 
 namespace etg {
 namespace {
@@ -27,10 +28,9 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int kTile = 256;      // output tile (rows and columns)
+constexpr int kTile = kTileM;   // output tile (rows and columns)
 constexpr int kDepth = 32;      // k per step (one MFMA step)
-constexpr int kXcds = 8;
-constexpr int kGroupM = 8;
+constexpr int64_t kCus = 256;
 
 // ---------------------------------------------------------------------------
 // pack: both splits of op(X) (rows_p x Kp per batch entry) in the order the
@@ -177,23 +177,17 @@ struct Params {
   double* C;
   float* Cf;                         // C in FP32 instead (beta = 0)
   int64_t ldc, strideC;
-  double* W;                         // split-K partials (m x n per split and batch entry)
+  // Output tiles (of all batch entries, one entry after another): the first `whole`
+  // are one workgroup's work each; each of the `rest` after them is that of `splits`
+  // workgroups with ks_per_split steps, whose sums go to W (a tile's splits one after
+  // another, each 64 KB x 4 in fragment order).
+  TileMap tiles;
+  int64_t whole, rest;
+  int splits;
   int64_t ks_per_split;
-  int tiles_m, tiles_n;
-  int vec_rows;                      // W / C / Cf rows written four at a time (alignment checked on the host)
+  f4* W;
+  int vec_rows;                      // C / Cf rows written four at a time (alignment checked on the host)
 };
-
-__device__ inline void map_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int nb = tiles_m * tiles_n;
-  const int per = nb / kXcds, rem = nb % kXcds;
-  const int xcd = bid % kXcds, idx = bid / kXcds;
-  const int logical = (xcd < rem) ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-  const int group = kGroupM * tiles_n;
-  const int first_m = (logical / group) * kGroupM;
-  const int gsize = min(tiles_m - first_m, kGroupM);
-  tm = first_m + (logical % group) % gsize;
-  tn = (logical % group) / gsize;
-}
 
 __device__ inline f4 mfma(bf8 a, bf8 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -216,6 +210,7 @@ __device__ inline f4 mfma(bf8 a, bf8 b, f4 c) {
 // k the workgroup moves 1/64 operand bytes.
 // ---------------------------------------------------------------------------
 constexpr int kProductThreads = 512;
+constexpr int kTileF4 = kTile * kTile / 4;       // 16-byte pieces of a tile's FP32 sums
 
 __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params p) {
   __shared__ u4 lds[2][4096];        // per buffer: A chunks 0..31, B chunks 32..63 (1 KB each)
@@ -223,11 +218,23 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave & 1, wn = wave >> 1;     // rows 128 wm.., columns 64 wn..
-  int tile_m, tile_n;
-  map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  const int64_t bz = blockIdx.z, split = blockIdx.y;
-  const int64_t ks0 = split * p.ks_per_split;
-  const int64_t ks1 = min(p.KS, ks0 + p.ks_per_split);
+  // batch entry and slot of the tile, and its range of k steps
+  const int64_t count = p.tiles.count, bid = blockIdx.x;
+  const bool partial = bid >= p.whole;
+  int64_t bz, ks0 = 0, ks1 = p.KS;
+  int slot, piece = 0, tile_m, tile_n;
+  if (!partial) {
+    bz = bid / count;
+    slot = slot_of(int(bid - bz * count), int(min(count, p.whole - bz * count)));
+  } else {
+    piece = slot_of(int(bid - p.whole), int(p.rest) * p.splits);
+    const int64_t u = p.whole + piece % int(p.rest);
+    bz = u / count;
+    slot = int(u - bz * count);
+    ks0 = piece / int(p.rest) * p.ks_per_split;
+    ks1 = min(p.KS, ks0 + p.ks_per_split);
+  }
+  if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
   const int64_t nsteps = ks1 - ks0;
   const int64_t astride = p.KS * 128;          // u4 units from one row block to the next
 
@@ -312,37 +319,17 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
     compute(int(s & 1));
   }
 
-  const int lrow = lane >> 4, lcol = lane & 15;
-  const int64_t r0 = int64_t(tile_m) * kTile + wm * 128, c0 = int64_t(tile_n) * kTile + wn * 64;
-  if (p.W) {
-    double* W = p.W + (split + bz * gridDim.y) * p.m * p.n;
-    if (p.vec_rows) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int64_t row = r0 + i * 16 + 4 * lrow;
-          const int64_t col = c0 + j * 16 + lcol;
-          if (row < p.m && col < p.n) {
-            double2* w = reinterpret_cast<double2*>(W + row + col * p.m);
-            w[0] = double2{double(acc[i][j][0]), double(acc[i][j][1])};
-            w[1] = double2{double(acc[i][j][2]), double(acc[i][j][3])};
-          }
-        }
-      return;
-    }
+  if (partial) {
+    const int rest = int(p.rest);
+    f4* W = p.W + (int64_t(piece % rest) * p.splits + piece / rest) * kTileF4 + wave * 2048 + lane;
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t row = r0 + i * 16 + 4 * lrow + r;
-          const int64_t col = c0 + j * 16 + lcol;
-          if (row < p.m && col < p.n) W[row + col * p.m] = double(acc[i][j][r]);
-        }
+      for (int j = 0; j < 4; ++j) W[(i * 4 + j) * 64] = acc[i][j];
     return;
   }
+  const int lrow = lane >> 4, lcol = lane & 15;
+  const int64_t r0 = int64_t(tile_m) * kTile + wm * 128, c0 = int64_t(tile_n) * kTile + wn * 64;
   if (p.Cf) {
     float* C = p.Cf + bz * p.strideC;
     if (p.vec_rows) {
@@ -413,24 +400,31 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
       }
 }
 
-// C = alpha * sum_s W_s + beta * C
-__global__ void splitk_reduce_bf(const double* __restrict__ W, int splits, int64_t m, int64_t n,
-                                 double alpha, double beta, double* C, float* Cf, int64_t ldc,
-                                 int64_t strideC) {
-  const int64_t bz = blockIdx.z;
-  const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (idx >= m * n) return;
-  const int64_t row = idx % m, col = idx / m;
-  const double* w = W + bz * splits * m * n + idx;
-  double s = 0.0;
-  for (int q = 0; q < splits; ++q) s += w[int64_t(q) * m * n];
-  const double v = alpha * s;
-  if (Cf) {
-    Cf[bz * strideC + row + col * ldc] = float(v);
-    return;
+// C = alpha * sum_s W_s + beta * C on the tiles whose k range was split: a lane
+// adds up (in FP64) four consecutive rows of one column.  Bound by HBM.
+__global__ __launch_bounds__(256) void splitk_reduce_bf(Params p) {
+  const int64_t u = p.whole + blockIdx.y, bz = u / p.tiles.count;
+  int tile_m, tile_n;
+  if (!tile_of(p.tiles, int(u - bz * p.tiles.count), tile_m, tile_n)) return;
+  const int q = int(blockIdx.x) * 256 + int(threadIdx.x);               // wave (3 bits), block row (3), block column (2), lane (6)
+  const int wave = q >> 11, lane = q & 63;
+  const int64_t row = int64_t(tile_m) * kTile + (wave & 1) * 128 + ((q >> 8) & 7) * 16 + 4 * (lane >> 4);
+  const int64_t col = int64_t(tile_n) * kTile + (wave >> 1) * 64 + ((q >> 6) & 3) * 16 + (lane & 15);
+  if (row >= p.m || col >= p.n) return;
+  const f4* W = p.W + int64_t(blockIdx.y) * p.splits * kTileF4 + q;
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int s = 0; s < p.splits; ++s) {
+    const f4 w = W[int64_t(s) * kTileF4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] += double(w[r]);
   }
-  double* c = C + bz * strideC + row + col * ldc;
-  *c = (beta == 0.0) ? v : v + beta * *c;
+  const int64_t at = bz * p.strideC + row + col * p.ldc;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    if (row + r >= p.m) return;
+    if (p.Cf) p.Cf[at + r] = float(p.alpha * v[r]);
+    else p.C[at + r] = p.beta == 0.0 ? p.alpha * v[r] : p.alpha * v[r] + p.beta * p.C[at + r];
+  }
 }
 
 void pack(hipStream_t s, const double* X, int64_t ld, int64_t strideX, bool kcontig, int64_t rows,
@@ -497,13 +491,15 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
   const int64_t b_batch = g.strideB == 0 ? 1 : g.batch;
   __bf16* Ap = packed_a(stream, g, ws, m_p, Kp);
   const __bf16* Bp = static_cast<const __bf16*>(g.b_packed);
+  // op(A)^T and op(B) one array: packed once
+  if (Bp == nullptr && g.A == g.B && g.ta != g.tb && g.lda == g.ldb && g.m == g.n && g.batch == 1) Bp = Ap;
   if (Bp == nullptr) {
     const size_t b_elems = size_t(b_batch) * size_t(n_p) * size_t(Kp);
     if (ws->packB.resize(2 * b_elems * sizeof(__bf16))) ++ws->gen;
     __bf16* P = ws->packB.as<__bf16>();
     pack(stream, g.B, g.ldb, g.strideB, !g.tb, g.n, g.k, n_p, Kp, b_batch, P);
     Bp = P;
-  } else if (g.strideB != 0) {
+  } else if (g.b_packed != nullptr && g.strideB != 0) {
     fail("gemm: a prepacked B operand is shared by the whole batch");
   }
 
@@ -516,57 +512,53 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
   p.strideBp = g.strideB == 0 ? 0 : 2 * n_p * Kp;
   p.m = g.m; p.n = g.n; p.alpha = g.alpha; p.beta = g.beta;
   p.C = g.C; p.Cf = g.Cf; p.ldc = g.ldc; p.strideC = g.strideC;
-  p.tiles_m = int(m_p / kTile);
-  p.tiles_n = int(n_p / kTile);
+  p.tiles = map_tiles(g.m, g.n, kTile, g.lower, 0, 0);
+  // One workgroup per CU: the tiles that fill whole rounds of the chip are taken
+  // whole, those of the last round share it by splitting their k.  With every tile
+  // split so that rounds are 90 % full, partials of the whole output in FP64, before:
+  // m = n = k = 6080 1.26 -> 0.99 ms, k = 2541 0.72 -> 0.50, 23104 x 1600 x 2541 0.85
+  // -> 0.65, 820 x 17020 x 17020 2.35 -> 1.98, m = n = k = 1520 73 -> 60 us; 1600 x
+  // 1600 x 23104 0.49 -> 0.47 (49 tiles, five splits each either way).
+  const int64_t tiles = int64_t(p.tiles.count) * g.batch;
+  p.whole = tiles / kCus * kCus;
+  p.rest = tiles - p.whole;
+  p.splits = 1;
   p.ks_per_split = KS;
-  // One workgroup per CU.  Split K when the output has few tiles: the smallest
-  // split count whose rounds of 256 workgroups are at least 90 % full (at most
-  // 256 splits of at least 16 k steps each; partials of at most 256 tiles).
-  const int64_t tiles = int64_t(p.tiles_m) * p.tiles_n * g.batch;
-  int splits = 1;
-  if (tiles < 2048 && KS >= 32) {
-    const int64_t cus = 256, max_s = std::min<int64_t>(256, KS / 16);
-    int best = 1;
-    double best_eff = 0.0;
-    for (int64_t s = 1; s <= max_s; ++s) {
-      const double wgs = double(tiles * s);
-      const double eff = (wgs / cus) / double(ceil_div(tiles * s, cus));
-      if (eff > best_eff + 1e-9) { best_eff = eff; best = int(s); }
-      if (eff >= 0.9) { best = int(s); break; }
+  if (p.rest > 0 && KS >= 32) {
+    // microseconds of the last round: 2.3 per step, 0.107 to write and read a partial
+    // sum of a tile, 6 for the second launch
+    double best = 2.3 * double(KS);
+    for (int64_t s = 2; s <= std::min<int64_t>(kCus, KS / 16); ++s) {
+      const int64_t kps = ceil_div(KS, s), used = ceil_div(KS, kps);
+      const double t = 2.3 * double(kps * ceil_div(p.rest * used, kCus)) + 0.107 * double(p.rest * used) + 6.0;
+      if (t < best) {
+        best = t;
+        p.splits = int(used);
+        p.ks_per_split = kps;
+      }
     }
-    splits = best;
   }
-  if (splits > 1) {
-    const int64_t kps = ceil_div(KS, splits);
-    splits = int(ceil_div(KS, kps));
-    p.ks_per_split = kps;
-    if (ws->buf.resize(size_t(splits) * size_t(g.m) * size_t(g.n) * size_t(g.batch) * sizeof(double)))
-      ++ws->gen;
-    p.W = ws->buf.as<double>();
+  if (p.splits > 1) {
+    if (ws->buf.resize(size_t(p.rest) * size_t(p.splits) * kTileF4 * sizeof(f4))) ++ws->gen;
+    p.W = ws->buf.as<f4>();
+  } else {
+    p.whole = tiles;
+    p.rest = 0;
   }
   // rows four at a time: m, ldc and the batch stride multiples of 4 elements and
-  // the output 16 B (FP32) or 32 B (FP64) aligned; split-K partials (ld m, in the
-  // 256 B aligned workspace) need m a multiple of 4
-  if (splits > 1) {
-    p.vec_rows = g.m % 4 == 0 && reinterpret_cast<uintptr_t>(p.W) % 32 == 0;
-  } else {
-    const uintptr_t base = g.Cf ? reinterpret_cast<uintptr_t>(g.Cf) : reinterpret_cast<uintptr_t>(g.C);
-    p.vec_rows = g.m % 4 == 0 && g.ldc % 4 == 0 && (g.batch == 1 || g.strideC % 4 == 0) &&
-                 base % (g.Cf ? 16 : 32) == 0;
-  }
-  dim3 grid(unsigned(tiles / g.batch), unsigned(splits), unsigned(g.batch));
-  gemm_bf16x3_kernel<<<grid, kProductThreads, 0, stream>>>(p);
+  // the output 16 B (FP32) or 32 B (FP64) aligned
+  const uintptr_t base = g.Cf ? reinterpret_cast<uintptr_t>(g.Cf) : reinterpret_cast<uintptr_t>(g.C);
+  p.vec_rows = g.m % 4 == 0 && g.ldc % 4 == 0 && (g.batch == 1 || g.strideC % 4 == 0) &&
+               base % (g.Cf ? 16 : 32) == 0;
+  gemm_bf16x3_kernel<<<unsigned(p.whole + p.rest * p.splits), kProductThreads, 0, stream>>>(p);
   ETG_LAUNCH("gemm_bf16x3");
-  if (splits > 1) {
-    const int64_t mn = g.m * g.n;
-    dim3 rgrid(unsigned(ceil_div(mn, 256)), 1, unsigned(g.batch));
-    splitk_reduce_bf<<<rgrid, 256, 0, stream>>>(p.W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.Cf, g.ldc,
-                                                g.strideC);
+  if (p.rest > 0) {
+    splitk_reduce_bf<<<dim3(kTileF4 / 256, unsigned(p.rest)), 256, 0, stream>>>(p);
     ETG_LAUNCH("splitk_reduce");
   }
   GemmLaunch info;
   info.kernel = "gemm_bf16x3<256x256>";
-  info.splits = splits;
+  info.splits = p.splits;
   return info;
 }
 
