@@ -401,8 +401,7 @@ void CCSD::program_omega(Ops& X, Prec prec) {
   double* U = X.buf(SL_U, "u_aibj", N * N);
   X.squareup(t_.as<double>() + n_t1, T, N);
   const int64_t d[4] = {n_v, n_o, n_v, n_o};
-  X.sort4(T, d, "1234", U, 2.0, 0.0);
-  X.sort4(T, d, "1432", U, -1.0, 1.0);
+  X.sort4(T, d, "1432", U, -1.0, 0.0, T, 2.0);
   // singles: F_ai + doubles A1, B1, C1
   omega_singles(X, prec, U);
   // doubles: E2, symmetric sum, B2, 1/2 diagonal, pack, then C2/D2 and A2
@@ -452,26 +451,23 @@ void CCSD::omega_e2_b2(Ops& X, Prec prec, const double* T, const double* U) {
   double* u_e2 = X.buf(SL_A, "e2_u", N * N);   // u_kl^bd = 2 t_bkdl - t_bldk = u(b,k,d,l)
   X.sort4(U, d, "1432", u_e2, 1.0, 0.0);
   double* om = X.buf(SL_B, "e2_omega", N * N);
-  X.fill0(om, N * N);
   double* Xbc = X.buf(SL_SMALL0, "e2_X", v * v);
   double* Ykj = X.buf(SL_SMALL1, "e2_Y", o * o);
   X.copy_sub(F + o + n * o, n, Xbc, v, v, v, 1.0, 0.0);
   X.gemm('N', 'N', v, v, o * v * o, -1.0, u_e2, v, g_ovov, o * v * o, 1.0, Xbc, v, prec);
-  X.gemm('N', 'N', v, o * v * o, v, 1.0, Xbc, v, T, v, 1.0, om, v, prec);
+  X.gemm('N', 'N', v, o * v * o, v, 1.0, Xbc, v, T, v, 0.0, om, v, prec);
   X.copy_sub(F, n, Ykj, o, o, o, 1.0, 0.0);
   X.gemm('N', 'N', o, o, v * o * v, 1.0, g_ovov, o, u_e2, v * o * v, 1.0, Ykj, o, prec);
   X.gemm('N', 'N', v * o * v, o, o, -1.0, T, v * o * v, Ykj, o, 1.0, om, v * o * v, prec);
   // symmetric sum
   double* om2 = X.buf(SL_C, "e2_omega_sym", N * N);
   X.symsum(om, om2, N);
-  // B2 in (a,b,i,j) order (omega_ccsd.F90:483-583)
+  // B2 in (a,b,i,j) order (omega_ccsd.F90:483-583), its g_aibj added before the sort
+  X.gemm('T', 'N', N, N, J, 1.0, Lt_vo_.as<double>(), J, Lt_vo_.as<double>(), J, 1.0, om2, N, prec);
   double* om_abij = X.buf(SL_A, "b2_omega_abij", N * N);
   X.sort4(om2, d, "1324", om_abij, 1.0, 0.0);
   double* t_abij = X.buf(SL_B, "b2_t_abij", N * N);
   X.sort4(T, d, "1324", t_abij, 1.0, 0.0);
-  double* g_vovo = X.buf(SL_C, "b2_g_vovo", N * N);
-  X.gemm('T', 'N', N, N, J, 1.0, Lt_vo_.as<double>(), J, Lt_vo_.as<double>(), J, 0.0, g_vovo, N, prec);
-  X.sort4(g_vovo, d, "1324", om_abij, 1.0, 1.0);
   double* g_kilj = X.buf(SL_SMALL3, "b2_g_kilj", o * o * o * o);
   double* X_klij = X.buf(SL_SMALL2, "b2_X", o * o * o * o);
   X.gemm('T', 'N', o * o, o * o, J, 1.0, Lt_oo_.as<double>(), J, Lt_oo_.as<double>(), J, 0.0, g_kilj,
@@ -503,19 +499,17 @@ void CCSD::omega_c2_d2(Ops& X, Prec prec, const double* Tfull, const double* U) 
          v * v, prec);                                       // g_abij
   const int64_t d_vvoo[4] = {v, v, o, o};
   X.sort4(g_vvoo, d_vvoo, "2314", C, 1.0, 0.0);             // C(b,i,a,j) = g_abij
-  X.sort4(C, d, "1234", D, -1.0, 0.0);                      // D = -C
   double* g_voov = X.buf(SL_B, "c2_g_voov", N * N);
   X.gemm('T', 'N', N, N, J, 1.0, Lt_vo_.as<double>(), J, Lmo_ov_.as<double>(), J, 0.0, g_voov, N,
          prec);                                              // g_aijb
   const int64_t d_voov[4] = {v, o, o, v};
-  X.sort4(g_voov, d_voov, "4312", D, 2.0, 1.0);             // D(c,k,a,i) += 2 g_aikc
+  X.sort4(g_voov, d_voov, "4312", D, 2.0, 0.0, C, -1.0);    // D(c,k,a,i) = 2 g_aikc - C
   double* G = X.buf(SL_B, "c2_G", N * N);
   const int64_t d_ovov[4] = {o, v, o, v};
   X.sort4(g_ovov_.as<double>(), d_ovov, "2341", G, 1.0, 0.0);   // G(c,l,d,k) = g_kcld
   X.gemm('N', 'N', N, N, N, -0.5, G, N, Tm, N, 1.0, C, N, prec);
   double* Gc = X.buf(SL_E, "c2_Gc", N * N);                 // 2 G(p,s,r,q) - G(p,q,r,s)
-  X.sort4(G, d, "1432", Gc, 2.0, 0.0);
-  X.sort4(G, d, "1234", Gc, -1.0, 1.0);
+  X.sort4(G, d, "1432", Gc, 2.0, 0.0, G, -1.0);
   X.gemm('N', 'N', N, N, N, 0.5, Gc, N, U, N, 1.0, D, N, prec);
   double* W = X.buf(SL_B, "c2_W", N * N);
   X.gemm('N', 'N', N, N, N, -1.5, Tm, N, C, N, 0.0, W, N, prec);

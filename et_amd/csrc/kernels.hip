@@ -37,9 +37,11 @@ __device__ inline int64_t pidx(int64_t x, int64_t y) {
 // element-wise divisions then cost a fraction of the 64-bit ones)
 template <typename I>
 __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict__ y, I e0, I e1, I e2,
-                                I e3, I s0, I s1, I s2, I s3, double alpha, double beta, int64_t sx, int64_t sy) {
+                                I e3, I s0, I s1, I s2, I s3, double alpha, double beta, int64_t sx, int64_t sy,
+                                const double* z, double gamma, int64_t sz) {
   x += int64_t(blockIdx.z) * sx;
   y += int64_t(blockIdx.z) * sy;
+  z += int64_t(blockIdx.z) * sz;
   const I n = e0 * e1 * e2 * e3;
   for (I idx = I(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += I(gridDim.x) * blockDim.x) {
     I r = idx;
@@ -47,7 +49,8 @@ __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict
     const I o1 = r % e1; r /= e1;
     const I o2 = r % e2;
     const I o3 = r / e2;
-    const double v = alpha * x[o0 * s0 + o1 * s1 + o2 * s2 + o3 * s3];
+    double v = alpha * x[o0 * s0 + o1 * s1 + o2 * s2 + o3 * s3];
+    if (gamma != 0.0) v += gamma * z[idx];
     y[idx] = (beta == 0.0) ? v : v + beta * y[idx];
   }
 }
@@ -59,9 +62,11 @@ __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict
 __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __restrict__ y,
                                       int64_t e0, int64_t ep, int64_t eq, int64_t er, int64_t s0,
                                       int64_t sq, int64_t sr, int64_t yp, int64_t yq, int64_t yr,
-                                      double alpha, double beta, int64_t bx, int64_t by) {
+                                      double alpha, double beta, int64_t bx, int64_t by, const double* z,
+                                      double gamma, int64_t bz) {
   x += int64_t(blockIdx.z) * bx;
   y += int64_t(blockIdx.z) * by;
+  z += int64_t(blockIdx.z) * bz;
   __shared__ double tile[32][33];
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t nt0 = (e0 + 31) / 32;
@@ -79,7 +84,8 @@ __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __re
       const int64_t ip = tp * 32 + k, i0 = t0 * 32 + tx;
       if (i0 < e0 && ip < ep) {
         double* dst = yb + i0 + ip * yp;
-        const double v = alpha * tile[tx][k];
+        double v = alpha * tile[tx][k];
+        if (gamma != 0.0) v += gamma * z[dst - y];
         *dst = (beta == 0.0) ? v : v + beta * *dst;
       }
     }
@@ -480,9 +486,13 @@ __global__ void fill_kernel(double* __restrict__ x, int64_t n, double value) {
 }  // namespace
 
 void permute4(hipStream_t s, const double* x, double* y, const int64_t e[4], const int64_t st[4],
-              double alpha, double beta, const Batch& b) {
+              double alpha, double beta, const Batch& b, const double* z, double gamma) {
   const int64_t n = e[0] * e[1] * e[2] * e[3];
   if (n == 0) return;
+  if (z == nullptr) {
+    z = y;                                      // not read
+    gamma = 0.0;
+  }
   int p = -1;                                   // output position of the input-fastest index
   for (int k = 0; k < 4; ++k)
     if (st[k] == 1 && e[k] > 1) p = k;
@@ -496,7 +506,7 @@ void permute4(hipStream_t s, const double* x, double* y, const int64_t e[4], con
     dim3 grid(unsigned(tiles), unsigned(std::min<int64_t>(others, 65535)), unsigned(b.n));
     permute4_tiled_kernel<<<grid, kBlock, 0, s>>>(x, y, e[0], e[p], e[oth[0]], e[oth[1]], st[0],
                                                   st[oth[0]], st[oth[1]], ostride[p], ostride[oth[0]],
-                                                  ostride[oth[1]], alpha, beta, b.x, b.y);
+                                                  ostride[oth[1]], alpha, beta, b.x, b.y, z, gamma, b.z);
     ETG_LAUNCH("permute4_tiled");
     return;
   }
@@ -504,15 +514,15 @@ void permute4(hipStream_t s, const double* x, double* y, const int64_t e[4], con
   if (n + int64_t(kBlock) * grid_for(n) <= int64_t(UINT32_MAX))
     permute4_kernel<uint32_t><<<grid_z(n, b.n), kBlock, 0, s>>>(
         x, y, uint32_t(e[0]), uint32_t(e[1]), uint32_t(e[2]), uint32_t(e[3]), uint32_t(st[0]), uint32_t(st[1]),
-        uint32_t(st[2]), uint32_t(st[3]), alpha, beta, b.x, b.y);
+        uint32_t(st[2]), uint32_t(st[3]), alpha, beta, b.x, b.y, z, gamma, b.z);
   else
     permute4_kernel<int64_t><<<grid_z(n, b.n), kBlock, 0, s>>>(x, y, e[0], e[1], e[2], e[3], st[0], st[1], st[2],
-                                                               st[3], alpha, beta, b.x, b.y);
+                                                               st[3], alpha, beta, b.x, b.y, z, gamma, b.z);
   ETG_LAUNCH("permute4");
 }
 
 void sort4(hipStream_t s, const double* x, const int64_t d[4], const char* perm, double* y,
-           double alpha, double beta, const Batch& b) {
+           double alpha, double beta, const Batch& b, const double* z, double gamma) {
   if (std::strlen(perm) != 4) fail("sort4: permutation must have 4 digits");
   const int64_t in_stride[4] = {1, d[0], d[0] * d[1], d[0] * d[1] * d[2]};
   int64_t e[4], st[4];
@@ -524,7 +534,7 @@ void sort4(hipStream_t s, const double* x, const int64_t d[4], const char* perm,
     e[k] = d[q];
     st[k] = in_stride[q];
   }
-  permute4(s, x, y, e, st, alpha, beta, b);
+  permute4(s, x, y, e, st, alpha, beta, b, z, gamma);
 }
 
 void squareup(hipStream_t s, const double* packed, double* full, int64_t N, const Batch& b) {

@@ -10,26 +10,28 @@
 namespace etg {
 
 // The same operation on n vectors in one launch: vector k of the input at x + k b.x,
-// of the output at y + k b.y.  One launch per vector costs more than the work below
+// of the output at y + k b.y (a second input at z + k b.z).  One launch per vector costs more than the work below
 // a few thousand elements (three roots of H2O-He: 19.2 -> 16.6 ms with the launches
 // of a pass merged and its zero fills left out).
 struct Batch {
-  int64_t n = 1, x = 0, y = 0;
+  int64_t n = 1, x = 0, y = 0, z = 0;
 };
 // The ladder's: packed vectors (t or omega) and the +- arrays.
 struct LadderBatch {
   int64_t n = 1, vec = 0, plus = 0, minus = 0;
 };
 
-// y[o0,o1,o2,o3] = alpha * x[...] + beta * y, where output index k runs over
-// dims out_dim[k] and reads x at sum_k o_k * src_stride[k].
+// y[o0,o1,o2,o3] = alpha * x[...] + beta * y (+ gamma * z in y's order), where output
+// index k runs over dims out_dim[k] and reads x at sum_k o_k * src_stride[k].
 void permute4(hipStream_t s, const double* x, double* y, const int64_t out_dim[4],
-              const int64_t src_stride[4], double alpha, double beta, const Batch& b = {});
+              const int64_t src_stride[4], double alpha, double beta, const Batch& b = {},
+              const double* z = nullptr, double gamma = 0.0);
 
-// Helper: y = alpha * permute(x) + beta * y for x of dims d (column-major) and
-// y laid out in the order `perm` (1-based digits, e.g. "1324": y(p,r,q,s) = x(p,q,r,s)).
+// Helper: y = alpha * permute(x) + beta * y (+ gamma * z) for x of dims d (column-major) and
+// y (and z) laid out in the order `perm` (1-based digits, e.g. "1324": y(p,r,q,s) = x(p,q,r,s)).
 void sort4(hipStream_t s, const double* x, const int64_t d[4], const char* perm, double* y,
-           double alpha = 1.0, double beta = 0.0, const Batch& b = {});
+           double alpha = 1.0, double beta = 0.0, const Batch& b = {}, const double* z = nullptr,
+           double gamma = 0.0);
 
 // full N x N symmetric matrix from packed storage
 void squareup(hipStream_t s, const double* packed, double* full, int64_t N, const Batch& b = {});

@@ -3,6 +3,7 @@
 #include "ops.hpp"
 
 #include <algorithm>
+#include <array>
 #include <cstring>
 
 #include "ccsd.hpp"
@@ -21,8 +22,8 @@ double* DirectOps::buf(int slot, const char* name, int64_t elems) {
 void DirectOps::gemm(const Gemm& g, Prec prec) { wf_.run_gemm(g, prec); }
 
 void DirectOps::sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
-                      double beta) {
-  etg::sort4(wf_.stream(), x, d, perm, y, alpha, beta);
+                      double beta, const double* z, double gamma) {
+  etg::sort4(wf_.stream(), x, d, perm, y, alpha, beta, Batch{}, z, gamma);
 }
 
 void DirectOps::squareup(const double* packed, double* full, int64_t N) {
@@ -288,7 +289,10 @@ bool Tape::adjoint_writes_whole(const Op& op, int k) const {
         return g.lda == ra && (g.batch == 1 || g.strideA == ra * ca) && is(g.A, ra * ca * g.batch);
       return g.ldb == rb && (g.batch == 1 || g.strideB == rb * cb) && is(g.B, rb * cb * g.batch);
     }
-    case SORT4: return find(op.y) != k && is(op.x, op.d[0] * op.d[1] * op.d[2] * op.d[3]);
+    case SORT4: {
+      const int64_t n = op.d[0] * op.d[1] * op.d[2] * op.d[3];
+      return find(op.y) != k && (is(op.x, n) || (op.x2 && is(op.x2, n)));
+    }
     case SYMSUM: return is(op.x, op.N * op.N);
     case SYMPACK: return is(op.x, op.nv * op.no * op.nv * op.no);
     case COPY_SUB: return find(op.y) != k && op.lds == op.m && is(op.x, op.m * op.n);
@@ -307,7 +311,7 @@ void Tape::gemm(const Gemm& g, Prec prec) {
 }
 
 void Tape::sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
-                 double beta) {
+                 double beta, const double* z, double gamma) {
   Op op;
   op.kind = SORT4;
   op.x = x;
@@ -316,8 +320,10 @@ void Tape::sort4(const double* x, const int64_t d[4], const char* perm, double* 
   std::strncpy(op.perm, perm, 4);
   op.alpha = alpha;
   op.beta = beta;
+  op.x2 = z;
+  op.f1 = z ? gamma : 0.0;
   ops_.push_back(op);
-  DirectOps::sort4(x, d, perm, y, alpha, beta);
+  DirectOps::sort4(x, d, perm, y, alpha, beta, z, gamma);
 }
 
 void Tape::squareup(const double* packed, double* full, int64_t N) {
@@ -452,6 +458,7 @@ void Tape::op_io(const Op& op, const double* in[3], const double* out[2]) {
     case COPY_SUB:
       in[0] = op.x;
       if (op.beta != 0.0) in[1] = op.y;
+      if (op.kind == SORT4) in[2] = op.x2;
       out[0] = op.y;
       break;
     case SQUAREUP:
@@ -661,7 +668,9 @@ void Tape::run_recipe_op(const Op& op, int k, double* base) {
     return rslots_[size_t(sl)].mem.as<double>() + (p - bufs_[size_t(q)]->base);
   };
   switch (op.kind) {
-    case SORT4: etg::sort4(s, in(op.x), op.d, op.perm, out(op.y), op.alpha, op.beta); break;
+    case SORT4:
+      etg::sort4(s, in(op.x), op.d, op.perm, out(op.y), op.alpha, op.beta, Batch{}, op.x2 ? in(op.x2) : nullptr, op.f1);
+      break;
     case SQUAREUP: etg::squareup(s, in(op.x), out(op.y), op.N); break;
     case COPY_SUB: etg::copy_sub(s, in(op.x), op.lds, out(op.y), op.ldd, op.m, op.n, op.alpha, op.beta); break;
     case FILL0: fill(s, out(op.y), op.n, 0.0); break;
@@ -678,6 +687,11 @@ void Tape::run_recipe_op(const Op& op, int k, double* base) {
 // ---------------------------------------------------------------------------
 
 namespace {
+// dims of permute(x) for x of dims d
+std::array<int64_t, 4> permuted(const int64_t d[4], const char* perm) {
+  return {d[perm[0] - '1'], d[perm[1] - '1'], d[perm[2] - '1'], d[perm[3] - '1']};
+}
+
 int64_t dense_size(const int64_t d[4]) { return d[0] * d[1] * d[2] * d[3]; }
 
 }  // namespace
@@ -867,10 +881,14 @@ void Tape::tangent(Prec prec, int64_t nb) {
     double* dy = deriv(op.y);
     const Batch b{nb, op.x ? dstride(op.x) : 0, dstride(op.y)};
     switch (op.kind) {
-      case SORT4:
-        if (dx) etg::sort4(s, dx, op.d, op.perm, dy, op.alpha, op.beta, b);
+      case SORT4: {
+        const double* dz = op.x2 ? deriv(op.x2) : nullptr;
+        const int64_t sz = dz ? dstride(op.x2) : 0;
+        if (dx) etg::sort4(s, dx, op.d, op.perm, dy, op.alpha, op.beta, Batch{nb, b.x, b.y, sz}, dz, op.f1);
+        else if (dz) etg::sort4(s, dz, permuted(op.d, op.perm).data(), "1234", dy, op.f1, op.beta, Batch{nb, sz, b.y});
         else scale_vectors(dy, dense_size(op.d), b.y, nb, op.beta);
         break;
+      }
       case SQUAREUP:
         if (dx) etg::squareup(s, dx, dy, op.N, b);
         else scale_vectors(dy, op.N * op.N, b.y, nb, 0.0);
@@ -954,19 +972,26 @@ void Tape::adjoint(Prec prec, int64_t nb) {
     const bool y_ends = ends(op.y);
     const double acc = fresh.empty() ? 1.0 : 0.0;
     switch (op.kind) {
-      case SORT4:
+      case SORT4: {
+        double* zb = op.x2 ? deriv(op.x2) : nullptr;
+        auto onto = [&](const double* p) {
+          return std::find(fresh.begin(), fresh.end(), find(p)) != fresh.end() ? 0.0 : 1.0;
+        };
+        const auto e = permuted(op.d, op.perm);
         if (xb) {
-          int64_t e[4];
           char inv[5] = {0, 0, 0, 0, 0};
-          for (int q = 0; q < 4; ++q) {
-            const int r = op.perm[q] - '1';
-            e[q] = op.d[r];
-            inv[r] = char('1' + q);
-          }
-          etg::sort4(s, yb, e, inv, xb, op.alpha, acc, b);
+          for (int q = 0; q < 4; ++q) inv[op.perm[q] - '1'] = char('1' + q);
+          // z the same array: both terms at once
+          if (op.x2 == op.x)
+            etg::sort4(s, yb, e.data(), inv, xb, op.alpha, onto(op.x), Batch{nb, sy, sx, sy}, yb, op.f1);
+          else
+            etg::sort4(s, yb, e.data(), inv, xb, op.alpha, onto(op.x), b);
         }
+        if (zb && op.x2 != op.x)
+          etg::sort4(s, yb, e.data(), "1234", zb, op.f1, onto(op.x2), Batch{nb, sy, dstride(op.x2)});
         if (!y_ends) scale_vectors(yb, dense_size(op.d), sy, nb, op.beta);
         break;
+      }
       case SQUAREUP:
         if (xb) packsum(s, yb, xb, op.N, b);
         if (!y_ends) scale_vectors(yb, op.N * op.N, sy, nb, 0.0);

