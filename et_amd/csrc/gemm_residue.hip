@@ -127,9 +127,17 @@ __global__ __launch_bounds__(256) void row_exponents_finish_kernel(const double*
 // 2. Residue packs.  Per modulus one plane of 1 KB chunks (16 rows x 64 k: lane
 // l holds 16 consecutive k of row l % 16 from 16 (l / 16) on), row blocks
 // outermost, k steps contiguous.  One wave forms the 15 chunks of a (row block,
-// k step).  About 125 VALU operations per element (8 per modulus) against 8
-// bytes read and 15 written: close to balanced with HBM.
+// k step).  About 75 VALU operations per element (5 per modulus) against 8
+// bytes read and 15 written: bound by HBM, 37 M elements in 200 us.  (With 125
+// operations, residues formed in FP32, 215; products of 1520^3 133 -> 127 us.)
 // ---------------------------------------------------------------------------
+// The 16 values are formed here, in the order of the source, not where they are used.
+__device__ inline void pin(uint32_t (&x)[16]) {
+#pragma unroll
+  for (int j = 0; j < 16; ++j) asm volatile("" : "+v"(x[j]));
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 constexpr int kPackLd = kDepth + 2;           // LDS row of a staged chunk (doubles)
 
 __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restrict__ X, int64_t ld, int64_t strideX,
@@ -172,14 +180,27 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
   u4* dst = P + bz * kModuli * plane + (rb * KS + ks) * 64 + lane;
 #pragma unroll
   for (int i = 0; i < kModuli; ++i) {
+    // residue_byte of the 16 elements side by side: a byte dot product's result can
+    // be read three operations later, and the compiler would wait that out each time
+    uint32_t x[16];
+    if (residue::kMod[i] == 256) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = lo[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = residue::byte_dot(lo[j], kC.low[i], kC.offset[i]);
+      pin(x);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = residue::byte_dot(hi[j], kC.high[i], x[j]);
+      pin(x);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) x[j] = residue::low_byte(x[j], kC.invf[i], kC.c[i]);
+    }
     u4 w;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      uint32_t b[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = residue::residue_byte(lo[4 * q + j], hi[4 * q + j], i);
-      const uint32_t p01 = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
-      const uint32_t p23 = __builtin_amdgcn_perm(b[3], b[2], 0x0c0c0400u);
+      const uint32_t p01 = __builtin_amdgcn_perm(x[4 * q + 1], x[4 * q], 0x0c0c0400u);
+      const uint32_t p23 = __builtin_amdgcn_perm(x[4 * q + 3], x[4 * q + 2], 0x0c0c0400u);
       w[q] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
     }
     dst[i * plane] = w;

@@ -73,11 +73,15 @@ constexpr uint64_t fraction80(int i, bool high) {
   return high ? uint64_t(f >> 40) : uint64_t(f & ((uint64_t(1) << 40) - 1));
 }
 
+constexpr uint32_t kBits23 = 0x4b000000u;         // the float 2^23
+
 struct Constants {
   // residues of an integer given as 8 unsigned bytes of (a' + 2^63): weights of
-  // the low and high four bytes, 256^j mod m, and -2^63 mod m
+  // the low and high four bytes, 256^j mod m, and -2^63 - 2^23 mod m with the bits
+  // of the float 2^23 on top
   uint32_t low[kModuli], high[kModuli], offset[kModuli];
-  float mf[kModuli], invf[kModuli];
+  uint32_t c[kModuli];                            // 256 - m
+  float invf[kModuli];
   double md[kModuli], invd[kModuli];
   double fhi[kModuli], flo[kModuli];
 };
@@ -90,8 +94,8 @@ constexpr Constants make_constants() {
     for (int j = 0; j < 8; ++j) w[j / 4] |= uint32_t(pow2_mod(8 * j, m) & 0xff) << (8 * (j % 4));
     c.low[i] = w[0];
     c.high[i] = w[1];
-    c.offset[i] = uint32_t((m - pow2_mod(63, m)) % m);
-    c.mf[i] = float(m);
+    c.offset[i] = kBits23 + uint32_t((2 * m - pow2_mod(63, m) - pow2_mod(23, m)) % m);
+    c.c[i] = uint32_t(256 - m);
     c.invf[i] = 1.0f / float(m);
     c.md[i] = double(m);
     c.invd[i] = 1.0 / double(m);
@@ -140,21 +144,31 @@ ETG_HD inline uint32_t byte_dot(uint32_t a, uint32_t b, uint32_t c) {
 #endif
 }
 
-// Symmetric residue of the integer modulo m_i: its two's complement in the low
-// byte of the returned word.  The byte dot products are below 2^20, so the FP32
-// arithmetic is exact; rounding to the nearest multiple cannot err, as a tie
-// occurs for m = 256 only, where 128 and -128 are the same byte.
-ETG_HD inline uint32_t residue_byte(uint32_t lo, uint32_t hi, int i) {
-  constexpr float kMagic = 12582912.0f;           // 1.5 2^23: adding it rounds to an integer
-  const float f = float(byte_dot(hi, kC.high[i], byte_dot(lo, kC.low[i], kC.offset[i])));
-  const float q = fmaf(f, kC.invf[i], kMagic) - kMagic;
-  const float r = fmaf(-q, kC.mf[i], f) + kMagic;
-  uint32_t bits;
-  __builtin_memcpy(&bits, &r, sizeof(bits));
-  return bits;
+// Low byte of a number x = 2^23 + v congruent to the integer, in [-128, 127] and
+// congruent too, from the bits of the float x (v < 2^23).  x / m is rounded by adding
+// 1.5 2^23, which leaves the quotient in the low bits, and x - q m is x + (256 - m) q
+// in the low byte.  The FP32 quotient may be one off where x / m is near a half; that
+// the result is in range then was checked for every x and every m.
+ETG_HD inline uint32_t low_byte(uint32_t x, float inv, uint32_t c) {
+  float f;
+  __builtin_memcpy(&f, &x, sizeof(f));
+  f = fmaf(f, inv, 12582912.0f);
+  uint32_t q;
+  __builtin_memcpy(&q, &f, sizeof(q));
+  return (q & 0xffffffu) * c + x;
 }
 
-// The same of an int32 sum (FP64 arithmetic, exact).
+// Symmetric residue of the integer modulo m_i: its two's complement in the low
+// byte of the returned word.  Four operations (two byte dot products, a fused
+// multiply-add and an integer one); with the byte sum converted to float and the
+// remainder formed there it took seven.
+ETG_HD inline uint32_t residue_byte(uint32_t lo, uint32_t hi, int i) {
+  if (kMod[i] == 256) return lo;                  // 2^63 is a multiple
+  return low_byte(byte_dot(hi, kC.high[i], byte_dot(lo, kC.low[i], kC.offset[i])), kC.invf[i], kC.c[i]);
+}
+
+// The same of an int32 sum (FP64 arithmetic, exact; the matrix cores are busy beside it,
+// and the four-operation form gained nothing there).
 ETG_HD inline uint32_t residue_byte_of_sum(int32_t s, double m, double inv) {
   constexpr double kMagic = 6755399441055744.0;   // 1.5 2^52
   const double t = double(s);
