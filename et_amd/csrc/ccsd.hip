@@ -39,7 +39,12 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   omega_.resize(sizeof(double) * (n_t1 + n_t2));
   g_ovov_.resize(sizeof(double) * N * N);
   red_partial_.resize(sizeof(double) * kReduceBlocks * kDotBatch);
-  red_result_.resize(sizeof(double) * 8);
+  try {
+    red_result_.resize_host(sizeof(double) * kResults);
+  } catch (const Error&) {                // no pinned memory: results are copied
+    (void)hipGetLastError();
+    red_result_.resize(sizeof(double) * kResults);
+  }
   work_.resize(kBigSlots);
   // small scratch, sized once for every use in the programs below
   small_[0].resize(sizeof(double) * n * n);
@@ -76,6 +81,22 @@ void CCSD::require(bool ok, const char* what) const {
 }
 
 void CCSD::synchronize() { ETG_HIP(hipStreamSynchronize(stream_)); }
+
+// n of the numbers that kernels left at `res` (in red_result_), after all that is queued.
+// The kernels write them to pinned host memory themselves: a copy costs a launch and a
+// staging round of its own, about 10 us for each of a solver's scalars.
+void CCSD::results(const double* res, int64_t n, double* host) {
+  if (!red_result_.on_host())
+    ETG_HIP(hipMemcpyAsync(host, res, sizeof(double) * n, hipMemcpyDeviceToHost, stream_));
+  synchronize();
+  if (red_result_.on_host()) std::copy(res, res + n, host);
+}
+
+double CCSD::result(const double* res) {
+  double v = 0.0;
+  results(res, 1, &v);
+  return v;
+}
 
 double* CCSD::scratch(int slot, int64_t elems, const char* name) {
   if (slot < kBigSlots) {
@@ -351,19 +372,13 @@ double CCSD::calculate_energy() {
   double* res = red_result_.as<double>();
   ccsd_energy(stream_, t_.as<double>(), t_.as<double>() + n_t1, g_ovov_.as<double>(), n_o, n_v,
               red_partial_.as<double>(), res);
-  double e = 0.0;
-  ETG_HIP(hipMemcpyAsync(&e, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-  synchronize();
-  return e;
+  return result(res);
 }
 
 double CCSD::omega_norm() {
   double* res = red_result_.as<double>() + 1;
   sum_squares(stream_, omega_.as<double>(), n_t1 + n_t2, red_partial_.as<double>(), res);
-  double e = 0.0;
-  ETG_HIP(hipMemcpyAsync(&e, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-  synchronize();
-  return std::sqrt(e);
+  return std::sqrt(result(res));
 }
 
 void CCSD::set_t2_to_mp2_guess() {

@@ -14,12 +14,12 @@
 namespace etg {
 
 // Lowest n_want eigenpairs of a small non-symmetric matrix on the device (one
-// wavefront; dimension <= 128): G (device, ld ldg) -> wr, wi (host, k values by
+// wavefront per root; dimension <= 128): G (device, ld ldg) -> wr, wi (host, k values by
 // ascending real part), X (device, k x n_want, ld ldx).  Throws on complex
 // wanted roots or QR non-convergence.
 void reduced_eigen_solve(hipStream_t stream, DeviceBuffer& workspace, const double* G_dev, int64_t k,
                          int64_t ldg, int64_t n_want, double* wr, double* wi, double* X_dev,
-                         int64_t ldx);
+                         int64_t ldx, double* pinned = nullptr);
 // The same solve with its workspace in a static device array (no allocation;
 // dimension <= 128).  Calls that overlap on one GPU share that array and race.
 void reduced_eigen_solve_noalloc(hipStream_t stream, const double* G_dev, int64_t k, int64_t ldg,
@@ -218,7 +218,13 @@ class CCSD {
   DeviceBuffer Lt_oo_, Lt_vo_, Lt_vv_, Lt_vvT_;   // L_t1 ov block equals L_mo ov
   DeviceBuffer h_, eps_, F_, t_, omega_, diff_;
   DeviceBuffer g_ovov_;                           // independent of t1 (ov block is not dressed)
-  DeviceBuffer red_partial_, red_result_;
+  DeviceBuffer red_partial_;
+  // numbers for the host, in pinned memory where there is some: scalars, then from
+  // kBlockResults on a Davidson block's and its eigenvalues
+  static constexpr int64_t kBlockResults = 16, kResults = 512;
+  DeviceBuffer red_result_;
+  void results(const double* res, int64_t n, double* host);
+  double result(const double* res);
   DeviceBuffer small_[4];
   std::vector<DeviceBuffer> work_;                // (ov)^2 scratch slots
 

@@ -300,7 +300,8 @@ __global__ __launch_bounds__(kLanes) void reduced_eigenvalues_kernel(const doubl
                                                                      int ldg, double* __restrict__ wr_out,
                                                                      double* __restrict__ wi_out,
                                                                      double* __restrict__ norm_out,
-                                                                     int* __restrict__ info) {
+                                                                     int* __restrict__ info,
+                                                                     double* __restrict__ host_out) {
   __shared__ double H[kLdH * kMaxRed];
   __shared__ double wr[kMaxRed], wi[kMaxRed], ort[kMaxRed];
   const int lane = threadIdx.x;
@@ -357,6 +358,7 @@ __global__ __launch_bounds__(kLanes) void reduced_eigenvalues_kernel(const doubl
   if (lane == 0) {
     *norm_out = anorm;
     *info = st;
+    if (host_out) host_out[2 * kMaxRed] = double(st);
   }
   if (st != 0) return;
   for (int i = lane; i < k; i += kLanes) {
@@ -367,6 +369,10 @@ __global__ __launch_bounds__(kLanes) void reduced_eigenvalues_kernel(const doubl
     }
     wr_out[rank] = wr[i];
     wi_out[rank] = wi[i];
+    if (host_out) {
+      host_out[rank] = wr[i];
+      host_out[kMaxRed + rank] = wi[i];
+    }
   }
 }
 
@@ -562,9 +568,11 @@ constexpr size_t kEigenWork = 2 * kMaxRed + 4 * kMaxRed * kMaxRed + 2;
 static __device__ __align__(256) double scratch[kEigenWork];
 
 // Launches the solve with its workspace at `base` (kEigenWork doubles) and
-// returns wr, wi to the host; throws on QR non-convergence.
+// returns wr, wi to the host (through 2 kMaxRed + 1 doubles of pinned memory where
+// the caller has some); throws on QR non-convergence.
 void reduced_eigen_launch(hipStream_t stream, double* base, const double* G_dev, int64_t k, int64_t ldg,
-                          int64_t n_want, double* wr, double* wi, double* X_dev, int64_t ldx) {
+                          int64_t n_want, double* wr, double* wi, double* X_dev, int64_t ldx,
+                          double* pinned = nullptr) {
   if (k < 1 || k > kMaxRed) fail("reduced eigenproblem: dimension must be in [1, 128]");
   if (n_want < 0 || n_want > k) fail("reduced eigenproblem: invalid number of wanted roots");
   if (ldg < k || ldx < k) fail("reduced eigenproblem: leading dimension below the dimension");
@@ -573,20 +581,22 @@ void reduced_eigen_launch(hipStream_t stream, double* base, const double* G_dev,
   double* dnorm = dwi + kMaxRed;
   int* dinfo = reinterpret_cast<int*>(dnorm + 1);
   double* work = dnorm + 2;                 // (2k)^2: a complex pair's system
-  reduced_eigenvalues_kernel<<<1, kLanes, 0, stream>>>(G_dev, int(k), int(ldg), dwr, dwi, dnorm, dinfo);
+  reduced_eigenvalues_kernel<<<1, kLanes, 0, stream>>>(G_dev, int(k), int(ldg), dwr, dwi, dnorm, dinfo, pinned);
   ETG_LAUNCH("reduced_eigenvalues");
   if (n_want > 0) {
     reduced_eigenvectors_kernel<<<unsigned(n_want + 1), kLanes, 0, stream>>>(
         G_dev, int(k), int(ldg), int(n_want), dwr, dwi, dnorm, dinfo, X_dev, int(ldx), work);
     ETG_LAUNCH("reduced_eigenvectors");
   }
-  double host[2 * kMaxRed + 2];
-  ETG_HIP(hipMemcpyAsync(host, base, sizeof host, hipMemcpyDeviceToHost, stream));
+  double copy[2 * kMaxRed + 2];
+  if (!pinned) ETG_HIP(hipMemcpyAsync(copy, base, sizeof copy, hipMemcpyDeviceToHost, stream));
   ETG_HIP(hipStreamSynchronize(stream));
+  int info = 0;
+  if (!pinned) std::memcpy(&info, copy + 2 * kMaxRed + 1, sizeof info);
+  const double* host = pinned ? pinned : copy;
   std::copy(host, host + k, wr);
   std::copy(host + kMaxRed, host + kMaxRed + k, wi);
-  int info = 0;
-  std::memcpy(&info, host + 2 * kMaxRed + 1, sizeof info);
+  if (pinned) info = int(pinned[2 * kMaxRed]);
   if (info == 1) fail("reduced eigenproblem: QR iteration did not converge");
 }
 
@@ -613,10 +623,10 @@ double* scratch_address() {
 
 void reduced_eigen_solve(hipStream_t stream, DeviceBuffer& workspace, const double* G_dev, int64_t k,
                          int64_t ldg, int64_t n_want, double* wr, double* wi, double* X_dev,
-                         int64_t ldx) {
+                         int64_t ldx, double* pinned) {
   if (k < 1 || k > kMaxRed) fail("reduced eigenproblem: dimension must be in [1, 128]");
   workspace.resize(sizeof(double) * kEigenWork);
-  reduced_eigen_launch(stream, workspace.as<double>(), G_dev, k, ldg, n_want, wr, wi, X_dev, ldx);
+  reduced_eigen_launch(stream, workspace.as<double>(), G_dev, k, ldg, n_want, wr, wi, X_dev, ldx, pinned);
 }
 
 void reduced_eigen_solve_noalloc(hipStream_t stream, const double* G_dev, int64_t k, int64_t ldg,
@@ -629,7 +639,9 @@ void reduced_eigen_solve_noalloc(hipStream_t stream, const double* G_dev, int64_
 
 void CCSD::reduced_eigen(const double* G_dev, int64_t k, int64_t ldg, int64_t n_want, double* wr,
                          double* wi, double* X_dev, int64_t ldx) {
-  reduced_eigen_solve(stream_, red_eig_, G_dev, k, ldg, n_want, wr, wi, X_dev, ldx);
+  static_assert(kBlockResults + 2 * kMaxRed + 1 <= kResults, "room for the eigenvalues");
+  reduced_eigen_solve(stream_, red_eig_, G_dev, k, ldg, n_want, wr, wi, X_dev, ldx,
+                      red_result_.on_host() ? red_result_.as<double>() + kBlockResults : nullptr);
 }
 
 int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max_iterations,
@@ -659,7 +671,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   // otherwise AV, and then V as well, in pinned host memory that the kernels
   // read and write over PCIe (etg_set_davidson_space overrides the choice).
   dav_Y_.resize(sizeof(double) * size_t(n) * size_t(3 * s1));
-  dav_small_.resize(sizeof(double) * size_t(max_dim * max_dim + 2 * max_dim * s1 + 3 * s1 + max_dim + 2 * s1 * s1 + 2 * s1 + 2));
+  dav_small_.resize(sizeof(double) * size_t(max_dim * max_dim + 2 * max_dim * s1 + 3 * s1 + max_dim + 2 * s1 * s1 + s1));
   {
     const size_t space = sizeof(double) * size_t(n) * size_t(max_dim);
     size_t free_b = 0, total_b = 0;
@@ -705,8 +717,8 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   double* cvec = coef + 3 * s1;              // Gram-Schmidt coefficients (max_dim)
   double* gram = cvec + max_dim;             // Gram matrix of a block (s1 x s1)
   double* tmat = gram + s1 * s1;             // inverse Cholesky factor of a block (s1 x s1)
-  double* sums = tmat + s1 * s1;             // squared norms (2 s1)
-  double* flags = sums + 2 * s1;             // success of the two Cholesky factorisations
+  double* sums = tmat + s1 * s1;             // squared norms of the new vectors (s1)
+  double* flags = red_result_.as<double>() + 5;   // success of the two Cholesky factorisations
   diff_.resize(sizeof(double) * n);
   double* d = diff_.as<double>();
   orbital_differences(stream_, eps_.as<double>(), d, n_o, n_v, n);
@@ -714,10 +726,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   auto dot_host = [&](const double* a, const double* b) {
     double* res = red_result_.as<double>() + 3;
     dot(stream_, a, b, n, red_partial_.as<double>(), res);
-    double v = 0.0;
-    ETG_HIP(hipMemcpyAsync(&v, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-    synchronize();
-    return v;
+    return result(res);
   };
   // Cholesky QR twice of q columns at X, through W: X T with T = R^-1, R^T R =
   // X^T X, both times (and XA T alongside, through WA, when XA is given).  It gives
@@ -738,8 +747,7 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     multiply(X, XA, W, WA);
     factor(W, flags + 1);
     double ok[2];
-    ETG_HIP(hipMemcpyAsync(ok, flags, sizeof ok, hipMemcpyDeviceToHost, stream_));
-    synchronize();
+    results(flags, 2, ok);
     if (ok[0] == 0.0 || ok[1] == 0.0) return false;
     multiply(W, WA, X, XA);
     return true;
@@ -829,11 +837,11 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
     ritz_residual_kernel<<<grid_for_d(n * se), kBlock, 0, stream_>>>(AY, Y, coef, n, int(se), Rb);
     ETG_LAUNCH("ritz_residual");
     // squared norms of the Ritz vectors and of the residuals
-    dots(stream_, Y, n, Y, n, n, se, red_partial_.as<double>(), sums, 1);
-    dots(stream_, Rb, n, Rb, n, n, se, red_partial_.as<double>(), sums + se, 1);
+    double* sq = red_result_.as<double>() + kBlockResults;
+    dots(stream_, Y, n, Y, n, n, se, red_partial_.as<double>(), sq, 1);
+    dots(stream_, Rb, n, Rb, n, n, se, red_partial_.as<double>(), sq + se, 1);
     std::vector<double> ynorm(2 * se);
-    ETG_HIP(hipMemcpyAsync(ynorm.data(), sums, sizeof(double) * 2 * se, hipMemcpyDeviceToHost, stream_));
-    synchronize();                        // also: packed (host) is read by the copy above
+    results(sq, 2 * se, ynorm.data());    // also waits: packed (host) is read by the copy above
     const double* rnorm = ynorm.data() + se;
     bool converged = true;
     for (int64_t j = 0; j < se; ++j) {

@@ -64,7 +64,8 @@ __global__ void mirror_row_kernel(double* G, int ld, int s, int dim) {
 // One wavefront, a column of the augmented matrix per lane in LDS.  (One thread with the
 // matrix in its scratch memory took 35 us of a 0.7 ms iteration at dimension 8; 11 us.)
 __global__ __launch_bounds__(64) void diis_solve_kernel(const double* __restrict__ G, int ld, int dim,
-                                                        double* __restrict__ w, int* __restrict__ info) {
+                                                        double* __restrict__ w, int* __restrict__ info,
+                                                        double* __restrict__ info_out) {
   constexpr int kMax = CCSD::kMaxDiis + 1;
   static_assert(kMax < 64, "one lane per column");
   __shared__ double A[kMax][kMax + 2];
@@ -106,7 +107,10 @@ __global__ __launch_bounds__(64) void diis_solve_kernel(const double* __restrict
     }
     for (int i = 0; i < dim; ++i) w[i] = A[i][n];
   }
-  if (j == 0) *info = status;
+  if (j == 0) {
+    *info = status;
+    *info_out = double(status);
+  }
 }
 
 // x = sum_s w_s X_s over the dim records (diis_tool construct_extrapolated_vector).
@@ -218,7 +222,8 @@ void CCSD::diis_step(DiisSpace& d, const double* e, double* x) {
     ETG_LAUNCH("diis_mirror_row");
   };
   new_row();
-  diis_solve_kernel<<<1, 64, 0, stream_>>>(G, kMaxDiis, dim, d.w.as<double>(), d.info.as<int>());
+  double* info = red_result_.as<double>() + 4;
+  diis_solve_kernel<<<1, 64, 0, stream_>>>(G, kMaxDiis, dim, d.w.as<double>(), d.info.as<int>(), info);
   ETG_LAUNCH("diis_solve");
   extrapolate_kernel<<<grid_for_n(n), kBlock, 0, stream_>>>(X, n, dim, d.w.as<double>(),
                                                             d.info.as<int>(), x);
@@ -230,10 +235,7 @@ void CCSD::diis_step(DiisSpace& d, const double* e, double* x) {
     ETG_LAUNCH("diis_crop_error");
     new_row();
   }
-  int info = 0;
-  ETG_HIP(hipMemcpyAsync(&info, d.info.as<int>(), sizeof(int), hipMemcpyDeviceToHost, stream_));
-  synchronize();
-  if (info != 0) fail("diis_update: could not solve the DIIS matrix equation (zero pivot)");
+  if (result(info) != 0.0) fail("diis_update: could not solve the DIIS matrix equation (zero pivot)");
   ++d.count;
 }
 

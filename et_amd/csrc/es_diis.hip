@@ -58,10 +58,7 @@ int64_t CCSD::diis_excited_states(int side, int64_t n_states, double residual_th
   auto dot_host = [&](const double* a, const double* b) {
     double* res = red_result_.as<double>() + 3;
     dot(stream_, a, b, n, red_partial_.as<double>(), res);
-    double v = 0.0;
-    ETG_HIP(hipMemcpyAsync(&v, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-    synchronize();
-    return v;
+    return result(res);
   };
   if (start) {
     ETG_HIP(hipMemcpyAsync(X, start, sizeof(double) * n * s, hipMemcpyDefault, stream_));

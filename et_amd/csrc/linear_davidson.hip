@@ -93,10 +93,7 @@ int64_t CCSD::linear_davidson(int side, const double* F, const double* start, do
   auto dot_host = [&](const double* a, const double* b) {
     double* res = red_result_.as<double>() + 3;
     dot(stream_, a, b, n, red_partial_.as<double>(), res);
-    double v = 0.0;
-    ETG_HIP(hipMemcpyAsync(&v, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-    synchronize();
-    return v;
+    return result(res);
   };
   // y (host, k) -> out = M y for M = V or AV
   auto combine = [&](const double* M, const std::vector<double>& y, int64_t k, double* out) {

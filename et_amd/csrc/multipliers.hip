@@ -132,10 +132,7 @@ double CCSD::multiplier_residual_norm() {
   require(have_mres_, "multiplier_residual_norm: the multiplier equation has not been constructed");
   double* res = red_result_.as<double>() + 2;
   sum_squares(stream_, mres_.as<double>(), n_t1 + n_t2, red_partial_.as<double>(), res);
-  double e = 0.0;
-  ETG_HIP(hipMemcpyAsync(&e, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-  synchronize();
-  return std::sqrt(e);
+  return std::sqrt(result(res));
 }
 
 void CCSD::multiplier_quasi_newton_update() {
@@ -176,9 +173,7 @@ double CCSD::one_electron_expectation(const double* X) {
   tape_->tangent(Prec::F64, 1);
   double* res = red_result_.as<double>() + 3;
   dot(stream_, tbar_.as<double>(), tape_->deriv(omega_.as<double>()), n, red_partial_.as<double>(), res);
-  double lag = 0.0;
-  ETG_HIP(hipMemcpyAsync(&lag, res, sizeof(double), hipMemcpyDeviceToHost, stream_));
-  synchronize();
+  const double lag = result(res);
   double e = 0.0;
   for (int64_t i = 0; i < n_o; ++i) e += 2.0 * X[i + nm * i];
   for (int64_t i = 0; i < n_o; ++i)
