@@ -50,7 +50,7 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   small_[0].resize(sizeof(double) * n * n);
   small_[1].resize(sizeof(double) * n * n);
   small_[2].resize(sizeof(double) * std::max(std::max(n * n, J), o * o * o * o));
-  small_[3].resize(sizeof(double) * std::max(std::max(J * N, J * o * o), o * o * o * o));
+  small_[3].resize(sizeof(double) * std::max(J * o * n, o * o * o * o));
   // one workspace for the products that run as int8 ones, direct and in the
   // transformation passes (one stream): a whole (ov)^3 product takes 45 n_t1^2 bytes
   // (1.7 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
@@ -331,29 +331,18 @@ void CCSD::program_fock(Ops& X) {
   // Coulomb: F_pq += 2 sum_J L_pq X_J,  X_J = sum_k L_kk
   double* XJ = X.buf(SL_SMALL2, "fock_XJ", J);
   X.trace_oo(Loo, XJ);
-  double* c = X.buf(SL_SMALL0, "fock_coul_oo", o * o);
-  X.gemm('T', 'N', o * o, 1, J, 2.0, Loo, J, XJ, J, 0.0, c, o * o, Prec::F64);
-  X.copy_sub(c, o, F, n, o, o, 1.0, 1.0);
-  c = X.buf(SL_SMALL0, "fock_coul_ov", o * v);
-  X.gemm('T', 'N', o * v, 1, J, 2.0, Lov, J, XJ, J, 0.0, c, o * v, Prec::F64);
-  X.copy_sub(c, o, F + n * o, n, o, v, 1.0, 1.0);
-  c = X.buf(SL_SMALL0, "fock_coul_vo", v * o);
-  X.gemm('T', 'N', v * o, 1, J, 2.0, Lt_vo_.as<double>(), J, XJ, J, 0.0, c, v * o, Prec::F64);
-  X.copy_sub(c, v, F + o, n, v, o, 1.0, 1.0);
-  c = X.buf(SL_SMALL0, "fock_coul_vv", v * v);
-  X.gemm('T', 'N', v * v, 1, J, 2.0, Lt_vv_.as<double>(), J, XJ, J, 0.0, c, v * v, Prec::F64);
-  X.copy_sub(c, v, F + o + n * o, n, v, v, 1.0, 1.0);
-  // Exchange: F_pq -= sum_{J,k} L_pk L_kq with left factors reordered to (J, k, p)
-  double* Lleft = X.buf(SL_SMALL3, "fock_Lleft_oo", J * o * o);
-  const int64_t d_oo[4] = {J, o, o, 1};
-  X.sort4(Loo, d_oo, "1324", Lleft, 1.0, 0.0);                        // (J, k, i)
-  X.gemm('T', 'N', o, o, J * o, -1.0, Lleft, J * o, Loo, J * o, 1.0, F, n, Prec::F64);
-  X.gemm('T', 'N', o, v, J * o, -1.0, Lleft, J * o, Lov, J * o, 1.0, F + n * o, n, Prec::F64);
-  Lleft = X.buf(SL_SMALL3, "fock_Lleft_vo", J * o * v);
-  const int64_t d_vo[4] = {J, v, o, 1};
-  X.sort4(Lt_vo_.as<double>(), d_vo, "1324", Lleft, 1.0, 0.0);       // (J, k, a)
-  X.gemm('T', 'N', v, o, J * o, -1.0, Lleft, J * o, Loo, J * o, 1.0, F + o, n, Prec::F64);
-  X.gemm('T', 'N', v, v, J * o, -1.0, Lleft, J * o, Lov, J * o, 1.0, F + o + n * o, n, Prec::F64);
+  X.add_coulomb(Loo, o, o, XJ, F, "fock_coul_oo");
+  X.add_coulomb(Lov, o, v, XJ, F + n * o, "fock_coul_ov");
+  X.add_coulomb(Lt_vo_.as<double>(), v, o, XJ, F + o, "fock_coul_vo");
+  X.add_coulomb(Lt_vv_.as<double>(), v, v, XJ, F + o + n * o, "fock_coul_vv");
+  // Exchange: F_pq -= sum_{J,k} L_pk L_kq with left factors reordered to (J, k, p), p over
+  // the occupied and then the virtual orbitals: two products for the four blocks
+  double* Lleft = X.buf(SL_SMALL3, "fock_Lleft", J * o * n);
+  const int64_t d_oo[4] = {J, o, o, 1}, d_vo[4] = {J, v, o, 1};
+  X.sort4(Loo, d_oo, "1324", Lleft, 1.0, 0.0);                                       // (J, k, i)
+  X.sort4(Lt_vo_.as<double>(), d_vo, "1324", Lleft + J * o * o, 1.0, 0.0);           // (J, k, a)
+  X.gemm('T', 'N', n, o, J * o, -1.0, Lleft, J * o, Loo, J * o, 1.0, F, n, Prec::F64);
+  X.gemm('T', 'N', n, v, J * o, -1.0, Lleft, J * o, Lov, J * o, 1.0, F + n * o, n, Prec::F64);
 }
 
 void CCSD::construct_fock() {

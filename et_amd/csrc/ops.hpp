@@ -51,6 +51,9 @@ class Ops {
   virtual void trace_oo(const double* Loo, double* XJ) = 0;
   // f(b + v j) = F(j, o + b)
   virtual void fock_ov_vec(const double* F, double* f) = 0;
+  // F(p, q) += 2 sum_J L(J, p, q) x(J) on a rows x cols block of the Fock matrix
+  virtual void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
+                           const char* name) = 0;
   // packed Omega doubles += ladder term sum_cd g_acbd t_cidj (g from the (J, c, a) vv block)
   virtual void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) = 0;
 
@@ -103,6 +106,8 @@ class DirectOps : public Ops {
   void t1_xy(const double* t1, double* X, double* Y) override;
   void trace_oo(const double* Loo, double* XJ) override;
   void fock_ov_vec(const double* F, double* f) override;
+  void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
+                   const char* name) override;
   void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) override;
 
  protected:
@@ -130,6 +135,8 @@ class Tape : public DirectOps {
   void t1_xy(const double* t1, double* X, double* Y) override;
   void trace_oo(const double* Loo, double* XJ) override;
   void fock_ov_vec(const double* F, double* f) override;
+  void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
+                   const char* name) override;
   void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) override;
 
   // Buffers that exist outside the tape.  Constant ones carry no derivative;
