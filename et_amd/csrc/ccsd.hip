@@ -290,11 +290,11 @@ void CCSD::program_t1_cholesky(Ops& X) {
   double* Lvo = Lt_vo_.as<double>();
   double* Lvv = Lt_vv_.as<double>();
   // oo: L_ij = L_ij + sum_a L_ia t_aj          ((J i) x a) (a x j)
-  X.copy_sub(Lmo_oo_.as<double>(), J * o * o, Loo, J * o * o, J * o * o, 1, 1.0, 0.0);
-  X.gemm('N', 'N', J * o, o, v, 1.0, Lmo_ov_.as<double>(), J * o, t1, v, 1.0, Loo, J * o, Prec::F64);
+  X.gemm_from(Lmo_oo_.as<double>(), J * o, make_gemm('N', 'N', J * o, o, v, 1.0, Lmo_ov_.as<double>(), J * o, t1, v, 0.0, Loo,
+                                                     J * o), Prec::F64);
   // vo: L_ai = L_ai + sum_b L_ab t_bi - sum_j t_aj L'_ji   (L' = dressed oo block)
-  X.copy_sub(Lmo_vo_.as<double>(), J * v * o, Lvo, J * v * o, J * v * o, 1, 1.0, 0.0);
-  X.gemm('N', 'N', J * v, o, v, 1.0, Lmo_vv_.as<double>(), J * v, t1, v, 1.0, Lvo, J * v, Prec::F64);
+  X.gemm_from(Lmo_vo_.as<double>(), J * v, make_gemm('N', 'N', J * v, o, v, 1.0, Lmo_vv_.as<double>(), J * v, t1, v, 0.0, Lvo,
+                                                     J * v), Prec::F64);
   X.gemm_batched('N', 'T', J, v, o, -1.0, Loo, J, J * o, t1, v, 0, 1.0, Lvo, J, J * v, o, Prec::F64);
   // vv: L_ab = L_ab - sum_j t_aj L_jb         batched over b: (J x j)(j x a)
   X.copy_sub(Lmo_vv_.as<double>(), J * v * v, Lvv, J * v * v, J * v * v, 1, 1.0, 0.0);
@@ -427,11 +427,11 @@ void CCSD::omega_singles(Ops& X, Prec prec, const double* U) {
   const int64_t o = n_o, v = n_v, J = n_J, N = n_t1, n = n_mo;
   double* om1 = omega_.as<double>();
   // Omega_ai = F_ai                                    (omega_ccs.F90:62-86)
-  X.copy_sub(F_.as<double>() + o, n, om1, v, v, o, 1.0, 0.0);
   // A1: X_Jbi = sum_cj L^mo_Jcj u_cjbi ; Omega_ai += sum_Jb L^T1_Jab X_Jbi   (omega_doubles.F90:36-139)
   double* Xj = X.buf(SL_SMALL3, "a1_X", J * N);
   X.gemm('N', 'N', J, N, N, 1.0, Lmo_vo_.as<double>(), J, U, N, 0.0, Xj, J, prec);
-  X.gemm('T', 'N', v, o, J * v, 1.0, Lt_vvT_.as<double>(), J * v, Xj, J * v, 1.0, om1, v, prec);
+  X.gemm_from(F_.as<double>() + o, n, make_gemm('T', 'N', v, o, J * v, 1.0, Lt_vvT_.as<double>(), J * v, Xj, J * v, 0.0, om1, v),
+              prec);
   // B1: Omega_ai -= sum_jbk u_ajbk g_kbji             (omega_doubles.F90:141-205)
   double* g_kbji = X.buf(SL_A, "b1_g_kbji", o * v * o * o);
   double* g_jbki = X.buf(SL_B, "b1_g_jbki", o * v * o * o);
@@ -457,11 +457,9 @@ void CCSD::omega_e2_b2(Ops& X, Prec prec, const double* T, const double* U) {
   double* om = X.buf(SL_B, "e2_omega", N * N);
   double* Xbc = X.buf(SL_SMALL0, "e2_X", v * v);
   double* Ykj = X.buf(SL_SMALL1, "e2_Y", o * o);
-  X.copy_sub(F + o + n * o, n, Xbc, v, v, v, 1.0, 0.0);
-  X.gemm('N', 'N', v, v, o * v * o, -1.0, u_e2, v, g_ovov, o * v * o, 1.0, Xbc, v, prec);
+  X.gemm_from(F + o + n * o, n, make_gemm('N', 'N', v, v, o * v * o, -1.0, u_e2, v, g_ovov, o * v * o, 0.0, Xbc, v), prec);
   X.gemm('N', 'N', v, o * v * o, v, 1.0, Xbc, v, T, v, 0.0, om, v, prec);
-  X.copy_sub(F, n, Ykj, o, o, o, 1.0, 0.0);
-  X.gemm('N', 'N', o, o, v * o * v, 1.0, g_ovov, o, u_e2, v * o * v, 1.0, Ykj, o, prec);
+  X.gemm_from(F, n, make_gemm('N', 'N', o, o, v * o * v, 1.0, g_ovov, o, u_e2, v * o * v, 0.0, Ykj, o), prec);
   X.gemm('N', 'N', v * o * v, o, o, -1.0, T, v * o * v, Ykj, o, 1.0, om, v * o * v, prec);
   // symmetric sum
   double* om2 = X.buf(SL_C, "e2_omega_sym", N * N);
@@ -641,7 +639,9 @@ void CCSD::ladder_G(const Block& b, const double* LT, Prec prec, bool fp32, uint
     whole.C = nullptr;
     whole.Cf = gblk_.as<float>();
   }
-  if ((prec == Prec::BF16X3 && split_bf16_pays(whole)) || runs_as_residues(whole, prec, gws_cur_)) {
+  // (small blocks whole too: 361 x 361 x 279 is one launch of 5 us, as strips three)
+  if ((prec == Prec::BF16X3 && split_bf16_pays(whole)) || runs_as_residues(whole, prec, gws_cur_) ||
+      2.0 * double(v * b.la) * double(v * b.lb) * double(J) < 3e8) {
     run_gemm(whole, prec);
     return;
   }

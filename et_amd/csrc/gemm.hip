@@ -18,6 +18,7 @@
 // that tiles sharing A rows / B columns run close together in time on the
 // same L2.
 #include "gemm.hpp"
+#include "kernels.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -50,6 +51,8 @@ struct Params {
   double* W;
   int64_t k_per_split;
   int tiles_m, tiles_n;
+  const double* Cin;                 // Gemm::Cin (gemm_few_tiles; beta is 1)
+  int64_t ldcin;
 };
 
 __device__ inline void map_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
@@ -393,7 +396,8 @@ __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
       p.W[(split + bz * gridDim.y) * p.m * p.n + row + col * p.m] = v;
     } else {
       double* c = p.C + bz * p.strideC + row + col * p.ldc;
-      *c = (p.beta == 0.0) ? p.alpha * v : p.alpha * v + p.beta * *c;
+      const double* c0 = p.Cin ? p.Cin + row + col * p.ldcin : c;
+      *c = (p.beta == 0.0) ? p.alpha * v : p.alpha * v + p.beta * *c0;
     }
   }
 }
@@ -409,7 +413,8 @@ __global__ void scale_matrix(double* C, int64_t m, int64_t n, int64_t ldc, int64
 
 // C = alpha * sum_s W_s + beta * C for split-K partials.
 __global__ void splitk_reduce(const double* __restrict__ W, int splits, int64_t m, int64_t n,
-                              double alpha, double beta, double* C, int64_t ldc, int64_t strideC) {
+                              double alpha, double beta, double* C, int64_t ldc, int64_t strideC,
+                              const double* Cin, int64_t ldcin) {
   const int64_t bz = blockIdx.z;
   const int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (idx >= m * n) return;
@@ -418,8 +423,9 @@ __global__ void splitk_reduce(const double* __restrict__ W, int splits, int64_t 
   double s = 0.0;
   for (int q = 0; q < splits; ++q) s += w[int64_t(q) * m * n];
   double* c = C + bz * strideC + row + col * ldc;
+  const double* c0 = Cin ? Cin + row + col * ldcin : c;
   const double v = alpha * s;
-  *c = (beta == 0.0) ? v : v + beta * *c;
+  *c = (beta == 0.0) ? v : v + beta * *c0;
 }
 
 // The same for many splits of few outputs: 32 outputs per workgroup, eight threads
@@ -427,7 +433,7 @@ __global__ void splitk_reduce(const double* __restrict__ W, int splits, int64_t 
 // output would wait for a load per split: 95 us for 380 splits of 400 outputs).
 __global__ __launch_bounds__(256) void splitk_reduce_deep(const double* __restrict__ W, int splits, int64_t m, int64_t n,
                                                           double alpha, double beta, double* C, int64_t ldc,
-                                                          int64_t strideC) {
+                                                          int64_t strideC, const double* Cin, int64_t ldcin) {
   __shared__ double part[8][32];
   const int64_t bz = blockIdx.z;
   const int o = threadIdx.x & 31, g = threadIdx.x >> 5;
@@ -443,18 +449,19 @@ __global__ __launch_bounds__(256) void splitk_reduce_deep(const double* __restri
   if (g != 0 || idx >= m * n) return;
   for (int q = 1; q < 8; ++q) s += part[q][o];
   double* c = C + bz * strideC + (idx % m) + (idx / m) * ldc;
+  const double* c0 = Cin ? Cin + (idx % m) + (idx / m) * ldcin : c;
   const double v = alpha * s;
-  *c = (beta == 0.0) ? v : v + beta * *c;
+  *c = (beta == 0.0) ? v : v + beta * *c0;
 }
 
 void reduce_splits(hipStream_t stream, const Gemm& g, const double* W, int splits) {
   const int64_t mn = g.m * g.n;
   if (splits >= 16)
     splitk_reduce_deep<<<dim3(unsigned(ceil_div(mn, 32)), 1, unsigned(g.batch)), 256, 0, stream>>>(
-        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC);
+        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC, g.Cin, g.ldcin);
   else
     splitk_reduce<<<dim3(unsigned(ceil_div(mn, 256)), 1, unsigned(g.batch)), 256, 0, stream>>>(
-        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC);
+        W, splits, g.m, g.n, g.alpha, g.beta, g.C, g.ldc, g.strideC, g.Cin, g.ldcin);
   ETG_LAUNCH("splitk_reduce");
 }
 
@@ -544,6 +551,7 @@ Params split_params(const Gemm& g, GemmWorkspace* ws, int want, int* splits) {
   p.A = g.A; p.lda = g.lda; p.strideA = g.strideA;
   p.B = g.B; p.ldb = g.ldb; p.strideB = g.strideB;
   p.C = g.C; p.ldc = g.ldc; p.strideC = g.strideC;
+  p.Cin = g.Cin; p.ldcin = g.ldcin;
   p.W = nullptr;
   p.k_per_split = g.k;
   *splits = want;
@@ -1010,6 +1018,18 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
   if (g.ldb < std::max<int64_t>(1, rowsB)) fail("gemm: ldb too small");
   if (g.ldc < std::max<int64_t>(1, g.m)) fail("gemm: ldc too small");
   if (g.batch > 65535) fail("gemm: batch too large");
+  if (g.Cin != nullptr) {
+    if (g.batch != 1 || g.ldcin < g.m) fail("gemm: inconsistent input C");
+    Gemm h = g;
+    h.beta = 1.0;
+    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) && few_tiles_pay(g) &&
+                     !(prec == Prec::BF16X3 && split_bf16_pays(g)) &&
+                     !(prec != Prec::F32 && runs_as_residues(g, Prec::F64, ws));
+    if (few) return prec == Prec::F32 ? launch_typed<float>(stream, h, ws) : launch_typed<double>(stream, h, ws);
+    copy_sub(stream, g.Cin, g.ldcin, g.C, g.ldc, g.m, g.n, 1.0, 0.0);
+    h.Cin = nullptr;
+    return gemm(stream, h, prec, ws);
+  }
   if (g.k == 0) {
     const int64_t mn = g.m * g.n;
     dim3 grid(unsigned(ceil_div(mn, 256)), 1, unsigned(g.batch));

@@ -31,6 +31,10 @@ struct Gemm {
   double* C = nullptr;
   int64_t ldc = 0, strideC = 0;
   int64_t batch = 1;
+  // When set: C = alpha op(A) op(B) + Cin instead (no batch; Cin m x n apart from C, beta
+  // ignored).  The products of few tiles read it themselves, for the others it is copied.
+  const double* Cin = nullptr;
+  int64_t ldcin = 0;
   // Nonzero: the caller guarantees that A holds the same data whenever it passes
   // this tag, so the split-bf16 path may reuse the packed A of an earlier call.
   uint64_t a_tag = 0;

@@ -21,6 +21,13 @@ double* DirectOps::buf(int slot, const char* name, int64_t elems) {
 
 void DirectOps::gemm(const Gemm& g, Prec prec) { wf_.run_gemm(g, prec); }
 
+void DirectOps::gemm_from(const double* src, int64_t lds, const Gemm& g, Prec prec) {
+  Gemm h = g;
+  h.Cin = src;
+  h.ldcin = lds;
+  wf_.run_gemm(h, prec);
+}
+
 void DirectOps::sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
                       double beta, const double* z, double gamma) {
   etg::sort4(wf_.stream(), x, d, perm, y, alpha, beta, Batch{}, z, gamma);
@@ -316,6 +323,25 @@ void Tape::gemm(const Gemm& g, Prec prec) {
   op.prec = prec;
   ops_.push_back(op);
   DirectOps::gemm(g, prec);
+}
+
+// The derivative of a constant src is zero: the passes have a product that writes.  Any
+// other src is recorded as the copy and the product that it stands for.
+void Tape::gemm_from(const double* src, int64_t lds, const Gemm& g, Prec prec) {
+  if (!bufs_[size_t(find(src))]->constant) {
+    copy_sub(src, lds, g.C, g.ldc, g.m, g.n, 1.0, 0.0);
+    Gemm h = g;
+    h.beta = 1.0;
+    gemm(h, prec);
+    return;
+  }
+  Op op;
+  op.kind = GEMM;
+  op.g = g;
+  op.g.beta = 0.0;
+  op.prec = prec;
+  ops_.push_back(op);
+  DirectOps::gemm_from(src, lds, g, prec);
 }
 
 void Tape::sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,

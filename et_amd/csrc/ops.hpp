@@ -31,6 +31,9 @@ class Ops {
   // scratch buffer: `slot` is the reuse slot of the direct program, `name` its identity on a tape
   virtual double* buf(int slot, const char* name, int64_t elems) = 0;
   virtual void gemm(const Gemm& g, Prec prec) = 0;
+  // C = src (ld lds) + alpha op(A) op(B): a small product reads src itself, one launch
+  // instead of a copy and a product (4.6 us in a chain of small ones)
+  virtual void gemm_from(const double* src, int64_t lds, const Gemm& g, Prec prec) = 0;
   // y = alpha * permute(x) + beta * y (+ gamma * z)   (kernels.hpp sort4 semantics).
   // With z one pass replaces a copy and an accumulating sort: (H2O)8 0.31 -> 0.18 ms.
   virtual void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
@@ -92,6 +95,7 @@ class DirectOps : public Ops {
   double* buf(int slot, const char* name, int64_t elems) override;
   void gemm(const Gemm& g, Prec prec) override;
   using Ops::gemm;
+  void gemm_from(const double* src, int64_t lds, const Gemm& g, Prec prec) override;
   void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
              double beta, const double* z = nullptr, double gamma = 0.0) override;
   void squareup(const double* packed, double* full, int64_t N) override;
@@ -121,6 +125,7 @@ class Tape : public DirectOps {
   double* buf(int slot, const char* name, int64_t elems) override;
   void gemm(const Gemm& g, Prec prec) override;
   using Ops::gemm;
+  void gemm_from(const double* src, int64_t lds, const Gemm& g, Prec prec) override;
   void sort4(const double* x, const int64_t d[4], const char* perm, double* y, double alpha,
              double beta, const double* z = nullptr, double gamma = 0.0) override;
   void squareup(const double* packed, double* full, int64_t N) override;
