@@ -403,9 +403,7 @@ void CCSD::program_omega(Ops& X, Prec prec) {
   // t_aibj (full) and u_aibj = 2 t_aibj - t_ajbi      (omega_ccsd.F90:881-914)
   double* T = X.buf(SL_T, "t_aibj", N * N);
   double* U = X.buf(SL_U, "u_aibj", N * N);
-  X.squareup(t_.as<double>() + n_t1, T, N);
-  const int64_t d[4] = {n_v, n_o, n_v, n_o};
-  X.sort4(T, d, "1432", U, -1.0, 0.0, T, 2.0);
+  X.amplitudes(t_.as<double>() + n_t1, T, U);
   // singles: F_ai + doubles A1, B1, C1
   omega_singles(X, prec, U);
   // doubles: E2, symmetric sum, B2, 1/2 diagonal, pack, then C2/D2 and A2
@@ -462,12 +460,11 @@ void CCSD::omega_e2_b2(Ops& X, Prec prec, const double* T, const double* U) {
   X.gemm_from(F, n, make_gemm('N', 'N', o, o, v * o * v, 1.0, g_ovov, o, u_e2, v * o * v, 0.0, Ykj, o), prec);
   X.gemm('N', 'N', v * o * v, o, o, -1.0, T, v * o * v, Ykj, o, 1.0, om, v * o * v, prec);
   // symmetric sum
+  // and B2 in (a,b,i,j) order (omega_ccsd.F90:483-583), half of its g_aibj added before
+  X.gemm('T', 'N', N, N, J, 0.5, Lt_vo_.as<double>(), J, Lt_vo_.as<double>(), J, 1.0, om, N, prec);
   double* om2 = X.buf(SL_C, "e2_omega_sym", N * N);
-  X.symsum(om, om2, N);
-  // B2 in (a,b,i,j) order (omega_ccsd.F90:483-583), its g_aibj added before the sort
-  X.gemm('T', 'N', N, N, J, 1.0, Lt_vo_.as<double>(), J, Lt_vo_.as<double>(), J, 1.0, om2, N, prec);
   double* om_abij = X.buf(SL_A, "b2_omega_abij", N * N);
-  X.sort4(om2, d, "1324", om_abij, 1.0, 0.0);
+  X.symsum_abij(om, om2, om_abij);
   double* t_abij = X.buf(SL_B, "b2_t_abij", N * N);
   X.sort4(T, d, "1324", t_abij, 1.0, 0.0);
   double* g_kilj = X.buf(SL_SMALL3, "b2_g_kilj", o * o * o * o);
@@ -482,10 +479,7 @@ void CCSD::omega_e2_b2(Ops& X, Prec prec, const double* T, const double* U) {
   X.gemm('N', 'N', o * o, o * o, v * v, 1.0, g_klcd, o * o, t_abij, v * v, 1.0, X_klij, o * o, prec);
   X.gemm('N', 'N', v * v, o * o, o * o, 1.0, t_abij, v * v, X_klij, o * o, 1.0, om_abij, v * v, prec);
   // back to (a,i,b,j), 1/2 on the diagonal and pack into omega2   (omega_ccsd.F90:97-102)
-  double* om_aibj = X.buf(SL_C, "b2_omega_aibj", N * N);
-  const int64_t d_vvoo[4] = {v, v, o, o};
-  X.sort4(om_abij, d_vvoo, "1324", om_aibj, 1.0, 0.0);
-  X.packin(om_aibj, omega_.as<double>() + n_t1, N, 1.0, 0.0, 0.5);
+  X.packin_abij(om_abij, X.buf(SL_C, "b2_omega_aibj", N * N), omega_.as<double>() + n_t1);
 }
 
 void CCSD::omega_c2_d2(Ops& X, Prec prec, const double* Tfull, const double* U) {
@@ -515,10 +509,9 @@ void CCSD::omega_c2_d2(Ops& X, Prec prec, const double* Tfull, const double* U) 
   X.gemm('N', 'N', N, N, N, 0.5, Gc, N, U, N, 1.0, D, N, prec);
   double* W = X.buf(SL_B, "c2_W", N * N);
   X.gemm('N', 'N', N, N, N, -1.5, Tm, N, C, N, 0.0, W, N, prec);
-  X.sympack(W, omega_.as<double>() + n_t1, v, o, 1.0, 1.0 / 3.0, 2.0 / 3.0);
-  double* V = X.buf(SL_B, "c2_V", N * N);
+  double* V = X.buf(SL_C, "c2_V", N * N);
   X.gemm('N', 'N', N, N, N, 0.5, U, N, D, N, 0.0, V, N, prec);
-  X.sympack(V, omega_.as<double>() + n_t1, v, o, 1.0, 1.0, 0.0);
+  X.sympack_two(W, 1.0, 1.0 / 3.0, 2.0 / 3.0, V, omega_.as<double>() + n_t1);
 }
 
 // ---------------------------------------------------------------------------

@@ -167,13 +167,17 @@ __global__ void symmetric_sum_kernel(const double* __restrict__ x, double* __res
 // X block) stages x(Y, X) (read along Y), x(X, Y) (along X) and, when f2 != 0,
 // the two exchange terms x(p + v s, r + v q) (along p) and x(r + v q, p + v s)
 // (along r) for Y = p + v q, X = r + v s, then adds to packed element
-// X (X + 1) / 2 + Y, contiguous in Y for each X.
+// X (X + 1) / 2 + Y, contiguous in Y for each X.  TWO: `plain` is a second array,
+// added with alpha = f1 = 1, f2 = 0 (no batch).
+template <bool TWO>
 __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const double* __restrict__ x,
                                                                         double* __restrict__ y, int64_t n_v,
                                                                         int64_t N, double alpha, double f1,
-                                                                        double f2, int64_t sx, int64_t sy) {
+                                                                        double f2, int64_t sx, int64_t sy,
+                                                                        const double* __restrict__ plain) {
   x += int64_t(blockIdx.z) * sx;
   y += int64_t(blockIdx.z) * sy;
+  __shared__ double E[TWO ? 32 : 1][33], F[TWO ? 32 : 1][33];   // of plain, as A and B
   __shared__ double A[32][33], B[32][33];              // A[xl][yl] = x(Y, X), B[yl][xl] = x(X, Y)
   __shared__ double C[32][33], D[32][33];              // C[xl][yl] = x(p + v s, r + v q), D[yl][xl] = mirror
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
@@ -187,6 +191,10 @@ __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const do
     const int64_t Xr = X0 + tx, Yc = Y0 + k;            // B[k][tx] = x(X0 + tx, Y0 + k)
     const bool okB = Xr < N && Yc < N;
     B[k][tx] = okB ? x[Xr + N * Yc] : 0.0;
+    if constexpr (TWO) {
+      E[k][tx] = okA ? plain[Yr + N * Xc] : 0.0;
+      F[k][tx] = okB ? plain[Xr + N * Yc] : 0.0;
+    }
     if (exch) {
       // C[k][tx]: Y = Yr = p + v q, X = Xc = r + v s  ->  x(p + v s, r + v q)
       const int64_t p = Yr % n_v, q = Yr / n_v, r = Xc % n_v, sx = Xc / n_v;
@@ -208,6 +216,7 @@ __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const do
       if (exch) v += f2 * (C[k][tx] + D[tx][k]);
       v *= alpha;
     }
+    if constexpr (TWO) v += X == Y ? E[k][tx] : E[k][tx] + F[tx][k];
     y[X * (X + 1) / 2 + Y] += v;
   }
 }
@@ -230,6 +239,72 @@ __global__ void symmetrize_and_pack_kernel(const double* __restrict__ x, double*
     double v = f1 * (x[Y + N * X] + x[X + N * Y]);
     if (f2 != 0.0) v += f2 * (x[(p + n_v * s) + N * (r + n_v * q)] + x[(r + n_v * q) + N * (p + n_v * s)]);
     y[k] += alpha * v;
+  }
+}
+
+// ---- steps of the direct residual taken together (the recorded program keeps them apart) ----
+
+// full = t (N x N, symmetric) from packed storage, and u(ai, bj) = 2 t(ai, bj) - t(aj, bi).
+// As squareup_tiled, with the exchange terms of the tile read along X: for i >= j they lie
+// contiguously in a.
+__global__ __launch_bounds__(256) void squareup_and_u_kernel(const double* __restrict__ packed, double* __restrict__ full,
+                                                             double* __restrict__ u, int64_t n_v, int64_t N) {
+  __shared__ double P[32][33], Q[32][33];               // P[xl][yl] = t(X, Y), Q[yl][xl] = t(aj, bi)
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int64_t xb = tri_root(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
+  const int64_t X0 = xb * 32, Y0 = yb * 32;
+  for (int k = ty; k < 32; k += 8) {
+    const int64_t X = X0 + k, Y = Y0 + tx;
+    P[k][tx] = (X < N && Y <= X) ? packed[X * (X + 1) / 2 + Y] : 0.0;
+    const int64_t Xr = X0 + tx, Yc = Y0 + k;            // Xr = a + v i, Yc = b + v j
+    const int64_t a = Xr % n_v, i = Xr / n_v, b = Yc % n_v, j = Yc / n_v;
+    Q[k][tx] = (Xr < N && Yc <= Xr) ? packed[pidx(a + n_v * j, b + n_v * i)] : 0.0;
+  }
+  __syncthreads();
+  for (int k = ty; k < 32; k += 8) {
+    const int64_t X = X0 + k, Y = Y0 + tx;              // (Y, X), along Y
+    if (X < N && Y <= X) {
+      full[Y + N * X] = P[k][tx];
+      u[Y + N * X] = 2.0 * P[k][tx] - Q[tx][k];
+    }
+    const int64_t Xr = X0 + tx, Yc = Y0 + k;            // (Xr, Yc), along Xr
+    if (Xr < N && Yc <= Xr) {
+      full[Xr + N * Yc] = P[tx][k];
+      u[Xr + N * Yc] = 2.0 * P[tx][k] - Q[k][tx];
+    }
+  }
+}
+
+// y(a, b, i, j) = x(ai, bj) + x(bj, ai): one 32 x 32 tile of (a, b) for one (i, j) per workgroup.
+__global__ __launch_bounds__(256) void symsum_abij_kernel(const double* __restrict__ x, double* __restrict__ y,
+                                                          int64_t n_v, int64_t n_o) {
+  __shared__ double T[32][33];                          // T[a][b] = x(bj, ai)
+  const int64_t N = n_v * n_o, nt = (n_v + 31) / 32;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  const int64_t a0 = (blockIdx.x % nt) * 32, b0 = (blockIdx.x / nt) * 32;
+  for (int64_t ij = blockIdx.y; ij < n_o * n_o; ij += gridDim.y) {
+    const int64_t i = ij % n_o, j = ij / n_o;
+    for (int k = ty; k < 32; k += 8)
+      if (a0 + k < n_v && b0 + tx < n_v) T[k][tx] = x[(b0 + tx + n_v * j) + N * (a0 + k + n_v * i)];
+    __syncthreads();
+    for (int k = ty; k < 32; k += 8) {
+      const int64_t a = a0 + tx, b = b0 + k;
+      if (a < n_v && b < n_v) y[a + n_v * b + n_v * n_v * ij] = x[(a + n_v * i) + N * (b + n_v * j)] + T[tx][k];
+    }
+    __syncthreads();
+  }
+}
+
+// packin of the (a, i, b, j) order of x(a, b, i, j): packed element X = (a, i) >= Y = (b, j)
+// is x(b, a, j, i), contiguous in b, times diag_scale where X = Y.
+__global__ void packin_abij_kernel(const double* __restrict__ x, double* __restrict__ packed, int64_t n_v, int64_t n_o,
+                                   double diag_scale) {
+  const int64_t N = n_v * n_o, n = N * (N + 1) / 2;
+  for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < n; k += int64_t(gridDim.x) * blockDim.x) {
+    const int64_t X = tri_root(k), Y = k - X * (X + 1) / 2;
+    const int64_t i = X / n_v, a = X - i * n_v, j = Y / n_v, b = Y - j * n_v;
+    const double v = x[b + n_v * a + n_v * n_v * (j + n_o * i)];
+    packed[k] = X == Y ? diag_scale * v : v;
   }
 }
 
@@ -584,14 +659,40 @@ void symmetrize_and_pack(hipStream_t s, const double* x, double* packed, int64_t
   const int64_t N = n_v * n_o;
   if (N >= 32) {
     const int64_t nb = ceil_div(N, 32);
-    symmetrize_and_pack_tiled_kernel<<<dim3(unsigned(nb * (nb + 1) / 2), 1, unsigned(b.n)), kBlock, 0, s>>>(
-        x, packed, n_v, N, alpha, f1, f2, b.x, b.y);
+    symmetrize_and_pack_tiled_kernel<false><<<dim3(unsigned(nb * (nb + 1) / 2), 1, unsigned(b.n)), kBlock, 0, s>>>(
+        x, packed, n_v, N, alpha, f1, f2, b.x, b.y, nullptr);
     ETG_LAUNCH("symmetrize_and_pack_tiled");
     return;
   }
   symmetrize_and_pack_kernel<<<grid_z(N * (N + 1) / 2, b.n), kBlock, 0, s>>>(x, packed, n_v, n_o, alpha, f1, f2, b.x,
                                                                              b.y);
   ETG_LAUNCH("symmetrize_and_pack");
+}
+
+void symmetrize_and_pack_two(hipStream_t s, const double* x, const double* plain, double* packed, int64_t n_v,
+                             int64_t n_o, double alpha, double f1, double f2) {
+  const int64_t N = n_v * n_o, nb = ceil_div(N, 32);
+  symmetrize_and_pack_tiled_kernel<true><<<unsigned(nb * (nb + 1) / 2), kBlock, 0, s>>>(x, packed, n_v, N, alpha, f1, f2, 0, 0,
+                                                                                  plain);
+  ETG_LAUNCH("symmetrize_and_pack_two");
+}
+
+void squareup_and_u(hipStream_t s, const double* packed, double* full, double* u, int64_t n_v, int64_t n_o) {
+  const int64_t N = n_v * n_o, nb = ceil_div(N, 32);
+  squareup_and_u_kernel<<<unsigned(nb * (nb + 1) / 2), kBlock, 0, s>>>(packed, full, u, n_v, N);
+  ETG_LAUNCH("squareup_and_u");
+}
+
+void symsum_abij(hipStream_t s, const double* x, double* y, int64_t n_v, int64_t n_o) {
+  const int64_t nt = ceil_div(n_v, 32);
+  symsum_abij_kernel<<<dim3(unsigned(nt * nt), unsigned(std::min<int64_t>(n_o * n_o, 65535))), kBlock, 0, s>>>(x, y, n_v, n_o);
+  ETG_LAUNCH("symsum_abij");
+}
+
+void packin_abij(hipStream_t s, const double* x, double* packed, int64_t n_v, int64_t n_o, double diag_scale) {
+  const int64_t N = n_v * n_o;
+  packin_abij_kernel<<<grid_for(N * (N + 1) / 2), kBlock, 0, s>>>(x, packed, n_v, n_o, diag_scale);
+  ETG_LAUNCH("packin_abij");
 }
 
 void ladder_t_pm(hipStream_t s, const double* t2, double* tp, double* tm, int64_t n_o, int64_t n_v,

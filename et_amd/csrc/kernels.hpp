@@ -49,6 +49,17 @@ void symmetric_sum(hipStream_t s, const double* x, double* y, int64_t N, const B
 void symmetrize_and_pack(hipStream_t s, const double* x, double* packed, int64_t n_v, int64_t n_o,
                          double alpha, double f1, double f2, const Batch& b = {});
 
+// Steps of the direct residual taken together; each saves a pass over an (ov)^2 array and
+// a launch.  Both symmetrize_and_pack of x and of plain (alpha = f1 = 1, f2 = 0):
+void symmetrize_and_pack_two(hipStream_t s, const double* x, const double* plain, double* packed, int64_t n_v,
+                             int64_t n_o, double alpha, double f1, double f2);
+// squareup, and u = 2 t(ai, bj) - t(aj, bi)
+void squareup_and_u(hipStream_t s, const double* packed, double* full, double* u, int64_t n_v, int64_t n_o);
+// y(a, b, i, j) = x(ai, bj) + x(bj, ai)
+void symsum_abij(hipStream_t s, const double* x, double* y, int64_t n_v, int64_t n_o);
+// packin of x(a, b, i, j) taken in the order (a, i, b, j)
+void packin_abij(hipStream_t s, const double* x, double* packed, int64_t n_v, int64_t n_o, double diag_scale);
+
 // Ladder (+/-) helpers ------------------------------------------------------
 // t+ (o+ x v+): (1 - d_cd/2)(t_cidj + t_cjdi), rows ij (i <= j), cols cd (c <= d)
 // t- (o- x v-): t_cidj - t_cjdi, rows i < j, cols c < d

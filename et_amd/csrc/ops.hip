@@ -78,6 +78,24 @@ void DirectOps::add_coulomb(const double* L, int64_t rows, int64_t cols, const d
   gemm_batched('T', 'N', rows, 1, J, 2.0, L, J, J * rows, x, J, 0, 1.0, F, n, n, cols, Prec::F64);
 }
 
+void DirectOps::amplitudes(const double* t2, double* T, double* U) {
+  etg::squareup_and_u(wf_.stream(), t2, T, U, wf_.n_v, wf_.n_o);
+}
+
+void DirectOps::symsum_abij(const double* x, double* sym, double* abij) {
+  (void)sym;
+  etg::symsum_abij(wf_.stream(), x, abij, wf_.n_v, wf_.n_o);
+}
+
+void DirectOps::packin_abij(const double* abij, double* aibj, double* packed) {
+  (void)aibj;
+  etg::packin_abij(wf_.stream(), abij, packed, wf_.n_v, wf_.n_o, 0.5);
+}
+
+void DirectOps::sympack_two(const double* W, double alpha, double f1, double f2, const double* V, double* packed) {
+  etg::symmetrize_and_pack_two(wf_.stream(), W, V, packed, wf_.n_v, wf_.n_o, alpha, f1, f2);
+}
+
 void DirectOps::ladder(const double* t2, const double* LvvT, double* om2, Prec prec) {
   wf_.ladder_primal(t2, LvvT, om2, prec);
 }
@@ -469,6 +487,29 @@ void Tape::add_coulomb(const double* L, int64_t rows, int64_t cols, const double
   double* c = buf(SL_SMALL0, name, rows * cols);
   gemm('T', 'N', rows * cols, 1, J, 2.0, L, J, x, J, 0.0, c, rows * cols, Prec::F64);
   copy_sub(c, rows, F, wf_.n_mo, rows, cols, 1.0, 1.0);
+}
+
+void Tape::amplitudes(const double* t2, double* T, double* U) {
+  const int64_t d[4] = {wf_.n_v, wf_.n_o, wf_.n_v, wf_.n_o};
+  squareup(t2, T, wf_.n_t1);
+  sort4(T, d, "1432", U, -1.0, 0.0, T, 2.0);
+}
+
+void Tape::symsum_abij(const double* x, double* sym, double* abij) {
+  const int64_t d[4] = {wf_.n_v, wf_.n_o, wf_.n_v, wf_.n_o};
+  symsum(x, sym, wf_.n_t1);
+  sort4(sym, d, "1324", abij, 1.0, 0.0);
+}
+
+void Tape::packin_abij(const double* abij, double* aibj, double* packed) {
+  const int64_t d[4] = {wf_.n_v, wf_.n_v, wf_.n_o, wf_.n_o};
+  sort4(abij, d, "1324", aibj, 1.0, 0.0);
+  packin(aibj, packed, wf_.n_t1, 1.0, 0.0, 0.5);
+}
+
+void Tape::sympack_two(const double* W, double alpha, double f1, double f2, const double* V, double* packed) {
+  sympack(W, packed, wf_.n_v, wf_.n_o, alpha, f1, f2);
+  sympack(V, packed, wf_.n_v, wf_.n_o, 1.0, 1.0, 0.0);
 }
 
 void Tape::ladder(const double* t2, const double* LvvT, double* om2, Prec prec) {

@@ -57,6 +57,14 @@ class Ops {
   // F(p, q) += 2 sum_J L(J, p, q) x(J) on a rows x cols block of the Fock matrix
   virtual void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
                            const char* name) = 0;
+  // T = full matrix of the packed t2, U(ai, bj) = 2 T(ai, bj) - T(aj, bi)
+  virtual void amplitudes(const double* t2, double* T, double* U) = 0;
+  // abij(a, b, i, j) = x(ai, bj) + x(bj, ai); sym is the (ov)^2 scratch of a program in two steps
+  virtual void symsum_abij(const double* x, double* sym, double* abij) = 0;
+  // packed = abij in the order (a, i, b, j), half its diagonal; aibj is scratch likewise
+  virtual void packin_abij(const double* abij, double* aibj, double* packed) = 0;
+  // packed += sympack of W (alpha, f1, f2) and of V (1, 1, 0)
+  virtual void sympack_two(const double* W, double alpha, double f1, double f2, const double* V, double* packed) = 0;
   // packed Omega doubles += ladder term sum_cd g_acbd t_cidj (g from the (J, c, a) vv block)
   virtual void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) = 0;
 
@@ -112,6 +120,10 @@ class DirectOps : public Ops {
   void fock_ov_vec(const double* F, double* f) override;
   void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
                    const char* name) override;
+  void amplitudes(const double* t2, double* T, double* U) override;
+  void symsum_abij(const double* x, double* sym, double* abij) override;
+  void packin_abij(const double* abij, double* aibj, double* packed) override;
+  void sympack_two(const double* W, double alpha, double f1, double f2, const double* V, double* packed) override;
   void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) override;
 
  protected:
@@ -142,6 +154,10 @@ class Tape : public DirectOps {
   void fock_ov_vec(const double* F, double* f) override;
   void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
                    const char* name) override;
+  void amplitudes(const double* t2, double* T, double* U) override;
+  void symsum_abij(const double* x, double* sym, double* abij) override;
+  void packin_abij(const double* abij, double* aibj, double* packed) override;
+  void sympack_two(const double* W, double alpha, double f1, double f2, const double* V, double* packed) override;
   void ladder(const double* t2, const double* LvvT, double* om2, Prec prec) override;
 
   // Buffers that exist outside the tape.  Constant ones carry no derivative;
