@@ -188,9 +188,12 @@ void CCSD::run_gemm(const Gemm& g, Prec prec) {
     // algorithmic HBM bytes: read A and B once (once in all for an operand shared
     // by the batch), write C once (and read it if beta != 0)
     const double mn = double(g.m) * double(g.n), nbat = double(g.batch);
-    const double bytes = 8.0 * (double(g.m) * double(g.k) * (g.strideA == 0 ? 1.0 : nbat) +
-                                double(g.k) * double(g.n) * (g.strideB == 0 ? 1.0 : nbat) +
-                                (g.beta != 0.0 ? 2.0 : 1.0) * mn * nbat);
+    double bytes = 8.0 * (double(g.m) * double(g.k) * (g.strideA == 0 ? 1.0 : nbat) +
+                          double(g.k) * double(g.n) * (g.strideB == 0 ? 1.0 : nbat) +
+                          (g.beta != 0.0 || g.Cin != nullptr ? 2.0 : 1.0) * mn * nbat);
+    if (g.A2 != nullptr)
+      bytes += 8.0 * (double(g.m) * double(g.k) * (g.strideA2 == 0 ? 1.0 : nbat) +
+                      double(g.k) * double(g.n) * (g.strideB2 == 0 ? 1.0 : nbat));
     ledger_recs_.push_back(LedgerRec{info.kernel, gemm_flops(g), bytes, a, b});
   }
   last_omega_flops += gemm_flops(g);

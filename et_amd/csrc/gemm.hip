@@ -53,6 +53,10 @@ struct Params {
   int tiles_m, tiles_n;
   const double* Cin;                 // Gemm::Cin (gemm_few_tiles; beta is 1)
   int64_t ldcin;
+  // Gemm::A2, B2 (gemm_few_tiles): k runs over the first pair, padded to kpad (whole
+  // chunks of 16), then over the second
+  const double *A2, *B2;
+  int64_t strideA2, strideB2, kpad;
 };
 
 __device__ inline void map_tile(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
@@ -304,19 +308,23 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p) {
 // the waves' sums meet in LDS (summed in wave order).  Within a chunk lane group
 // l / 16 holds k = 4 (l / 16) .. + 3 and MFMA step s takes element s of each: every
 // lane reads 32 contiguous bytes of a k-contiguous operand, 16 lanes 128 of the other.
-template <typename T, bool TA, bool TB, int TM, int TN, int WK>
+// TWO: two pairs of operands of the same shape are summed, as one k range (a tangent
+// pass's dA B + A dB: one launch of a chain of small kernels, 4.6 us, instead of two).
+template <typename T, bool TA, bool TB, int TM, int TN, int WK, bool TWO>
 __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   __shared__ double red[WK][TM * TN * 256];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lcol = lane & 15, lk = 4 * (lane >> 4);
   const int64_t m0 = int64_t(blockIdx.x % p.tiles_m) * (16 * TM), n0 = int64_t(blockIdx.x / p.tiles_m) * (16 * TN);
   const int64_t bz = blockIdx.z, split = blockIdx.y;
-  const int64_t kbeg = split * p.k_per_split, kend = min(p.k, kbeg + p.k_per_split);
+  const int64_t kbeg = split * p.k_per_split, kend = min(TWO ? 2 * p.kpad : p.k, kbeg + p.k_per_split);
   const int64_t sa = TA ? 1 : p.lda, sb = TB ? p.ldb : 1;   // from one k to the next
   const double* pa[TM];
   const double* pb[TN];
+  const int64_t to_a2 = TWO ? (p.A2 + bz * p.strideA2) - (p.A + bz * p.strideA) : 0;
+  const int64_t to_b2 = TWO ? (p.B2 + bz * p.strideB2) - (p.B + bz * p.strideB) : 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i) {                           // rows past the edge repeat the last one
     const int64_t r = min(m0 + 16 * i + lcol, p.m - 1);
@@ -334,24 +342,33 @@ __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
     for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
   T a[2][TM][4], b[2][TN][4];
   auto load = [&](int at, int64_t k0) {
-    if (k0 + 16 <= kend) {
+    int64_t da = 0, db = 0, limit = kend;
+    if constexpr (TWO) {
+      limit = p.k;
+      if (k0 >= p.kpad) {
+        k0 -= p.kpad;
+        da = to_a2;
+        db = to_b2;
+      }
+    }
+    if (k0 + 16 <= limit) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) a[at][i][s] = M::cvt(pa[i][(k0 + lk + s) * sa]);
+        for (int s = 0; s < 4; ++s) a[at][i][s] = M::cvt(pa[i][da + (k0 + lk + s) * sa]);
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) b[at][j][s] = M::cvt(pb[j][(k0 + lk + s) * sb]);
+        for (int s = 0; s < 4; ++s) b[at][j][s] = M::cvt(pb[j][db + (k0 + lk + s) * sb]);
     } else {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const bool ok = k0 + lk + s < kend;
-        const int64_t k = ok ? k0 + lk + s : kbeg;
+        const bool ok = k0 + lk + s < limit;
+        const int64_t k = ok ? k0 + lk + s : (TWO ? 0 : kbeg);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[at][i][s] = ok ? M::cvt(pa[i][k * sa]) : T(0);
+        for (int i = 0; i < TM; ++i) a[at][i][s] = ok ? M::cvt(pa[i][da + k * sa]) : T(0);
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b[at][j][s] = ok ? M::cvt(pb[j][k * sb]) : T(0);
+        for (int j = 0; j < TN; ++j) b[at][j][s] = ok ? M::cvt(pb[j][db + k * sb]) : T(0);
       }
     }
   };
@@ -580,15 +597,15 @@ GemmLaunch run_choice(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, Choi
   return info;
 }
 
-template <typename T, int TM, int TN, int WK>
+template <typename T, int TM, int TN, int WK, bool TWO>
 const char* launch_few(hipStream_t stream, const Gemm& g, Params p, int splits) {
   p.tiles_m = int(ceil_div(g.m, 16 * TM));
   p.tiles_n = int(ceil_div(g.n, 16 * TN));
   const dim3 grid(unsigned(p.tiles_m) * unsigned(p.tiles_n), unsigned(splits), unsigned(g.batch));
-  if (!g.ta && !g.tb) gemm_few_tiles<T, false, false, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
-  else if (!g.ta && g.tb) gemm_few_tiles<T, false, true, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
-  else if (g.ta && !g.tb) gemm_few_tiles<T, true, false, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
-  else gemm_few_tiles<T, true, true, TM, TN, WK><<<grid, 64 * WK, 0, stream>>>(p);
+  if (!g.ta && !g.tb) gemm_few_tiles<T, false, false, TM, TN, WK, TWO><<<grid, 64 * WK, 0, stream>>>(p);
+  else if (!g.ta && g.tb) gemm_few_tiles<T, false, true, TM, TN, WK, TWO><<<grid, 64 * WK, 0, stream>>>(p);
+  else if (g.ta && !g.tb) gemm_few_tiles<T, true, false, TM, TN, WK, TWO><<<grid, 64 * WK, 0, stream>>>(p);
+  else gemm_few_tiles<T, true, true, TM, TN, WK, TWO><<<grid, 64 * WK, 0, stream>>>(p);
   ETG_LAUNCH("gemm_few_tiles");
   return sizeof(T) == 8 ? "gemm_few_tiles<f64>" : "gemm_few_tiles<f32>";
 }
@@ -715,6 +732,25 @@ bool few_tiles_pay(const Gemm& g) {
   return g.k > 128 || double(g.m) * double(g.n) * double(g.batch) < 4e5;
 }
 
+// Two pairs of few tiles as one k range.
+template <typename T>
+GemmLaunch launch_two(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
+  Gemm both = g;
+  both.k = 2 * (ceil_div(g.k, 16) * 16);
+  const FewChoice c = choose_few(both, ws != nullptr);
+  int splits = 1;
+  Params p = split_params(both, ws, c.splits, &splits);
+  p.k = g.k;
+  p.kpad = both.k / 2;
+  p.A2 = g.A2; p.strideA2 = g.strideA2;
+  p.B2 = g.B2; p.strideB2 = g.strideB2;
+  GemmLaunch info;
+  info.splits = splits;
+  info.kernel = c.tile == 16 ? launch_few<T, 1, 1, 4, true>(stream, g, p, splits) : launch_few<T, 2, 2, 4, true>(stream, g, p, splits);
+  if (splits > 1) reduce_splits(stream, g, p.W, splits);
+  return info;
+}
+
 template <typename T>
 GemmLaunch launch_rows(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
   if (few_tiles_pay(g)) {
@@ -723,7 +759,8 @@ GemmLaunch launch_rows(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
     const Params p = split_params(g, ws, c.splits, &splits);
     GemmLaunch info;
     info.splits = splits;
-    info.kernel = c.tile == 16 ? launch_few<T, 1, 1, 4>(stream, g, p, splits) : launch_few<T, 2, 2, 4>(stream, g, p, splits);
+    info.kernel = c.tile == 16 ? launch_few<T, 1, 1, 4, false>(stream, g, p, splits)
+                               : launch_few<T, 2, 2, 4, false>(stream, g, p, splits);
     if (splits > 1) reduce_splits(stream, g, p.W, splits);
     return info;
   }
@@ -1018,6 +1055,20 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
   if (g.ldb < std::max<int64_t>(1, rowsB)) fail("gemm: ldb too small");
   if (g.ldc < std::max<int64_t>(1, g.m)) fail("gemm: ldc too small");
   if (g.batch > 65535) fail("gemm: batch too large");
+  if (g.A2 != nullptr) {
+    if (g.Cin != nullptr || g.Cf != nullptr || g.b_packed != nullptr || g.a_tag != 0) fail("gemm: two operand pairs take no options");
+    Gemm one = g;
+    one.A2 = one.B2 = nullptr;
+    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) && few_tiles_pay(g) &&
+                     !(prec == Prec::BF16X3 && split_bf16_pays(one)) &&
+                     !(prec != Prec::F32 && runs_as_residues(one, Prec::F64, ws));
+    if (few) return prec == Prec::F32 ? launch_two<float>(stream, g, ws) : launch_two<double>(stream, g, ws);
+    gemm(stream, one, prec, ws);
+    one.A = g.A2; one.strideA = g.strideA2;
+    one.B = g.B2; one.strideB = g.strideB2;
+    one.beta = 1.0;
+    return gemm(stream, one, prec, ws);
+  }
   if (g.Cin != nullptr) {
     if (g.batch != 1 || g.ldcin < g.m) fail("gemm: inconsistent input C");
     Gemm h = g;

@@ -31,6 +31,11 @@ struct Gemm {
   double* C = nullptr;
   int64_t ldc = 0, strideC = 0;
   int64_t batch = 1;
+  // When set: C = alpha (op(A) op(B) + op(A2) op(B2)) + beta C, the second pair with the
+  // first one's shapes and leading dimensions.  Products of few tiles form both in one
+  // launch, others one after the other.
+  const double *A2 = nullptr, *B2 = nullptr;
+  int64_t strideA2 = 0, strideB2 = 0;
   // When set: C = alpha op(A) op(B) + Cin instead (no batch; Cin m x n apart from C, beta
   // ignored).  The products of few tiles read it themselves, for the others it is copied.
   const double* Cin = nullptr;
@@ -171,6 +176,7 @@ inline Gemm make_gemm(char ta, char tb, int64_t m, int64_t n, int64_t k, double 
 // Floating-point operations the product performs (2 m n k per batch entry; of a
 // lower block triangle those of its blocks).
 inline double gemm_flops(const Gemm& g) {
+  if (g.A2 != nullptr) return 4.0 * double(g.m) * double(g.n) * double(g.k) * double(g.batch);
   if (g.lower > 0) return double(g.m + g.lower) * double(g.n) * double(g.k);
   return 2.0 * double(g.m) * double(g.n) * double(g.k) * double(g.batch);
 }

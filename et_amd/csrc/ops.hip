@@ -811,14 +811,27 @@ void Tape::tangent_gemm(const Gemm& g, Prec prec, int64_t nb) {
       z.beta = g.beta;
       wf_.run_gemm(z, prec);
     }
-    double beta = g.beta;                 // of the first product; the second adds to it
+    if (dA && dB) {                       // dA B, then A dB
+      Gemm h = base;
+      h.A = dA + k * sA;
+      h.A2 = pA;
+      h.strideA2 = base.strideA;
+      h.B2 = dB + k * sB;
+      h.strideB2 = base.strideB;
+      if (vec_batch) {
+        h.strideA = sA;
+        h.strideB2 = sB;
+      }
+      wf_.run_gemm(h, prec);
+      continue;
+    }
+    const double beta = g.beta;
     if (dA) {
       Gemm h = base;
       h.A = dA + k * sA;
       if (vec_batch) h.strideA = sA;
       h.beta = beta;
       wf_.run_gemm(h, prec);
-      beta = 1.0;
     }
     if (dB) {
       Gemm h = base;
