@@ -334,10 +334,7 @@ void CCSD::program_fock(Ops& X) {
   // Coulomb: F_pq += 2 sum_J L_pq X_J,  X_J = sum_k L_kk
   double* XJ = X.buf(SL_SMALL2, "fock_XJ", J);
   X.trace_oo(Loo, XJ);
-  X.add_coulomb(Loo, o, o, XJ, F, "fock_coul_oo");
-  X.add_coulomb(Lov, o, v, XJ, F + n * o, "fock_coul_ov");
-  X.add_coulomb(Lt_vo_.as<double>(), v, o, XJ, F + o, "fock_coul_vo");
-  X.add_coulomb(Lt_vv_.as<double>(), v, v, XJ, F + o + n * o, "fock_coul_vv");
+  X.coulomb(Loo, Lov, Lt_vo_.as<double>(), Lt_vv_.as<double>(), XJ, F);
   // Exchange: F_pq -= sum_{J,k} L_pk L_kq with left factors reordered to (J, k, p), p over
   // the occupied and then the virtual orbitals: two products for the four blocks
   double* Lleft = X.buf(SL_SMALL3, "fock_Lleft", J * o * n);

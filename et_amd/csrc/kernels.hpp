@@ -60,6 +60,10 @@ void symsum_abij(hipStream_t s, const double* x, double* y, int64_t n_v, int64_t
 // packin of x(a, b, i, j) taken in the order (a, i, b, j)
 void packin_abij(hipStream_t s, const double* x, double* packed, int64_t n_v, int64_t n_o, double diag_scale);
 
+// F(p, q) += 2 sum_J L(J, p, q) x(J), L in its oo, ov, vo and vv blocks
+void fock_coulomb(hipStream_t s, const double* Loo, const double* Lov, const double* Lvo, const double* Lvv,
+                  const double* x, int64_t n_J, int64_t n_o, int64_t n_v, double* F);
+
 // Ladder (+/-) helpers ------------------------------------------------------
 // t+ (o+ x v+): (1 - d_cd/2)(t_cidj + t_cjdi), rows ij (i <= j), cols cd (c <= d)
 // t- (o- x v-): t_cidj - t_cjdi, rows i < j, cols c < d

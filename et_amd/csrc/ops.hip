@@ -70,12 +70,9 @@ void DirectOps::fock_ov_vec(const double* F, double* f) {
   etg::fock_ov_vector(wf_.stream(), F, f, wf_.n_o, wf_.n_v);
 }
 
-// A batch of products, one per column of the block: straight into F, a launch instead of
-// a product and an addition (a launch of a small residual's chain is 4.6 us).
-void DirectOps::add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F, const char* name) {
-  (void)name;
-  const int64_t J = wf_.n_J, n = wf_.n_mo;
-  gemm_batched('T', 'N', rows, 1, J, 2.0, L, J, J * rows, x, J, 0, 1.0, F, n, n, cols, Prec::F64);
+void DirectOps::coulomb(const double* Loo, const double* Lov, const double* Lvo, const double* Lvv, const double* x,
+                        double* F) {
+  etg::fock_coulomb(wf_.stream(), Loo, Lov, Lvo, Lvv, x, wf_.n_J, wf_.n_o, wf_.n_v, F);
 }
 
 void DirectOps::amplitudes(const double* t2, double* T, double* U) {
@@ -480,13 +477,20 @@ void Tape::fock_ov_vec(const double* F, double* f) {
   DirectOps::fock_ov_vec(F, f);
 }
 
-// As one product and an addition, which run for all vectors of a pass at once (a recorded
-// batch would run vector by vector).
-void Tape::add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F, const char* name) {
-  const int64_t J = wf_.n_J;
-  double* c = buf(SL_SMALL0, name, rows * cols);
-  gemm('T', 'N', rows * cols, 1, J, 2.0, L, J, x, J, 0.0, c, rows * cols, Prec::F64);
-  copy_sub(c, rows, F, wf_.n_mo, rows, cols, 1.0, 1.0);
+// Per block a product and an addition, which have rules for the passes and run for all
+// their vectors at once.
+void Tape::coulomb(const double* Loo, const double* Lov, const double* Lvo, const double* Lvv, const double* x,
+                   double* F) {
+  const int64_t J = wf_.n_J, n = wf_.n_mo, o = wf_.n_o, v = wf_.n_v;
+  auto block = [&](const double* L, int64_t rows, int64_t cols, double* Fb, const char* name) {
+    double* c = buf(SL_SMALL0, name, rows * cols);
+    gemm('T', 'N', rows * cols, 1, J, 2.0, L, J, x, J, 0.0, c, rows * cols, Prec::F64);
+    copy_sub(c, rows, Fb, n, rows, cols, 1.0, 1.0);
+  };
+  block(Loo, o, o, F, "fock_coul_oo");
+  block(Lov, o, v, F + n * o, "fock_coul_ov");
+  block(Lvo, v, o, F + o, "fock_coul_vo");
+  block(Lvv, v, v, F + o + n * o, "fock_coul_vv");
 }
 
 void Tape::amplitudes(const double* t2, double* T, double* U) {

@@ -54,9 +54,9 @@ class Ops {
   virtual void trace_oo(const double* Loo, double* XJ) = 0;
   // f(b + v j) = F(j, o + b)
   virtual void fock_ov_vec(const double* F, double* f) = 0;
-  // F(p, q) += 2 sum_J L(J, p, q) x(J) on a rows x cols block of the Fock matrix
-  virtual void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
-                           const char* name) = 0;
+  // F(p, q) += 2 sum_J L(J, p, q) x(J) on all four blocks of the Fock matrix
+  virtual void coulomb(const double* Loo, const double* Lov, const double* Lvo, const double* Lvv, const double* x,
+                       double* F) = 0;
   // T = full matrix of the packed t2, U(ai, bj) = 2 T(ai, bj) - T(aj, bi)
   virtual void amplitudes(const double* t2, double* T, double* U) = 0;
   // abij(a, b, i, j) = x(ai, bj) + x(bj, ai); sym is the (ov)^2 scratch of a program in two steps
@@ -118,8 +118,8 @@ class DirectOps : public Ops {
   void t1_xy(const double* t1, double* X, double* Y) override;
   void trace_oo(const double* Loo, double* XJ) override;
   void fock_ov_vec(const double* F, double* f) override;
-  void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
-                   const char* name) override;
+  void coulomb(const double* Loo, const double* Lov, const double* Lvo, const double* Lvv, const double* x,
+               double* F) override;
   void amplitudes(const double* t2, double* T, double* U) override;
   void symsum_abij(const double* x, double* sym, double* abij) override;
   void packin_abij(const double* abij, double* aibj, double* packed) override;
@@ -152,8 +152,8 @@ class Tape : public DirectOps {
   void t1_xy(const double* t1, double* X, double* Y) override;
   void trace_oo(const double* Loo, double* XJ) override;
   void fock_ov_vec(const double* F, double* f) override;
-  void add_coulomb(const double* L, int64_t rows, int64_t cols, const double* x, double* F,
-                   const char* name) override;
+  void coulomb(const double* Loo, const double* Lov, const double* Lvo, const double* Lvv, const double* x,
+               double* F) override;
   void amplitudes(const double* t2, double* T, double* U) override;
   void symsum_abij(const double* x, double* sym, double* abij) override;
   void packin_abij(const double* abij, double* aibj, double* packed) override;
