@@ -184,28 +184,48 @@ __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const do
   const int64_t xb = tri_root(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
   const int64_t X0 = xb * 32, Y0 = yb * 32;
   const bool exch = f2 != 0.0;
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t Yr = Y0 + tx, Xc = X0 + k;            // A[k][tx] = x(Y0 + tx, X0 + k)
-    const bool okA = Yr < N && Xc < N;
-    A[k][tx] = okA ? x[Yr + N * Xc] : 0.0;
-    const int64_t Xr = X0 + tx, Yc = Y0 + k;            // B[k][tx] = x(X0 + tx, Y0 + k)
-    const bool okB = Xr < N && Yc < N;
-    B[k][tx] = okB ? x[Xr + N * Yc] : 0.0;
+  // all loads first, none under a condition (rows past the edge repeat the last one): as
+  // conditional loads each waits for the one before it
+  double la[4], lb[4], lc[4], ld[4], le[4], lf[4], ly[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = ty + 8 * i;
+    const int64_t Yr = min(Y0 + tx, N - 1), Xc = min(X0 + k, N - 1);    // A[k][tx] = x(Y0 + tx, X0 + k)
+    la[i] = x[Yr + N * Xc];
+    const int64_t Xr = min(X0 + tx, N - 1), Yc = min(Y0 + k, N - 1);    // B[k][tx] = x(X0 + tx, Y0 + k)
+    lb[i] = x[Xr + N * Yc];
     if constexpr (TWO) {
-      E[k][tx] = okA ? plain[Yr + N * Xc] : 0.0;
-      F[k][tx] = okB ? plain[Xr + N * Yc] : 0.0;
+      le[i] = plain[Yr + N * Xc];
+      lf[i] = plain[Xr + N * Yc];
     }
     if (exch) {
       // C[k][tx]: Y = Yr = p + v q, X = Xc = r + v s  ->  x(p + v s, r + v q)
-      const int64_t p = Yr % n_v, q = Yr / n_v, r = Xc % n_v, sx = Xc / n_v;
-      C[k][tx] = okA ? x[(p + n_v * sx) + N * (r + n_v * q)] : 0.0;
+      const int64_t q = Yr / n_v, p = Yr - q * n_v, s = Xc / n_v, r = Xc - s * n_v;
+      lc[i] = x[(p + n_v * s) + N * (r + n_v * q)];
       // D[k][tx]: X = Xr = r' + v s', Y = Yc = p' + v q'  ->  x(r' + v q', p' + v s')
-      const int64_t p2 = Yc % n_v, q2 = Yc / n_v, r2 = Xr % n_v, s2 = Xr / n_v;
-      D[k][tx] = okB ? x[(r2 + n_v * q2) + N * (p2 + n_v * s2)] : 0.0;
+      const int64_t q2 = Yc / n_v, p2 = Yc - q2 * n_v, s2 = Xr / n_v, r2 = Xr - s2 * n_v;
+      ld[i] = x[(r2 + n_v * q2) + N * (p2 + n_v * s2)];
+    }
+    ly[i] = y[Xc * (Xc + 1) / 2 + min(Yr, Xc)];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = ty + 8 * i;
+    A[k][tx] = la[i];
+    B[k][tx] = lb[i];
+    if constexpr (TWO) {
+      E[k][tx] = le[i];
+      F[k][tx] = lf[i];
+    }
+    if (exch) {
+      C[k][tx] = lc[i];
+      D[k][tx] = ld[i];
     }
   }
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = ty + 8 * i;
     const int64_t X = X0 + k, Y = Y0 + tx;
     if (X >= N || Y > X) continue;
     double v;
@@ -217,7 +237,7 @@ __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const do
       v *= alpha;
     }
     if constexpr (TWO) v += X == Y ? E[k][tx] : E[k][tx] + F[tx][k];
-    y[X * (X + 1) / 2 + Y] += v;
+    y[X * (X + 1) / 2 + Y] = ly[i] + v;
   }
 }
 
