@@ -129,7 +129,8 @@ __global__ __launch_bounds__(256) void row_exponents_finish_kernel(const double*
 // outermost, k steps contiguous.  One wave forms the 15 chunks of a (row block,
 // k step).  About 75 VALU operations per element (5 per modulus) against 8
 // bytes read and 15 written: bound by HBM, 37 M elements in 200 us.  (With 125
-// operations, residues formed in FP32, 215; products of 1520^3 133 -> 127 us.)
+// operations, residues formed in FP32, 215; products of 1520^3 133 -> 127 us,
+// with unconditional loads 121.)
 // ---------------------------------------------------------------------------
 // The 16 values are formed here, in the order of the source, not where they are used.
 __device__ inline void pin(uint32_t (&x)[16]) {
@@ -158,9 +159,14 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
     const double* x = X + bz * strideX + rb * 16 * ld;
     const int64_t kl = ks * kDepth + lane;
     double* t = stage[wave];
+    // (loads at clamped indices: under a condition each would wait for the one before it;
+    // with those the products of 17020 x 820 x 17020 took 4.89 -> 4.55 ms)
+    const int64_t last = rows - 1 - rb * 16, kc = min(kl, K - 1);
+    double v[16];
 #pragma unroll
-    for (int rr = 0; rr < 16; ++rr)
-      t[rr * kPackLd + lane] = (rb * 16 + rr < rows && kl < K) ? x[rr * ld + kl] : 0.0;
+    for (int rr = 0; rr < 16; ++rr) v[rr] = x[min(int64_t(rr), last) * ld + kc];
+#pragma unroll
+    for (int rr = 0; rr < 16; ++rr) t[rr * kPackLd + lane] = (rr <= last && kl < K) ? v[rr] : 0.0;
     __syncthreads();
     const double2* src = reinterpret_cast<const double2*>(&t[(lane & 15) * kPackLd + 16 * (lane >> 4)]);
     const bool ok = ex != residue::kNotFinite;
@@ -171,10 +177,14 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
       residue::to_integer(ok ? v.y : 0.0, ex, lo[2 * j + 1], hi[2 * j + 1]);
     }
   } else {
-    const double* x = X + bz * strideX + r + k0 * ld;
+    const double* x = X + bz * strideX + min(r, rows - 1) + min(k0, K - 1) * ld;
     const int n = (r < rows && ex != residue::kNotFinite && k0 < K) ? int(min<int64_t>(16, K - k0)) : 0;
+    const int64_t last = max(int64_t(0), K - 1 - k0);
+    double v[16];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) residue::to_integer(j < n ? x[j * ld] : 0.0, ex, lo[j], hi[j]);
+    for (int j = 0; j < 16; ++j) v[j] = x[min(int64_t(j), last) * ld];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) residue::to_integer(j < n ? v[j] : 0.0, ex, lo[j], hi[j]);
   }
   if (ks >= KS) return;
   u4* dst = P + bz * kModuli * plane + (rb * KS + ks) * 64 + lane;

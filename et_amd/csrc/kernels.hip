@@ -168,7 +168,9 @@ __global__ void symmetric_sum_kernel(const double* __restrict__ x, double* __res
 // the two exchange terms x(p + v s, r + v q) (along p) and x(r + v q, p + v s)
 // (along r) for Y = p + v q, X = r + v s, then adds to packed element
 // X (X + 1) / 2 + Y, contiguous in Y for each X.  TWO: `plain` is a second array,
-// added with alpha = f1 = 1, f2 = 0 (no batch).
+// added with alpha = f1 = 1, f2 = 0 (no batch).  All loads come first and at clamped
+// indices: with each under its own edge condition they waited for one another, and the
+// two-array form took 437 us instead of 186 at (H2O)8.
 template <bool TWO>
 __global__ __launch_bounds__(256) void symmetrize_and_pack_tiled_kernel(const double* __restrict__ x,
                                                                         double* __restrict__ y, int64_t n_v,
