@@ -59,6 +59,10 @@ __global__ void permute4_kernel(const double* __restrict__ x, double* __restrict
 // tiles of the (output dim 0, output dim p) plane go through LDS, where p is the
 // output position of the input-fastest index, so reads (along dim p) and writes
 // (along dim 0) are both unit-stride.  q, r: the other two output dims.
+// Bound by HBM.  As in the other tiled kernels, the four loads of a lane come together and
+// at clamped indices: each under its own edge condition waited for the one before (the four
+// reorderings of the (H2O)8 residual 514 -> 443 us, squareup_and_u 161 -> 147, symsum_abij
+// 172 -> 150; ladder_g_pm_tiled, which loops over pairs, loses by it: 1146 -> 1315).
 __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __restrict__ y,
                                       int64_t e0, int64_t ep, int64_t eq, int64_t er, int64_t s0,
                                       int64_t sq, int64_t sr, int64_t yp, int64_t yq, int64_t yr,
@@ -75,18 +79,27 @@ __global__ void permute4_tiled_kernel(const double* __restrict__ x, double* __re
     const int64_t iq = o % eq, ir = o / eq;
     const double* xb = x + iq * sq + ir * sr;
     double* yb = y + iq * yq + ir * yr;
-    for (int k = ty; k < 32; k += 8) {
-      const int64_t i0 = t0 * 32 + k, ip = tp * 32 + tx;
-      tile[k][tx] = (i0 < e0 && ip < ep) ? xb[i0 * s0 + ip] : 0.0;
-    }
+    double v[4], w[4] = {}, g[4] = {};
+    const int64_t j0 = min(t0 * 32 + tx, e0 - 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      v[k] = xb[min(t0 * 32 + ty + 8 * k, e0 - 1) * s0 + min(tp * 32 + tx, ep - 1)];
+    if (gamma != 0.0)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) g[k] = z[yb - y + j0 + min(tp * 32 + ty + 8 * k, ep - 1) * yp];
+    if (beta != 0.0)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k] = yb[j0 + min(tp * 32 + ty + 8 * k, ep - 1) * yp];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tile[ty + 8 * k][tx] = v[k];
     __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-      const int64_t ip = tp * 32 + k, i0 = t0 * 32 + tx;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t ip = tp * 32 + ty + 8 * k, i0 = t0 * 32 + tx;
       if (i0 < e0 && ip < ep) {
-        double* dst = yb + i0 + ip * yp;
-        double v = alpha * tile[tx][k];
-        if (gamma != 0.0) v += gamma * z[dst - y];
-        *dst = (beta == 0.0) ? v : v + beta * *dst;
+        double u = alpha * tile[tx][ty + 8 * k];
+        if (gamma != 0.0) u += gamma * g[k];
+        yb[i0 + ip * yp] = (beta == 0.0) ? u : u + beta * w[k];
       }
     }
     __syncthreads();
@@ -115,10 +128,14 @@ __global__ __launch_bounds__(256) void squareup_tiled_kernel(const double* __res
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t xb = tri_root(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
   const int64_t X0 = xb * 32, Y0 = yb * 32;
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t X = X0 + k, Y = Y0 + tx;
-    P[k][tx] = (X < N && Y <= X) ? packed[X * (X + 1) / 2 + Y] : 0.0;
+  double p[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t X = min(X0 + ty + 8 * k, N - 1);
+    p[k] = packed[X * (X + 1) / 2 + min(Y0 + tx, X)];
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) P[ty + 8 * k][tx] = p[k];
   __syncthreads();
   for (int k = ty; k < 32; k += 8) {
     const int64_t X = X0 + k, Y = Y0 + tx;              // full(Y, X), along Y
@@ -152,14 +169,19 @@ __global__ void symmetric_sum_kernel(const double* __restrict__ x, double* __res
   const int64_t bx = blockIdx.x, by = blockIdx.y;
   const int tx = threadIdx.x, ty = threadIdx.y;  // 32 x 8
   // load transposed block (by, bx) of x: rows by*32.., cols bx*32..
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t r = by * 32 + tx, c = bx * 32 + k;
-    tile[k][tx] = (r < N && c < N) ? x[r + N * c] : 0.0;
+  double t[4], v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    t[k] = x[min(by * 32 + tx, N - 1) + N * min(bx * 32 + ty + 8 * k, N - 1)];
+    v[k] = x[min(bx * 32 + tx, N - 1) + N * min(by * 32 + ty + 8 * k, N - 1)];
   }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) tile[ty + 8 * k][tx] = t[k];
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t r = bx * 32 + tx, c = by * 32 + k;
-    if (r < N && c < N) y[r + N * c] = x[r + N * c] + tile[tx][k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t r = bx * 32 + tx, c = by * 32 + ty + 8 * k;
+    if (r < N && c < N) y[r + N * c] = v[k] + tile[tx][ty + 8 * k];
   }
 }
 
@@ -275,12 +297,21 @@ __global__ __launch_bounds__(256) void squareup_and_u_kernel(const double* __res
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t xb = tri_root(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
   const int64_t X0 = xb * 32, Y0 = yb * 32;
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t X = X0 + k, Y = Y0 + tx;
-    P[k][tx] = (X < N && Y <= X) ? packed[X * (X + 1) / 2 + Y] : 0.0;
-    const int64_t Xr = X0 + tx, Yc = Y0 + k;            // Xr = a + v i, Yc = b + v j
-    const int64_t a = Xr % n_v, i = Xr / n_v, b = Yc % n_v, j = Yc / n_v;
-    Q[k][tx] = (Xr < N && Yc <= Xr) ? packed[pidx(a + n_v * j, b + n_v * i)] : 0.0;
+  double p[4], q[4];
+  const int64_t Xr = min(X0 + tx, N - 1);               // a + v i
+  const int64_t i = Xr / n_v, a = Xr - i * n_v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t X = min(X0 + ty + 8 * k, N - 1);
+    p[k] = packed[X * (X + 1) / 2 + min(Y0 + tx, X)];
+    const int64_t Yc = min(Y0 + ty + 8 * k, N - 1);     // b + v j
+    const int64_t j = Yc / n_v, b = Yc - j * n_v;
+    q[k] = packed[pidx(a + n_v * j, b + n_v * i)];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    P[ty + 8 * k][tx] = p[k];
+    Q[ty + 8 * k][tx] = q[k];
   }
   __syncthreads();
   for (int k = ty; k < 32; k += 8) {
@@ -306,12 +337,19 @@ __global__ __launch_bounds__(256) void symsum_abij_kernel(const double* __restri
   const int64_t a0 = (blockIdx.x % nt) * 32, b0 = (blockIdx.x / nt) * 32;
   for (int64_t ij = blockIdx.y; ij < n_o * n_o; ij += gridDim.y) {
     const int64_t i = ij % n_o, j = ij / n_o;
-    for (int k = ty; k < 32; k += 8)
-      if (a0 + k < n_v && b0 + tx < n_v) T[k][tx] = x[(b0 + tx + n_v * j) + N * (a0 + k + n_v * i)];
+    double t[4], v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      t[k] = x[(min(b0 + tx, n_v - 1) + n_v * j) + N * (min(a0 + ty + 8 * k, n_v - 1) + n_v * i)];
+      v[k] = x[(min(a0 + tx, n_v - 1) + n_v * i) + N * (min(b0 + ty + 8 * k, n_v - 1) + n_v * j)];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) T[ty + 8 * k][tx] = t[k];
     __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-      const int64_t a = a0 + tx, b = b0 + k;
-      if (a < n_v && b < n_v) y[a + n_v * b + n_v * n_v * ij] = x[(a + n_v * i) + N * (b + n_v * j)] + T[tx][k];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t a = a0 + tx, b = b0 + ty + 8 * k;
+      if (a < n_v && b < n_v) y[a + n_v * b + n_v * n_v * ij] = v[k] + T[tx][ty + 8 * k];
     }
     __syncthreads();
   }
@@ -885,16 +923,25 @@ __global__ void symmetric_sum_acc_kernel(const double* __restrict__ x, double* _
   __shared__ double tile[32][33];
   const int64_t bx = blockIdx.x, by = blockIdx.y;
   const int tx = threadIdx.x, ty = threadIdx.y;
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t r = by * 32 + tx, c = bx * 32 + k;
-    tile[k][tx] = (r < N && c < N) ? x[r + N * c] : 0.0;
+  double t[4], v[4], w[4] = {};
+  const int64_t rc = min(bx * 32 + tx, N - 1);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    t[k] = x[min(by * 32 + tx, N - 1) + N * min(bx * 32 + ty + 8 * k, N - 1)];
+    v[k] = x[rc + N * min(by * 32 + ty + 8 * k, N - 1)];
   }
+  if (beta != 0.0)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) w[k] = y[rc + N * min(by * 32 + ty + 8 * k, N - 1)];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) tile[ty + 8 * k][tx] = t[k];
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t r = bx * 32 + tx, c = by * 32 + k;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t r = bx * 32 + tx, c = by * 32 + ty + 8 * k;
     if (r < N && c < N) {
-      const double v = x[r + N * c] + tile[tx][k];
-      y[r + N * c] = (beta == 0.0) ? v : v + beta * y[r + N * c];
+      const double u = v[k] + tile[tx][ty + 8 * k];
+      y[r + N * c] = (beta == 0.0) ? u : u + beta * w[k];
     }
   }
 }
@@ -960,16 +1007,28 @@ __global__ __launch_bounds__(256) void sympack_adjoint_tiled_kernel(const double
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
   const int64_t xb = tri_root2(blockIdx.x), yb = int64_t(blockIdx.x) - xb * (xb + 1) / 2;
   const int64_t X0 = xb * 32, Y0 = yb * 32;
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t X = X0 + k, Y = Y0 + tx;
-    P[k][tx] = (X < N && Y <= X) ? p[X * (X + 1) / 2 + Y] * (X == Y ? alpha : alpha * f1) : 0.0;
+  double v[4], w1[4] = {}, w2[4] = {};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t X = min(X0 + ty + 8 * k, N - 1);
+    v[k] = p[X * (X + 1) / 2 + min(Y0 + tx, X)];
   }
+  if (acc)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w1[k] = x[min(Y0 + tx, N - 1) + N * min(X0 + ty + 8 * k, N - 1)];
+      w2[k] = x[min(X0 + tx, N - 1) + N * min(Y0 + ty + 8 * k, N - 1)];
+    }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) P[ty + 8 * k][tx] = v[k] * (X0 + ty + 8 * k == Y0 + tx ? alpha : alpha * f1);
   __syncthreads();
-  for (int k = ty; k < 32; k += 8) {
-    const int64_t X = X0 + k, Y = Y0 + tx;              // x(Y, X), along Y
-    if (X < N && Y <= X) x[Y + N * X] = acc ? x[Y + N * X] + P[k][tx] : P[k][tx];
-    const int64_t Xr = X0 + tx, Yc = Y0 + k;            // x(Xr, Yc), along Xr (the diagonal once)
-    if (Xr < N && Yc < Xr) x[Xr + N * Yc] = acc ? x[Xr + N * Yc] + P[tx][k] : P[tx][k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int64_t X = X0 + ty + 8 * k, Y = Y0 + tx;     // x(Y, X), along Y
+    const double u1 = P[ty + 8 * k][tx], u2 = P[tx][ty + 8 * k];
+    if (X < N && Y <= X) x[Y + N * X] = acc ? w1[k] + u1 : u1;
+    const int64_t Xr = X0 + tx, Yc = Y0 + ty + 8 * k;   // x(Xr, Yc), along Xr (the diagonal once)
+    if (Xr < N && Yc < Xr) x[Xr + N * Yc] = acc ? w2[k] + u2 : u2;
   }
 }
 
