@@ -65,11 +65,17 @@ __global__ __launch_bounds__(256) void pack_split_bf16_kernel(const double* __re
     const int64_t rb0 = tr * 4;
     const int64_t r = rb0 * 16 + row;
     bf8 h, l;
+    // the eight loads at clamped indices and first: under a condition each would wait
+    // for the one before it ((H2O)8, split-bf16: residual 32.7 -> 31.7 ms, the left
+    // transformation of twelve vectors 253.6 -> 251.9)
+    const int64_t k0 = ks * kDepth + 8 * kq, rc = min(r, rows - 1);
+    const int64_t step_r = kcontig ? ld : 1, step_k = kcontig ? 1 : ld;
+    double v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = Xb[rc * step_r + min(k0 + e, K - 1) * step_k];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int64_t k = ks * kDepth + 8 * kq + e;
-      double x = 0.0;
-      if (r < rows && k < K) x = kcontig ? Xb[k + r * ld] : Xb[r + k * ld];
+      const double x = (r < rows && k0 + e < K) ? v[e] : 0.0;
       const __bf16 xh = __bf16(float(x));
       h[e] = xh;
       l[e] = __bf16(float(x - double(float(xh))));
