@@ -1181,7 +1181,9 @@ __global__ void copy_sub_kernel2(const double* src, int64_t lds, double* dst, in
   dst += int64_t(blockIdx.z) * sy;
   GRID_LOOP(k, m * n) {
     const int64_t r = k % m, c = k / m;
-    const double v = alpha * src[r + lds * c];
+    // alpha = 0 scales dst alone: src is dst then, and may hold anything (an infinity or
+    // NaN times 0 would stay in a derivative that starts here)
+    const double v = alpha == 0.0 ? 0.0 : alpha * src[r + lds * c];
     dst[r + ldd * c] = (beta == 0.0) ? v : v + beta * dst[r + ldd * c];
   }
 }

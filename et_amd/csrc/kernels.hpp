@@ -160,7 +160,7 @@ void quasi_newton_step(hipStream_t s, const double* eps, const double* residual,
 // dst (m x n, ld ldd) += sum over b < nbatch of the contiguous m x n blocks part_b
 void batch_sum_acc(hipStream_t s, const double* part, int64_t nbatch, int64_t m, int64_t n, double* dst,
                    int64_t ldd);
-// dst (m x n) = alpha * src + beta * dst
+// dst (m x n) = alpha * src + beta * dst; src is not read when alpha = 0, dst not when beta = 0
 void copy_sub(hipStream_t s, const double* src, int64_t lds, double* dst, int64_t ldd, int64_t m,
               int64_t n, double alpha, double beta, const Batch& b = {});
 
