@@ -340,7 +340,8 @@ __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
-  T a[2][TM][4], b[2][TN][4];
+  // (converted where they are used: at the load each FP32 value would wait for its own)
+  double a[2][TM][4], b[2][TN][4];
   auto load = [&](int at, int64_t k0) {
     int64_t da = 0, db = 0, limit = kend;
     if constexpr (TWO) {
@@ -355,20 +356,20 @@ __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) a[at][i][s] = M::cvt(pa[i][da + (k0 + lk + s) * sa]);
+        for (int s = 0; s < 4; ++s) a[at][i][s] = pa[i][da + (k0 + lk + s) * sa];
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) b[at][j][s] = M::cvt(pb[j][db + (k0 + lk + s) * sb]);
+        for (int s = 0; s < 4; ++s) b[at][j][s] = pb[j][db + (k0 + lk + s) * sb];
     } else {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const bool ok = k0 + lk + s < limit;
         const int64_t k = ok ? k0 + lk + s : (TWO ? 0 : kbeg);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[at][i][s] = ok ? M::cvt(pa[i][da + k * sa]) : T(0);
+        for (int i = 0; i < TM; ++i) a[at][i][s] = ok ? pa[i][da + k * sa] : 0.0;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) b[at][j][s] = ok ? M::cvt(pb[j][db + k * sb]) : T(0);
+        for (int j = 0; j < TN; ++j) b[at][j][s] = ok ? pb[j][db + k * sb] : 0.0;
       }
     }
   };
@@ -378,7 +379,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_few_tiles(Params p) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = M::run(a[at][i][s], b[at][j][s], acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = M::run(M::cvt(a[at][i][s]), M::cvt(b[at][j][s]), acc[i][j]);
   };
   int64_t k0 = kbeg + 16 * wave;
   if (k0 < kend) load(0, k0);
