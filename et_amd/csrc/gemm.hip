@@ -723,14 +723,42 @@ FewChoice choose_few(const Gemm& g, bool can_split) {
   return best;
 }
 
-// Products that run on gemm_few_tiles: at most 1.5 GFLOP (us, tiled and this:
-// 95 x 95 x 279 18 and 4, 19 x 5 x 5301 19 and 6, 380^3 25 and 8, 741^3 41 and 32, 76 x 20
-// x 96520 40 and 26; beyond, 400 x 400 x 5776 63 and 64, 210 x 2926 x 2926 99 and 112),
-// except short k over many outputs, which the larger tiles read fewer times
-// (76 x 30400 x 76: 20 and 26).
-bool few_tiles_pay(const Gemm& g) {
+// Microseconds of a small product on the tiled kernel and on gemm_few_tiles, fitted to
+// 458 shapes of each type between 2 MFLOP and 1.5 GFLOP (m, n = 8 .. 5800, k = 8 .. 65536,
+// all four transpositions; 12-19 % rms).  The tiled kernel: its k steps of 16, longer when
+// a CU holds more of its workgroups (FP32 products half as long), then C or the partial
+// sums.  gemm_few_tiles: as in choose_few, C or the partial sums in the output's width;
+// the two types alike, since it is bound by the operands' loads.
+double tiled_us(const Gemm& g, bool f32, bool can_split) {
+  const Choice c = choose_tiling(g, f32 ? 157.3e12 : 78.6e12, can_split);
+  const double mn = double(g.m) * double(g.n) * double(g.batch);
+  const double wgs = double(ceil_div(g.m, c.bm)) * double(ceil_div(g.n, c.bm)) * double(g.batch) * c.splits;
+  const double slots = c.bm == 64 ? 1024.0 : 512.0;
+  const double crowd = std::max(0.0, std::min(wgs, slots) / 256.0 - 1.0);
+  const double step = c.bm == 64 ? (f32 ? 0.65 + 0.42 * crowd : 0.85 + 0.65 * crowd) : (f32 ? 3.0 : 4.7);
+  const double steps = double(ceil_div(ceil_div(g.k, c.splits), 16));
+  const double out = c.splits > 1 ? (f32 ? 6.5 + 7.0e-6 * c.splits * mn : 5.7 + 3.5e-6 * c.splits * mn)
+                                  : (f32 ? 3.2e-6 : 1.95e-6) * mn;
+  return 3.4 + steps * step * std::max(1.0, wgs / slots) + out;
+}
+
+double few_us(const Gemm& g, const FewChoice& c) {
+  const double b = double(g.batch), mn = double(g.m) * double(g.n) * b;
+  const double work = 2e-6 * double(ceil_div(g.m, c.tile) * c.tile) * double(ceil_div(g.n, c.tile) * c.tile) * double(g.k) * b;
+  const double chunks = double(ceil_div(ceil_div(ceil_div(g.k, c.splits), 16) * 16, 64));
+  const double out = c.splits > 1 ? 2.75 + 10.9e-6 * c.splits * mn : 5.8e-6 * mn;
+  return (c.tile == 16 ? 2.7 + 0.216 * chunks + work / 25.0 : 4.3 + 0.342 * chunks + work / 46.5) + out;
+}
+
+// Products that run on gemm_few_tiles: up to 1.5 GFLOP, where its estimate is a tenth
+// below the tiled kernel's (us, tiled and this: FP64 95 x 95 x 279 19 and 4, 380^3 25 and
+// 8, 741^3 40 and 32, 1526 x 1201 x 141 19 and 29; FP32 300^3 16 and 6, 741^3 36 and 33,
+// 1526 x 1201 x 141 17 and 23).  With this rule 4 of 1000 products are more than 5 % slower
+// than on the tiled kernel (worst 1.17 times); by FLOPs and k > 128 alone, the same for
+// both types, 69 were (worst 3.1 times, FP32).
+bool few_tiles_pay(const Gemm& g, bool f32, bool can_split) {
   if (gemm_flops(g) > 1.5e9 || ceil_div(g.m, 16) * ceil_div(g.n, 16) > (int64_t(1) << 30)) return false;
-  return g.k > 128 || double(g.m) * double(g.n) * double(g.batch) < 4e5;
+  return 1.1 * few_us(g, choose_few(g, can_split)) < tiled_us(g, f32, can_split);
 }
 
 // Two pairs of few tiles as one k range.
@@ -754,7 +782,7 @@ GemmLaunch launch_two(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
 
 template <typename T>
 GemmLaunch launch_rows(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
-  if (few_tiles_pay(g)) {
+  if (few_tiles_pay(g, sizeof(T) == 4, ws != nullptr)) {
     const FewChoice c = choose_few(g, ws != nullptr);
     int splits = 1;
     const Params p = split_params(g, ws, c.splits, &splits);
@@ -1060,7 +1088,8 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
     if (g.Cin != nullptr || g.Cf != nullptr || g.b_packed != nullptr || g.a_tag != 0) fail("gemm: two operand pairs take no options");
     Gemm one = g;
     one.A2 = one.B2 = nullptr;
-    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) && few_tiles_pay(g) &&
+    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) &&
+                     few_tiles_pay(g, prec == Prec::F32, ws != nullptr) &&
                      !(prec == Prec::BF16X3 && split_bf16_pays(one)) &&
                      !(prec != Prec::F32 && runs_as_residues(one, Prec::F64, ws));
     if (few) return prec == Prec::F32 ? launch_two<float>(stream, g, ws) : launch_two<double>(stream, g, ws);
@@ -1074,7 +1103,8 @@ GemmLaunch gemm(hipStream_t stream, const Gemm& g, Prec prec, GemmWorkspace* ws)
     if (g.batch != 1 || g.ldcin < g.m) fail("gemm: inconsistent input C");
     Gemm h = g;
     h.beta = 1.0;
-    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) && few_tiles_pay(g) &&
+    const bool few = g.k > 0 && std::max(g.lda, g.ldb) < (int64_t(1) << 24) &&
+                     few_tiles_pay(g, prec == Prec::F32, ws != nullptr) &&
                      !(prec == Prec::BF16X3 && split_bf16_pays(g)) &&
                      !(prec != Prec::F32 && runs_as_residues(g, Prec::F64, ws));
     if (few) return prec == Prec::F32 ? launch_typed<float>(stream, h, ws) : launch_typed<double>(stream, h, ws);
