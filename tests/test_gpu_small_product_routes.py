@@ -23,6 +23,15 @@ def test_fp32_is_not_slower_than_fp64(m, n, k, ta, tb):
     assert t32 < 1.25 * t64, (t32, t64)
 
 
+def test_short_k_over_many_outputs_is_tiled():
+    """Three times the k (past the rule's range) takes 2.2 times as long as the tiled kernel, 1.4 times as
+    long as the products of few tiles."""
+    def seconds(k):
+        return min(ccsd.bench_gemm(1526, 1201, k, ccsd.FP64, reps=20, ta='T', tb='T') for _ in range(5))
+    t, t3 = seconds(141), seconds(423)
+    assert t < 0.57 * t3, (t, t3)
+
+
 @pytest.mark.parametrize('m,n,k,ta,tb', SHAPES)
 @pytest.mark.parametrize('precision', [ccsd.FP64, ccsd.FP32])
 def test_product(precision, m, n, k, ta, tb):
