@@ -325,17 +325,19 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
     compute(int(s & 1));
   }
 
+  const int lrow = lane >> 4, lcol = lane & 15;
+  const int64_t r0 = int64_t(tile_m) * kTile + wm * 128, c0 = int64_t(tile_n) * kTile + wn * 64;
   if (partial) {
     const int rest = int(p.rest);
     f4* W = p.W + (int64_t(piece % rest) * p.splits + piece / rest) * kTileF4 + wave * 2048 + lane;
+    // (only blocks that hold outputs: the whole tile costs 1592 x 12 x 4813 59.6 us, this 56.6)
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) W[(i * 4 + j) * 64] = acc[i][j];
+      for (int j = 0; j < 4; ++j)
+        if (r0 + i * 16 < p.m && c0 + j * 16 < p.n) W[(i * 4 + j) * 64] = acc[i][j];
     return;
   }
-  const int lrow = lane >> 4, lcol = lane & 15;
-  const int64_t r0 = int64_t(tile_m) * kTile + wm * 128, c0 = int64_t(tile_n) * kTile + wn * 64;
   if (p.Cf) {
     float* C = p.Cf + bz * p.strideC;
     if (p.vec_rows) {
