@@ -184,13 +184,14 @@ struct Params {
   float* Cf;                         // C in FP32 instead (beta = 0)
   int64_t ldc, strideC;
   // Output tiles (of all batch entries, one entry after another): the first `whole`
-  // are one workgroup's work each; each of the `rest` after them is that of `splits`
-  // workgroups with ks_per_split steps, whose sums go to W (a tile's splits one after
-  // another, each 64 KB x 4 in fragment order).
+  // are one workgroup's work each, in `pieces` FP32 chains of `chain` steps one after
+  // another; each of the `rest` after them is that of `splits` workgroups with
+  // ks_per_split steps.  One chain's sums go to C; those of several to W (a tile's one
+  // after another, each 64 KB x 4 in fragment order).
   TileMap tiles;
   int64_t whole, rest;
-  int splits;
-  int64_t ks_per_split;
+  int pieces, splits;
+  int64_t chain, ks_per_split;
   f4* W;
   int vec_rows;                      // C / Cf rows written four at a time (alignment checked on the host)
 };
@@ -218,6 +219,8 @@ __device__ inline f4 mfma(bf8 a, bf8 b, f4 c) {
 constexpr int kProductThreads = 512;
 constexpr int kTileF4 = kTile * kTile / 4;       // 16-byte pieces of a tile's FP32 sums
 
+// kPieces: whole tiles too add up several chains.
+template <bool kPieces>
 __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params p) {
   __shared__ u4 lds[2][4096];        // per buffer: A chunks 0..31, B chunks 32..63 (1 KB each)
 
@@ -314,28 +317,45 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
     }
   };
 
-  // Step s computes from buffer s % 2 while the slabs of step s + 1 land in the
-  // other buffer (issued at the start of step s, after the barrier that ended
-  // every wave's reads of that buffer).
-  if (nsteps > 0) load(0, ks0);
-  for (int64_t s = 0; s < nsteps; ++s) {
-    __builtin_amdgcn_s_waitcnt(0);             // this wave's copies of step s have landed
-    __syncthreads();                           // everyone's have; buffer (s + 1) % 2 is free
-    if (s + 1 < nsteps) load(int((s + 1) & 1), ks0 + s + 1);
-    compute(int(s & 1));
-  }
-
   const int lrow = lane >> 4, lcol = lane & 15;
   const int64_t r0 = int64_t(tile_m) * kTile + wm * 128, c0 = int64_t(tile_n) * kTile + wn * 64;
-  if (partial) {
-    const int rest = int(p.rest);
-    f4* W = p.W + (int64_t(piece % rest) * p.splits + piece / rest) * kTileF4 + wave * 2048 + lane;
-    // (only blocks that hold outputs: the whole tile costs 1592 x 12 x 4813 59.6 us, this 56.6)
+  // sums of one chain
+  f4* W = p.W + wave * 2048 + lane;
+  if (partial)
+    W += ((kPieces ? p.whole * p.pieces : 0) + int64_t(piece % int(p.rest)) * p.splits + piece / int(p.rest)) * kTileF4;
+  else if (kPieces)
+    W += (bz * count + slot) * p.pieces * kTileF4;
+  // (only blocks that hold outputs: the whole tile costs 1592 x 12 x 4813 59.6 us, this 56.6)
+  auto write_sums = [&] {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (r0 + i * 16 < p.m && c0 + j * 16 < p.n) W[(i * 4 + j) * 64] = acc[i][j];
+  };
+
+  // Step s computes from buffer s % 2 while the slabs of step s + 1 land in the
+  // other buffer (issued at the start of step s, after the barrier that ended
+  // every wave's reads of that buffer).
+  if (nsteps > 0) load(0, ks0);
+  int64_t chain_end = kPieces && !partial ? p.chain : nsteps;
+  for (int64_t s = 0; s < nsteps; ++s) {
+    __builtin_amdgcn_s_waitcnt(0);             // this wave's copies of step s have landed
+    __syncthreads();                           // everyone's have; buffer (s + 1) % 2 is free
+    if (s + 1 < nsteps) load(int((s + 1) & 1), ks0 + s + 1);
+    compute(int(s & 1));
+    if (kPieces && s + 1 == chain_end && s + 1 < nsteps) {
+      write_sums();
+      W += kTileF4;
+      chain_end += p.chain;
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+  if (kPieces || partial) {
+    write_sums();
     return;
   }
   if (p.Cf) {
@@ -408,10 +428,13 @@ __global__ __launch_bounds__(kProductThreads, 1) void gemm_bf16x3_kernel(Params 
       }
 }
 
-// C = alpha * sum_s W_s + beta * C on the tiles whose k range was split: a lane
-// adds up (in FP64) four consecutive rows of one column.  Bound by HBM.
+// C = alpha * sum_s W_s + beta * C on the tiles of several chains: a lane adds up
+// (in FP64) four consecutive rows of one column.  Bound by HBM.
 __global__ __launch_bounds__(256) void splitk_reduce_bf(Params p) {
-  const int64_t u = p.whole + blockIdx.y, bz = u / p.tiles.count;
+  const bool all = p.pieces > 1;
+  const int64_t u = (all ? 0 : p.whole) + blockIdx.y, bz = u / p.tiles.count;
+  const int sums = u < p.whole ? p.pieces : p.splits;
+  const int64_t first = u < p.whole ? u * p.pieces : (all ? p.whole * p.pieces : 0) + (u - p.whole) * p.splits;
   int tile_m, tile_n;
   if (!tile_of(p.tiles, int(u - bz * p.tiles.count), tile_m, tile_n)) return;
   const int q = int(blockIdx.x) * 256 + int(threadIdx.x);               // wave (3 bits), block row (3), block column (2), lane (6)
@@ -419,9 +442,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_bf(Params p) {
   const int64_t row = int64_t(tile_m) * kTile + (wave & 1) * 128 + ((q >> 8) & 7) * 16 + 4 * (lane >> 4);
   const int64_t col = int64_t(tile_n) * kTile + (wave >> 1) * 64 + ((q >> 6) & 3) * 16 + (lane & 15);
   if (row >= p.m || col >= p.n) return;
-  const f4* W = p.W + int64_t(blockIdx.y) * p.splits * kTileF4 + q;
+  const f4* W = p.W + first * kTileF4 + q;
   double v[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int s = 0; s < p.splits; ++s) {
+  for (int s = 0; s < sums; ++s) {
     const f4 w = W[int64_t(s) * kTileF4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) v[r] += double(w[r]);
@@ -521,13 +544,32 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
   p.m = g.m; p.n = g.n; p.alpha = g.alpha; p.beta = g.beta;
   p.C = g.C; p.Cf = g.Cf; p.ldc = g.ldc; p.strideC = g.strideC;
   p.tiles = map_tiles(g.m, g.n, kTile, g.lower, 0, 0);
-  // One workgroup per CU: the tiles that fill whole rounds of the chip are taken
-  // whole, those of the last round share it by splitting their k.  With every tile
-  // split so that rounds are 90 % full, partials of the whole output in FP64, before:
-  // m = n = k = 6080 1.26 -> 0.99 ms, k = 2541 0.72 -> 0.50, 23104 x 1600 x 2541 0.85
-  // -> 0.65, 820 x 17020 x 17020 2.35 -> 1.98, m = n = k = 1520 73 -> 60 us; 1600 x
-  // 1600 x 23104 0.49 -> 0.47 (49 tiles, five splits each either way).
+  // One workgroup per CU: the tiles that fill whole rounds of the chip are taken by
+  // one workgroup each, those of the last round share it by splitting their k.  With
+  // every tile split over workgroups so that rounds are 90 % full, and partials of the
+  // whole output in FP64, before: m = n = k = 6080 1.24 -> 1.12 ms, k = 2541 0.70 -> 0.60,
+  // 820 x 17020 x 17020 2.34 -> 2.12, m = n = k = 1520 74 -> 60 us; 1600 x 1600 x 23104
+  // 0.49 -> 0.46 (49 tiles, five splits each either way).
   const int64_t tiles = int64_t(p.tiles.count) * g.batch;
+  // An FP32 chain's rounding grows with its length (by its square root where the terms'
+  // signs are random, in proportion where they agree), so no tile's chain is longer than
+  // it would be with every tile's k cut alike for rounds that are at least 90 % full
+  // (products of 2048 tiles and more: one chain), and chains meet in FP64.  Whole tiles in
+  // one chain, operands of one sign: rms error 6.5e-7 of the sum at 4352 x 4096 x 6144 and
+  // 8.9e-7 at 820 x 17020 x 8510; so 1.5e-7 both.  The further partial sums cost m = n = k =
+  // 6080 0.98 -> 1.12 ms, k = 2541 0.47 -> 0.60, 820 x 17020 x 17020 1.97 -> 2.12.
+  p.chain = KS;
+  if (tiles < 2048 && KS >= 32) {
+    double best = 0.0;
+    for (int64_t s = 1; s <= std::min<int64_t>(kCus, KS / 16); ++s) {
+      const double full = double(tiles * s) / double(kCus * ceil_div(tiles * s, kCus));
+      if (full <= best + 1e-9) continue;
+      best = full;
+      p.chain = ceil_div(KS, s);
+      if (full >= 0.9) break;
+    }
+  }
+  p.pieces = int(ceil_div(KS, p.chain));
   p.whole = tiles / kCus * kCus;
   p.rest = tiles - p.whole;
   p.splits = 1;
@@ -538,6 +580,7 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
     double best = 2.3 * double(KS);
     for (int64_t s = 2; s <= std::min<int64_t>(kCus, KS / 16); ++s) {
       const int64_t kps = ceil_div(KS, s), used = ceil_div(KS, kps);
+      if (kps > p.chain) continue;
       const double t = 2.3 * double(kps * ceil_div(p.rest * used, kCus)) + 0.107 * double(p.rest * used) + 6.0;
       if (t < best) {
         best = t;
@@ -546,27 +589,32 @@ GemmLaunch gemm_bf16x3(hipStream_t stream, const Gemm& g, GemmWorkspace* ws) {
       }
     }
   }
-  if (p.splits > 1) {
-    if (ws->buf.resize(size_t(p.rest) * size_t(p.splits) * kTileF4 * sizeof(f4))) ++ws->gen;
-    p.W = ws->buf.as<f4>();
-  } else {
+  if (p.splits == 1) {
     p.whole = tiles;
     p.rest = 0;
+  }
+  if (p.whole == 0) p.pieces = 1;
+  const int64_t sums = (p.pieces > 1 ? p.whole * p.pieces : 0) + p.rest * p.splits;
+  if (sums > 0) {
+    if (ws->buf.resize(size_t(sums) * kTileF4 * sizeof(f4))) ++ws->gen;
+    p.W = ws->buf.as<f4>();
   }
   // rows four at a time: m, ldc and the batch stride multiples of 4 elements and
   // the output 16 B (FP32) or 32 B (FP64) aligned
   const uintptr_t base = g.Cf ? reinterpret_cast<uintptr_t>(g.Cf) : reinterpret_cast<uintptr_t>(g.C);
   p.vec_rows = g.m % 4 == 0 && g.ldc % 4 == 0 && (g.batch == 1 || g.strideC % 4 == 0) &&
                base % (g.Cf ? 16 : 32) == 0;
-  gemm_bf16x3_kernel<<<unsigned(p.whole + p.rest * p.splits), kProductThreads, 0, stream>>>(p);
+  const unsigned workgroups = unsigned(p.whole + p.rest * p.splits);
+  if (p.pieces > 1) gemm_bf16x3_kernel<true><<<workgroups, kProductThreads, 0, stream>>>(p);
+  else gemm_bf16x3_kernel<false><<<workgroups, kProductThreads, 0, stream>>>(p);
   ETG_LAUNCH("gemm_bf16x3");
-  if (p.rest > 0) {
-    splitk_reduce_bf<<<dim3(kTileF4 / 256, unsigned(p.rest)), 256, 0, stream>>>(p);
+  if (sums > 0) {
+    splitk_reduce_bf<<<dim3(kTileF4 / 256, unsigned(p.pieces > 1 ? tiles : p.rest)), 256, 0, stream>>>(p);
     ETG_LAUNCH("splitk_reduce");
   }
   GemmLaunch info;
   info.kernel = "gemm_bf16x3<256x256>";
-  info.splits = p.splits;
+  info.splits = std::max(p.pieces, p.splits);
   return info;
 }
 
