@@ -53,6 +53,16 @@ class HostCopy {
         done[size_t(i)].store(true, std::memory_order_release);
       }
     };
+    auto issue = [&](int i) {
+      ETG_HIP(hipMemcpyAsync(slot(i), static_cast<const char*>(src) + size_t(i) * piece, length(i), hipMemcpyDeviceToHost,
+                             stream));
+      ETG_HIP(hipEventRecord(events_[size_t(i % kRing)], stream));
+    };
+    int issued = 0;
+    for (; issued < std::min(n, kRing); ++issued) issue(issued);
+    // the work queued before the copy may take seconds: the threads start when its first
+    // piece is here (started before, they turned over in sched_yield: eight busy cores)
+    ETG_HIP(hipEventSynchronize(events_[0]));
     struct Team {                         // joined on every way out
       std::atomic<bool>& stop;
       std::vector<std::thread> threads;
@@ -70,13 +80,6 @@ class HostCopy {
       ETG_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
       return;
     }
-    auto issue = [&](int i) {
-      ETG_HIP(hipMemcpyAsync(slot(i), static_cast<const char*>(src) + size_t(i) * piece, length(i), hipMemcpyDeviceToHost,
-                             stream));
-      ETG_HIP(hipEventRecord(events_[size_t(i % kRing)], stream));
-    };
-    int issued = 0;
-    for (; issued < std::min(n, kRing); ++issued) issue(issued);
     for (int i = 0; i < n; ++i) {
       ETG_HIP(hipEventSynchronize(events_[size_t(i % kRing)]));
       ready.store(i + 1, std::memory_order_release);
