@@ -21,6 +21,7 @@ struct Error : std::runtime_error {
 
 inline void check_hip(hipError_t e, const char* what, const char* file, int line) {
   if (e != hipSuccess) {
+    (void)hipGetLastError();         // reported here, not again by the next launch
     fail(std::string("HIP error in ") + what + " (" + file + ":" + std::to_string(line) +
          "): " + hipGetErrorString(e));
   }
