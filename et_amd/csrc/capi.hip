@@ -23,6 +23,9 @@ thread_local std::string g_last_error;
 
 template <typename F>
 int guarded(F&& f) {
+  struct Scope {                     // no spare memory outside the entry point (set by wf_of)
+    ~Scope() { etg::g_spare = nullptr; }
+  } scope;
   try {
     f();
     return 0;
@@ -38,6 +41,7 @@ int guarded(F&& f) {
 
 etg::CCSD& wf_of(etg_handle* h) {
   if (h == nullptr || h->wf == nullptr) etg::fail("null etg handle");
+  etg::g_spare = h->wf;
   return *h->wf;
 }
 

@@ -54,7 +54,7 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   // one workspace for the products that run as int8 ones, direct and in the
   // transformation passes (one stream): a whole (ov)^3 product takes 45 n_t1^2 bytes
   // (1.7 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
-  // 4 GB, 0.87 s with 2.5 GB)
+  // 4 GB, 0.87 s with 2.5 GB); allocated by the first of them, freed by give_back()
   const double residue_bytes = std::min(4.0e9, std::max(0.4e9, 64.0 * double(N) * double(N)));
   gws_.residue = gws_pass_.residue = std::make_shared<ResidueWorkspace>(size_t(residue_bytes));
   // default ladder batch: G blocks of at most ~12 GB
@@ -96,6 +96,25 @@ double CCSD::result(const double* res) {
   double v = 0.0;
   results(res, 1, &v);
   return v;
+}
+
+// The int8 products' workspace is the one buffer that nothing depends on (the FP64
+// kernels need none): a system that fits without it runs without it.
+bool CCSD::give_back() {
+  ResidueWorkspace* r = gws_.residue.get();
+  if (r == nullptr || r->buf.bytes() == 0) return false;
+  (void)hipDeviceSynchronize();           // queued products use it
+  r->buf.release();
+  r->refused = true;
+  ++gws_.gen;                             // captured passes hold its address
+  ++gws_pass_.gen;
+  return true;
+}
+
+int64_t CCSD::free_memory() const {
+  size_t free_b = 0, total_b = 0;
+  ETG_HIP(hipMemGetInfo(&free_b, &total_b));
+  return int64_t(free_b + gws_.residue->buf.bytes());
 }
 
 double* CCSD::scratch(int slot, int64_t elems, const char* name) {
@@ -924,10 +943,8 @@ void CCSD::jacobian_transpose_transform(const double* b, double* sigma) {
 // 35 % of the free HBM (the record's derivative buffers and the ladder's
 // per-vector work, per vector), at most kMaxTransformBatch or the caller's limit.
 int64_t CCSD::transform_batch_capacity() {
-  size_t free_b = 0, total_b = 0;
-  ETG_HIP(hipMemGetInfo(&free_b, &total_b));
   const double per_vec = 8.0 * double(tape_->derivative_elems() + ladder_vector_elems() + 2 * (n_t1 + n_t2));
-  int64_t nb = int64_t(0.35 * double(free_b) / per_vec);
+  int64_t nb = int64_t(0.35 * double(free_memory()) / per_vec);
   nb = std::max<int64_t>(1, std::min<int64_t>(nb, kMaxTransformBatch));
   if (transform_batch_limit_ > 0) nb = std::min(nb, transform_batch_limit_);
   return nb;
@@ -1108,7 +1125,11 @@ void CCSD::transform_batch(int side, int64_t n_vec, const double* X, double* R, 
     if (graphs && tg != nullptr) {
       ETG_HIP(hipGraphLaunch(tg->exec, stream_));
     } else {
+      const bool int8 = !gws_pass_.residue->refused;
       transform_body(side, prec, nb);
+      // without the int8 products' workspace from some point on: the FP64 kernels' own
+      // workspace is sized by a pass that uses them throughout
+      if (graphs && int8 && gws_pass_.residue->refused) transform_body(side, prec, nb);
       if (graphs) {
         synchronize();                  // buffers are sized; capture the same sequence
         const uint64_t gen = gws_pass_.gen;

@@ -35,10 +35,11 @@ struct DiisSpace {
   DeviceBuffer e, x, G, w, info;
 };
 
-class CCSD {
+class CCSD final : public Spare {
  public:
   CCSD(int64_t n_o, int64_t n_v, int64_t n_J);
   ~CCSD();
+  bool give_back() override;                      // the int8 products' workspace
 
   int64_t n_o, n_v, n_J, n_mo, n_t1, n_t2;
 
@@ -213,6 +214,7 @@ class CCSD {
   hipStream_t stream_ = nullptr;
   HostCopy host_copy_;
   GemmWorkspace gws_;
+  int64_t free_memory() const;                    // of the device, with what give_back() frees
 
   DeviceBuffer Lmo_oo_, Lmo_ov_, Lmo_vo_, Lmo_vv_;
   DeviceBuffer Lt_oo_, Lt_vo_, Lt_vv_, Lt_vvT_;   // L_t1 ov block equals L_mo ov

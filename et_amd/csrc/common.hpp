@@ -30,6 +30,17 @@ inline void check_hip(hipError_t e, const char* what, const char* file, int line
 #define ETG_HIP(call) ::etg::check_hip((call), #call, __FILE__, __LINE__)
 #define ETG_LAUNCH(what) ::etg::check_hip(hipGetLastError(), what, __FILE__, __LINE__)
 
+// Device memory that its owner can do without.  An allocation that fails asks for the
+// spare memory of the object whose entry point the calling thread is in, and tries again.
+class Spare {
+ public:
+  virtual bool give_back() = 0;      // true when some was freed
+
+ protected:
+  ~Spare() = default;
+};
+inline thread_local Spare* g_spare = nullptr;
+
 // Owning device allocation (bytes); moves only.
 class DeviceBuffer {
  public:
@@ -80,9 +91,15 @@ class DeviceBuffer {
     if (host)
       ETG_HIP(hipHostMalloc(&ptr_, bytes, hipHostMallocDefault));
     else
-      ETG_HIP(hipMalloc(&ptr_, bytes));
+      ETG_HIP(allocate(bytes));
     bytes_ = bytes;
     return true;
+  }
+  hipError_t allocate(size_t bytes) {
+    const hipError_t e = hipMalloc(&ptr_, bytes);
+    if (e != hipErrorOutOfMemory || g_spare == nullptr || !g_spare->give_back()) return e;
+    (void)hipGetLastError();
+    return hipMalloc(&ptr_, bytes);
   }
   void* ptr_ = nullptr;
   size_t bytes_ = 0;

@@ -674,10 +674,8 @@ int64_t CCSD::davidson(int side, int64_t n_states, double threshold, int64_t max
   dav_small_.resize(sizeof(double) * size_t(max_dim * max_dim + 2 * max_dim * s1 + 3 * s1 + max_dim + 2 * s1 * s1 + s1));
   {
     const size_t space = sizeof(double) * size_t(n) * size_t(max_dim);
-    size_t free_b = 0, total_b = 0;
-    ETG_HIP(hipMemGetInfo(&free_b, &total_b));
     const size_t held = (dav_V_.on_host() ? 0 : dav_V_.bytes()) + (dav_AV_.on_host() ? 0 : dav_AV_.bytes());
-    const double avail = 0.5 * double(free_b + held);
+    const double avail = 0.5 * double(size_t(free_memory()) + held);
     bool v_host = false, av_host = false;
     if (dav_space_ == 2) {
       v_host = av_host = true;

@@ -85,8 +85,9 @@ struct PackedOperand {
 
 // Packs, products and exponents of the FP64 products that run as int8 ones
 // (gemm_residue.hip).  Allocated once, at its first use, `capacity` bytes long:
-// larger products run in panels, and its address never changes (captured launch
-// sequences hold it).  Products queued on one stream only.
+// larger products run in panels.  Its address never changes while it is there (captured
+// launch sequences hold it); it is freed when another allocation fails (Spare), and not
+// allocated again.  Products queued on one stream only.
 struct ResidueWorkspace {
   explicit ResidueWorkspace(size_t bytes) : capacity(bytes) {}
   size_t capacity;
