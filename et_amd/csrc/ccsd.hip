@@ -52,8 +52,8 @@ CCSD::CCSD(int64_t no, int64_t nv, int64_t nJ) : n_o(no), n_v(nv), n_J(nJ) {
   small_[2].resize(sizeof(double) * std::max(std::max(n * n, J), o * o * o * o));
   small_[3].resize(sizeof(double) * std::max(J * o * n, o * o * o * o));
   // one workspace for the products that run as int8 ones, direct and in the
-  // transformation passes (one stream): a whole (ov)^3 product takes 45 n_t1^2 bytes
-  // (1.7 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
+  // transformation passes (one stream): a whole (ov)^3 product takes 50 n_t1^2 bytes
+  // (1.8 GB at (H2O)8), larger ones run in panels (n_t1 = 14400: residual 0.82 s with
   // 4 GB, 0.87 s with 2.5 GB); allocated by the first of them, freed by give_back()
   const double residue_bytes = std::min(4.0e9, std::max(0.4e9, 64.0 * double(N) * double(N)));
   gws_.residue = gws_pass_.residue = std::make_shared<ResidueWorkspace>(size_t(residue_bytes));

@@ -19,6 +19,7 @@
 // same L2.
 #include "gemm.hpp"
 #include "kernels.hpp"
+#include "tile_map.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -26,6 +27,7 @@
 #include <mutex>
 #include <string>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 namespace etg {
@@ -35,8 +37,6 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kXcds = 8;
-constexpr int kGroupM = 8;
 
 struct Params {
   int64_t m, n, k;
@@ -122,12 +122,20 @@ struct TileLayout {
   static __device__ inline int at(int mn, int k) { return KCONTIG ? mn * LD + k : k * LD + mn; }
 };
 
+struct EveryTile {};
+struct FlaggedBlocks {
+  TileMap tiles;
+  const int* flags;
+  int64_t stride;
+};
+
 // T: arithmetic type of the products (double or float); operands are FP64 in memory.
 // Two workgroups per CU: the FP64 128 x 128 tile fits its 128 accumulator
 // registers and operand staging in 256 VGPRs and 72 KB of LDS, so one
 // workgroup's barrier and LDS refill overlap the other's matrix-core work.
-template <typename T, bool TA, bool TB, int BM, int BN, int BK, bool WIDE>
-__global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p) {
+// F: which tiles, EveryTile or the flagged ones of an int8 product (FlaggedBlocks).
+template <typename T, bool TA, bool TB, int BM, int BN, int BK, bool WIDE, typename F>
+__global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p, F f) {
   using M = Mfma<T>;
   using acc_t = typename M::acc_t;
   constexpr int WM = BM / 2, WN = BN / 2;  // wave sub-tile
@@ -144,11 +152,28 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave & 1, wn = wave >> 1;
-  int tile_m, tile_n;
-  map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
-  const int64_t m0 = int64_t(tile_m) * BM, n0 = int64_t(tile_n) * BN;
   const int64_t bz = blockIdx.z;
   const int64_t split = blockIdx.y;
+  int tile_m, tile_n;
+  int64_t m0, n0;
+  if constexpr (std::is_same_v<F, FlaggedBlocks>) {
+    static_assert(BM == BN && (BM == 128 || BM == 64), "a tile in one flagged block");
+    constexpr int kRows = kTileM / BM;
+    const int per_tile = kRows * (f.tiles.tile_n / BN);
+    // (in dispatch order, round-robin over the XCDs: flagged blocks lie together, and with
+    // a range of tiles per XCD one of them had nearly all the work)
+    const int slot = int(blockIdx.x) / per_tile, part = int(blockIdx.x) % per_tile;
+    if (!tile_of(f.tiles, slot, tile_m, tile_n)) return;
+    const int mi = part % kRows * BM, ni = part / kRows * BN;
+    if (f.flags[bz * f.stride + int64_t(slot) * kFlaggedBlocks + mi / 128 + ni / 128 * 2] == 0) return;
+    m0 = int64_t(tile_m) * kTileM + mi;
+    n0 = int64_t(tile_n) * f.tiles.tile_n + ni;
+    if (m0 >= p.m || n0 >= p.n) return;
+  } else {
+    map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
+    m0 = int64_t(tile_m) * BM;
+    n0 = int64_t(tile_n) * BN;
+  }
   const double* A = p.A + bz * p.strideA;
   const double* B = p.B + bz * p.strideB;
   const int64_t kbeg = split * p.k_per_split;
@@ -498,16 +523,16 @@ const char* launch_cfg(hipStream_t stream, const Gemm& g, Params p, int splits) 
   dim3 grid(p.tiles_m * p.tiles_n, splits, unsigned(g.batch));
   const char* name;
   if (!g.ta && !g.tb) {
-    gemm_mfma16<T, false, false, BM, BN, BK, WIDE><<<grid, kThreads, 0, stream>>>(p);
+    gemm_mfma16<T, false, false, BM, BN, BK, WIDE, EveryTile><<<grid, kThreads, 0, stream>>>(p, EveryTile{});
     name = kernel_name<T, false, false, BM, BN, WIDE>();
   } else if (!g.ta && g.tb) {
-    gemm_mfma16<T, false, true, BM, BN, BK, WIDE><<<grid, kThreads, 0, stream>>>(p);
+    gemm_mfma16<T, false, true, BM, BN, BK, WIDE, EveryTile><<<grid, kThreads, 0, stream>>>(p, EveryTile{});
     name = kernel_name<T, false, true, BM, BN, WIDE>();
   } else if (g.ta && !g.tb) {
-    gemm_mfma16<T, true, false, BM, BN, BK, WIDE><<<grid, kThreads, 0, stream>>>(p);
+    gemm_mfma16<T, true, false, BM, BN, BK, WIDE, EveryTile><<<grid, kThreads, 0, stream>>>(p, EveryTile{});
     name = kernel_name<T, true, false, BM, BN, WIDE>();
   } else {
-    gemm_mfma16<T, true, true, BM, BN, BK, WIDE><<<grid, kThreads, 0, stream>>>(p);
+    gemm_mfma16<T, true, true, BM, BN, BK, WIDE, EveryTile><<<grid, kThreads, 0, stream>>>(p, EveryTile{});
     name = kernel_name<T, true, true, BM, BN, WIDE>();
   }
   ETG_LAUNCH("gemm_mfma16");
@@ -1062,6 +1087,31 @@ void set_gemm_autotune(bool on) { g_autotune.store(on); }
 int64_t gemm_tuned_shapes() {
   std::lock_guard<std::mutex> lock(g_tune_mu);
   return int64_t(g_tuned.size());
+}
+
+namespace {
+template <int BM, bool WIDE>
+void launch_flagged(hipStream_t stream, const Gemm& g, const Params& p, const FlaggedBlocks& f) {
+  const int64_t per_tile = int64_t(kTileM / BM) * (f.tiles.tile_n / BM);
+  const dim3 grid(unsigned(f.tiles.count * per_tile), 1, unsigned(g.batch));
+  using F = FlaggedBlocks;
+  if (!g.ta && !g.tb) gemm_mfma16<double, false, false, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else if (!g.ta && g.tb) gemm_mfma16<double, false, true, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else if (g.ta && !g.tb) gemm_mfma16<double, true, false, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else gemm_mfma16<double, true, true, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  ETG_LAUNCH("gemm_mfma16");
+}
+}  // namespace
+
+void gemm_flagged_blocks(hipStream_t stream, const Gemm& g, const TileMap& tiles, const int* flags, int64_t flag_stride) {
+  int splits = 1;
+  const Params p = split_params(g, nullptr, 1, &splits);
+  const FlaggedBlocks f{tiles, flags, flag_stride};
+  // 64 x 64 where 128 x 128 would leave CUs idle with all blocks flagged
+  const bool small = int64_t(tiles.count) * (kTileM / 128) * (tiles.tile_n / 128) * g.batch < 512;
+  const bool wide = std::max(g.lda, g.ldb) >= (int64_t(1) << 21);
+  if (small) wide ? launch_flagged<64, true>(stream, g, p, f) : launch_flagged<64, false>(stream, g, p, f);
+  else wide ? launch_flagged<128, true>(stream, g, p, f) : launch_flagged<128, false>(stream, g, p, f);
 }
 
 bool runs_as_residues(const Gemm& g, Prec prec, const GemmWorkspace* ws) {

@@ -1,19 +1,25 @@
-// FP64 products on the int8 matrix cores, exact modulo 15 coprime moduli
+// FP64 products on the int8 matrix cores, exact modulo 16 coprime moduli
 // (residue.hpp has the arithmetic and its error).
 //
 // The FP64 matrix cores reach 78 TFLOP/s on this chip and the FP64 kernels 62
-// of them; the int8 matrix cores run v_mfma_i32_16x16x64_i8 at 4.2-4.9 POP/s,
-// so 15 int8 products per FP64 product are worth up to 280 TFLOP/s.  A product
-// runs as
+// of them; the int8 products here run at 2.4-2.6 POP/s (the kernel's 2548 TOP/s
+// on random bytes; 3491 on zeros, where the power limit does not bind), so 17 of them
+// per FP64 product are worth up to 150 TFLOP/s.  A product runs as
 //   1. row norms of op(A) and op(B)^T            (reads each operand once)
-//   2. residue packs: 15 bytes per element, in the order the matrix cores read
-//   3. 15 int8 products, each sum reduced to one byte per output
-//   4. reconstruction of C from its 15 bytes     (writes C once)
+//   2. residue packs: 17 bytes per element, in the order the matrix cores read
+//      (a byte per modulus, and the magnitude)
+//   3. 16 int8 products, each sum reduced to one byte per output, and before
+//      them the product of the magnitudes, which flags the 128 x 128 blocks that
+//      need the FP64 kernel
+//   4. reconstruction of C from its 16 bytes     (writes C once)
+//   5. the flagged blocks on the FP64 kernel
 // on panels of A and B whose packs fit a bounded workspace.
 #include <algorithm>
 #include <string>
+#include <type_traits>
 
 #include "gemm.hpp"
+#include "kernels.hpp"
 #include "residue.hpp"
 #include "tile_map.hpp"
 
@@ -25,9 +31,11 @@ using residue::kModuli;
 
 typedef int i4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kDepth = 64;                    // k per step (one MFMA step)
+constexpr int kPlanes = kModuli + 1;          // of a pack: the residues and the magnitudes
 
 // ---------------------------------------------------------------------------
 // 1. Scale exponents.  Element (r, k) of the rows x K operand is X[k + r ld]
@@ -37,7 +45,8 @@ constexpr int kDepth = 64;                    // k per step (one MFMA step)
 // One workgroup per row.
 __global__ __launch_bounds__(256) void row_exponents_kcontig_kernel(const double* __restrict__ X, int64_t ld,
                                                                     int64_t strideX, int64_t K,
-                                                                    int64_t exp_stride, int* __restrict__ e) {
+                                                                    int64_t exp_stride, int* __restrict__ e,
+                                                                    float* __restrict__ nrm) {
   __shared__ double ss[4];
   __shared__ unsigned long long mm[4];
   const int64_t r = blockIdx.x, bz = blockIdx.y;
@@ -67,6 +76,7 @@ __global__ __launch_bounds__(256) void row_exponents_kcontig_kernel(const double
       mx = mm[q] > mx ? mm[q] : mx;
     }
     e[bz * exp_stride + r] = residue::scale_exponent(s, mx, K);
+    nrm[bz * exp_stride + r] = residue::scaled_norm(s, mx);
   }
 }
 
@@ -110,7 +120,8 @@ __global__ __launch_bounds__(256) void row_norms_partial_kernel(const double* __
 __global__ __launch_bounds__(256) void row_exponents_finish_kernel(const double* __restrict__ ps,
                                                                    const unsigned long long* __restrict__ pm,
                                                                    int64_t rows, int parts, int64_t K,
-                                                                   int64_t exp_stride, int* __restrict__ e) {
+                                                                   int64_t exp_stride, int* __restrict__ e,
+                                                                    float* __restrict__ nrm) {
   const int64_t r = int64_t(blockIdx.x) * 256 + threadIdx.x, bz = blockIdx.y;
   if (r >= rows) return;
   double s = 0.0;
@@ -121,16 +132,16 @@ __global__ __launch_bounds__(256) void row_exponents_finish_kernel(const double*
     mx = pm[at] > mx ? pm[at] : mx;
   }
   e[bz * exp_stride + r] = residue::scale_exponent(s, mx, K);
+  nrm[bz * exp_stride + r] = residue::scaled_norm(s, mx);
 }
 
 // ---------------------------------------------------------------------------
 // 2. Residue packs.  Per modulus one plane of 1 KB chunks (16 rows x 64 k: lane
 // l holds 16 consecutive k of row l % 16 from 16 (l / 16) on), row blocks
-// outermost, k steps contiguous.  One wave forms the 15 chunks of a (row block,
-// k step).  About 75 VALU operations per element (5 per modulus) against 8
-// bytes read and 15 written: bound by HBM, 37 M elements in 200 us.  (With 125
-// operations, residues formed in FP32, 215; products of 1520^3 133 -> 127 us,
-// with unconditional loads 121.)
+// outermost, k steps contiguous.  One wave forms the 17 chunks of a (row block,
+// k step).  Some 90 VALU operations per element (four per modulus, and the bytes'
+// packing) against 8 bytes read and 17 written: bound by HBM, 37 M elements in
+// 154 us (6.0 TB/s).
 // ---------------------------------------------------------------------------
 // The 16 values are formed here, in the order of the source, not where they are used.
 __device__ inline void pin(uint32_t (&x)[16]) {
@@ -139,18 +150,35 @@ __device__ inline void pin(uint32_t (&x)[16]) {
   __builtin_amdgcn_sched_barrier(0);
 }
 
+// The low bytes of 16 words.
+__device__ inline u4 pack_bytes(const uint32_t (&x)[16]) {
+  u4 w;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint32_t p01 = __builtin_amdgcn_perm(x[4 * q + 1], x[4 * q], 0x0c0c0400u);
+    const uint32_t p23 = __builtin_amdgcn_perm(x[4 * q + 3], x[4 * q + 2], 0x0c0c0400u);
+    w[q] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+  }
+  return w;
+}
+
 constexpr int kPackLd = kDepth + 2;           // LDS row of a staged chunk (doubles)
 
 __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restrict__ X, int64_t ld, int64_t strideX,
                                                            int kcontig, int64_t rows, int64_t K, int64_t KS,
                                                            int64_t plane, const int* __restrict__ e,
-                                                           int64_t exp_stride, u4* __restrict__ P) {
+                                                           int64_t exp_stride, u4* __restrict__ P,
+                                                           int* __restrict__ flags, int64_t n_flags) {
   __shared__ __attribute__((aligned(16))) double stage[4][16 * kPackLd];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t ks = int64_t(blockIdx.x) * 4 + wave;
   const int64_t rb = blockIdx.y, bz = blockIdx.z;
   const int64_t r = rb * 16 + (lane & 15), k0 = ks * kDepth + 16 * (lane >> 4);
   const int ex = r < rows ? e[bz * exp_stride + r] : 0;
+  // the products' flags, cleared on the way
+  for (int64_t f = ((bz * gridDim.y + rb) * gridDim.x + blockIdx.x) * 256 + threadIdx.x; f < n_flags;
+       f += int64_t(gridDim.x) * gridDim.y * gridDim.z * 256)
+    flags[f] = 0;
   uint32_t lo[16], hi[16];
   if (kcontig) {
     // whole rows of the chunk (512 contiguous bytes per load) through LDS: read by
@@ -187,7 +215,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
     for (int j = 0; j < 16; ++j) residue::to_integer(j < n ? v[j] : 0.0, ex, lo[j], hi[j]);
   }
   if (ks >= KS) return;
-  u4* dst = P + bz * kModuli * plane + (rb * KS + ks) * 64 + lane;
+  u4* dst = P + bz * kPlanes * plane + (rb * KS + ks) * 64 + lane;
 #pragma unroll
   for (int i = 0; i < kModuli; ++i) {
     // residue_byte of the 16 elements side by side: a byte dot product's result can
@@ -206,15 +234,12 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
 #pragma unroll
       for (int j = 0; j < 16; ++j) x[j] = residue::low_byte(x[j], kC.invf[i], kC.c[i]);
     }
-    u4 w;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const uint32_t p01 = __builtin_amdgcn_perm(x[4 * q + 1], x[4 * q], 0x0c0c0400u);
-      const uint32_t p23 = __builtin_amdgcn_perm(x[4 * q + 3], x[4 * q + 2], 0x0c0c0400u);
-      w[q] = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
-    }
-    dst[i * plane] = w;
+    dst[i * plane] = pack_bytes(x);
   }
+  uint32_t q[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) q[j] = residue::magnitude_byte(hi[j]);
+  dst[kModuli * plane] = pack_bytes(q);
 }
 
 // ---------------------------------------------------------------------------
@@ -227,7 +252,7 @@ __global__ __launch_bounds__(256) void residue_pack_kernel(const double* __restr
 // read in the step before.  A step is 32 MFMAs (512 cycles) per wave against 12
 // KB of LDS reads.  Two workgroups per CU hide barriers, the first copies and the
 // byte epilogue under each other's products, but drift apart along k until their
-// tiles no longer meet in the L2: TOP/s with 15 moduli of random bytes for
+// tiles no longer meet in the L2: TOP/s with 15 planes of random bytes for
 //   m = n = 6912, k =    1600    3200    14400   28800      m = n = k = 1536
 //   256 x 128            2360    2400     1780    1990                  1790
 //   256 x 256            2170    2440     2560    2480                  1470
@@ -239,6 +264,7 @@ constexpr int64_t kShortDepth = 3200;
 
 constexpr int kWaveM = 8, kWaveN = 4;         // 16 x 16 blocks of a wave
 constexpr int kBlocksM = kTileM / 16;
+constexpr int kFlags = kFlaggedBlocks;        // 128 x 128 blocks of a tile (two of them in 256 x 128)
 
 struct Params {
   const u4 *A, *B;                 // packs (planes of the first modulus)
@@ -247,6 +273,14 @@ struct Params {
   int64_t planeA, planeB, planeR;  // from one modulus to the next (u4, u4, u32 units)
   int64_t strideA, strideB, strideR;   // from one batch entry to the next
   TileMap tiles;
+  // per tile its 128 x 128 blocks (kFlags, row by row) that are left to the FP64 kernel:
+  // zero before the launch, set by the product of the magnitudes
+  int* flags;
+  int64_t strideF;
+  // of the guard product
+  int64_t m, n;
+  const float *na, *nb;            // norms of the rows
+  int64_t na_stride, nb_stride;
 };
 
 // Waits until at most N of this wave's vector-memory operations are outstanding.
@@ -258,6 +292,19 @@ __device__ inline void wait_copies() {
   asm volatile("" ::: "memory");
 }
 
+// 16 x 16 sums of products of 8-bit floats (5 exponent bits), half h of a chunk's k.
+__device__ inline i4 mfma_magnitudes(i4 a, i4 b, int h, i4 c) {
+  typedef int i2 __attribute__((ext_vector_type(2)));
+  const i2 ah = h ? i2{a[2], a[3]} : i2{a[0], a[1]}, bh = h ? i2{b[2], b[3]} : i2{b[0], b[1]};
+  return __builtin_bit_cast(i4, __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8(__builtin_bit_cast(long, ah), __builtin_bit_cast(long, bh),
+                                                                          __builtin_bit_cast(f4, c), 0, 0, 0));
+}
+
+// blockIdx.y = 0: the product of the magnitudes, which flags the blocks with an output
+// below the threshold or with a row that is not finite.  It comes first, and a product
+// that finds its blocks flagged already has nothing to do; one that started before gives
+// residues that nobody reads.  (A launch of its own left CUs idle: 820 x 17020 x 17020
+// 6.19 ms with 15 moduli, 5.43 in one.)
 template <int WN, int kStages>
 __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_kernel(Params p) {
   constexpr int kBlocksN = WN * kWaveN;
@@ -268,8 +315,16 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
   const int slot = slot_of(blockIdx.x, gridDim.x);
   int tile_m, tile_n;
   if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
-  const int z = blockIdx.y;
+  const bool guard = blockIdx.y == 0;
+  const int z = guard ? kModuli : int(blockIdx.y) - 1;
   const int64_t bz = blockIdx.z;
+  int* flags = p.flags + bz * p.strideF + int64_t(slot) * kFlags;
+  if (!guard) {
+    int all = 1;
+#pragma unroll
+    for (int q = 0; q < WN; ++q) all &= __hip_atomic_load(&flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(all)) return;
+  }
   const u4* sa = p.A + bz * p.strideA + z * p.planeA + int64_t(tile_m) * kBlocksM * p.KS * 64;
   const u4* sb = p.B + bz * p.strideB + z * p.planeB + int64_t(tile_n) * kBlocksN * p.KS * 64;
   const __amdgpu_buffer_rsrc_t ra =
@@ -298,8 +353,9 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
 #pragma unroll
     for (int j = 0; j < kWaveN; ++j) acc[i][j] = i4{0, 0, 0, 0};
   // the four B fragments, then each row block's products with the next block's A
-  // fragment read ahead of them (order pinned by the scheduling groups)
-  auto compute = [&](int stage) {
+  // fragment read ahead of them (order pinned by the scheduling groups); the magnitudes'
+  // 64 k are two products of 32 k, sums in FP32
+  auto compute = [&](int stage, auto magnitudes) {
     const u4* As = &lds[stage][wm * kWaveM * 64];
     const u4* Bs = &lds[stage][(kBlocksM + wn * kWaveN) * 64];
     i4 a[2], b[kWaveN];
@@ -309,31 +365,77 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
 #pragma unroll
     for (int i = 0; i < kWaveM; ++i) {
       if (i + 1 < kWaveM) a[(i + 1) & 1] = __builtin_bit_cast(i4, As[(i + 1) * 64 + lane]);
+      if constexpr (magnitudes) {
 #pragma unroll
-      for (int j = 0; j < kWaveN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i & 1], b[j], acc[i][j], 0, 0, 0);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < kWaveN; ++j) acc[i][j] = mfma_magnitudes(a[i & 1], b[j], h, acc[i][j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kWaveN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[i & 1], b[j], acc[i][j], 0, 0, 0);
+      }
       if (i == 0) __builtin_amdgcn_sched_group_barrier(0x100, kWaveN + 2, 0);
       else if (i + 1 < kWaveM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, kWaveN, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, magnitudes ? 2 * kWaveN : kWaveN, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
+
   const int64_t ns = p.KS;
 #pragma unroll
   for (int s = 0; s < kStages - 1; ++s)
     if (s < ns) load(s, s);
-  int stage = 0;
-  int64_t s = 0;
-  for (; s + kStages - 1 < ns; ++s) {
-    wait_copies<(kStages - 2) * (kCopiesA + kCopiesB)>();
-    load(stage == 0 ? kStages - 1 : stage - 1, s + kStages - 1);
-    compute(stage);
-    stage = stage + 1 == kStages ? 0 : stage + 1;
-  }
-  for (; s < ns; ++s) {
-    wait_copies<0>();
-    compute(stage);
-    stage = stage + 1 == kStages ? 0 : stage + 1;
+  auto steps = [&](auto magnitudes) {
+    int stage = 0;
+    int64_t s = 0;
+    for (; s + kStages - 1 < ns; ++s) {
+      wait_copies<(kStages - 2) * (kCopiesA + kCopiesB)>();
+      load(stage == 0 ? kStages - 1 : stage - 1, s + kStages - 1);
+      compute(stage, magnitudes);
+      stage = stage + 1 == kStages ? 0 : stage + 1;
+    }
+    for (; s < ns; ++s) {
+      wait_copies<0>();
+      compute(stage, magnitudes);
+      stage = stage + 1 == kStages ? 0 : stage + 1;
+    }
+  };
+  if (!guard) steps(std::false_type{});
+  if (guard) {
+    steps(std::true_type{});
+    // (in the copies' LDS: beside a second array the compiler waits for every copy in
+    // flight before each read of a stage, 1.7 times the kernel's time)
+    int* found = reinterpret_cast<int*>(&lds[0][0]);
+    __syncthreads();
+    const int64_t row0 = int64_t(tile_m) * kTileM + wm * (kWaveM * 16) + 4 * (lane >> 4);
+    const int64_t col0 = (int64_t(tile_n) * kBlocksN + wn * kWaveN) * 16 + (lane & 15);
+    if (tid < kFlags)                          // blocks past the edge have nothing to do
+      found[tid] = int64_t(tile_m) * kTileM + (tid & 1) * 128 >= p.m || int64_t(tile_n) * (kBlocksN * 16) + (tid >> 1) * 128 >= p.n;
+    __syncthreads();
+    // (norms of rows past the edge: inside the padded array, not used)
+    const f4* na = reinterpret_cast<const f4*>(p.na + bz * p.na_stride + row0);
+    const float* nb = p.nb + bz * p.nb_stride + col0;
+    f4 nr[kWaveM];
+#pragma unroll
+    for (int i = 0; i < kWaveM; ++i) nr[i] = na[i * 4];
+    bool lost = false;
+#pragma unroll
+    for (int j = 0; j < kWaveN; ++j) {
+      const float nc = col0 + j * 16 < p.n ? nb[j * 16] : residue::kZeroNorm;
+#pragma unroll
+      for (int i = 0; i < kWaveM; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int bits = acc[i][j][r];       // (bit_cast of the element itself takes the first one)
+          lost |= row0 + i * 16 + r < p.m && nr[i][r] > 0.0f && nc > 0.0f &&
+                  !(__builtin_bit_cast(float, bits) >= residue::kThreshold * fmaxf(nr[i][r], nc));
+        }
+    }
+    if (__ballot(lost) != 0 && lane == 0) found[wm + 2 * (wn / 2)] = 1;
+    __syncthreads();
+    if (tid < WN) __hip_atomic_store(&flags[tid], found[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
   }
   const double m = kC.md[z], inv = kC.invd[z];
   uint32_t* R = p.R + bz * p.strideR + z * p.planeR +
@@ -353,11 +455,10 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
 }
 
 // ---------------------------------------------------------------------------
-// 4. Reconstruction: C = alpha op(A) op(B) + beta C from the 15 bytes of each
+// 4. Reconstruction: C = alpha op(A) op(B) + beta C from the 16 bytes of each
 // output.  A lane takes the four rows of one column that its word of each plane
-// holds.  Bound by HBM (15 bytes read, 8 written, 8 more read with beta).  A
-// row or column with an infinity or NaN is summed term by term from the
-// operands instead.
+// holds.  Bound by HBM (16 bytes read, 8 written, 8 more read with beta).
+// Flagged blocks are the FP64 kernel's (gemm_flagged_blocks).
 // ---------------------------------------------------------------------------
 struct Output {
   const uint32_t* R;
@@ -370,19 +471,9 @@ struct Output {
   double* C;
   int64_t ldc, strideC;
   int vec_rows;                           // rows written four at a time (alignment checked on the host)
-  const double *A, *B;                    // panel operands, for the rows that are not finite
-  int64_t lda, strideA, ldb, strideB;
-  int a_kcontig, b_kcontig;
+  const int* flags;                       // as in Params
+  int64_t strideF;
 };
-
-__device__ double plain_sum(const Output& p, int64_t bz, int64_t row, int64_t col) {
-  const double* a = p.A + bz * p.strideA + (p.a_kcontig ? row * p.lda : row);
-  const double* b = p.B + bz * p.strideB + (p.b_kcontig ? col * p.ldb : col);
-  const int64_t sa = p.a_kcontig ? 1 : p.lda, sb = p.b_kcontig ? 1 : p.ldb;
-  double s = 0.0;
-  for (int64_t k = 0; k < p.K; ++k) s += a[k * sa] * b[k * sb];
-  return s;
-}
 
 __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
   const int lane = threadIdx.x & 63;
@@ -393,6 +484,7 @@ __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
   int tile_m, tile_n;
   if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
   const int64_t bz = blockIdx.y;
+  if (p.flags[bz * p.strideF + int64_t(slot) * kFlags + (blk % kBlocksM) / 8 + blk / kBlocksM / 8 * 2]) return;
   const int64_t row = int64_t(tile_m) * kTileM + (blk % kBlocksM) * 16 + 4 * (lane >> 4);
   const int64_t col = (int64_t(tile_n) * blocks_n + blk / kBlocksM) * 16 + (lane & 15);
   if (row >= p.m || col >= p.n) return;
@@ -413,12 +505,7 @@ __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
       hi = fma(b, kC.fhi[i], hi);
       lo = fma(b, kC.flo[i], lo);
     }
-    v[r] = 0.0;
-    if (r < rows) {
-      const int e = ea[r];
-      v[r] = (e == residue::kNotFinite || eb == residue::kNotFinite) ? plain_sum(p, bz, row + r, col)
-                                                                    : residue::reconstruct(hi, lo, e, eb);
-    }
+    v[r] = r < rows ? residue::reconstruct(hi, lo, ea[r], eb) : 0.0;
   }
   double* c = p.C + bz * p.strideC + row + col * p.ldc;
   if (p.vec_rows) {
@@ -450,8 +537,8 @@ struct Panels {
   int64_t a_entries, b_entries;               // batch entries packed per group (1 for a shared operand)
   int64_t rm_p, rn_p;                         // panel rows padded to whole tiles
   int64_t parts;                              // k ranges of the row norms
-  size_t bytes_a, bytes_b, bytes_r, bytes_e, bytes_n;
-  size_t total() const { return bytes_a + bytes_b + bytes_r + bytes_e + bytes_n; }
+  size_t bytes_a, bytes_b, bytes_r, bytes_e, bytes_n, bytes_f;
+  size_t total() const { return bytes_a + bytes_b + bytes_r + bytes_e + bytes_n + bytes_f; }
 };
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
@@ -465,13 +552,19 @@ bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
   p.a_entries = g.strideA == 0 ? 1 : p.batch;
   p.b_entries = g.strideB == 0 ? 1 : p.batch;
   if (p.same) p.rm_p = p.rn_p = std::max(p.rm_p, p.rn_p);
-  p.bytes_a = align256(size_t(p.a_entries * kModuli) * size_t(p.rm_p * p.KS * kDepth));
-  p.bytes_b = p.same ? 0 : align256(size_t(p.b_entries * kModuli) * size_t(p.rn_p * p.KS * kDepth));
-  p.bytes_e = align256(sizeof(int) * size_t(p.a_entries * p.rm_p + p.b_entries * p.rn_p));
+  p.bytes_a = align256(size_t(p.a_entries * kPlanes) * size_t(p.rm_p * p.KS * kDepth));
+  p.bytes_b = p.same ? 0 : align256(size_t(p.b_entries * kPlanes) * size_t(p.rn_p * p.KS * kDepth));
+  p.bytes_e = align256((sizeof(int) + sizeof(float)) * size_t(p.a_entries * p.rm_p + p.b_entries * p.rn_p));
   p.bytes_n = align256(16 * size_t(std::max(p.a_entries * p.rm_p, p.b_entries * p.rn_p) * p.parts));
-  p.bytes_r = 0;
+  p.bytes_r = p.bytes_f = 0;
   if (p.total() >= capacity) return false;
-  const int64_t room = int64_t(capacity - p.total()) / (p.batch * kModuli) - 256;   // outputs
+  // outputs: a byte per modulus, and the flags of a tile
+  const int64_t room = int64_t(double(capacity - p.total()) / (double(p.batch) * (kModuli + 0.001))) - 512;
+  auto residues_of = [&](int64_t outputs) {
+    p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(outputs));
+    p.bytes_f = align256(sizeof(int) * kFlags * size_t(p.batch) * size_t(outputs / (int64_t(kTileM) * p.tile_n)));
+    return p.total() <= capacity;
+  };
   p.out_m = p.rm_p;
   p.out_n = p.rn_p;
   // a quarter of the capacity (or all) for the residues: thinner pieces leave CUs idle
@@ -488,16 +581,14 @@ bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
     }
     if (fit * p.tile_n >= std::min<int64_t>(p.rn_p, 512)) {
       p.out_n = fit * p.tile_n;
-      p.bytes_r = align256(size_t(kModuli) * size_t(outputs(p.out_n)));
-      return p.total() <= capacity;
+      return residues_of(outputs(p.out_n));
     }
   }
   const int64_t least = std::min<int64_t>(p.out_n, 512);
   if (p.out_m * p.out_n > room) p.out_n = std::max(least, room / p.out_m / p.tile_n * p.tile_n);
   if (p.out_m * p.out_n > room) p.out_m = room / p.out_n / kTileM * kTileM;
   if (p.out_m < std::min<int64_t>(p.rm_p, 1024)) return false;
-  p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(p.out_m * p.out_n));
-  return p.total() <= capacity;
+  return residues_of(p.out_m * p.out_n);
 }
 
 // The whole product where its packs fit the capacity, else equal groups of the
@@ -532,9 +623,10 @@ bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
 
 // One operand panel: exponents, then the pack.
 void pack_operand(hipStream_t s, const double* X, int64_t ld, int64_t strideX, bool kcontig, int64_t rows, int64_t K,
-                  int64_t KS, int64_t rows_p, int64_t entries, int64_t parts, void* norms, int* e, u4* P) {
+                  int64_t KS, int64_t rows_p, int64_t entries, int64_t parts, void* norms, int* e, float* nrm, u4* P, int* flags,
+                  int64_t n_flags) {
   if (kcontig) {
-    row_exponents_kcontig_kernel<<<dim3(unsigned(rows), unsigned(entries)), 256, 0, s>>>(X, ld, strideX, K, rows_p, e);
+    row_exponents_kcontig_kernel<<<dim3(unsigned(rows), unsigned(entries)), 256, 0, s>>>(X, ld, strideX, K, rows_p, e, nrm);
     ETG_LAUNCH("row_exponents");
   } else {
     const int64_t k_per = ceil_div(K, parts);
@@ -544,11 +636,12 @@ void pack_operand(hipStream_t s, const double* X, int64_t ld, int64_t strideX, b
         X, ld, strideX, rows, K, k_per, ps, pm);
     ETG_LAUNCH("row_norms");
     row_exponents_finish_kernel<<<dim3(unsigned(ceil_div(rows, 256)), unsigned(entries)), 256, 0, s>>>(
-        ps, pm, rows, int(parts), K, rows_p, e);
+        ps, pm, rows, int(parts), K, rows_p, e, nrm);
     ETG_LAUNCH("row_exponents");
   }
   residue_pack_kernel<<<dim3(unsigned(ceil_div(KS, 4)), unsigned(ceil_div(rows, 16)), unsigned(entries)), 256, 0, s>>>(
-      X, ld, strideX, kcontig ? 1 : 0, rows, K, KS, rows_p * KS * (kDepth / 16), e, rows_p, P);
+      X, ld, strideX, kcontig ? 1 : 0, rows, K, KS, rows_p * KS * (kDepth / 16), e, rows_p, P,
+      flags, n_flags);
   ETG_LAUNCH("residue_pack");
 }
 
@@ -599,7 +692,10 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
   uint32_t* R = reinterpret_cast<uint32_t*>(base + p.bytes_a + p.bytes_b);
   int* ea = reinterpret_cast<int*>(base + p.bytes_a + p.bytes_b + p.bytes_r);
   int* eb = p.same ? ea : ea + p.a_entries * p.rm_p;
+  float* na = reinterpret_cast<float*>(ea + p.a_entries * p.rm_p + p.b_entries * p.rn_p);
+  float* nrm_b = p.same ? na : na + p.a_entries * p.rm_p;
   void* norms = base + p.bytes_a + p.bytes_b + p.bytes_r + p.bytes_e;
+  int* flags = reinterpret_cast<int*>(base + p.bytes_a + p.bytes_b + p.bytes_r + p.bytes_e + p.bytes_n);
   const bool a_kcontig = g.ta, b_kcontig = !g.tb;
   const int64_t pm = ceil_div(g.m, p.rows_m), pn = ceil_div(g.n, p.rows_n);
   // one panel of op(A), group of batch entries and panel of op(B); an operand is
@@ -611,12 +707,18 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
     const double* A = g.A + b0 * g.strideA + (a_kcontig ? m0 * g.lda : m0);
     const double* B = g.B + b0 * g.strideB + (b_kcontig ? n0 * g.ldb : n0);
     const int64_t a_want = mi + (g.strideA == 0 ? 0 : pm * bi), b_want = ni + (g.strideB == 0 ? 0 : pn * bi);
-    if (a_want != a_is)
+    const int64_t n_flags = int64_t(p.bytes_f / sizeof(int));
+    bool clear = false;                  // the flags of the next launch
+    if (a_want != a_is) {
       pack_operand(stream, A, g.lda, g.strideA, a_kcontig, m, g.k, p.KS, p.rm_p, g.strideA == 0 ? 1 : nb, p.parts, norms,
-                   ea, PA);
-    if (b_want != b_is && !p.same)
+                   ea, na, PA, flags, n_flags);
+      clear = true;
+    }
+    if (b_want != b_is && !p.same) {
       pack_operand(stream, B, g.ldb, g.strideB, b_kcontig, n, g.k, p.KS, p.rn_p, g.strideB == 0 ? 1 : nb, p.parts, norms,
-                   eb, PB);
+                   eb, nrm_b, PB, flags, clear ? 0 : n_flags);
+      clear = true;
+    }
     a_is = a_want;
     b_is = b_want;
     for (int64_t c0 = 0; c0 < n; c0 += p.out_n) {
@@ -633,11 +735,19 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
         q.planeA = p.rm_p * p.KS * (kDepth / 16);
         q.planeB = p.rn_p * p.KS * (kDepth / 16);
         q.planeR = int64_t(q.tiles.count) * kTileM * p.tile_n / 4;
-        q.strideA = g.strideA == 0 ? 0 : kModuli * q.planeA;
-        q.strideB = g.strideB == 0 ? 0 : kModuli * q.planeB;
+        q.strideA = g.strideA == 0 ? 0 : kPlanes * q.planeA;
+        q.strideB = g.strideB == 0 ? 0 : kPlanes * q.planeB;
         q.strideR = kModuli * q.planeR;
+        q.flags = flags;
+        q.strideF = int64_t(q.tiles.count) * kFlags;
+        q.m = mo; q.n = no;
+        q.na = na + r0; q.nb = nrm_b + c0;
+        q.na_stride = g.strideA == 0 ? 0 : p.rm_p;
+        q.nb_stride = g.strideB == 0 ? 0 : p.rn_p;
         const unsigned tiles = unsigned(q.tiles.count);
-        const dim3 grid(tiles, kModuli, unsigned(nb));
+        const dim3 grid(tiles, kPlanes, unsigned(nb));
+        if (!clear) fill(stream, reinterpret_cast<double*>(flags), nb * q.strideF / 2, 0.0);
+        clear = false;
         if (p.tile_n == 128)
           residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
         else
@@ -650,17 +760,24 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
         o.tiles = q.tiles;
         o.m = mo; o.n = no; o.K = g.k;
         o.ea = ea + r0; o.eb = eb + c0;
-        o.ea_stride = g.strideA == 0 ? 0 : p.rm_p;
-        o.eb_stride = g.strideB == 0 ? 0 : p.rn_p;
+        o.ea_stride = q.na_stride;
+        o.eb_stride = q.nb_stride;
         o.alpha = g.alpha; o.beta = g.beta;
         o.C = g.C + b0 * g.strideC + m0 + r0 + (n0 + c0) * g.ldc;
         o.ldc = g.ldc; o.strideC = g.strideC;
         o.vec_rows = mo % 4 == 0 && g.ldc % 2 == 0 && (g.batch == 1 || g.strideC % 2 == 0) &&
                      reinterpret_cast<uintptr_t>(o.C) % 16 == 0;
-        o.A = A + (a_kcontig ? r0 * g.lda : r0); o.lda = g.lda; o.strideA = g.strideA; o.a_kcontig = a_kcontig ? 1 : 0;
-        o.B = B + (b_kcontig ? c0 * g.ldb : c0); o.ldb = g.ldb; o.strideB = g.strideB; o.b_kcontig = b_kcontig ? 1 : 0;
+        o.flags = flags;
+        o.strideF = q.strideF;
         residue_reconstruct_kernel<<<dim3(tiles * unsigned(kBlocksM * p.tile_n / 64), unsigned(nb)), 256, 0, stream>>>(o);
         ETG_LAUNCH("residue_reconstruct");
+        Gemm f = g;
+        f.m = mo; f.n = no;
+        f.A = A + (a_kcontig ? r0 * g.lda : r0);
+        f.B = B + (b_kcontig ? c0 * g.ldb : c0);
+        f.C = o.C;
+        f.batch = nb;
+        gemm_flagged_blocks(stream, f, q.tiles, flags, q.strideF);
       }
     }
   };

@@ -4,19 +4,19 @@
 // A row a of op(A) and a column b of op(B) are scaled by powers of two and
 // rounded to integers, a' = rint(2^ea a), b' = rint(2^eb b), with ||a'||_2 and
 // ||b'||_2 at most 2^kNormBits.  By Cauchy-Schwarz |a'.b'| < M / 2 for
-// M = m_0 m_1 ... m_14, the product of 15 pairwise coprime moduli of at most 8
+// M = m_0 m_1 ... m_15, the product of 16 pairwise coprime moduli of at most 8
 // bits, so the integer a'.b' is determined by its residues, and each residue
 // is an int8 product with int32 accumulation, without any rounding
 // (Chinese remainder theorem; the scheme is Ozaki, Uchino and Imamura's
 // "Ozaki scheme II", 2025).  The only errors are the rounding of the operands
-// to integers, at most 2^-(kNormBits - 1) ||a|| relative to a row's norm per
-// element, and one final rounding to double.
+// to integers, at most 2^-kNormBits ||a|| per element, and one final rounding to
+// double.
 //
-// An FP64 sum of k products rounds every partial sum: for terms of random sign
-// its error is about 2^-56 to 2^-55 of ||a|| ||b||, whatever k.  Rounding the
-// operands here costs about 2^-59 of ||a|| ||b|| (0.4 / 2^57.5), so 15 moduli
-// are about ten times closer to the exact product than the FP64 kernels;
-// 14 (2^-55) would not be.
+// So the error is fixed in the norm, 0.41 2^-kNormBits ||a|| ||b|| rms for norms of
+// 2^kNormBits (two to four times that for smaller ones), while an FP64 sum of terms of
+// random sign has about 0.4 2^-53 of sum |a_k b_k|.  Rows and columns whose large elements
+// meet are far more exact than in FP64 (normal ones 15 times); where large elements meet
+// small ones the FP64 sum would be, and such outputs go to it: see the guard below.
 #pragma once
 
 #include <cmath>
@@ -33,9 +33,9 @@
 namespace etg {
 namespace residue {
 
-constexpr int kModuli = 15;
-constexpr int kMod[kModuli] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197};
-constexpr int kNormBits = 58;                     // 2 kNormBits < log2(M / 2) = 116.78
+constexpr int kModuli = 16;
+constexpr int kMod[kModuli] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227, 223, 217, 211, 199, 197, 193};
+constexpr int kNormBits = 62;                     // 2 kNormBits < log2(M / 2) = 124.37
 // |residue| <= 128 on both sides: the int32 sums hold this many terms
 constexpr int64_t kMaxDepth = (int64_t(1) << 17) - 1;
 constexpr int kNotFinite = INT32_MIN;             // exponent of a row with an infinity or NaN
@@ -64,9 +64,9 @@ constexpr int cofactor_inverse(int i) {
 }
 
 // X = sum_i r_i inv_i (M / m_i)  (mod M), so X / M = sum_i r_i f_i (mod 1) with
-// f_i = inv_i / m_i.  f_i = (kHi + kLo 2^-40) 2^-40 to 2^-81: sums of 15 terms
-// |r_i| <= 128 of either part are exact in FP64, and the 2^-73 M that is left
-// out is below 2^-12 of the operands' rounding.
+// f_i = inv_i / m_i.  f_i = (kHi + kLo 2^-40) 2^-40 to 2^-81: sums of 16 terms
+// |r_i| <= 128 of either part are exact in FP64, and the 2^-70 M at most that is left
+// out (2^-74 rms) is below 2^-5 of the operands' rounding.
 constexpr uint64_t fraction80(int i, bool high) {
   const unsigned __int128 num = (unsigned __int128)(unsigned(cofactor_inverse(i))) << 81;
   const unsigned __int128 f = (num / unsigned(kMod[i]) + 1) >> 1;   // rounded to 2^-80
@@ -177,6 +177,45 @@ ETG_HD inline uint32_t residue_byte_of_sum(int32_t s, double m, double inv) {
   uint64_t bits;
   __builtin_memcpy(&bits, &r, sizeof(bits));
   return uint32_t(bits);
+}
+
+// The guard.  The rounding of the operands has an rms error of 0.41 2^kNormBits in a'.b'
+// (1/2 / sqrt(3) per element, norms up to 2^kNormBits) whatever the sum, while an FP64
+// sum's error goes with sum |a_k b_k|.  Where large elements of the row meet small ones of
+// the column that sum is far below ||a|| ||b||, and digits that FP64 would keep are lost.
+// So a product also forms Q = sum qa qb of the magnitudes q = |a'| 2^-47, rounded to 8-bit
+// floats (5 exponent and 2 fraction bits, 2^30 below the row's norm; at most a ninth up):
+// Q is at most 1.24 times sum |a'_k b'_k| 2^-94.  With the rows' norms na and nb in units
+// of 2^kNormBits, an output with Q below kThreshold max(na, nb) is formed in FP64; elsewhere
+// sum |a'_k b'_k| is at least max(na, nb) 2^(kNormBits + kGuardBits), and the rms error at
+// most 0.41 2^-kGuardBits of sum |a_k b_k|, about what an FP64 sum of terms of random sign has.
+// With 15 moduli (58 bits) that limit is reached in most 128 x 128 blocks of a molecule's
+// products.
+constexpr int kGuardBits = 52;                    // 0.82 2^-53
+constexpr float kThreshold = 1.24f * float(uint64_t(1) << (kNormBits + kGuardBits - 94));
+static_assert(kNormBits <= 62, "the largest magnitude is an 8-bit float");
+constexpr float kZeroNorm = -1.0f;                // of a row of zeros: nothing to lose
+
+// Norm of the scaled row in units of 2^kNormBits (1 where it is only bounded; infinite for
+// a row that is not finite).
+ETG_HD inline float scaled_norm(double sumsq, uint64_t max_bits) {
+  if (max_bits == 0) return kZeroNorm;
+  if (max_bits >= 0x7ff0000000000000ull) return float(HUGE_VAL);
+  if (!(sumsq > 1e-270 && sumsq < 1e290)) return 1.0f;
+  int x;
+  const double f = frexp(sumsq, &x);
+  return float(sqrt((x & 1) ? 0.5 * f : f)) * (1.0f + 0x1p-20f);
+}
+
+// From the high half of the integer, floor(a' / 2^32) + 2^31: the top of the FP32 number
+// |a'| 2^-32, its exponent from 2^0 on.
+ETG_HD inline uint32_t magnitude_byte(uint32_t hi) {
+  const int32_t h = int32_t(hi ^ 0x80000000u);
+  const float f = float(uint32_t(h ^ (h >> 31)));
+  uint32_t bits;
+  __builtin_memcpy(&bits, &f, sizeof(bits));
+  const int32_t q = int32_t((bits + 0x100000u) >> 21) - (127 << 2);
+  return uint32_t(q > 0 ? q : 0);
 }
 
 // a'.b' 2^-(ea + eb) from the sums hi = sum_i r_i kHi_i and lo = sum_i r_i kLo_i.
