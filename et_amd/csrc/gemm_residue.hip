@@ -15,6 +15,7 @@
 //   5. the flagged blocks on the FP64 kernel
 // on panels of A and B whose packs fit a bounded workspace.
 #include <algorithm>
+#include <cmath>
 #include <string>
 #include <type_traits>
 
@@ -544,6 +545,11 @@ struct Panels {
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 int64_t round_up(int64_t x, int64_t to) { return ceil_div(x, to) * to; }
 
+// op(A)^T and op(B) are one array.
+bool one_operand(const Gemm& g) {
+  return g.A == g.B && g.ta != g.tb && g.lda == g.ldb && g.m == g.n && g.batch == 1;
+}
+
 // Buffer sizes of the panels; what the packs leave is the room for the residues,
 // which go by columns (at least 512, or all), then rows.  False when that does not fit.
 bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
@@ -603,7 +609,7 @@ bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
   p.rows_m = g.m;
   p.rows_n = g.n;
   p.batch = g.batch;
-  p.same = g.A == g.B && g.ta != g.tb && g.lda == g.ldb && g.m == g.n && g.batch == 1;
+  p.same = one_operand(g);
   int64_t groups = 1, pm = 1, pn = 1;
   while (!size_panels(g, capacity, p)) {
     if (p.same) {
@@ -647,24 +653,27 @@ void pack_operand(hipStream_t s, const double* X, int64_t ld, int64_t strideX, b
 
 }  // namespace
 
-// Estimated seconds of the int8 path (2400 TOP/s over whole tiles, 7.4 ps per
-// operand element and 5.1 ps per output of packs and reconstruction, 45 us of
-// launches) against those of the FP64 kernels (`fp64_seconds`, at least the 35
-// TFLOP/s that products of a few hundred rows reach).  Measured per product, FP64
-// and int8: 1024^3 56 and 75 us, 1280^3 107 and 99, 1520^3 175 and 133, 2048^3
-// 311 and 193, 4096^3 2200 and 1069 us; m = n = 4096 with k = 279 / 600 / 1270:
-// 196 and 233, 364 and 295, 716 and 443 us; 210 x 2926 x 2926 100 and 132 us.
-// The estimate follows these to 20 % on either side of the crossing.
+// Estimated microseconds of the int8 path against those of the FP64 kernels
+// (`fp64_seconds`, at least the 50 TFLOP/s that products of a few hundred rows reach).
+// Products: rounds of 512 or 256 workgroups, each 0.69 or 0.74 us per step of 64 k and 2.1
+// to begin and end; the last of a few rounds counts half as a whole one (its workgroups
+// run faster alone).  Packs 7.3 ps per operand element with the norms, an operand shared
+// by both sides once; 7.6 ps per output; 35 us of launches.  Fitted to 260 products of
+// m, n = 128 .. 19000, k = 128 .. 32768 (0.6 .. 400 GFLOP): 9 % rms.  Of these the rule sends
+// none to the slower path by more than 5 %, and leaves seven that would gain as much on the
+// FP64 kernels; without the rounds and with the constants of 15 moduli it sent twelve
+// (5559 x 3230 x 313 1.31 times slower, 424 x 2101 x 26993 912 against 1050 us).
 bool residue_pays(const Gemm& g, double fp64_seconds) {
   if (g.k > residue::kMaxDepth || std::min(g.m, g.n) < 128 || g.k < 128) return false;
   const double b = double(g.batch), m = double(g.m), n = double(g.n), k = double(g.k);
-  const int64_t tile_n = g.k <= kShortDepth ? 128 : 256;
-  const double mp = double(ceil_div(g.m, kTileM) * kTileM), np = double(ceil_div(g.n, tile_n) * tile_n);
-  const double kp = double(ceil_div(g.k, kDepth) * kDepth);
-  const double products = 2.0 * kModuli * mp * np * kp * b / 2400e12;
-  const double packs = 7.4e-12 * ((g.strideA == 0 ? 1.0 : b) * m * k + (g.strideB == 0 ? 1.0 : b) * n * k);
-  const double output = 5.1e-12 * m * n * b;
-  return products + packs + output + 45e-6 < 0.95 * std::min(fp64_seconds, 2.0 * m * n * k * b / 35e12);
+  const bool small = g.k <= kShortDepth;
+  const double tiles = double(ceil_div(g.m, kTileM)) * double(ceil_div(g.n, small ? 128 : 256)) * b;
+  const double q = tiles * kPlanes / (small ? 512.0 : 256.0);
+  const double rounds = q > 8.0 ? q : 0.5 * std::ceil(q) + 0.5 * std::max(1.0, q);
+  const double products = rounds * ((small ? 0.69 : 0.74) * double(ceil_div(g.k, kDepth)) + 2.1);
+  const double elements = (g.strideA == 0 ? 1.0 : b) * m * k + (one_operand(g) ? 0.0 : (g.strideB == 0 ? 1.0 : b) * n * k);
+  const double us = 35.0 + products + 7.3e-6 * elements + 7.6e-6 * m * n * b;
+  return us < 0.95e6 * std::min(fp64_seconds, 2.0 * m * n * k * b / 50e12);
 }
 
 bool residue_fits(const Gemm& g, const GemmWorkspace* ws) {
