@@ -157,17 +157,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_mfma16(Params p, F f) {
   int tile_m, tile_n;
   int64_t m0, n0;
   if constexpr (std::is_same_v<F, FlaggedBlocks>) {
-    static_assert(BM == BN && (BM == 128 || BM == 64), "a tile in one flagged block");
-    constexpr int kRows = kTileM / BM;
-    const int per_tile = kRows * (f.tiles.tile_n / BN);
+    static_assert(BM == 64 && BN == 64, "a flagged block");
+    const int per_tile = 4 * (f.tiles.tile_n / 64);
     // (in dispatch order, round-robin over the XCDs: flagged blocks lie together, and with
     // a range of tiles per XCD one of them had nearly all the work)
     const int slot = int(blockIdx.x) / per_tile, part = int(blockIdx.x) % per_tile;
     if (!tile_of(f.tiles, slot, tile_m, tile_n)) return;
-    const int mi = part % kRows * BM, ni = part / kRows * BN;
-    if (f.flags[bz * f.stride + int64_t(slot) * kFlaggedBlocks + mi / 128 + ni / 128 * 2] == 0) return;
-    m0 = int64_t(tile_m) * kTileM + mi;
-    n0 = int64_t(tile_n) * f.tiles.tile_n + ni;
+    if ((f.flags[bz * f.stride + slot] >> part & 1) == 0) return;
+    m0 = int64_t(tile_m) * kTileM + part % 4 * 64;
+    n0 = int64_t(tile_n) * f.tiles.tile_n + part / 4 * 64;
     if (m0 >= p.m || n0 >= p.n) return;
   } else {
     map_tile(blockIdx.x, p.tiles_m, p.tiles_n, tile_m, tile_n);
@@ -1090,28 +1088,26 @@ int64_t gemm_tuned_shapes() {
 }
 
 namespace {
-template <int BM, bool WIDE>
+template <bool WIDE>
 void launch_flagged(hipStream_t stream, const Gemm& g, const Params& p, const FlaggedBlocks& f) {
-  const int64_t per_tile = int64_t(kTileM / BM) * (f.tiles.tile_n / BM);
-  const dim3 grid(unsigned(f.tiles.count * per_tile), 1, unsigned(g.batch));
+  const dim3 grid(unsigned(f.tiles.count * 4 * (f.tiles.tile_n / 64)), 1, unsigned(g.batch));
   using F = FlaggedBlocks;
-  if (!g.ta && !g.tb) gemm_mfma16<double, false, false, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
-  else if (!g.ta && g.tb) gemm_mfma16<double, false, true, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
-  else if (g.ta && !g.tb) gemm_mfma16<double, true, false, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
-  else gemm_mfma16<double, true, true, BM, BM, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  if (!g.ta && !g.tb) gemm_mfma16<double, false, false, 64, 64, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else if (!g.ta && g.tb) gemm_mfma16<double, false, true, 64, 64, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else if (g.ta && !g.tb) gemm_mfma16<double, true, false, 64, 64, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
+  else gemm_mfma16<double, true, true, 64, 64, 16, WIDE, F><<<grid, kThreads, 0, stream>>>(p, f);
   ETG_LAUNCH("gemm_mfma16");
 }
 }  // namespace
 
+// Blocks of 64 x 64: a few flagged ones of 128 x 128 take as long as one workgroup needs
+// for its k (1.8 ms at 6080), and more of the output lies in flagged blocks of that size.
 void gemm_flagged_blocks(hipStream_t stream, const Gemm& g, const TileMap& tiles, const int* flags, int64_t flag_stride) {
   int splits = 1;
   const Params p = split_params(g, nullptr, 1, &splits);
   const FlaggedBlocks f{tiles, flags, flag_stride};
-  // 64 x 64 where 128 x 128 would leave CUs idle with all blocks flagged
-  const bool small = int64_t(tiles.count) * (kTileM / 128) * (tiles.tile_n / 128) * g.batch < 512;
-  const bool wide = std::max(g.lda, g.ldb) >= (int64_t(1) << 21);
-  if (small) wide ? launch_flagged<64, true>(stream, g, p, f) : launch_flagged<64, false>(stream, g, p, f);
-  else wide ? launch_flagged<128, true>(stream, g, p, f) : launch_flagged<128, false>(stream, g, p, f);
+  if (std::max(g.lda, g.ldb) >= (int64_t(1) << 21)) launch_flagged<true>(stream, g, p, f);
+  else launch_flagged<false>(stream, g, p, f);
 }
 
 bool runs_as_residues(const Gemm& g, Prec prec, const GemmWorkspace* ws) {

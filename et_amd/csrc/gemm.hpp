@@ -138,10 +138,10 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
 // Whether gemm() would run g so (the caller then need not cut g.lower's triangle itself).
 bool runs_as_residues(const Gemm& g, Prec prec, const GemmWorkspace* ws);
 
-// C = alpha op(A) op(B) + beta C on the FP64 kernel, in the 128 x 128 blocks that are
-// flagged: kFlaggedBlocks per tile of the map (rows first), batch entries at flag_stride.
+// C = alpha op(A) op(B) + beta C on the FP64 kernel, in the 64 x 64 blocks that are
+// flagged: a bit each (row block + 4 column block) of one word per tile of the map, batch
+// entries at flag_stride.
 struct TileMap;
-constexpr int kFlaggedBlocks = 4;
 void gemm_flagged_blocks(hipStream_t stream, const Gemm& g, const TileMap& tiles, const int* flags, int64_t flag_stride);
 
 // bf16 values of the split-bf16 pack of a rows x k operand (both splits, padded

@@ -9,7 +9,7 @@
 //   2. residue packs: 17 bytes per element, in the order the matrix cores read
 //      (a byte per modulus, and the magnitude)
 //   3. 16 int8 products, each sum reduced to one byte per output, and before
-//      them the product of the magnitudes, which flags the 128 x 128 blocks that
+//      them the product of the magnitudes, which flags the 64 x 64 blocks that
 //      need the FP64 kernel
 //   4. reconstruction of C from its 16 bytes     (writes C once)
 //   5. the flagged blocks on the FP64 kernel
@@ -265,7 +265,6 @@ constexpr int64_t kShortDepth = 3200;
 
 constexpr int kWaveM = 8, kWaveN = 4;         // 16 x 16 blocks of a wave
 constexpr int kBlocksM = kTileM / 16;
-constexpr int kFlags = kFlaggedBlocks;        // 128 x 128 blocks of a tile (two of them in 256 x 128)
 
 struct Params {
   const u4 *A, *B;                 // packs (planes of the first modulus)
@@ -274,8 +273,8 @@ struct Params {
   int64_t planeA, planeB, planeR;  // from one modulus to the next (u4, u4, u32 units)
   int64_t strideA, strideB, strideR;   // from one batch entry to the next
   TileMap tiles;
-  // per tile its 128 x 128 blocks (kFlags, row by row) that are left to the FP64 kernel:
-  // zero before the launch, set by the product of the magnitudes
+  // per tile the 64 x 64 blocks that are left to the FP64 kernel (bit: row block + 4 column
+  // block): zero before the launch, set by the product of the magnitudes
   int* flags;
   int64_t strideF;
   // of the guard product
@@ -319,13 +318,10 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
   const bool guard = blockIdx.y == 0;
   const int z = guard ? kModuli : int(blockIdx.y) - 1;
   const int64_t bz = blockIdx.z;
-  int* flags = p.flags + bz * p.strideF + int64_t(slot) * kFlags;
-  if (!guard) {
-    int all = 1;
-#pragma unroll
-    for (int q = 0; q < WN; ++q) all &= __hip_atomic_load(&flags[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__builtin_amdgcn_readfirstlane(all)) return;
-  }
+  int* flags = p.flags + bz * p.strideF + slot;
+  constexpr int kAllBlocks = (1 << (4 * WN)) - 1;
+  if (!guard && __builtin_amdgcn_readfirstlane(__hip_atomic_load(flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == kAllBlocks)
+    return;
   const u4* sa = p.A + bz * p.strideA + z * p.planeA + int64_t(tile_m) * kBlocksM * p.KS * 64;
   const u4* sb = p.B + bz * p.strideB + z * p.planeB + int64_t(tile_n) * kBlocksN * p.KS * 64;
   const __amdgpu_buffer_rsrc_t ra =
@@ -411,16 +407,13 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
     __syncthreads();
     const int64_t row0 = int64_t(tile_m) * kTileM + wm * (kWaveM * 16) + 4 * (lane >> 4);
     const int64_t col0 = (int64_t(tile_n) * kBlocksN + wn * kWaveN) * 16 + (lane & 15);
-    if (tid < kFlags)                          // blocks past the edge have nothing to do
-      found[tid] = int64_t(tile_m) * kTileM + (tid & 1) * 128 >= p.m || int64_t(tile_n) * (kBlocksN * 16) + (tid >> 1) * 128 >= p.n;
-    __syncthreads();
     // (norms of rows past the edge: inside the padded array, not used)
     const f4* na = reinterpret_cast<const f4*>(p.na + bz * p.na_stride + row0);
     const float* nb = p.nb + bz * p.nb_stride + col0;
     f4 nr[kWaveM];
 #pragma unroll
     for (int i = 0; i < kWaveM; ++i) nr[i] = na[i * 4];
-    bool lost = false;
+    bool lost[2] = {false, false};             // the wave's two blocks
 #pragma unroll
     for (int j = 0; j < kWaveN; ++j) {
       const float nc = col0 + j * 16 < p.n ? nb[j * 16] : residue::kZeroNorm;
@@ -429,13 +422,25 @@ __global__ __launch_bounds__(128 * WN, WN == 2 ? 2 : 1) void residue_product_ker
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int bits = acc[i][j][r];       // (bit_cast of the element itself takes the first one)
-          lost |= row0 + i * 16 + r < p.m && nr[i][r] > 0.0f && nc > 0.0f &&
-                  !(__builtin_bit_cast(float, bits) >= residue::kThreshold * fmaxf(nr[i][r], nc));
+          lost[i / 4] |= row0 + i * 16 + r < p.m && nr[i][r] > 0.0f && nc > 0.0f &&
+                         !(__builtin_bit_cast(float, bits) >= residue::kThreshold * fmaxf(nr[i][r], nc));
         }
     }
-    if (__ballot(lost) != 0 && lane == 0) found[wm + 2 * (wn / 2)] = 1;
+    static_assert(kWaveM == 8 && kWaveN == 4, "two 64 x 64 blocks of a wave");
+    int mine = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {              // blocks past the edge have nothing to do
+      const bool past = int64_t(tile_m) * kTileM + (wm * 2 + h) * 64 >= p.m || (int64_t(tile_n) * WN + wn) * 64 >= p.n;
+      if (past || __ballot(lost[h]) != 0) mine |= 1 << (wm * 2 + h + 4 * wn);
+    }
+    if (lane == 0) found[wave] = mine;
     __syncthreads();
-    if (tid < WN) __hip_atomic_store(&flags[tid], found[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+      int all = 0;
+#pragma unroll
+      for (int w = 0; w < 2 * WN; ++w) all |= found[w];
+      __hip_atomic_store(flags, all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     return;
   }
   const double m = kC.md[z], inv = kC.invd[z];
@@ -485,7 +490,7 @@ __global__ __launch_bounds__(256) void residue_reconstruct_kernel(Output p) {
   int tile_m, tile_n;
   if (!tile_of(p.tiles, slot, tile_m, tile_n)) return;
   const int64_t bz = blockIdx.y;
-  if (p.flags[bz * p.strideF + int64_t(slot) * kFlags + (blk % kBlocksM) / 8 + blk / kBlocksM / 8 * 2]) return;
+  if (p.flags[bz * p.strideF + slot] >> ((blk % kBlocksM) / 4 + blk / kBlocksM / 4 * 4) & 1) return;
   const int64_t row = int64_t(tile_m) * kTileM + (blk % kBlocksM) * 16 + 4 * (lane >> 4);
   const int64_t col = (int64_t(tile_n) * blocks_n + blk / kBlocksM) * 16 + (lane & 15);
   if (row >= p.m || col >= p.n) return;
@@ -568,7 +573,7 @@ bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
   const int64_t room = int64_t(double(capacity - p.total()) / (double(p.batch) * (kModuli + 0.001))) - 512;
   auto residues_of = [&](int64_t outputs) {
     p.bytes_r = align256(size_t(p.batch * kModuli) * size_t(outputs));
-    p.bytes_f = align256(sizeof(int) * kFlags * size_t(p.batch) * size_t(outputs / (int64_t(kTileM) * p.tile_n)));
+    p.bytes_f = align256(sizeof(int) * size_t(p.batch) * size_t(outputs / (int64_t(kTileM) * p.tile_n)));
     return p.total() <= capacity;
   };
   p.out_m = p.rm_p;
@@ -748,14 +753,14 @@ bool gemm_residue(hipStream_t stream, const Gemm& g, GemmWorkspace* ws, bool may
         q.strideB = g.strideB == 0 ? 0 : kPlanes * q.planeB;
         q.strideR = kModuli * q.planeR;
         q.flags = flags;
-        q.strideF = int64_t(q.tiles.count) * kFlags;
+        q.strideF = q.tiles.count;
         q.m = mo; q.n = no;
         q.na = na + r0; q.nb = nrm_b + c0;
         q.na_stride = g.strideA == 0 ? 0 : p.rm_p;
         q.nb_stride = g.strideB == 0 ? 0 : p.rn_p;
         const unsigned tiles = unsigned(q.tiles.count);
         const dim3 grid(tiles, kPlanes, unsigned(nb));
-        if (!clear) fill(stream, reinterpret_cast<double*>(flags), nb * q.strideF / 2, 0.0);
+        if (!clear) fill(stream, reinterpret_cast<double*>(flags), ceil_div(nb * q.strideF, 2), 0.0);
         clear = false;
         if (p.tile_n == 128)
           residue_product_kernel<2, 3><<<grid, 256, 0, stream>>>(q);
