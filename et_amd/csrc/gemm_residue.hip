@@ -665,7 +665,7 @@ void pack_operand(hipStream_t s, const double* X, int64_t ld, int64_t strideX, b
 // run faster alone).  Packs 7.3 ps per operand element with the norms, an operand shared
 // by both sides once; 7.6 ps per output; 35 us of launches.  Fitted to 260 products of
 // m, n = 128 .. 19000, k = 128 .. 32768 (0.6 .. 400 GFLOP): 9 % rms.  Of these the rule sends
-// none to the slower path by more than 5 %, and leaves seven that would gain as much on the
+// none to the slower path by more than 5 %, and leaves two that would gain as much on the
 // FP64 kernels; without the rounds and with the constants of 15 moduli it sent twelve
 // (5559 x 3230 x 313 1.31 times slower, 424 x 2101 x 26993 912 against 1050 us).
 bool residue_pays(const Gemm& g, double fp64_seconds) {
@@ -678,7 +678,7 @@ bool residue_pays(const Gemm& g, double fp64_seconds) {
   const double products = rounds * ((small ? 0.69 : 0.74) * double(ceil_div(g.k, kDepth)) + 2.1);
   const double elements = (g.strideA == 0 ? 1.0 : b) * m * k + (one_operand(g) ? 0.0 : (g.strideB == 0 ? 1.0 : b) * n * k);
   const double us = 35.0 + products + 7.3e-6 * elements + 7.6e-6 * m * n * b;
-  return us < 0.95e6 * std::min(fp64_seconds, 2.0 * m * n * k * b / 50e12);
+  return us < 1e6 * std::min(fp64_seconds, 2.0 * m * n * k * b / 50e12);
 }
 
 bool residue_fits(const Gemm& g, const GemmWorkspace* ws) {
