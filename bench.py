@@ -39,8 +39,8 @@ from et_amd import synthetic as syn  # noqa: E402
 METRIC = 'CCSD omega evals/s & time-to-solution, mixed vs FP64 GPU at |ΔE|≤1e-8 Eh'
 # dense matrix-core peaks; split-bf16 counts its three bf16 products per term
 PEAKS = {'fp64': 78.6e12, 'fp32': 157.3e12, 'bf16x3': 2.5e15 / 3}
-# FP64 products that run as 15 exact int8 products (5 POP/s dense)
-RESIDUE_PEAK = 5.0e15 / 15
+# FP64 products that run as 16 exact int8 products and one of 8-bit floats (5 POP/s dense)
+RESIDUE_PEAK = 5.0e15 / 17
 
 
 def peak_of(kernel, precision):
@@ -54,12 +54,13 @@ CPU_SINGLE_THREAD = dict(n_o=40, n_v=152, n_J=2541, seed=0)
 HARTREE_TO_EV = 27.21138602          # CODATA 2014, the factor eT prints
 _PN = {ccsd.BF16X3: 'bf16x3', ccsd.FP32: 'fp32', ccsd.FP64: 'fp64'}
 WORKLOAD_NAME = 'omega_o48_v400_J1600_seed0'
-# HBM bytes per launch of the residual's dominant kernel on this workload: rocprofv3
-# --pmc FETCH_SIZE and --pmc WRITE_SIZE (KiB per dispatch, averaged over the kernel's
-# launches in the last of three residual evaluations), each scaled by what the counter reads for a
-# plain 1 GiB device copy (bench.py --copy-calibration: FETCH_SIZE x 2.000,
-# WRITE_SIZE x 1.000).  Summary and commands: profiles/omega_fp64_o48_v400_J1600_hbm_traffic.md
-MEASURED_TRAFFIC = {(WORKLOAD_NAME, 'gemm_mfma16<f64,NN,128x128>'): 1.067e11}
+# HBM bytes per ledger launch of the residual's dominant product on this workload, with its
+# packs and reconstruction: rocprofv3 --pmc FETCH_SIZE and --pmc WRITE_SIZE (KiB per dispatch,
+# summed over these kernels in the last of three residual evaluations, over 33 launches), each
+# scaled by what the counter reads for a plain 1 GiB device copy (bench.py --copy-calibration:
+# FETCH_SIZE x 2.000, WRITE_SIZE x 1.000).  Summary and commands:
+# profiles/omega_fp64_o48_v400_J1600_hbm_traffic.md
+MEASURED_TRAFFIC = {(WORKLOAD_NAME, 'gemm_residue<256x256>'): 1.186e11}
 
 
 def log(*a):

@@ -4,7 +4,8 @@
 // The FP64 matrix cores reach 78 TFLOP/s on this chip and the FP64 kernels 62
 // of them; the int8 products here run at 2.4-2.6 POP/s (the kernel's 2548 TOP/s
 // on random bytes; 3491 on zeros, where the power limit does not bind), so 17 of them
-// per FP64 product are worth up to 150 TFLOP/s.  A product runs as
+// per FP64 product are worth up to 150 TFLOP/s (with the product of 8-bit floats, whose
+// instruction has half the k, 2.2 POP/s and 130 in a residual).  A product runs as
 //   1. row norms of op(A) and op(B)^T            (reads each operand once)
 //   2. residue packs: 17 bytes per element, in the order the matrix cores read
 //      (a byte per modulus, and the magnitude)
@@ -604,9 +605,9 @@ bool size_panels(const Gemm& g, size_t capacity, Panels& p) {
 
 // The whole product where its packs fit the capacity, else equal groups of the
 // batch, else (one entry at a time) equal panels of rows, the longer panel split
-// first.  A panel more of one operand packs the other once more: 7.4 ps per element
-// against the 12.5 fs of products that each of its elements has with every row
-// of the panel, so panels of 2560 rows cost a quarter, of 6912 rows a twelfth.
+// first.  A panel more of one operand packs the other once more: 7.3 ps per element
+// against the 13.3 fs of products that each of its elements has with every row
+// of the panel, so panels of 2560 rows cost a fifth, of 6912 rows a twelfth.
 bool plan_panels(const Gemm& g, size_t capacity, Panels& p) {
   p.KS = ceil_div(g.k, kDepth);
   p.tile_n = g.k <= kShortDepth ? 128 : 256;
